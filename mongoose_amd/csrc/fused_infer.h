@@ -9,6 +9,7 @@
 
 #include <cstdint>
 #include <string>
+#include <mutex>
 #include <vector>
 
 namespace mg {
@@ -101,10 +102,17 @@ public:
         if (mode == 3 || mode == 4) flowBroken = false;      // asked for again by name: a wait that ran out earlier no longer bars it
         execMode = mode;
         if (mode != 0) q4ActQuant = false;      // only the op-by-op loop has the integer matvecs
-        if (mode != 3 && mode != 4) releaseFlow();
     }
     void flowRegeometry();
-    void releaseFlow();
+    // Persistent launches of several contexts on one device take turns (fused_infer.hip).
+    int takeFlowTurn();                     // under flowTurnMutex(), before the launch
+    std::mutex& flowTurnMutex() const;
+    int launchFlowGraph(hipGraphExec_t ex);
+    int launchTokenGraph(hipGraphExec_t ex);
+    void leaveFlowTurns();
+    int flowDevice = 0;
+    hipEvent_t flowTurnEvent = nullptr;     // created with the launch's buffers
+    bool capturing = false;                 // a graph capture of this context is under way (holds flowTurnMutex())
 
     // shape
     int dim, kvDim, headDim, nHeads, nKVHeads, ffnDim, vocabSize, nLayers, maxSeq;
@@ -170,6 +178,7 @@ public:
         unsigned generation = 0;
         hipGraph_t g = nullptr;
         hipGraphExec_t ex = nullptr;
+        bool flow = false;         // captured with the persistent launch
     };
     int LayerGraphCapture(LayerGraph& lg);                 // (re)captures lg.l0 .. lg.l1 on the context's stream
     int LayerGraphLaunch(LayerGraph& lg, int pos);         // sets the device position, replays; asynchronous
