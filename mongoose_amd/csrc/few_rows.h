@@ -1,0 +1,60 @@
+// few_rows.h -- launchers of the few-row prefill kernels (few_rows.hip): a handful of positions through the layers.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace mg {
+
+// One launch over a tile of 16 or 32 weight rows x 16, 32 or 64 activation rows a workgroup; what follows the product is
+// the epilogue of the mode.
+enum FewMode {
+    FEW_STORE = 0,   // Y (+)= v * scale + bias
+    FEW_RESID = 1,   // Y += v * scale + bias; optionally the next projection's split of Y * nextGain and the rows' sums of squares
+    FEW_SWIGLU = 2,  // seg0 = gate, seg1 = up: silu(g) * u as the split of the down projection's input
+    FEW_QKV = 3,     // seg0 = q, seg1 = k, seg2 = v: bias, RoPE, q rows to seg0.Y, K / V rows into the caches at pos0 + row
+};
+struct FewSeg { const signed char* W; const float* scales; const float* bias; float* Y; int N; };
+struct FewParams {
+    FewSeg seg[3];
+    const unsigned short* Ahi;       // split activations in the order few_rows.hip describes (for this launch's weight format)
+    const unsigned short* Alo;
+    int T, K;
+    int q4;                          // weights: 0 = int8 rows with scales, 1 = Q4_0 in the split layout
+    int accumulate;                  // FEW_STORE: Y += instead of Y =
+    // the rows' RMS factor, applied to the finished sums: sumSq holds sumParts partial sums of squares of every row,
+    // sumStride floats apart (NULL: no factor)
+    const float* sumSq;
+    int sumParts, sumStride;
+    float eps;
+    // FEW_RESID (optional), FEW_SWIGLU
+    const float* nextGain;
+    unsigned short* nextHi;
+    unsigned short* nextLo;
+    int nextQ4;                      // weight format of the projection that reads them
+    float* nextSumSq;                // [tiles of the launch][sumStride]; few_rows_sum_parts(N, T, K) of them
+    // FEW_QKV
+    void* Kc;
+    void* Vc;
+    const float* cosTab;
+    const float* sinTab;
+    int pos0, headDim, kvHalf;
+    // filled by the launcher
+    int nTiles;
+};
+int few_rows_sum_parts(int N, int T, int K);
+// K a multiple of 32, W and the planes 16-byte aligned; FEW_QKV: headDim 64 or 128, N multiples of it.
+hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s);
+
+// Rows of the embedding table (kinds as launch_embed_rows) into x, their split times `gain` and their sums of squares
+// (one part).  tokens may be pinned host memory.
+hipError_t launch_embed_split(int kind, const void* table, const float* scales, const int* tokens, float* x, const float* gain,
+                              unsigned short* hi, unsigned short* lo, float* sumSq, int T, int dim, int vocab, int q4, hipStream_t s);
+// Rows of fp32 activations split for a launch over weights of format q4.
+hipError_t launch_few_split(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4, hipStream_t s);
+
+// Causal attention of T query rows (rotated) at positions pos0 .. over the cache rows [0, pos0 + T), all products and sums
+// in fp32; the result goes out as the split the output projection reads.
+hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
+                                int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4,
+                                hipStream_t s);
+
+}  // namespace mg

@@ -1,0 +1,739 @@
+// few_rows.hip -- a layer over a handful of positions (short prompts, further turns of a conversation, small batches of
+// rows through one matrix).
+//
+// Up to some hundred rows a projection is bound by its weight bytes and by launch latency, not by the matrix cores: what
+// counts is that every weight byte is requested once and early, by enough workgroups, and that a layer is few launches.
+// A layer is five here -- norm + q|k|v + RoPE + cache rows, attention, Wo + residual, norm + gate|up + SwiGLU, down +
+// residual -- where the tiled GEMMs of prefill.hip with their K splits need ten (0.5B shape, 37 rows behind 200: 78 us a
+// layer before).
+//
+// Arithmetic is that of prefill.hip: int8 weights (Q4_0: nibble - 8) exact in bf16, activations as two bf16 terms, fp32
+// accumulation on v_mfma_f32_16x16x32_bf16.  The RMS factor is applied to the finished sums: whoever produces a row of
+// the hidden state also leaves its split times the next gain and, per tile, the row's sum of squares.
+#include "kernels.h"
+#include "prefill.h"
+#include "few_rows.h"
+#include "device_util.h"
+
+namespace mg {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+constexpr int FR_WAVES = 8, FR_WG = 64 * FR_WAVES;
+
+// two floats -> two bf16, round to nearest even
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+    const float2_t f = {a, b};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f, bf16x2_t));
+}
+__device__ __forceinline__ unsigned short bf16_one(float a) { return (unsigned short)(bf16_pair(a, 0.f) & 0xffffu); }
+__device__ __forceinline__ float bf16_value(unsigned short h) { return __builtin_bit_cast(float, (unsigned)h << 16); }
+__device__ __forceinline__ unsigned pack_exact(float lo, float hi) {      // small whole numbers: truncation is exact
+    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x07060302u);
+}
+// 8 int8 -> 8 bf16
+__device__ __forceinline__ bf16x8_t frag_i8(int lo, int hi) {
+    uint4 u;
+    u.x = pack_exact((float)(signed char)(lo), (float)(signed char)(lo >> 8));
+    u.y = pack_exact((float)(signed char)(lo >> 16), (float)(lo >> 24));
+    u.z = pack_exact((float)(signed char)(hi), (float)(signed char)(hi >> 8));
+    u.w = pack_exact((float)(signed char)(hi >> 16), (float)(hi >> 24));
+    return __builtin_bit_cast(bf16x8_t, u);
+}
+// the low (sh = 0) or high (sh = 4) nibbles of 8 bytes, minus 8 -> 8 bf16
+__device__ __forceinline__ bf16x8_t frag_nib(int2 w, unsigned sh) {
+    const unsigned a = ((unsigned)w.x >> sh) & 0x0f0f0f0fu, b = ((unsigned)w.y >> sh) & 0x0f0f0f0fu;
+    uint4 u;
+    u.x = pack_exact(cvt_ubyte<0>(a) - 8.0f, cvt_ubyte<1>(a) - 8.0f);
+    u.y = pack_exact(cvt_ubyte<2>(a) - 8.0f, cvt_ubyte<3>(a) - 8.0f);
+    u.z = pack_exact(cvt_ubyte<0>(b) - 8.0f, cvt_ubyte<1>(b) - 8.0f);
+    u.w = pack_exact(cvt_ubyte<2>(b) - 8.0f, cvt_ubyte<3>(b) - 8.0f);
+    return __builtin_bit_cast(bf16x8_t, u);
+}
+// The split planes of these kernels are stored as the MFMA operand is held: per 16 rows and 64 k two steps of 1 KB, in
+// each the lane's 8 values at lane * 16 bytes (lane = 16 q + row % 16), so that an operand is one contiguous load.  (Row
+// by row, a lane per row, every load touches 16 lines per quarter wave: 37 rows through an 896 x 4864 matrix 19.8 us
+// instead of 12.3.)  The k of a step: 16 q + 8 s .. + 7 for int8 weights, whose row then is one 16-byte load a lane, or
+// 32 s + 8 q .. + 7 for Q4_0, where a step has to be one block.
+__device__ __forceinline__ size_t few_index(int t, int k, int K, int q4) {
+    const int kk = k & 63;
+    const int s = q4 ? kk >> 5 : (kk >> 3) & 1, q = q4 ? (kk >> 3) & 3 : kk >> 4;
+    return ((size_t)(t >> 4) * ((K + 63) >> 6) + (k >> 6)) * 1024 + s * 512 + (q * 16 + (t & 15)) * 8 + (k & 7);
+}
+
+// ---------------------------------------------------------------------------
+// Y[T,N] = (Ahi + Alo)[T,K] . W[N,K]^T with the mode's epilogue.  A workgroup = 8 waves that split K: wave w takes the
+// 64-k chunks w, w + 8, ...; a chunk of 16 weight rows is one 16-byte load a lane (Q4_0: two of 8 bytes), a chunk of 16
+// activation rows two of each plane, straight from the blocked planes into MFMA operands -- no operand is wanted by two
+// waves, so nothing goes through LDS before the sums of the eight waves do.  D register sets keep D - 1 chunks of loads
+// in flight a wave.
+//   MT: 16-row blocks of activations, NB: 16-row blocks of weights a workgroup.
+// The k of a chunk an operand's quarter (lane / 16) holds: 16 q .. 16 q + 15 in two steps of 8 (Q8), or 8 q .. 8 q + 7 of
+// each of the two Q4_0 blocks -- any order serves as long as both operands have the same.
+// ---------------------------------------------------------------------------
+//   LOOP = 0: K of at most 16 chunks, two a wave: both are requested at once, no ring.
+template <int MODE, int MT, int NB, int Q4, int LOOP>
+__global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
+    constexpr int D = !LOOP || MT * NB >= 6 || MT == 4 ? 2 : (MT * NB >= 3 ? 3 : 4);
+    constexpr int NCOL = 16 * NB, MROW = 16 * MT, LST = MROW + 4;
+    static_assert(NCOL * (MROW / 4) <= FR_WG, "four results a thread");
+    extern __shared__ __attribute__((aligned(16))) float part[];      // [wave][column][LST]: the waves' sums
+    __shared__ float sumq[FR_WAVES][MROW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fq = lane >> 4;
+    const int numM = (p.T + MROW - 1) / MROW;
+    const int L = blockIdx.x, grp = L / (8 * numM), rem = L % (8 * numM);
+    const int nTile = grp * 8 + (rem & 7), mTile = rem >> 3;          // the row tiles of a weight tile on one XCD
+    if (nTile >= p.nTiles) return;
+    const int m0 = mTile * MROW, K = p.K, T = p.T;
+    const int mRows = min(MROW, T - m0);
+
+    // the tile's matrix, its first row there, and the distance of its two 16-row blocks
+    int sgi = 0, r0 = nTile * NCOL, blk = 16;
+    int head0 = 0, jj0 = 0;                                           // FEW_QKV: first element of the head, index in the half
+    if (MODE == FEW_SWIGLU) r0 = nTile * (NCOL / 2);                   // the first NB/2 blocks are gate rows, the others the same up rows
+    if (MODE == FEW_QKV) {
+        const int half = p.headDim >> 1, tq = p.seg[0].N >> 5, tk = p.seg[1].N >> 5;
+        const int t = nTile < tq ? nTile : (nTile < tq + tk ? nTile - tq : nTile - tq - tk);
+        sgi = nTile < tq ? 0 : (nTile < tq + tk ? 1 : 2);
+        if (sgi == 2) r0 = t * 32;
+        else {
+            const int per = half >> 4;
+            head0 = (t / per) * p.headDim;
+            jj0 = (t % per) * 16;
+            r0 = head0 + jj0;
+            blk = half;
+        }
+    }
+    FewSeg sg = p.seg[0];
+    if (MODE == FEW_QKV) { if (sgi == 1) sg = p.seg[1]; if (sgi == 2) sg = p.seg[2]; }
+    const int N = sg.N;
+
+    const int chunks = K >> 6, planeChunks = (K + 63) >> 6;           // whole chunks; a last half one is multiplied after them
+    // A lane's weights of a chunk: row fr of the block, 16 of its 64 bytes (Q4_0: 8 bytes of each of two blocks).  Loaded
+    // like that a quarter wave touches 16 rows; so lane 16 Q + R loads piece R % 4 of row 4 Q + R / 4 instead (whole
+    // rows of 64 bytes) and the pieces change lanes (ds_bpermute).
+    const signed char* wP[NB];
+    const unsigned short* dP[NB];
+    const int ldRow = 4 * fq + (fr >> 2), ldPiece = fr & 3;
+    const int from = 4 * (16 * (fr >> 2) + 4 * (fr & 3) + (Q4 ? fq & 1 : fq));      // (bytes: ds_bpermute's lane address)
+    auto blockRow = [&](int b, int i) __attribute__((always_inline)) {
+        return min((MODE == FEW_SWIGLU ? r0 + (b % (NB / 2 > 0 ? NB / 2 : 1)) * 16 : r0 + b * blk) + i, N - 1);
+    };
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const signed char* W = (MODE == FEW_SWIGLU && b >= NB / 2) ? p.seg[1].W : sg.W;
+        wP[b] = Q4 ? W + (size_t)blockRow(b, ldRow) * (K >> 1) + ldPiece * 8 : W + (size_t)blockRow(b, ldRow) * K + ldPiece * 16;
+        dP[b] = Q4 ? reinterpret_cast<const unsigned short*>(W + (size_t)N * (K >> 1)) + (size_t)blockRow(b, fr) * (K >> 5) : nullptr;
+    }
+    const size_t aBlk = (size_t)planeChunks * 1024;                   // elements from one 16-row block to the next
+    const unsigned short* aH[MT];
+    const unsigned short* aL[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {                                    // (blocks past the last row repeat the last one)
+        const size_t o = (size_t)min((m0 >> 4) + i, (T - 1) >> 4) * aBlk + lane * 8;
+        aH[i] = p.Ahi + o;
+        aL[i] = p.Alo + o;
+    }
+
+    // What the epilogue needs is requested before the products' operands: the rows' sums of squares (for the RMS factor;
+    // 64 / MROW lanes share a row's parts), and this thread's scale, bias, gain, residual rows and RoPE factors.
+    constexpr int G = MT == 1 ? 4 : (MT == 2 ? 2 : 1), SQN = 4;     // (MT = 3: lanes past the rows repeat the last one)
+    const int sqRow = min(m0 + (G == 1 ? lane : lane % MROW), T - 1), sq0 = wave * G + (G == 1 ? 0 : lane / MROW);
+    float sqv[SQN];
+#pragma unroll
+    for (int j = 0; j < SQN; j++) {
+        const int i = sq0 + j * FR_WAVES * G;
+        sqv[j] = 0.f;
+        if (p.sumSq && i < p.sumParts) sqv[j] = p.sumSq[(size_t)i * p.sumStride + sqRow];
+    }
+    const int n = tid % NCOL, mq = (tid / NCOL) * 4;                  // this thread's results: column n, rows mq .. mq + 3
+    const int b = n >> 4, i16 = n & 15;
+    const bool isUp = MODE == FEW_SWIGLU && n >= NCOL / 2;
+    const int row = MODE == FEW_SWIGLU ? r0 + n % (NCOL / 2) : r0 + b * blk + i16;      // row of the weight matrix = column of the result
+    const bool okN = row < N, mine = mq < mRows;
+    const float* scales = isUp ? p.seg[1].scales : sg.scales;
+    const int rowC = min(row, N - 1);
+    const float sc = Q4 ? 1.0f : scales[rowC], bi = (MODE != FEW_SWIGLU && sg.bias) ? sg.bias[rowC] : 0.f;
+    float gain = 1.0f, old[4] = {0.f, 0.f, 0.f, 0.f}, cs[4], sn[4];
+    if (MODE == FEW_RESID || MODE == FEW_STORE) {
+        if (MODE == FEW_RESID && p.nextGain) gain = p.nextGain[rowC];
+        if (MODE == FEW_RESID || p.accumulate)
+#pragma unroll
+            for (int e = 0; e < 4; e++) old[e] = sg.Y[(size_t)min(m0 + mq + e, T - 1) * N + rowC];
+    }
+    if (MODE == FEW_QKV) {
+        const int half = p.headDim >> 1;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const size_t o = (size_t)(p.pos0 + min(m0 + mq + e, T - 1)) * half + jj0 + i16;
+            cs[e] = p.cosTab[o];
+            sn[e] = p.sinTab[o];
+        }
+    }
+
+    float4_t acc[MT][NB];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][b][e] = 0.f;
+
+    uint4 vh[D][MT][2], vl[D][MT][2];
+    int4 vw[D][NB];
+    unsigned vd[D][NB];
+    auto load = [&](int c, uint4 (&h)[MT][2], uint4 (&l)[MT][2], int4 (&w)[NB], unsigned (&d)[NB]) __attribute__((always_inline)) {
+        const int cc = max(min(c, chunks - 1), 0);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (Q4) {
+                const int2 x = *reinterpret_cast<const int2*>(wP[b] + cc * 32);
+                w[b] = make_int4(x.x, x.y, 0, 0);
+                d[b] = (unsigned)dP[b][cc * 2] | ((unsigned)dP[b][cc * 2 + 1] << 16);
+            } else {
+                w[b] = *reinterpret_cast<const int4*>(wP[b] + cc * 64);
+            }
+        }
+        // (every load is unconditional: one under a branch, even a branch that is always taken, makes the compiler's waits
+        // drain the ring; rows past T are whatever the buffer holds, and their results are dropped)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                h[i][s] = *reinterpret_cast<const uint4*>(aH[i] + cc * 1024 + s * 512);
+                l[i][s] = *reinterpret_cast<const uint4*>(aL[i] + cc * 1024 + s * 512);
+            }
+        asm volatile("" ::: "memory");                                // (the loads stay here, ahead of the products before them)
+    };
+    // a 32-k step: weight fragments f (Q4_0: block scales d) against activation blocks
+    auto product = [&](const bf16x8_t (&f)[NB], const float (&d)[NB], int i, uint4 h, uint4 l) __attribute__((always_inline)) {
+        const bf16x8_t ah = __builtin_bit_cast(bf16x8_t, h), al = __builtin_bit_cast(bf16x8_t, l);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (Q4) {
+                // a Q4_0 block's sum, then its fp16 scale (not foldable into a bf16 weight without loss)
+                float4_t t = {0.f, 0.f, 0.f, 0.f};
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, f[b], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, f[b], t, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[i][b][e] = fmaf(d[b], t[e], acc[i][b][e]);
+            } else {
+                acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, f[b], acc[i][b], 0, 0, 0);
+                acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, f[b], acc[i][b], 0, 0, 0);
+            }
+        }
+    };
+    auto multiply = [&](const uint4 (&h)[MT][2], const uint4 (&l)[MT][2], const int4 (&w)[NB], const unsigned (&d)[NB]) __attribute__((always_inline)) {
+        int4 x[NB];                                                   // this lane's own pieces
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            x[b].x = __builtin_amdgcn_ds_bpermute(from, w[b].x);
+            x[b].y = __builtin_amdgcn_ds_bpermute(from, w[b].y);
+            x[b].z = __builtin_amdgcn_ds_bpermute(Q4 ? from + 8 : from, Q4 ? w[b].x : w[b].z);      // (Q4_0: pieces 2 and 3 are the second block)
+            x[b].w = __builtin_amdgcn_ds_bpermute(Q4 ? from + 8 : from, Q4 ? w[b].y : w[b].w);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            bf16x8_t f[NB];
+            float dd[NB];
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                f[b] = Q4 ? frag_nib(s ? make_int2(x[b].z, x[b].w) : make_int2(x[b].x, x[b].y), fq >= 2 ? 4u : 0u)
+                          : frag_i8(s ? x[b].z : x[b].x, s ? x[b].w : x[b].y);
+                dd[b] = Q4 ? half_bits_to_float((unsigned short)(s ? d[b] >> 16 : d[b] & 0xffffu)) : 1.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < MT; i++) product(f, dd, i, h[i][s], l[i][s]);
+        }
+    };
+    if (!LOOP) {
+        load(wave, vh[0], vl[0], vw[0], vd[0]);
+        load(wave + FR_WAVES, vh[1], vl[1], vw[1], vd[1]);
+        if (wave < chunks) multiply(vh[0], vl[0], vw[0], vd[0]);
+        if (wave + FR_WAVES < chunks) multiply(vh[1], vl[1], vw[1], vd[1]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < D - 1; j++) load(wave + j * FR_WAVES, vh[j], vl[j], vw[j], vd[j]);
+        for (int c = wave; c < chunks; c += D * FR_WAVES) {
+#pragma unroll
+            for (int j = 0; j < D; j++) {
+                constexpr int DM = D - 1;
+                load(c + (j + DM) * FR_WAVES, vh[(j + DM) % D], vl[(j + DM) % D], vw[(j + DM) % D], vd[(j + DM) % D]);
+                if (c + j * FR_WAVES < chunks) multiply(vh[j], vl[j], vw[j], vd[j]);
+            }
+        }
+    }
+
+    if ((K & 32) && wave == (chunks & (FR_WAVES - 1))) {              // the last 32 k: 8 a quarter
+        bf16x8_t f[NB];
+        float dd[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (Q4) {
+                const signed char* W = (MODE == FEW_SWIGLU && b >= NB / 2) ? p.seg[1].W : sg.W;
+                f[b] = frag_nib(*reinterpret_cast<const int2*>(W + (size_t)blockRow(b, fr) * (K >> 1) + chunks * 32 + (fq & 1) * 8), fq >= 2 ? 4u : 0u);
+                dd[b] = half_bits_to_float(dP[b][chunks * 2]);
+            } else {
+                const signed char* W = (MODE == FEW_SWIGLU && b >= NB / 2) ? p.seg[1].W : sg.W;
+                const int2 x = *reinterpret_cast<const int2*>(W + (size_t)blockRow(b, fr) * K + chunks * 64 + 8 * fq);
+                f[b] = frag_i8(x.x, x.y);
+                dd[b] = 1.0f;
+            }
+        }
+        const int at = chunks * 1024 + (Q4 ? 0 : (fq & 1) * 512 + ((fq >> 1) * 16 + fr) * 8 - lane * 8);      // k = 8 q .. 8 q + 7
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+            product(f, dd, i, *reinterpret_cast<const uint4*>(aH[i] + at), *reinterpret_cast<const uint4*>(aL[i] + at));
+    }
+
+    // C layout: lane holds column fr, rows 4 fq .. 4 fq + 3 of a block
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+            *reinterpret_cast<float4_t*>(&part[(wave * NCOL + b * 16 + fr) * LST + i * 16 + 4 * fq]) = acc[i][b];
+    {
+        float sq = (sqv[0] + sqv[1]) + (sqv[2] + sqv[3]);
+        if (p.sumSq)
+            for (int i = sq0 + SQN * FR_WAVES * G; i < p.sumParts; i += FR_WAVES * G) sq += p.sumSq[(size_t)i * p.sumStride + sqRow];
+        if (G == 4) sq = rows_sum(sq);
+        if (G == 2) sq += __shfl_xor(sq, 32, 64);
+        if (lane < MROW) sumq[wave][lane] = sq;
+    }
+    __syncthreads();
+    if (NB < 8 && !mine) return;                                      // (NB = 8: 128 columns x 16 rows, all threads have results)
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < FR_WAVES; w++) {
+        const float4_t t = *reinterpret_cast<const float4_t*>(&part[(w * NCOL + n) * LST + mq]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] += t[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        float rs = 1.0f;
+        if (p.sumSq) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < FR_WAVES; w++) t += sumq[w][mq + e];
+            rs = 1.0f / sqrtf(t / (float)K + p.eps);
+        }
+        v[e] = v[e] * sc * rs + bi;
+    }
+    if (MODE == FEW_STORE) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int m = m0 + mq + e;
+            if (okN && m < T) {
+                float* y = sg.Y + (size_t)m * N + row;
+                *y = old[e] + v[e];
+            }
+        }
+    } else if (MODE == FEW_RESID) {
+        float q2[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int m = m0 + mq + e;
+            q2[e] = 0.f;
+            if (okN && m < T) {
+                const float x = old[e] + v[e];
+                sg.Y[(size_t)m * N + row] = x;
+                q2[e] = x * x;
+                if (p.nextHi) {
+                    const float a = x * gain;
+                    const unsigned short h = bf16_one(a);
+                    const size_t o = few_index(m, row, N, p.nextQ4);
+                    p.nextHi[o] = h;
+                    p.nextLo[o] = bf16_one(a - bf16_value(h));
+                }
+            }
+        }
+        if (p.nextSumSq) {
+            // the tile's share of the rows' sums of squares: over the 16 lanes of a block, then the blocks
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                q2[e] = row_sum16(q2[e]);
+                if (NB >= 2) q2[e] += __shfl_xor(q2[e], 16, 64);
+                if (NB == 4) q2[e] += __shfl_xor(q2[e], 32, 64);
+            }
+            if (n == 0)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (m0 + mq + e < T) p.nextSumSq[(size_t)nTile * p.sumStride + m0 + mq + e] = q2[e];
+        }
+    } else if (MODE == FEW_SWIGLU) {
+        // the up value of a gate value's column is NCOL / 2 threads away: in the wave, or (64 columns of each) in the next
+        float up[4];
+        if (NB < 8) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) up[e] = __shfl_xor(v[e], NCOL / 2, 64);
+        } else {
+            __syncthreads();                                          // (all sums are read; every thread is here: see `mine`)
+            *reinterpret_cast<float4_t*>(&part[(n * (MROW / 4) + mq / 4) * 4]) = float4_t{v[0], v[1], v[2], v[3]};
+            __syncthreads();
+            const float4_t t = *reinterpret_cast<const float4_t*>(&part[((n ^ (NCOL / 2)) * (MROW / 4) + mq / 4) * 4]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) up[e] = t[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float u = up[e];
+            const int m = m0 + mq + e;
+            if (!isUp && okN && m < T) {
+                const float g = v[e];
+                const float a = g * (1.0f / (1.0f + expf(-g))) * u;          // mongoose.cu:949-956
+                const unsigned short h = bf16_one(a);
+                const size_t o = few_index(m, row, N, p.nextQ4);
+                p.nextHi[o] = h;
+                p.nextLo[o] = bf16_one(a - bf16_value(h));
+            }
+        }
+    } else {
+        // RoPE on the pairs (j, j + half) of q and k (mongoose.cu:991-1006): the partner is 16 lanes away
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float other = __shfl_xor(v[e], 16, 64);
+            const int m = m0 + mq + e;
+            if (m >= T) continue;
+            const size_t pos = (size_t)(p.pos0 + m);
+            float x = v[e];
+            if (sgi < 2) x = b == 0 ? v[e] * cs[e] - other * sn[e] : other * sn[e] + v[e] * cs[e];
+            if (sgi == 0) sg.Y[(size_t)m * N + row] = x;
+            else {
+                void* cache = sgi == 1 ? p.Kc : p.Vc;
+                if (p.kvHalf) static_cast<_Float16*>(cache)[pos * N + row] = (_Float16)x;
+                else static_cast<float*>(cache)[pos * N + row] = x;
+            }
+        }
+    }
+}
+
+template <int MODE, int MT, int NB, int Q4, int LOOP>
+static hipError_t launch_few_l(const FewParams& p, hipStream_t s) {
+    constexpr int bytes = FR_WAVES * 16 * NB * (16 * MT + 4) * 4;
+    if (bytes > 48 * 1024) {
+        static bool raised = false;                                    // (more than the default cap on dynamic LDS)
+        if (!raised) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_rows_kernel<MODE, MT, NB, Q4, LOOP>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+            if (e != hipSuccess) return e;
+            raised = true;
+        }
+    }
+    const int numM = (p.T + 16 * MT - 1) / (16 * MT);
+    const unsigned grid = (unsigned)((p.nTiles + 7) / 8 * 8) * (unsigned)numM;
+    hipLaunchKernelGGL((few_rows_kernel<MODE, MT, NB, Q4, LOOP>), dim3(grid), dim3(FR_WG), bytes, s, p);
+    return hipGetLastError();
+}
+
+template <int MODE, int MT, int NB, int Q4>
+static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
+    return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1>(p, s);
+}
+
+// The tile of a launch (16 MT activation rows x 16 NB weight rows a workgroup).  A CU pulls some 53 bytes a nanosecond
+// through its load path here, whether they come from its L2 or from beyond it, and a round of workgroups pays 2.5 us of
+// start-up and end of its own: the tile with the shortest rounds * (start-up + bytes) is taken, with a workgroup on every CU
+// in mind.  (0.5B shape, 37 rows: gate | up in 304 workgroups of 48 x 16 + 16 rows 15.5 us, of 32 x 32 + 32 rows
+// 11.3 us, in 228 of 16 x 64 + 64 rows 10.5 us.)
+struct FewTile { int mt, nb; };
+static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast) {
+    const int b16 = (T + 15) / 16;
+    FewTile best{1, nbFirst};
+    double least = 1e30;
+    for (int nb = nbFirst; nb <= nbLast; nb *= 2)
+        for (int mt = 1; mt <= 4 && mt <= b16 && mt * nb <= 8; mt++) {
+            const long long wgs = (long long)((rowsN + 16 * nb - 1) / (16 * nb)) * ((b16 + mt - 1) / mt);
+            const double bytes = (64.0 * mt + 16.0 * nb) * K;
+            const double cost = (double)((wgs + 255) / 256) * (2500.0 + bytes / 53.0) + bytes * (double)wgs * 1e-9;
+            if (cost < least) { least = cost; best = FewTile{mt, nb}; }
+        }
+    return best;
+}
+int few_rows_sum_parts(int N, int T, int K) { const int b = few_tile(N, T, K, 1, 4).nb; return (N + 16 * b - 1) / (16 * b); }
+
+template <int MODE, int MT, int NB>
+static hipError_t launch_few_fmt(const FewParams& p, hipStream_t s) {
+    return p.q4 ? launch_few_t<MODE, MT, NB, 1>(p, s) : launch_few_t<MODE, MT, NB, 0>(p, s);
+}
+template <int MODE, int NB>
+static hipError_t launch_few_mt(int mt, const FewParams& p, hipStream_t s) {
+    if (mt == 1) return launch_few_fmt<MODE, 1, NB>(p, s);
+    if constexpr (NB <= 4)
+        if (mt == 2) return launch_few_fmt<MODE, 2, NB>(p, s);
+    if constexpr (NB <= 2) {
+        if (mt == 3) return launch_few_fmt<MODE, 3, NB>(p, s);
+        if (mt == 4) return launch_few_fmt<MODE, 4, NB>(p, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
+    if (p.T <= 0) return hipSuccess;
+    if (p.K <= 0 || p.K % 32 || !p.Ahi || !p.Alo || p.seg[0].N <= 0) return hipErrorInvalidValue;
+    const int N = p.seg[0].N;
+    if (mode == FEW_STORE || mode == FEW_RESID) {
+        const FewTile t = few_tile(N, p.T, p.K, 1, 4);
+        p.nTiles = (N + 16 * t.nb - 1) / (16 * t.nb);
+        if (mode == FEW_STORE) return t.nb == 1 ? launch_few_mt<FEW_STORE, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_STORE, 2>(t.mt, p, s) : launch_few_mt<FEW_STORE, 4>(t.mt, p, s);
+        return t.nb == 1 ? launch_few_mt<FEW_RESID, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_RESID, 2>(t.mt, p, s) : launch_few_mt<FEW_RESID, 4>(t.mt, p, s);
+    }
+    if (mode == FEW_SWIGLU) {
+        if (p.seg[1].N != N || !p.nextHi || !p.nextLo) return hipErrorInvalidValue;
+        const FewTile t = few_tile(2 * N, p.T, p.K, 2, 8);
+        p.nTiles = (N + 8 * t.nb - 1) / (8 * t.nb);
+        return t.nb == 2 ? launch_few_mt<FEW_SWIGLU, 2>(t.mt, p, s) : t.nb == 4 ? launch_few_mt<FEW_SWIGLU, 4>(t.mt, p, s) : launch_few_mt<FEW_SWIGLU, 8>(t.mt, p, s);
+    }
+    if (mode == FEW_QKV) {
+        if ((p.headDim != 64 && p.headDim != 128) || N % p.headDim || p.seg[1].N <= 0 || p.seg[1].N % p.headDim ||
+            p.seg[2].N != p.seg[1].N || !p.Kc || !p.Vc) return hipErrorInvalidValue;
+        p.nTiles = (N + 2 * p.seg[1].N) / 32;
+        return launch_few_mt<FEW_QKV, 2>(few_tile(N + 2 * p.seg[1].N, p.T, p.K, 2, 2).mt, p, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------------------
+// Embedding rows, their split times the first gain, their sums of squares: one workgroup a row.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(WG) void embed_split_kernel(int kind, const void* table, const float* scales, const int* tokens, float* x,
+                                                         const float* gain, unsigned short* hi, unsigned short* lo, float* sumSq,
+                                                         int dim, int vocab, int q4) {
+    __shared__ float red[4];
+    const int t = blockIdx.x;
+    int tok = tokens[t];
+    tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);
+    float ss = 0.f;
+    for (int i = threadIdx.x; i < dim; i += WG) {
+        const float v = embed_value(kind, table, scales, tok, dim, vocab, i);
+        x[(size_t)t * dim + i] = v;
+        ss += v * v;
+        const float a = v * gain[i];
+        const unsigned short h = bf16_one(a);
+        const size_t o = few_index(t, i, dim, q4);
+        hi[o] = h;
+        lo[o] = bf16_one(a - bf16_value(h));
+    }
+    ss = block_sum(ss, red);
+    if (threadIdx.x == 0) sumSq[t] = ss;
+}
+hipError_t launch_embed_split(int kind, const void* table, const float* scales, const int* tokens, float* x, const float* gain,
+                              unsigned short* hi, unsigned short* lo, float* sumSq, int T, int dim, int vocab, int q4, hipStream_t s) {
+    if (T <= 0) return hipSuccess;
+    hipLaunchKernelGGL(embed_split_kernel, dim3((unsigned)T), dim3(WG), 0, s, kind, table, scales, tokens, x, gain, hi, lo, sumSq, dim, vocab, q4);
+    return hipGetLastError();
+}
+
+// Rows of a caller's activations (per-op GEMM), one workgroup per 16 rows x 256 k: the planes are written whole lanes at a
+// time, rows past T as zeros.
+__global__ __launch_bounds__(WG) void few_split_kernel(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4) {
+    const int k = blockIdx.x * 256 + (threadIdx.x >> 4) * 8, r = threadIdx.x & 15;
+    const int t = blockIdx.y * 16 + r;
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        const int kk = k + half * 128;
+        if (kk >= K) continue;
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f), c = a;
+        if (t < T) {
+            a = *reinterpret_cast<const float4*>(in + (size_t)t * K + kk);
+            c = *reinterpret_cast<const float4*>(in + (size_t)t * K + kk + 4);
+        }
+        const float v[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+        unsigned h[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            h[i] = bf16_pair(v[2 * i], v[2 * i + 1]);
+            l[i] = bf16_pair(v[2 * i] - bf16_value((unsigned short)(h[i] & 0xffffu)), v[2 * i + 1] - bf16_value((unsigned short)(h[i] >> 16)));
+        }
+        const size_t o = few_index(t, kk, K, q4);
+        *reinterpret_cast<uint4*>(hi + o) = make_uint4(h[0], h[1], h[2], h[3]);
+        *reinterpret_cast<uint4*>(lo + o) = make_uint4(l[0], l[1], l[2], l[3]);
+    }
+}
+hipError_t launch_few_split(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4, hipStream_t s) {
+    if (T <= 0) return hipSuccess;
+    if (K % 32 || ((uintptr_t)in & 15)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(few_split_kernel, dim3((unsigned)((K + 255) / 256), (unsigned)((T + 15) / 16)), dim3(WG), 0, s, in, hi, lo, T, K, q4);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Causal attention over fp32 (or fp16) cache rows in fp32, on v_mfma_f32_16x16x4_f32: no split of the operands, no pass
+// over the cache rows beforehand.  A workgroup = one query head x 16 queries; its 8 waves take the 16-position tiles in
+// turn, each with a running maximum / sum / output of its own, combined through LDS at the end.
+//   S^T[kpos][q] = K . Q^T   A = K rows (lane: row l%16), B = Q rows; the quarter l/16 of a lane holds the head elements
+//                            HD/4 * (l/16) + s, s = 0 .. HD/4 - 1, of both
+//   O^T[d][q]    = V^T . P^T a lane holds S^T rows 4 (l/16) + e of its query: as the B operand of step e it is position
+//                            4 (l/16) + e, which is the V row the lane loads; its elements HD/16 * (l%16) + b make up
+//                            row l%16 of output block b
+// ---------------------------------------------------------------------------
+template <bool KVH>
+__device__ __forceinline__ float4 ld_row4(const void* base, size_t i) {
+    if (!KVH) return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
+    const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(base) + i);
+    return make_float4(half_bits_to_float((unsigned short)(u.x & 0xffffu)), half_bits_to_float((unsigned short)(u.x >> 16)),
+                       half_bits_to_float((unsigned short)(u.y & 0xffffu)), half_bits_to_float((unsigned short)(u.y >> 16)));
+}
+
+template <int HD, bool KVH>
+__global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, const void* Kc, const void* Vc, unsigned short* hi,
+                                                             unsigned short* lo, int T, int pos0, int dim, int kvDim, int nHeads,
+                                                             int nKVHeads, int q4) {
+    constexpr int KF = HD / 16, VF = HD / 16;              // K: float4 a lane and row (HD/4 elements); V: elements a lane and row
+    constexpr int OST = 17;
+    extern __shared__ float ob[];                          // [wave][HD][OST]
+    __shared__ float wm[FR_WAVES][16], wl[FR_WAVES][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fq = lane >> 4;
+    const int head = blockIdx.x % nHeads, q0 = ((int)gridDim.x / nHeads - 1 - (int)blockIdx.x / nHeads) * 16;    // the longest ranges first
+    const int kvh = head / (nHeads / nKVHeads);
+    const int myq = min(q0 + fr, T - 1), qpos = pos0 + myq;
+    const int last = pos0 + min(q0 + 15, T - 1), nTiles = last / 16 + 1;
+    const float scale = 1.0f / sqrtf((float)HD);
+    float4 qf[KF];
+#pragma unroll
+    for (int i = 0; i < KF; i++) {
+        qf[i] = *reinterpret_cast<const float4*>(q + (size_t)myq * dim + (size_t)head * HD + (HD / 4) * fq + 4 * i);
+        qf[i].x *= scale; qf[i].y *= scale; qf[i].z *= scale; qf[i].w *= scale;
+    }
+    float4_t o[VF];
+#pragma unroll
+    for (int b = 0; b < VF; b++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[b][e] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    float4 kf[2][KF], vf[2][4][VF / 4];
+    auto load = [&](int t, float4 (&k)[KF], float4 (&v)[4][VF / 4]) __attribute__((always_inline)) {
+        const int t0 = min(t, nTiles - 1) * 16;
+        // K: whole rows at a time, HD/4 lanes a row (they change lanes through LDS when they are wanted)
+#pragma unroll
+        for (int i = 0; i < KF; i++)
+            k[i] = ld_row4<KVH>(Kc, (size_t)min(t0 + i * (256 / HD) + lane / (HD / 4), last) * kvDim + (size_t)kvh * HD + 4 * (lane % (HD / 4)));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const size_t vr = (size_t)min(t0 + 4 * fq + e, last) * kvDim + (size_t)kvh * HD + VF * fr;
+#pragma unroll
+            for (int i = 0; i < VF / 4; i++) v[e][i] = ld_row4<KVH>(Vc, vr + 4 * i);
+        }
+    };
+    float* kt = ob + wave * (HD * OST);                    // this wave's K tile: 16 rows of HD + HD/16 floats
+    constexpr int KST = HD + HD / 16;
+    auto step = [&](int t, const float4 (&kl)[KF], const float4 (&v)[4][VF / 4]) __attribute__((always_inline)) {
+        float4 k[KF];
+#pragma unroll
+        for (int i = 0; i < KF; i++)
+            *reinterpret_cast<float4*>(&kt[(i * (256 / HD) + lane / (HD / 4)) * KST + 4 * (lane % (HD / 4))]) = kl[i];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < KF; i++) k[i] = *reinterpret_cast<const float4*>(&kt[fr * KST + (HD / 4) * fq + 4 * i]);
+        __builtin_amdgcn_wave_barrier();
+        float4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};         // two chains for the matrix pipe
+#pragma unroll
+        for (int i = 0; i < KF; i++) {
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i].x, qf[i].x, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i].y, qf[i].y, s1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i].z, qf[i].z, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i].w, qf[i].w, s1, 0, 0, 0);
+        }
+        float sv[4], tmax = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int kpos = t * 16 + 4 * fq + e;
+            sv[e] = kpos <= qpos ? s0[e] + s1[e] : -INFINITY;
+            tmax = fmaxf(tmax, sv[e]);
+        }
+        tmax = rows_max(tmax);
+        const float mNew = fmaxf(m, tmax);
+        const float corr = m == -INFINITY ? 0.f : exp_neg(m - mNew);
+        float ps = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            sv[e] = sv[e] == -INFINITY ? 0.f : exp_neg(sv[e] - mNew);
+            ps += sv[e];
+        }
+        l = l * corr + rows_sum(ps);
+        m = mNew;
+#pragma unroll
+        for (int b = 0; b < VF; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[b][e] *= corr;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < VF / 4; i++) {
+                o[4 * i + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].x, sv[e], o[4 * i + 0], 0, 0, 0);
+                o[4 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].y, sv[e], o[4 * i + 1], 0, 0, 0);
+                o[4 * i + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].z, sv[e], o[4 * i + 2], 0, 0, 0);
+                o[4 * i + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].w, sv[e], o[4 * i + 3], 0, 0, 0);
+            }
+    };
+    load(wave, kf[0], vf[0]);
+    for (int t = wave; t < nTiles; t += 2 * FR_WAVES) {
+        load(t + FR_WAVES, kf[1], vf[1]);
+        step(t, kf[0], vf[0]);
+        load(t + 2 * FR_WAVES, kf[0], vf[0]);
+        if (t + FR_WAVES < nTiles) step(t + FR_WAVES, kf[1], vf[1]);
+    }
+    __builtin_amdgcn_wave_barrier();
+    // O^T of block b: lane holds query fr, rows i = 4 fq + e, i.e. head element VF * i + b
+#pragma unroll
+    for (int b = 0; b < VF; b++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) ob[(wave * HD + VF * (4 * fq + e) + b) * OST + fr] = o[b][e];
+    if (fq == 0) { wm[wave][fr] = m; wl[wave][fr] = l; }
+    __syncthreads();
+    for (int i = tid; i < 16 * HD; i += FR_WG) {
+        const int qq = i / HD, d = i % HD;
+        if (q0 + qq >= T) continue;
+        float M = wm[0][qq];
+#pragma unroll
+        for (int w = 1; w < FR_WAVES; w++) M = fmaxf(M, wm[w][qq]);
+        float num = 0.f, den = 0.f;
+#pragma unroll
+        for (int w = 0; w < FR_WAVES; w++) {
+            const float g = wm[w][qq] == -INFINITY ? 0.f : exp_neg(wm[w][qq] - M);
+            num = fmaf(g, ob[(w * HD + d) * OST + qq], num);
+            den = fmaf(g, wl[w][qq], den);
+        }
+        const float a = num / den;
+        const unsigned short h = bf16_one(a);
+        const size_t ix = few_index(q0 + qq, head * HD + d, dim, q4);
+        hi[ix] = h;
+        lo[ix] = bf16_one(a - bf16_value(h));
+    }
+}
+
+template <int HD, bool KVH>
+static hipError_t launch_few_attn_t(unsigned grid, hipStream_t s, const float* q, const void* Kc, const void* Vc, unsigned short* hi,
+                                    unsigned short* lo, int T, int pos0, int dim, int kvDim, int nHeads, int nKVHeads, int q4) {
+    constexpr int bytes = FR_WAVES * HD * 17 * 4;
+    if (bytes > 48 * 1024) {
+        static bool raised = false;
+        if (!raised) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_attention_kernel<HD, KVH>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+            if (e != hipSuccess) return e;
+            raised = true;
+        }
+    }
+    hipLaunchKernelGGL((few_attention_kernel<HD, KVH>), dim3(grid), dim3(FR_WG), bytes, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    return hipGetLastError();
+}
+
+hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
+                                int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4, hipStream_t s) {
+    if (T <= 0) return hipSuccess;
+    if (nKVHeads <= 0 || nHeads % nKVHeads || pos0 < 0 || pos0 + T > rowLimit || dim != nHeads * headDim || kvDim != nKVHeads * headDim ||
+        (headDim != 64 && headDim != 128) || !hi || !lo) return hipErrorInvalidValue;
+    const unsigned grid = (unsigned)nHeads * (unsigned)((T + 15) / 16);
+    if (headDim == 64) return kvHalf ? launch_few_attn_t<64, true>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
+                                     : launch_few_attn_t<64, false>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    return kvHalf ? launch_few_attn_t<128, true>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
+                  : launch_few_attn_t<128, false>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+}
+
+}  // namespace mg

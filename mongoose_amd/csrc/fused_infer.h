@@ -151,6 +151,13 @@ private:
     void *pfHi = nullptr, *pfLo = nullptr, *pfHi2 = nullptr, *pfLo2 = nullptr;
     float* pfPartial = nullptr;
     int ensurePrefill(int rows, int kvRows);
+    float* pfSumSq = nullptr;               // few-row path: partial sums of squares of the rows
+    // Rows up to which a prefill takes the few-row kernels.  Microseconds a layer, few-row / tiled, measured: 0.5B shape 37 /
+    // 71 at 48 rows, 66 / 94 at 256, 126 / 134 at 640, 170 / 157 at 800; 1.1B 58 / 91 at 64, 127 / 165 at 320, 207 / 200 at
+    // 512; 8B 105 / 168 at 4, 257 / 265 at 128, 315 / 322 at 192, 422 / 321 at 256.
+    int fewRowsLimit() const { return 640 * 1024 / dim > 192 ? 640 * 1024 / dim : 192; }
+    int enqueuePrefillFew(int T, int pos0);
+    int enqueuePrefillTiles(int T, int pos0);
     std::vector<Slab> layerSlabs, kvSlabs;
     size_t slotOff[12] = {0};
     size_t layerSlabBytes = 0;

@@ -5,6 +5,7 @@
 #include "../../include/mongoose_hip.h"
 #include "host_util.h"
 #include "prefill.h"
+#include "few_rows.h"
 
 #include <chrono>
 #include <cmath>
@@ -1569,11 +1570,13 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     prefillCap = 0;
     const size_t T = ((size_t)rows + 127) / 128 * 128;
     const size_t plane = split_plane_elems((int)T, ffnDim > dim ? ffnDim : dim) * 2;
-    size_t bytes = alignUp256(T * 4) + 2 * alignUp256(T * dim * 4) + 2 * alignUp256(T * kvDim * 4) +
+    const size_t sums = (size_t)(dim / 16 + 1) * std::min<size_t>(T, (size_t)fewRowsLimit());
+    size_t bytes = alignUp256(sums * 4) + alignUp256(T * 4) + 2 * alignUp256(T * dim * 4) + 2 * alignUp256(T * kvDim * 4) +
                    2 * alignUp256(T * ffnDim * 4) + 4 * alignUp256(plane) + alignUp256(gemm_partial_floats() * 4) + 16 * 256;
     int rc = prefillSlab.init(bytes);
     if (rc) return rc;
     pfTokens = static_cast<int*>(prefillSlab.take(T * 4));
+    pfSumSq = static_cast<float*>(prefillSlab.take(sums * 4));
     pfX = static_cast<float*>(prefillSlab.take(T * dim * 4));
     pfQ = static_cast<float*>(prefillSlab.take(T * dim * 4));
     pfK = static_cast<float*>(prefillSlab.take(T * kvDim * 4));
@@ -1585,7 +1588,7 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     pfHi2 = prefillSlab.take(plane);      // second pair: written by the gate|up GEMM's own epilogue while it still reads the first
     pfLo2 = prefillSlab.take(plane);
     pfPartial = static_cast<float*>(prefillSlab.take(gemm_partial_floats() * 4));
-    if (!pfTokens || !pfX || !pfQ || !pfK || !pfV || !pfGate || !pfUp || !pfHi || !pfLo || !pfHi2 || !pfLo2 || !pfPartial) {
+    if (!pfTokens || !pfSumSq || !pfX || !pfQ || !pfK || !pfV || !pfGate || !pfUp || !pfHi || !pfLo || !pfHi2 || !pfLo2 || !pfPartial) {
         set_error("prefill slab too small");
         return MG_E_STATE;
     }
@@ -1593,25 +1596,8 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     return MG_OK;
 }
 
-int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* nextToken, float* logitsOut, float* elapsedMs) {
-    if (!built) return MG_E_NOT_BUILT;
-    ARGCHK(tokens && nTokens >= 1 && pos0 >= 0 && pos0 + nTokens <= maxSeq, "Prefill: bad token count or position");
-    for (int i = 0; i < nTokens; i++) ARGCHK(tokens[i] >= 0 && tokens[i] < vocabSize, "Prefill: token out of range");
-    int rc = checkReady(this);
-    if (rc) return rc;
-    for (const auto& L : layers) {
-        // q/k/v and gate/up share a launch: one weight format each
-        if (L.wq.kind != L.wk.kind || L.wk.kind != L.wv.kind || L.gate.kind != L.up.kind) {
-            set_error("Prefill: q/k/v (and gate/up) of a layer must share one weight format");
-            return MG_E_UNSUPPORTED;
-        }
-    }
-    rc = ensurePrefill(nTokens, pos0 + nTokens);
-    if (rc) return rc;
-    const int T = nTokens;
-    HIPCHK(hipStreamSynchronize(stream));
-    HIPCHK(hipMemcpy(pfTokens, tokens, sizeof(int) * (size_t)T, hipMemcpyHostToDevice));
-    HIPCHK(hipEventRecord(ev0, stream));
+// The layers over T rows through the tiled GEMMs of prefill.hip; the rows end up in pfX.
+int HIPFusedInference::enqueuePrefillTiles(int T, int pos0) {
     if (embedKind == 1 || embedKind == 2) {
         HIPCHK(launch_embed_rows(embedKind, embedTable, nullptr, pfTokens, pfX, T, dim, vocabSize, stream));
     } else {
@@ -1664,6 +1650,75 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
         normSplitDone = g.wroteNext != 0;
         g.Ahi = static_cast<const unsigned short*>(pfHi); g.Alo = static_cast<const unsigned short*>(pfLo);
     }
+    return MG_OK;
+}
+
+// The same through the few-row kernels (few_rows.hip): five launches a layer.
+int HIPFusedInference::enqueuePrefillFew(int T, int pos0) {
+    unsigned short *hi = static_cast<unsigned short*>(pfHi), *lo = static_cast<unsigned short*>(pfLo);         // normed rows
+    unsigned short *hi2 = static_cast<unsigned short*>(pfHi2), *lo2 = static_cast<unsigned short*>(pfLo2);     // attention output, SwiGLU rows
+    const bool table = embedKind == 1 || embedKind == 2;
+    HIPCHK(launch_embed_split(table ? embedKind : (lmHead.kind == WF_Q8 ? 0 : 3), table ? embedTable : lmHead.w, table ? nullptr : lmHead.scales,
+                              pfTokens, pfX, layers[0].norm1, hi, lo, pfSumSq, T, dim, vocabSize, layers[0].wq.kind == WF_Q4P, stream));
+    int parts = 1;
+    const int woParts = few_rows_sum_parts(dim, T, dim), downParts = few_rows_sum_parts(dim, T, ffnDim);
+    auto seg = [](const DevMat& m, const float* bias, float* y) {
+        return FewSeg{static_cast<const signed char*>(m.w), m.scales, bias, y, m.rows};
+    };
+    for (int l = 0; l < nLayers; l++) {
+        const LayerWeights& L = layers[l];
+        FewParams f{};
+        f.T = T; f.K = dim; f.Ahi = hi; f.Alo = lo; f.eps = eps;
+        f.sumSq = pfSumSq; f.sumParts = parts; f.sumStride = T;
+        f.q4 = L.wq.kind == WF_Q4P;
+        f.seg[0] = seg(L.wq, L.bq, pfQ); f.seg[1] = seg(L.wk, L.bk, nullptr); f.seg[2] = seg(L.wv, L.bv, nullptr);
+        f.Kc = kCache[l]; f.Vc = vCache[l]; f.cosTab = cosTab; f.sinTab = sinTab; f.pos0 = pos0; f.headDim = headDim; f.kvHalf = kvHalf;
+        HIPCHK(launch_few_rows(FEW_QKV, f, stream));
+        HIPCHK(launch_few_attention(pfQ, kCache[l], vCache[l], kvHalf, hi2, lo2, T, pos0, maxSeq, dim, kvDim, nHeads, nKVHeads, headDim,
+                                    L.wo.kind == WF_Q4P, stream));
+        FewParams r{};
+        r.T = T; r.sumStride = T; r.K = dim; r.Ahi = hi2; r.Alo = lo2;
+        r.q4 = L.wo.kind == WF_Q4P; r.seg[0] = seg(L.wo, nullptr, pfX);
+        r.nextGain = L.norm2; r.nextHi = hi; r.nextLo = lo; r.nextSumSq = pfSumSq; r.nextQ4 = L.gate.kind == WF_Q4P;
+        HIPCHK(launch_few_rows(FEW_RESID, r, stream));
+        parts = woParts;
+        FewParams g{};
+        g.T = T; g.K = dim; g.Ahi = hi; g.Alo = lo; g.eps = eps;
+        g.sumSq = pfSumSq; g.sumParts = parts; g.sumStride = T;
+        g.q4 = L.gate.kind == WF_Q4P; g.seg[0] = seg(L.gate, nullptr, nullptr); g.seg[1] = seg(L.up, nullptr, nullptr);
+        g.nextHi = hi2; g.nextLo = lo2; g.nextQ4 = L.down.kind == WF_Q4P;
+        HIPCHK(launch_few_rows(FEW_SWIGLU, g, stream));
+        r.K = ffnDim; r.q4 = L.down.kind == WF_Q4P; r.seg[0] = seg(L.down, nullptr, pfX);
+        if (l + 1 < nLayers) { r.nextGain = layers[l + 1].norm1; r.nextQ4 = layers[l + 1].wq.kind == WF_Q4P; }
+        else { r.nextGain = nullptr; r.nextHi = nullptr; r.nextLo = nullptr; r.nextSumSq = nullptr; }
+        HIPCHK(launch_few_rows(FEW_RESID, r, stream));
+        parts = downParts;
+    }
+    return MG_OK;
+}
+
+int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* nextToken, float* logitsOut, float* elapsedMs) {
+    if (!built) return MG_E_NOT_BUILT;
+    ARGCHK(tokens && nTokens >= 1 && pos0 >= 0 && pos0 + nTokens <= maxSeq, "Prefill: bad token count or position");
+    for (int i = 0; i < nTokens; i++) ARGCHK(tokens[i] >= 0 && tokens[i] < vocabSize, "Prefill: token out of range");
+    int rc = checkReady(this);
+    if (rc) return rc;
+    for (const auto& L : layers) {
+        // q/k/v and gate/up share a launch: one weight format each
+        if (L.wq.kind != L.wk.kind || L.wk.kind != L.wv.kind || L.gate.kind != L.up.kind) {
+            set_error("Prefill: q/k/v (and gate/up) of a layer must share one weight format");
+            return MG_E_UNSUPPORTED;
+        }
+    }
+    rc = ensurePrefill(nTokens, pos0 + nTokens);
+    if (rc) return rc;
+    const int T = nTokens;
+    const bool few = T <= fewRowsLimit();
+    HIPCHK(hipStreamSynchronize(stream));
+    HIPCHK(hipMemcpy(pfTokens, tokens, sizeof(int) * (size_t)T, hipMemcpyHostToDevice));
+    HIPCHK(hipEventRecord(ev0, stream));
+    rc = few ? enqueuePrefillFew(T, pos0) : enqueuePrefillTiles(T, pos0);
+    if (rc) return rc;
     // the last position continues on the decode path: final norm, lm_head, greedy token, state -> pos0 + T
     HIPCHK(hipMemcpyAsync(hidden[hiddenIdx], pfX + (size_t)(T - 1) * dim, (size_t)dim * 4, hipMemcpyDeviceToDevice, stream));
     { int rcs = setState(pos0 + T - 1, tokens[T - 1], 0, 0); if (rcs) return rcs; }

@@ -1,0 +1,66 @@
+"""The few-row prefill kernels (few_rows.hip) against the token-by-token path, at the edges of their tiles."""
+import numpy as np
+import pytest
+
+from mongoose_amd import configs
+from mongoose_amd import engine as E
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+# heads of 128 with a group of 3, widths that end inside a tile and inside a 64-wide step
+ODD = configs.TOY._replace(name="odd", nLayers=2, dim=384, nHeads=3, nKVHeads=1, headDim=128, ffnDim=1376 + 32, vocab=300, bias=True)
+SMALL = configs.TOY._replace(name="small", nLayers=2, dim=448, nHeads=7, nKVHeads=1, ffnDim=608, vocab=300, bias=True)
+
+
+WIDE = configs.TOY._replace(name="wide", nLayers=2, dim=512, ffnDim=9728, vocab=300)
+
+
+@pytest.mark.parametrize("shape,fmt,kv_f16,pos0,rows", [
+    (WIDE, "q8", False, 9, 37), (WIDE, "q4_0", False, 0, 64), (SMALL, "q8", False, 0, 1), (SMALL, "q8", False, 0, 16), (SMALL, "q8", False, 3, 17), (SMALL, "q8", False, 130, 64),
+    (SMALL, "q4_0", False, 5, 33), (SMALL, "q4_0", True, 0, 48), (ODD, "q8", False, 100, 15), (ODD, "q8", True, 17, 63),
+    (ODD, "q4_0", False, 250, 31)])
+def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
+    m = H.Model(shape, seed=rows, maxSeq=pos0 + rows + 3, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
+    toks = m.prompt(pos0 + rows + 1)
+    ref = np.empty(shape.vocab, np.float32)
+    for pos in range(pos0 + rows):
+        last = pos == pos0 + rows - 1
+        rc, nref = m.hip.DecodeToken(int(toks[pos]), pos, ref if last else None)
+        assert rc == 0, E.last_error()
+    after = np.empty(shape.vocab, np.float32)               # one more token: reads every K/V row
+    rc, _ = m.hip.DecodeToken(int(toks[-1]), pos0 + rows, after)
+    assert rc == 0
+    assert m.hip.ResetKV() == 0
+    for pos in range(pos0):
+        rc, _ = m.hip.DecodeToken(int(toks[pos]), pos)
+        assert rc == 0
+    rc, nxt, logits, _ = m.hip.Prefill(toks[pos0:pos0 + rows], pos0, wantLogits=True)
+    assert rc == 0, E.last_error()
+    bar = 1e-3 if kv_f16 else 1e-4
+    assert H.rel_err(logits, ref) < bar and nxt == nref
+    got = np.empty(shape.vocab, np.float32)
+    rc, _ = m.hip.DecodeToken(int(toks[-1]), pos0 + rows, got)
+    assert rc == 0 and H.rel_err(got, after) < bar
+    m.close()
+
+
+@pytest.mark.parametrize("rows,n,k,accumulate", [(1, 16, 32, 0), (17, 33, 96, 1), (64, 300, 1056, 0), (77, 129, 2080, 1), (130, 1000, 4864, 0),
+                                                 (513, 2900, 64, 0), (48, 9000, 64, 0), (300, 5632, 160, 1)])
+def test_few_row_gemm_matches_float64(hip, rows, n, k, accumulate):
+    rng = np.random.default_rng(rows)
+    a = rng.standard_normal((rows, k), dtype=np.float32)
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    sc = (0.01 * (1 + rng.random(n))).astype(np.float32)
+    bias = rng.standard_normal(n, dtype=np.float32)
+    y0 = rng.standard_normal((rows, n), dtype=np.float32)
+    ref = a.astype(np.float64) @ (w.astype(np.float64) * sc[:, None]).T + bias + (y0 if accumulate else 0)
+    ts = [hip.FromHost(a, a.shape), hip.UploadRawBytes(w), hip.FromHost(sc, sc.shape), hip.FromHost(bias, bias.shape), hip.FromHost(y0, y0.shape)]
+    nbytes = 4 * ((rows + 127) // 128 * 128) * ((k + 63) // 64 * 64)
+    ws = hip.UploadRawBytes(np.full(nbytes, 0xff, np.uint8))            # padding rows of the planes read as NaN
+    E.KQ8Gemm(ts[0], ts[1], ts[2], ts[3], ts[4], rows, n, k, accumulate, ws, nbytes)
+    E.KSync()
+    assert E.HIPCheck() == 0
+    assert H.rel_err(hip.ToHost(ts[4]).reshape(rows, n), ref) < 3e-5
+    for t in ts + [ws]:
+        t.Release()
