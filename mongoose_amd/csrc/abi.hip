@@ -4,6 +4,7 @@
 #include "../../include/mongoose_hip.h"
 #include "kernels.h"
 #include "prefill.h"
+#include "few_rows.h"
 #include "fused_infer.h"
 
 #include <atomic>
@@ -219,20 +220,38 @@ void mongoose_dequant_q8_rowscale(const void* w, const float* scales, float* out
 void mongoose_dequant_q4_0(const void* w, float* out, int rows, int cols, void* stream) {
     note(mg::launch_dequant_q4_0(w, out, rows, cols, S(stream)));
 }
+// The two launches of the multi-row product: the activations' split into the planes at `ws` (`plane` bytes each), the
+// product.  The few-row kernel serves up to 512 rows, more where the matrix is narrow: the tiled kernel has no room for K
+// splits here and leaves most CUs idle until N / 128 x T / 64 tiles fill them.  Microseconds a call, few-row / tiled:
+// 5632 x 2048 14 / 38 at 77 rows, 43 / 53 at 450, 70 / 66 at 800; 896 x 4864 13 / 78 at 77, 77 / 84 at 1500; 9000 x 8192
+// 53 / 129 at 77, 204 / 236 at 450, 276 / 254 at 600.
+static hipError_t q8_gemm_launches(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
+                                   int K, int accumulate, void* ws, size_t plane, hipStream_t s) {
+    void* hi = ws;
+    void* lo = static_cast<char*>(ws) + plane;
+    if (T > 0 && N > 0 && (T <= 512 || (long long)T * N <= 1500000) && aligned16(act)) {
+        hipError_t e = mg::launch_few_split(act, static_cast<unsigned short*>(hi), static_cast<unsigned short*>(lo), T, K, 0, s);
+        if (e != hipSuccess) return e;
+        mg::FewParams f{};
+        f.seg[0] = mg::FewSeg{static_cast<const signed char*>(w), scales, bias, out, N};
+        f.T = T; f.K = K; f.accumulate = accumulate;
+        f.Ahi = static_cast<const unsigned short*>(hi); f.Alo = static_cast<const unsigned short*>(lo);
+        return mg::launch_few_rows(mg::FEW_STORE, f, s);
+    }
+    hipError_t e = mg::launch_split_rows(act, nullptr, 0.f, T, K, hi, lo, s);
+    if (e != hipSuccess || T == 0 || N == 0) return e;
+    mg::GemmParams g{};
+    g.seg[0] = mg::GemmSeg{static_cast<const signed char*>(w), scales, bias, out, N, 0};
+    g.nseg = 1; g.T = T; g.K = K;
+    g.Ahi = static_cast<const unsigned short*>(hi); g.Alo = static_cast<const unsigned short*>(lo);
+    return mg::launch_gemm_q8(g, accumulate, s);
+}
 void mongoose_q8_gemm(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
                       int K, int accumulate, void* workspace, size_t workspaceBytes, void* stream) {
     const size_t plane = mg::split_plane_elems(T, K > 0 ? K : 64) * 2;     // a multiple of 16 KB
     if (T < 0 || N < 0 || K <= 0 || K % 32 != 0 || !workspace || workspaceBytes < 2 * plane ||
         ((uintptr_t)workspace & 15) || ((uintptr_t)w & 15)) { note(hipErrorInvalidValue); return; }
-    void* hi = workspace;
-    void* lo = static_cast<char*>(workspace) + plane;
-    note(mg::launch_split_rows(act, nullptr, 0.f, T, K, hi, lo, S(stream)));
-    if (T == 0 || N == 0) return;
-    mg::GemmParams g{};
-    g.seg[0] = mg::GemmSeg{static_cast<const signed char*>(w), scales, bias, out, N, 0};
-    g.nseg = 1; g.T = T; g.K = K;
-    g.Ahi = static_cast<const unsigned short*>(hi); g.Alo = static_cast<const unsigned short*>(lo);
-    note(mg::launch_gemm_q8(g, accumulate, S(stream)));
+    note(q8_gemm_launches(act, w, scales, bias, out, T, N, K, accumulate, workspace, plane, S(stream)));
 }
 // mongoose_q8_gemm with the split planes in the library's static scratch array: no allocation of any
 // kind on this path (no hipMalloc / hipFree, no workspace from the caller).
@@ -257,16 +276,7 @@ int mg_q8_gemm_noalloc(const float* act, const void* w, const float* scales, con
         (void)hipGetLastError();
         return MG_E_HIP;
     }
-    void* hi = base;
-    void* lo = static_cast<char*>(base) + plane;
-    e = mg::launch_split_rows(act, nullptr, 0.f, T, K, hi, lo, S(stream));
-    if (e == hipSuccess) {
-        mg::GemmParams g{};
-        g.seg[0] = mg::GemmSeg{static_cast<const signed char*>(w), scales, bias, out, N, 0};
-        g.nseg = 1; g.T = T; g.K = K;
-        g.Ahi = static_cast<const unsigned short*>(hi); g.Alo = static_cast<const unsigned short*>(lo);
-        e = mg::launch_gemm_q8(g, accumulate, S(stream));
-    }
+    e = q8_gemm_launches(act, w, scales, bias, out, T, N, K, accumulate, base, plane, S(stream));
     if (e != hipSuccess) {
         mg::set_error(std::string("mg_q8_gemm_noalloc: launch failed: ") + hipGetErrorString(e));
         (void)hipGetLastError();
