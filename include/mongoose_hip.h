@@ -267,9 +267,10 @@ int mg_hidden_idx(mg_ctx* ctx);
  * 4 = mode 3 with every workgroup computing (bit-identical results; for comparison).
  * A new context is in mode 3 (measured against mode 1: 0.5B shape 56 % more tokens per second, 1.1B
  * shape 59 %, 8B shape 20 %, also at contexts of thousands of positions).
- * The persistent launches of several contexts on one device take turns (two at once could each hold part of the
- * CUs and wait for workgroups that cannot start): one queued behind another context's waits on the device for
- * what that context has queued so far.
+ * On every device one context at a time owns the persistent launch -- the first that needs it, until it is
+ * destroyed or set to another mode (mg_flow_in_use).  Other contexts' launches take turns with the owner's (two at
+ * once could each hold part of the CUs and wait for workgroups that cannot start): one queued behind another
+ * context's waits on the device for what that context has queued so far.
  * The persistent launch needs all its workgroups resident at once: on a GPU shared with
  * other kernels its waits can run into their time limit; the call then returns MG_E_HIP,
  * and the context continues with the fused launches.  All modes give the same results to
@@ -389,7 +390,8 @@ int mg_bench_matvec(int wf, int N, int K, int nr, int ks, int grid, int copies, 
 int mg_flow_exchange(mg_ctx* ctx, int layer, float* out, size_t cap, int* geo);
 
 /* 1 when a step over all layers goes through the persistent launch of exec mode 3 (mode, model and
- * context as they are now), else 0. */
+ * context as they are now) and this context owns it, else 0 (mg_flow_tail_in_use and mg_flow_trace do not
+ * ask for the owner). */
 int mg_flow_in_use(mg_ctx* ctx);
 
 /* Timing diagnostic of exec mode 3: with enable != 0 every persistent launch records, per layer and

@@ -36,7 +36,8 @@ struct FlowTail {
     const float* cosTab; const float* sinTab;    // [maxSeq, headDim/2]
     StepState* state;            // read at the start (pos, token, count, nPrompt), written at the end of the launch
     int* history;                // greedy tokens go to history[count ..]
-    const int* prompt;           // while pos + 1 < nPrompt the next token is prompt[pos + 1] (optional)
+    const int* prompt;           // while pos + 1 < nPrompt the next token is prompt[pos + 1]; such a position's logits, argmax and
+                                 // history entry are left out
     float* amax;                 // argmax exchange: [2][grid] slots of FLOW_AMAX_STRIDE floats (value, index, rest unused),
                                  // part of the exchange allocation
     float* ropeCur;              // cos then sin row of the position after the launch (optional)
@@ -79,6 +80,8 @@ struct FlowParams {
     float eps;
     const StepState* state;      // position source (NULL -> posImm)
     int posImm;
+    int tokImm, nPromptImm;      // token mode, tokImm >= 0: position, token and prompt length come with the launch (posImm, these; no
+                                 // tokens emitted yet) instead of from the device state
     const float* cosRow;         // cos / sin row of the position [headDim/2]
     const float* sinRow;
     float* hidden;               // input of layer l0 and output of layer l1-1 [dim]
@@ -112,12 +115,13 @@ bool flow_grid_fits(int ffn, int nHeads, const FlowGeometry& g, int nCompute);
 // grid - p.nCompute of them prefetch (0, or a multiple of 8 with nCompute a multiple of 8 as well).
 hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s);
 // Fills the blocks of layers [l0, l1) (of the first half) with the "not written yet" pattern.
-hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, hipStream_t s);
+// hiddenIn != NULL: also dim floats of (page-locked host) memory into hidden.
+hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, const float* hiddenIn, float* hidden, int dim, hipStream_t s);
 // Floats of the whole exchange allocation: two halves of nLayers blocks (token mode alternates between them; launches
 // over a range of layers use the first) and the argmax exchange [2][grid] pairs behind them.
 size_t flow_xchg_floats(const FlowGeometry& g, int nLayers, int grid);
 inline float* flow_amax_area(float* xchg, const FlowGeometry& g, int nLayers) { return xchg + (size_t)2 * nLayers * g.stride; }
-// ... all of it (before the first token-mode launch after the position was set by the host).
+// ... all of it (before a token-mode launch that does not find its half as another left it).
 hipError_t launch_flow_reset_all(float* xchg, const FlowGeometry& g, int nLayers, int grid, hipStream_t s);
 // LDS a workgroup of the launch takes (an upper bound: dynamic part plus the variant's own arrays); token mode keeps
 // the token's embedding beside the staged vector.  Must stay within the CU's 160 KB.

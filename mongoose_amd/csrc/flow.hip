@@ -691,9 +691,12 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     const bool tokens = (FIX & 16) ? true : p.nTokens > 0;
     const int nTok = tokens ? p.nTokens : 1;
     const unsigned tw = tokens ? tail_words(p.tail, lane) : 0u;
-    int pos = p.state ? p.state->pos : p.posImm;
-    int tok = tokens ? p.state->token : 0;
-    const int count0 = tokens ? p.state->count : 0, nPrompt = tokens ? p.state->nPrompt : 0;
+    const bool imm = tokens && p.tokImm >= 0;
+    int pos = p.state && !imm ? p.state->pos : p.posImm;
+    int tok = imm ? p.tokImm : (tokens ? p.state->token : 0);
+    const int nPrompt = imm ? p.nPromptImm : (tokens ? p.state->nPrompt : 0);
+    // the token chosen at position np - 1 is entry hist0 + np of the history (np >= nPrompt)
+    const int hist0 = (tokens && !imm ? p.state->count : 0) - max(pos + 1, nPrompt);
     const size_t halfFloats = (size_t)p.nLayersTotal * G.stride;
     float* const xemb = reinterpret_cast<float*>(a4) + (dim > ffn ? dim : ffn);      // the token's embedding (token mode)
     for (int tk = 0; tk < nTok; tk++) {
@@ -1554,6 +1557,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
             int4 ring[RDT][NRT][CBT];
             float scl[RDT];
             const int nItemsAll = (vocab + NRT - 1) / NRT;
+            // (A position whose successor the prompt already has: no logits.  The exchange below stays, for the order it keeps.)
+            const bool head = np >= nPrompt;
             float bestV = -INFINITY;
             int bestI = INT_MAX;
             float acc[NRT];
@@ -1607,7 +1612,9 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
             // (256 waves) made the phase 15 us longer, eight an XCD brought the last workgroup 1.5 us closer to the median
             // and still cost 1.7 % of the step against this static mapping (0.3481 against 0.3422 ms).
             const int nb = (nchD + 64 * CBT - 1) / (64 * CBT);
-            if constexpr (RING) {
+            if (!head) {
+                resetOther();
+            } else if constexpr (RING) {
                 // Rows of more than 2048 weights (8B shape: 100 us of lm_head): the items of a workgroup -- its waves' first,
                 // second, ... items by the mapping above, numbered q = 8 round + slot -- are handed to its waves as they fall
                 // free, from a counter in LDS, after the two that every wave requests before the input is waited for.  The
@@ -1729,7 +1736,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
             const int* prompt = TW_PTR(const int, prompt);
             if (blockIdx.x == 0 && tid == 0) {
                 int* history = TW_PTR(int, history);
-                if (history && count0 + tk < TW_INT(historyCap)) history[count0 + tk] = ti;
+                const int h = hist0 + np;
+                if (history && head && h < TW_INT(historyCap)) history[h] = ti;
             }
             tok = (prompt && np < nPrompt) ? prompt[np] : ti;
             pos = np;
@@ -1746,7 +1754,11 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                 rc[half + j] = TW_PTR(const float, sinTab)[(size_t)pr * half + j];
             }
         }
-        if (tid == 0) { stw->pos = pos; stw->token = tok; stw->count = count0 + nTok; }
+        if (tid == 0) {
+            // (hist0 + pos + 1 tokens emitted, counted from the entry before the prompt's last position)
+            const int before = imm ? 0 : stw->count;
+            stw->pos = pos; stw->token = tok; stw->count = max(before, hist0 + pos + 1); stw->nPrompt = nPrompt;
+        }
     }
 }
 
@@ -1865,17 +1877,19 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
     return hipGetLastError();
 }
 
-__global__ void flow_reset_kernel(uint4* x, size_t n4) {
+__global__ void flow_reset_kernel(uint4* x, size_t n4, const float* hiddenIn, float* hidden, int dim) {
+    if (hiddenIn && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < dim; i += blockDim.x) hidden[i] = hiddenIn[i];
     const uint4 sent = make_uint4(XSENT, XSENT, XSENT, XSENT);
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) x[i] = sent;
 }
-hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, hipStream_t s) {
+hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, const float* hiddenIn, float* hidden, int dim, hipStream_t s) {
     if (l1 <= l0) return hipSuccess;
     const size_t n4 = (size_t)(l1 - l0) * g.stride / 4;
     size_t blocks = (n4 + WG - 1) / WG;
     if (blocks > 1024) blocks = 1024;
     hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s,
-                       reinterpret_cast<uint4*>(xchg + (size_t)l0 * g.stride), n4);
+                       reinterpret_cast<uint4*>(xchg + (size_t)l0 * g.stride), n4, hiddenIn, hidden, dim);
     return hipGetLastError();
 }
 
@@ -1886,7 +1900,8 @@ hipError_t launch_flow_reset_all(float* xchg, const FlowGeometry& g, int nLayers
     const size_t n4 = flow_xchg_floats(g, nLayers, grid) / 4;
     size_t blocks = (n4 + WG - 1) / WG;
     if (blocks > 1024) blocks = 1024;
-    hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s, reinterpret_cast<uint4*>(xchg), n4);
+    hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s, reinterpret_cast<uint4*>(xchg), n4,
+                       static_cast<const float*>(nullptr), static_cast<float*>(nullptr), 0);
     return hipGetLastError();
 }
 size_t flow_lds_bytes(int dim, int ffn, int headDim, int gqa, bool tokenMode) {

@@ -102,6 +102,7 @@ public:
         if (mode == 3 || mode == 4) flowBroken = false;      // asked for again by name: a wait that ran out earlier no longer bars it
         execMode = mode;
         if (mode != 0) q4ActQuant = false;      // only the op-by-op loop has the integer matvecs
+        if (mode != 3 && mode != 4) disownFlow();
     }
     void flowRegeometry();
     // Persistent launches of several contexts on one device take turns (fused_infer.hip).
@@ -146,7 +147,7 @@ private:
     int prefillCap = 0;             // rows the prefill buffers hold
     int prefillKVCap = 0;           // cache rows the attention's split planes hold
     void* pfKVSplit = nullptr;
-    int* pfTokens = nullptr;
+    const int* pfTokens = nullptr;
     float *pfX = nullptr, *pfQ = nullptr, *pfK = nullptr, *pfV = nullptr, *pfGate = nullptr, *pfUp = nullptr;
     void *pfHi = nullptr, *pfLo = nullptr, *pfHi2 = nullptr, *pfLo2 = nullptr;
     float* pfPartial = nullptr;
@@ -192,7 +193,8 @@ public:
     void LayerGraphDestroy(LayerGraph& lg);
     int UploadHidden(const float* data);                   // cuda_graph.go:650
     int ValidateGraphCapture(const float* hiddenIn, int layerStart, int layerEnd, float* maxDiff);   // :554-598
-    bool FlowInUse() const { return flowEligible(0, nLayers); }
+    bool FlowInUse() const;                                // goes through the persistent launch, as its owner on this device
+    void disownFlow() const;
     long long flowLimitTicks = 5000000;       // per wait of the persistent launch: 50 ms of the 100 MHz wall clock
     void SetFlowWaitLimit(long long ticks) { invalidateGraphs(); flowLimitTicks = ticks; }
     int statePosHost = -1;                    // the device state's position where the host knows it (set with the state, advanced
@@ -219,7 +221,14 @@ private:
     bool flowEligible(int l0, int l1) const;
     bool flowTailEligible() const;
     FlowTail* dFlowTail = nullptr;
-    int enqueueTokensFlow(int nTokens);
+    int enqueueTokensFlow(int nTokens, int pos = 0, int token = -1, int nPrompt = 0);
+    int flowClean = 0;              // halves of the exchange area known to be as a reset leaves them (bits 0 and 1)
+    int publish(const float* src, int n, const int* ints, int nInts);      // results on their way to hOut
+    int collect(float* out, int n, int* ints, int nInts);                  // ... waited for and copied to the caller
+    unsigned* hOut = nullptr;       // pinned: error word, flags of the slices from word 64, ints and floats at the offsets below
+    int hOutInts = 0, hOutFloats = 0;
+    unsigned hOutSeq = 0;
+    unsigned* hIn = nullptr;        // pinned: a call's tokens or hidden state on their way in
     int decodeRun(int nTokens, bool useGraph);      // nTokens decode steps from the device state
     bool runsInLaunch(bool useGraph) const;         // ... as runs of tokens inside the persistent launch
     int setState(int pos, int token, int count, int nPrompt);
@@ -227,7 +236,8 @@ private:
     bool q4ActQuant = false;      // exec mode 0: Q4_0 matrices through the int8-activation matvecs
     void* q8Scratch = nullptr;    // (max(dim, ffnDim)/32)*40 bytes of activation blocks (cuda_fused_infer.go:175-179)
     int ensureFlow();
-    int enqueueLayersFlow(int l0, int l1, const StepState* st, int posImm, bool resetFirst, int nTokens = 0);
+    int enqueueLayersFlow(int l0, int l1, const StepState* st, int posImm, bool resetFirst, int nTokens = 0, int tokImm = -1,
+                          int nPromptImm = 0, const float* hiddenIn = nullptr);
     int checkFlowError();
     int enqueueToken(bool withHead);      // embed -> layers -> final(+argmax) / advance, all from device state
 
@@ -253,7 +263,6 @@ private:
     int amaxParts = 0;
     int* dHistory = nullptr;
     int* dPrompt = nullptr;
-    int* hTokens = nullptr;         // pinned
     bool graphsUseFlow = false;       // the whole-token graphs were captured with the persistent layer launch
     unsigned graphGeneration = 0;     // bumped by whatever makes captured graphs stale (weights, caches, modes)
     hipGraph_t graphFull = nullptr, graphPrompt = nullptr;

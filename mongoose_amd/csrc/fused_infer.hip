@@ -153,8 +153,15 @@ HIPFusedInference* HIPFusedInference::New(int dim, int kvDim, int headDim, int n
     if (hipHostMalloc(&hp, 64, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) return fail("pinned alloc");
     f->hGate = static_cast<int*>(hp);
     *f->hGate = 1;
-    if (hipHostMalloc(&hp, sizeof(int) * ((size_t)maxSeq + 1), hipHostMallocDefault) != hipSuccess) return fail("pinned alloc");
-    f->hTokens = static_cast<int*>(hp);
+    // what calls hand over and take in: flags, error word, token ids, floats out; words in
+    f->hOutInts = 64 + 16 * PUBLISH_MAX_SLICES;
+    f->hOutFloats = (f->hOutInts + maxSeq + 1 + 63) / 64 * 64;
+    const size_t outWords = (size_t)f->hOutFloats + std::max(vocabSize, dim), inWords = (size_t)std::max(maxSeq, dim);
+    if (hipHostMalloc(&hp, outWords * 4, hipHostMallocDefault) != hipSuccess) return fail("pinned alloc");
+    f->hOut = static_cast<unsigned*>(hp);
+    std::memset(f->hOut, 0, (size_t)f->hOutInts * 4);
+    if (hipHostMalloc(&hp, inWords * 4, hipHostMallocDefault) != hipSuccess) return fail("pinned alloc");
+    f->hIn = static_cast<unsigned*>(hp);
 
     f->built = true;
     return f;
@@ -214,7 +221,8 @@ HIPFusedInference::~HIPFusedInference() {
     if (hFlowErr) (void)hipHostFree(hFlowErr);
     if (hState) (void)hipHostFree(hState);
     if (hGate) (void)hipHostFree(hGate);
-    if (hTokens) (void)hipHostFree(hTokens);
+    if (hOut) (void)hipHostFree(hOut);
+    if (hIn) (void)hipHostFree(hIn);
     for (hipEvent_t e : profEvents) (void)hipEventDestroy(e);
     if (copyStream) { (void)hipStreamSynchronize(copyStream); (void)hipStreamDestroy(copyStream); }
     if (computeDone) (void)hipEventDestroy(computeDone);
@@ -644,7 +652,9 @@ int HIPFusedInference::enqueueLayerFused(const LayerWeights& L, int layer, const
 // queued (an event recorded there only when the launch changes hands: a context that is alone on its device records and
 // waits for nothing).  The lock is held for the submission only.  Measured with three 0.5B contexts whose decode runs
 // alternate: 38.5 -> 24.1 ms a run of 16 + 64 tokens, where two of the three used the fused launches before.
-static struct FlowTurns { std::mutex m; HIPFusedInference* last = nullptr; } g_flowTurns[64];
+// One of the contexts owns the device's launch -- the first that asks, until it is destroyed, set to another mode or has
+// had a wait run out; what that means is only what FlowInUse reports, the others' launches take their turns all the same.
+static struct FlowTurns { std::mutex m; HIPFusedInference* last = nullptr; const HIPFusedInference* owner = nullptr; } g_flowTurns[64];
 
 int HIPFusedInference::takeFlowTurn() {
     HIPFusedInference*& last = g_flowTurns[flowDevice].last;
@@ -662,6 +672,7 @@ int HIPFusedInference::launchFlowGraph(hipGraphExec_t ex) {
     std::lock_guard<std::mutex> lk(flowTurnMutex());
     int rc = takeFlowTurn();
     if (rc) return rc;
+    flowClean = 0;                                  // (whatever the captured launches leave)
     HIPCHK(hipGraphLaunch(ex, stream));
     return MG_OK;
 }
@@ -672,8 +683,25 @@ int HIPFusedInference::launchTokenGraph(hipGraphExec_t ex) {
     return MG_OK;
 }
 
+bool HIPFusedInference::FlowInUse() const {
+    int dev = 0;
+    if (!flowEligible(0, nLayers)) return false;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { (void)hipGetLastError(); return false; }
+    FlowTurns& t = g_flowTurns[dev];
+    std::lock_guard<std::mutex> lk(t.m);
+    if (!t.owner) t.owner = this;
+    return t.owner == this;
+}
+void HIPFusedInference::disownFlow() const {
+    for (FlowTurns& t : g_flowTurns) {
+        std::lock_guard<std::mutex> lk(t.m);
+        if (t.owner == this) t.owner = nullptr;
+    }
+}
+
 // The context is about to go: nobody may wait for its stream any more.
 void HIPFusedInference::leaveFlowTurns() {
+    disownFlow();
     if (!flowTurnEvent) return;
     std::lock_guard<std::mutex> lk(flowTurnMutex());
     if (g_flowTurns[flowDevice].last == this) {
@@ -774,6 +802,7 @@ int HIPFusedInference::ensureFlow() {
         HIPCHK(hipMalloc(&v, sizeof(float) * flow_xchg_floats(flowGeo, nLayers, flowGrid)));
         flowXchg = static_cast<float*>(v);
         HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
+        flowClean = 3;
         HIPCHK(hipMalloc(&v, sizeof(FlowTail)));
         dFlowTail = static_cast<FlowTail*>(v);
         HIPCHK(hipMalloc(&v, FLOW_ERR_BYTES));
@@ -870,7 +899,8 @@ int HIPFusedInference::FlowTailTrace(long long* out, size_t cap, int* dims) {
     return MG_OK;
 }
 
-int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, int posImm, bool resetFirst, int nTokens) {
+int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, int posImm, bool resetFirst, int nTokens, int tokImm,
+                                         int nPromptImm, const float* hiddenIn) {
     if (l1 > nLayers) l1 = nLayers;
     FlowParams p{};
     p.layers = dFlowLayers; p.l0 = l0; p.l1 = l1; p.nLayersTotal = nLayers;
@@ -893,6 +923,8 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
     }
     p.eps = eps;
     p.state = st; p.posImm = posImm;
+    p.tokImm = tokImm; p.nPromptImm = nPromptImm;
+    if (tokImm >= 0) statePosHost = posImm;
     const int half = headDim / 2;
     p.cosRow = st ? ropeCur : cosTab + (size_t)posImm * half;
     p.sinRow = st ? ropeCur + half : sinTab + (size_t)posImm * half;
@@ -908,12 +940,21 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
         else if (statePosHost >= 0) posMax = (long long)statePosHost + (nTokens > 0 ? nTokens - 1 : 0);
         p.gqaCode = (posMax < 0 || (long long)nHeads * (posMax / FLOW_TILE + 1) > flowCompute) ? 1 : 0;
         p.generic = flowGeneric ? 1 : 0;
+        // the half of the exchange area a run of whole tokens starts in has to be as a reset leaves it: the launch before
+        // left the half of its last position's successor so (DecodeToken at consecutive positions resets nothing)
+        if (nTokens > 0 && !capturing) {
+            const int need = statePosHost >= 0 ? 1 << (statePosHost & 1) : 3;
+            if ((flowClean & need) != need) HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
+            flowClean = statePosHost >= 0 ? 1 << ((statePosHost + nTokens) & 1) : 0;
+        } else {
+            flowClean &= ~1;                                                          // (layers only: the first half)
+        }
         if (st && nTokens > 0 && statePosHost >= 0) statePosHost += nTokens;          // whole tokens advance the device state
         else if (st) statePosHost = -1;                                               // (what follows this launch advances it)
     }
     p.trace = flowTrace;
     if (nTokens > 0) { p.nTokens = nTokens; p.tail = dFlowTail; }
-    if (resetFirst) HIPCHK(launch_flow_reset(flowXchg, flowGeo, l0, l1, stream));
+    if (resetFirst) HIPCHK(launch_flow_reset(flowXchg, flowGeo, l0, l1, hiddenIn, hidden[hiddenIdx], dim, stream));
     if (mark(1)) return MG_E_HIP;
     if (capturing) { HIPCHK(launch_flow_layers(p, flowGrid, stream)); return MG_OK; }      // (the replay takes the turn)
     std::lock_guard<std::mutex> lk(flowTurnMutex());
@@ -923,11 +964,10 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
     return MG_OK;
 }
 
-// nTokens whole tokens from the device state in one launch: embedding, layers, final norm, lm_head, argmax; the
-// exchange area must be in its reset state for the first token's position (setState), the launch leaves it so for
-// the position after its last.
-int HIPFusedInference::enqueueTokensFlow(int nTokens) {
-    return enqueueLayersFlow(0, nLayers, dState, 0, false, nTokens);
+// nTokens whole tokens in one launch -- embedding, layers, final norm, lm_head, argmax -- from the device state, or (token
+// >= 0) from position pos and that token, nothing emitted yet; below nPrompt the tokens come from dPrompt.
+int HIPFusedInference::enqueueTokensFlow(int nTokens, int pos, int token, int nPrompt) {
+    return enqueueLayersFlow(0, nLayers, dState, pos, false, nTokens, token, nPrompt);
 }
 
 // Whole tokens in the launch need: the tail's operands set, the lm_head in the layers' format, room in LDS for the
@@ -953,8 +993,47 @@ int HIPFusedInference::SetTokensPerLaunch(int n) {
 int HIPFusedInference::setState(int pos, int token, int count, int nPrompt) {
     HIPCHK(launch_set_state(dState, pos, token, count, nPrompt, ropeRef(), stream));
     statePosHost = pos;
-    if (flowXchg && (execMode == 3 || execMode == 4)) HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
+    if (flowXchg && (execMode == 3 || execMode == 4)) {
+        HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
+        flowClean = 3;
+    }
     return MG_OK;
+}
+
+// ---- what a call hands to its caller ----
+// Queues n floats of src, nInts ints and the persistent launch's error word behind everything queued so far; collect()
+// waits for them.  One small launch writes them to page-locked memory and the host watches for its flags: a synchronous
+// copy each of logits, token and error word, behind a stream synchronisation, cost 125 us a token of the 1.1B shape.
+int HIPFusedInference::publish(const float* src, int n, const int* ints, int nInts) {
+    PublishParams p{};
+    p.src = src; p.dst = reinterpret_cast<float*>(hOut + hOutFloats); p.n = n;
+    p.ints = ints; p.intDst = reinterpret_cast<int*>(hOut + hOutInts); p.nInts = nInts;
+    p.err = dFlowErr; p.errDst = reinterpret_cast<int*>(hOut);
+    p.flags = hOut + 64; p.seq = ++hOutSeq;
+    HIPCHK(launch_publish(p, stream));
+    return MG_OK;
+}
+
+int HIPFusedInference::collect(float* out, int n, int* ints, int nInts) {
+    const int per = publish_slice_floats(n), slices = publish_slices(n);
+    const auto t0 = std::chrono::steady_clock::now();
+    bool waited = false;
+    for (int b = 0; b < slices; b++) {
+        const unsigned* flag = hOut + 64 + 16 * b;
+        for (unsigned spins = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != hOutSeq; spins++) {
+            __builtin_ia32_pause();
+            // (a run of many tokens: leave the waiting to the runtime after a while; it also reports a launch that failed)
+            if (spins % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+                if (waited) { set_error("a queued launch did not deliver its results"); return MG_E_HIP; }
+                HIPCHK(hipStreamSynchronize(stream));
+                waited = true;
+            }
+        }
+        const int i0 = b * per, i1 = std::min(n, i0 + per);
+        if (out && i1 > i0) std::memcpy(out + i0, hOut + hOutFloats + i0, (size_t)(i1 - i0) * 4);
+    }
+    if (ints && nInts) std::memcpy(ints, hOut + hOutInts, (size_t)nInts * 4);
+    return hOut[0] ? checkFlowError() : MG_OK;
 }
 
 // nTokens decode steps from the device state: runs of tokens inside the persistent launch where that is in use, else
@@ -988,9 +1067,11 @@ int HIPFusedInference::checkFlowError() {
     if (*hFlowErr == 0) return MG_OK;
     const int code = *hFlowErr;
     *hFlowErr = 0;
+    flowClean = 0;
     HIPCHK(hipMemsetAsync(dFlowErr, 0, sizeof(int), stream));
     HIPCHK(hipStreamSynchronize(stream));
     flowBroken = true;
+    disownFlow();
     invalidateGraphs();
     if (code == 3)
         set_error("persistent layer launch: the variant without grouped attention was given a position it does not cover; "
@@ -1058,43 +1139,37 @@ int HIPFusedInference::PartialStep(const float* hiddenIn, int pos, int layerStar
     ARGCHK(pos >= 0 && pos < maxSeq, "PartialStep: pos out of range");
     ARGCHK(layerStart >= 0, "PartialStep: negative layerStart");
     float* h = hidden[hiddenIdx];
-    if (hiddenIn) {
-        HIPCHK(hipStreamSynchronize(stream));
-        HIPCHK(hipMemcpy(h, hiddenIn, (size_t)dim * 4, hipMemcpyHostToDevice));      // :395
-    }
     const bool flow = flowEligible(layerStart, layerEnd);
     if (flow) {
+        // (the launch that resets the exchange area also brings the hidden state in, from page-locked memory: every call
+        // of this path waits for its end, so the words of the call before have been read)
+        if (hiddenIn) std::memcpy(hIn, hiddenIn, (size_t)dim * 4);
         int rc = ensureFlow();
-        if (rc == 0) rc = enqueueLayersFlow(layerStart, layerEnd, nullptr, pos, true);
+        if (rc == 0) rc = enqueueLayersFlow(layerStart, layerEnd, nullptr, pos, true, 0, -1, 0, hiddenIn ? reinterpret_cast<const float*>(hIn) : nullptr);
         if (rc) return rc;
     } else {
+        if (hiddenIn) {
+            HIPCHK(hipStreamSynchronize(stream));
+            HIPCHK(hipMemcpy(h, hiddenIn, (size_t)dim * 4, hipMemcpyHostToDevice));   // :395
+        }
         for (int l = layerStart; l < layerEnd && l < nLayers; l++) {
             if (!layers[l].norm1) continue;                                           // :415
             int rc = enqueueLayer(layers[l], l, nullptr, pos);
             if (rc) return rc;
         }
     }
-    if (layerEnd >= nLayers && logitsOut && finalNorm) {                              // :446
+    const bool wantLogits = layerEnd >= nLayers && logitsOut && finalNorm;            // :446
+    const bool wantHidden = hiddenOut && layerEnd < nLayers;                          // :452
+    if (wantLogits) {
         int rc = enqueueFinal(false);
-        if (rc) return rc;
-        HIPCHK(hipStreamSynchronize(stream));
-        HIPCHK(hipMemcpy(logitsOut, logits, (size_t)vocabSize * 4, hipMemcpyDeviceToHost));
-        rc = checkFlowError();
-        if (rc) return rc;
-    }
-    if (hiddenOut && layerEnd < nLayers) {                                            // :452
-        HIPCHK(hipStreamSynchronize(stream));
-        HIPCHK(hipMemcpy(hiddenOut, h, (size_t)dim * 4, hipMemcpyDeviceToHost));
-        int rc = checkFlowError();
         if (rc) return rc;
     }
     // Nothing read back: the launches stay queued (the reference does not sync here either) -- except after a
     // persistent launch, whose waits may have run out: that is reported by the call whose step it spoiled.
-    if (flow && !(layerEnd >= nLayers && logitsOut && finalNorm) && !(hiddenOut && layerEnd < nLayers)) {
-        HIPCHK(hipStreamSynchronize(stream));
-        return checkFlowError();
-    }
-    return MG_OK;
+    if (!wantLogits && !wantHidden && !flow) return MG_OK;
+    const int n = wantLogits ? vocabSize : (wantHidden ? dim : 0);
+    int rc = publish(wantLogits ? logits : h, n, nullptr, 0);
+    return rc ? rc : collect(wantLogits ? logitsOut : hiddenOut, n, nullptr, 0);
 }
 
 // ---- L3 bridge and mailbox (cuda_fused_infer.go:556-737) ----
@@ -1239,7 +1314,7 @@ int HIPFusedInference::enqueueToken(bool withHead) {
     HIPCHK(launch_advance_prompt(dState, dPrompt, ropeRef(), embedRef(), stream));
     // no lm_head launch to leave the exchange area reset for the next launch: a captured prompt step does it itself,
     // and so does any prompt step where whole tokens run in the launch (they expect to find it so)
-    if (flow && (fuseEmbed || flowTailEligible())) HIPCHK(launch_flow_reset(flowXchg, flowGeo, 0, nLayers, stream));
+    if (flow && (fuseEmbed || flowTailEligible())) HIPCHK(launch_flow_reset(flowXchg, flowGeo, 0, nLayers, nullptr, nullptr, 0, stream));
     return MG_OK;
 }
 
@@ -1257,24 +1332,30 @@ int HIPFusedInference::DecodeToken(int token, int pos, int* nextToken, float* lo
     ARGCHK(pos >= 0 && pos < maxSeq && token >= 0 && token < vocabSize, "DecodeToken: token or pos out of range");
     int rc = checkReady(this);
     if (rc) return rc;
-    { int rcs = setState(pos, token, 0, 0); if (rcs) return rcs; }
-    if (execMode == 0) {
-        rc = enqueueEmbed();
-        if (rc) return rc;
-        for (int l = 0; l < nLayers; l++) {
-            rc = enqueueLayerPerOp(layers[l], l, pos);
-            if (rc) return rc;
-        }
-        rc = enqueueFinal(true);
+    if (execMode != 0 && flowTailEligible()) {      // the whole token is one launch, position and token in its arguments
+        rc = ensureFlow();
+        if (rc == 0) rc = enqueueTokensFlow(1, pos, token, 0);
     } else {
-        rc = enqueueToken(true);
+        { int rcs = setState(pos, token, 0, 0); if (rcs) return rcs; }
+        if (execMode == 0) {
+            rc = enqueueEmbed();
+            if (rc) return rc;
+            for (int l = 0; l < nLayers; l++) {
+                rc = enqueueLayerPerOp(layers[l], l, pos);
+                if (rc) return rc;
+            }
+            rc = enqueueFinal(true);
+        } else {
+            rc = enqueueToken(true);
+        }
     }
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(hTokens, dHistory, sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    if (nextToken) *nextToken = hTokens[0];
-    if (logitsOut) HIPCHK(hipMemcpy(logitsOut, logits, (size_t)vocabSize * 4, hipMemcpyDeviceToHost));
-    return checkFlowError();
+    const int n = logitsOut ? vocabSize : 0;
+    int next = 0;
+    rc = publish(logits, n, dHistory, 1);
+    if (rc == 0) rc = collect(logitsOut, n, &next, 1);
+    if (nextToken) *nextToken = next;
+    return rc;
 }
 
 int HIPFusedInference::GraphCapture() {
@@ -1411,10 +1492,11 @@ int HIPFusedInference::GraphLaunch(int token, int pos, int* nextToken) {
     statePosHost = -1;
     rc = launchTokenGraph(execFull);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(hTokens, dHistory, sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    if (nextToken) *nextToken = hTokens[0];
-    return checkFlowError();
+    int next = 0;
+    rc = publish(nullptr, 0, dHistory, 1);
+    if (rc == 0) rc = collect(nullptr, 0, &next, 1);
+    if (nextToken) *nextToken = next;
+    return rc;
 }
 
 int HIPFusedInference::GraphValidate(int token, int pos, float* maxAbsDiff) {
@@ -1455,24 +1537,32 @@ int HIPFusedInference::Generate(const int* prompt, int nPrompt, int nDecode, int
         }
         return MG_OK;
     }
-    // (where runs of tokens go into one launch no graph is needed: the prompt steps are launched one by one)
-    const bool graphs = useGraph && !runsInLaunch(useGraph);
-    if (graphs) { rc = GraphCapture(); if (rc) return rc; }
-    HIPCHK(hipStreamSynchronize(stream));
-    HIPCHK(hipMemcpy(dPrompt, prompt, sizeof(int) * (size_t)nPrompt, hipMemcpyHostToDevice));
-    { int rcs = setState(0, prompt[0], 0, nPrompt); if (rcs) return rcs; }
-    if (graphs) { rc = primeGraph(); if (rc) return rc; }
-    for (int i = 0; i < nPrompt - 1; i++) {
-        if (graphs) { rc = launchTokenGraph(execPrompt); if (rc) return rc; }
-        else { rc = enqueueToken(false); if (rc) return rc; }
+    std::memcpy(hIn, prompt, sizeof(int) * (size_t)nPrompt);        // (every call that uses hIn waits for its end)
+    HIPCHK(launch_take_words(hIn, reinterpret_cast<unsigned*>(dPrompt), nPrompt, stream));
+    if (runsInLaunch(useGraph)) {
+        // prompt positions and decoded ones alike are tokens of the launches
+        rc = ensureFlow();
+        int done = 0;
+        for (const int total = nPrompt - 1 + nDecode; done < total && rc == MG_OK;) {
+            const int n = std::min(tokensPerLaunch, total - done);
+            rc = done == 0 ? enqueueTokensFlow(n, 0, prompt[0], nPrompt) : enqueueTokensFlow(n);
+            done += n;
+        }
+        if (rc) return rc;
+    } else {
+        if (useGraph) { rc = GraphCapture(); if (rc) return rc; }
+        { int rcs = setState(0, prompt[0], 0, nPrompt); if (rcs) return rcs; }
+        if (useGraph) { rc = primeGraph(); if (rc) return rc; }
+        for (int i = 0; i < nPrompt - 1; i++) {
+            if (useGraph) { rc = launchTokenGraph(execPrompt); if (rc) return rc; }
+            else { rc = enqueueToken(false); if (rc) return rc; }
+        }
+        statePosHost = nPrompt - 1;                 // one position a prompt step since setState(0, ..)
+        rc = decodeRun(nDecode, useGraph);
+        if (rc) return rc;
     }
-    statePosHost = nPrompt - 1;                     // one position a prompt step since setState(0, ..)
-    rc = decodeRun(nDecode, useGraph);
-    if (rc) return rc;
-    if (nDecode > 0) HIPCHK(hipMemcpyAsync(hTokens, dHistory, sizeof(int) * (size_t)nDecode, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    for (int i = 0; i < nDecode; i++) outTokens[i] = hTokens[i];
-    return checkFlowError();
+    rc = publish(nullptr, 0, dHistory, nDecode);
+    return rc ? rc : collect(nullptr, 0, outTokens, nDecode);
 }
 
 int HIPFusedInference::TimedDecode(int token, int pos, int steps, bool useGraph, float* elapsedMs) {
@@ -1571,11 +1661,10 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     const size_t T = ((size_t)rows + 127) / 128 * 128;
     const size_t plane = split_plane_elems((int)T, ffnDim > dim ? ffnDim : dim) * 2;
     const size_t sums = (size_t)(dim / 16 + 1) * std::min<size_t>(T, (size_t)fewRowsLimit());
-    size_t bytes = alignUp256(sums * 4) + alignUp256(T * 4) + 2 * alignUp256(T * dim * 4) + 2 * alignUp256(T * kvDim * 4) +
+    size_t bytes = alignUp256(sums * 4) + 2 * alignUp256(T * dim * 4) + 2 * alignUp256(T * kvDim * 4) +
                    2 * alignUp256(T * ffnDim * 4) + 4 * alignUp256(plane) + alignUp256(gemm_partial_floats() * 4) + 16 * 256;
     int rc = prefillSlab.init(bytes);
     if (rc) return rc;
-    pfTokens = static_cast<int*>(prefillSlab.take(T * 4));
     pfSumSq = static_cast<float*>(prefillSlab.take(sums * 4));
     pfX = static_cast<float*>(prefillSlab.take(T * dim * 4));
     pfQ = static_cast<float*>(prefillSlab.take(T * dim * 4));
@@ -1588,7 +1677,7 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     pfHi2 = prefillSlab.take(plane);      // second pair: written by the gate|up GEMM's own epilogue while it still reads the first
     pfLo2 = prefillSlab.take(plane);
     pfPartial = static_cast<float*>(prefillSlab.take(gemm_partial_floats() * 4));
-    if (!pfTokens || !pfSumSq || !pfX || !pfQ || !pfK || !pfV || !pfGate || !pfUp || !pfHi || !pfLo || !pfHi2 || !pfLo2 || !pfPartial) {
+    if (!pfSumSq || !pfX || !pfQ || !pfK || !pfV || !pfGate || !pfUp || !pfHi || !pfLo || !pfHi2 || !pfLo2 || !pfPartial) {
         set_error("prefill slab too small");
         return MG_E_STATE;
     }
@@ -1714,23 +1803,27 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
     if (rc) return rc;
     const int T = nTokens;
     const bool few = T <= fewRowsLimit();
-    HIPCHK(hipStreamSynchronize(stream));
-    HIPCHK(hipMemcpy(pfTokens, tokens, sizeof(int) * (size_t)T, hipMemcpyHostToDevice));
-    HIPCHK(hipEventRecord(ev0, stream));
+    std::memcpy(hIn, tokens, sizeof(int) * (size_t)T);              // (the embedding rows' launch reads them there)
+    pfTokens = reinterpret_cast<const int*>(hIn);
+    if (elapsedMs) HIPCHK(hipEventRecord(ev0, stream));
     rc = few ? enqueuePrefillFew(T, pos0) : enqueuePrefillTiles(T, pos0);
     if (rc) return rc;
     // the last position continues on the decode path: final norm, lm_head, greedy token, state -> pos0 + T
-    HIPCHK(hipMemcpyAsync(hidden[hiddenIdx], pfX + (size_t)(T - 1) * dim, (size_t)dim * 4, hipMemcpyDeviceToDevice, stream));
-    { int rcs = setState(pos0 + T - 1, tokens[T - 1], 0, 0); if (rcs) return rcs; }
+    HIPCHK(launch_prefill_tail(pfX + (size_t)(T - 1) * dim, hidden[hiddenIdx], dim, dState, pos0 + T - 1, tokens[T - 1], ropeRef(), stream));
     rc = enqueueFinal(true);
     if (rc) return rc;
     statePosHost = pos0 + T;                        // where the argmax's last kernel leaves the state
-    HIPCHK(hipEventRecord(ev1, stream));
-    HIPCHK(hipMemcpyAsync(hTokens, dHistory, sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    if (nextToken) *nextToken = hTokens[0];
-    if (logitsOut) HIPCHK(hipMemcpy(logitsOut, logits, (size_t)vocabSize * 4, hipMemcpyDeviceToHost));
-    if (elapsedMs) HIPCHK(hipEventElapsedTime(elapsedMs, ev0, ev1));
+    if (elapsedMs) HIPCHK(hipEventRecord(ev1, stream));
+    const int n = logitsOut ? vocabSize : 0;
+    int next = 0;
+    rc = publish(logits, n, dHistory, 1);
+    if (rc == 0) rc = collect(logitsOut, n, &next, 1);
+    if (rc) return rc;
+    if (nextToken) *nextToken = next;
+    if (elapsedMs) {
+        HIPCHK(hipEventSynchronize(ev1));
+        HIPCHK(hipEventElapsedTime(elapsedMs, ev0, ev1));
+    }
     return MG_OK;
 }
 
@@ -1747,10 +1840,8 @@ int HIPFusedInference::GeneratePrefill(const int* prompt, int nPrompt, int nDeco
     if (nDecode > 1 && graphs) { rc = primeGraph(); if (rc) return rc; }
     rc = decodeRun(nDecode - 1, true);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(hTokens, dHistory, sizeof(int) * (size_t)nDecode, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    for (int i = 0; i < nDecode; i++) outTokens[i] = hTokens[i];
-    return checkFlowError();
+    rc = publish(nullptr, 0, dHistory, nDecode);
+    return rc ? rc : collect(nullptr, 0, outTokens, nDecode);
 }
 
 }  // namespace mg

@@ -169,6 +169,26 @@ hipError_t launch_advance_prompt(StepState* state, const int* prompt, RopeCur ro
 // host-visible memory once everything queued before it on the stream has finished.
 hipError_t launch_signal_mailbox(unsigned* counter, unsigned value, hipStream_t s);
 
+// What a call hands to its caller -> page-locked host memory, behind everything queued before it on the stream: n floats of
+// src in publish_slices(n) slices, nInts ints, the error word.  A
+// slice's flag (64 bytes apart) takes the value seq once the slice is in host memory, so the host copies one slice on
+// while the next one crosses the link; the ints and the error word are there with the first.  Host addresses are what
+// hipHostMalloc returned.
+struct PublishParams {
+    const float* src; float* dst; int n;
+    const int* ints; int* intDst; int nInts;
+    const int* err; int* errDst;             // err NULL: 0 is stored
+    unsigned* flags; unsigned seq;
+};
+constexpr int PUBLISH_MAX_SLICES = 32;
+inline int publish_slice_floats(int n) { const int per = (n + PUBLISH_MAX_SLICES - 1) / PUBLISH_MAX_SLICES; return per < 1024 ? 1024 : (per + 255) / 256 * 256; }
+inline int publish_slices(int n) { return n > 0 ? (n + publish_slice_floats(n) - 1) / publish_slice_floats(n) : 1; }
+hipError_t launch_publish(const PublishParams& p, hipStream_t s);
+// n words of page-locked host memory -> device memory.
+hipError_t launch_take_words(const unsigned* src, unsigned* dst, int n, hipStream_t s);
+// The last row of a prefill -> the hidden buffer, and the step state for its lm_head.
+hipError_t launch_prefill_tail(const float* row, float* hidden, int dim, StepState* state, int pos, int token, RopeCur rope, hipStream_t s);
+
 // Stream gate for timing runs: waits for *flag != 0 (host-pinned) or limitTicks of the 100 MHz wall clock.
 hipError_t launch_gate(const int* flag, long long limitTicks, hipStream_t s);
 

@@ -1691,6 +1691,49 @@ hipError_t launch_signal_mailbox(unsigned* counter, unsigned value, hipStream_t 
     return hipGetLastError();
 }
 
+__global__ __launch_bounds__(WG) void publish_kernel(PublishParams p, int per) {
+    const int b = blockIdx.x;
+    const int i0 = b * per, i1 = min(p.n, i0 + per);
+    const float4* s4 = reinterpret_cast<const float4*>(p.src + i0);
+    float4* d4 = reinterpret_cast<float4*>(p.dst + i0);
+    const int n4 = (i1 - i0) >> 2;
+    for (int i = threadIdx.x; i < n4; i += WG) d4[i] = s4[i];
+    for (int i = i0 + n4 * 4 + threadIdx.x; i < i1; i += WG) p.dst[i] = p.src[i];
+    if (b == 0) {
+        for (int i = threadIdx.x; i < p.nInts; i += WG) p.intDst[i] = p.ints[i];
+        if (threadIdx.x == 0) *p.errDst = p.err ? *p.err : 0;
+    }
+    __threadfence_system();                          // every thread's own stores have reached the host's memory
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(p.flags + b * 16, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+hipError_t launch_publish(const PublishParams& p, hipStream_t s) {
+    hipLaunchKernelGGL(publish_kernel, dim3((unsigned)publish_slices(p.n)), dim3(WG), 0, s, p, publish_slice_floats(p.n));
+    return hipGetLastError();
+}
+
+__global__ void take_words_kernel(const unsigned* src, unsigned* dst, int n) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[i] = src[i];
+}
+hipError_t launch_take_words(const unsigned* src, unsigned* dst, int n, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(take_words_kernel, dim3((unsigned)((n + WG - 1) / WG)), dim3(WG), 0, s, src, dst, n);
+    return hipGetLastError();
+}
+
+__global__ void prefill_tail_kernel(const float* row, float* hidden, int dim, StepState* state, int pos, int token, RopeCur rope) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < dim) hidden[i] = row[i];
+    if (blockIdx.x == 0) {
+        copy_rope_row(rope, pos);
+        if (threadIdx.x == 0) { state->pos = pos; state->token = token; state->count = 0; state->nPrompt = 0; }
+    }
+}
+hipError_t launch_prefill_tail(const float* row, float* hidden, int dim, StepState* state, int pos, int token, RopeCur rope, hipStream_t s) {
+    hipLaunchKernelGGL(prefill_tail_kernel, dim3((unsigned)((dim + WG - 1) / WG)), dim3(WG), 0, s, row, hidden, dim, state, pos, token, rope);
+    return hipGetLastError();
+}
+
 __global__ void gate_kernel(const volatile int* flag, long long limitTicks) {
     const long long t0 = wall_clock64();
     while (__hip_atomic_load(const_cast<const int*>(flag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0) {

@@ -31,7 +31,7 @@ def test_contexts_take_turns(hip, per_launch):
     for m, p in zip(ms, prompts):
         rc, t = m.hip.Generate(p, 60, useGraph=True)
         assert rc == 0, E.last_error()
-        assert m.hip.FlowInUse()
+        assert m.hip.FlowTailInUse()
         alone.append(t.copy())
     for _ in range(4):
         for m, p, a in zip(ms, prompts, alone):
@@ -52,7 +52,7 @@ def test_contexts_take_turns(hip, per_launch):
         assert len(g) == 6
         for rc, t in g:
             assert rc == 0 and (t == a).all()
-    assert all(m.hip.FlowInUse() for m in ms)
+    assert all(m.hip.FlowTailInUse() for m in ms) and [m.hip.FlowInUse() for m in ms] == [True, False, False]
     ms[1].close()                                            # one leaves, the others go on
     rc, t = ms[0].hip.Generate(prompts[0], 60, useGraph=True)
     assert rc == 0 and (np.asarray(t) == alone[0]).all()
