@@ -64,3 +64,21 @@ def test_few_row_gemm_matches_float64(hip, rows, n, k, accumulate):
     assert H.rel_err(hip.ToHost(ts[4]).reshape(rows, n), ref) < 3e-5
     for t in ts + [ws]:
         t.Release()
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 4), (2, 2048), (3, 2052), (1, 4100), (2, 8192), (1, 8196), (2, 30)])
+def test_rmsnorm_rows_kept_in_registers_and_others(hip, rows, dim):
+    rng = np.random.default_rng(dim)
+    a, b = rng.standard_normal((2, rows, dim), dtype=np.float32)
+    w = rng.standard_normal(dim, dtype=np.float32)
+
+    def ref(x):
+        return x / np.sqrt((x * x).mean(axis=1, keepdims=True) + 1e-5) * w
+
+    ta, tb, tw, to = (hip.FromHost(v, v.shape) for v in (a, b, w, a))
+    E.KRMSNormOutEps(ta, to, tw, rows, dim, 1e-5)
+    assert H.rel_err(hip.ToHost(to).reshape(rows, dim), ref(a.astype(np.float64))) < 1e-6
+    E.KFusedAddRMSNormEps(ta, tb, tb, tw, rows, dim, 1e-5)                 # out may be an operand
+    assert H.rel_err(hip.ToHost(tb).reshape(rows, dim), ref(a.astype(np.float64) + b)) < 1e-6
+    for t in (ta, tb, tw, to):
+        t.Release()
