@@ -139,7 +139,13 @@ private:
     HIPFusedInference() = default;
     bool built = false;
     int invalidateGraphs();
-    int uploadMat(int idx, DevMat& m, int rows, int cols, const int8_t* q, const float* scales);
+    int uploadMat(int idx, DevMat& m, int rows, int cols, const float* src, const int8_t* q, const float* scales);
+    static constexpr size_t STAGE_BYTES = (size_t)4 << 20;
+    char* stage[2] = {nullptr, nullptr};             // pinned, made by the first upload
+    hipEvent_t stageFree[2] = {nullptr, nullptr};    // the copies out of them have ended
+    int stageAt = 0;
+    int stageBuffer(char** buf);                     // the buffer to fill next, once it is free
+    int stageSent();                                 // its copies are queued
     int uploadMatQ4(int idx, DevMat& m, int rows, int cols, const uint8_t* raw, size_t nbytes);
     int setVec(int idx, float*& dst, const float* data, size_t n, size_t expect);
     int slotAddr(int idx, char** out);

@@ -223,6 +223,10 @@ HIPFusedInference::~HIPFusedInference() {
     if (hGate) (void)hipHostFree(hGate);
     if (hOut) (void)hipHostFree(hOut);
     if (hIn) (void)hipHostFree(hIn);
+    for (int b = 0; b < 2; b++) {
+        if (stage[b]) (void)hipHostFree(stage[b]);
+        if (stageFree[b]) (void)hipEventDestroy(stageFree[b]);
+    }
     for (hipEvent_t e : profEvents) (void)hipEventDestroy(e);
     if (copyStream) { (void)hipStreamSynchronize(copyStream); (void)hipStreamDestroy(copyStream); }
     if (computeDone) (void)hipEventDestroy(computeDone);
@@ -262,27 +266,74 @@ DevMat* HIPFusedInference::matSlot(int idx, int* rows, int* cols) {
     return nullptr;
 }
 
+// ---- uploads ----
+// A matrix goes to the device in pieces of STAGE_BYTES through two page-locked buffers of the context: the worker threads
+// fill one (copy, quantize or regroup) while the other is on its way.  The copies are queued on the context's stream --
+// behind whatever still reads the slot -- and the call returns once the last piece has been taken from the caller's memory.
+// (Quantizing a matrix into fresh memory and copying it from there, pageable, waiting for each: 13.5 ms for 88 million
+// weights of the 0.5B shape, 4.0 ms now.)
+int HIPFusedInference::stageBuffer(char** buf) {
+    const int b = stageAt;
+    if (!stage[b]) {
+        void* v = nullptr;
+        HIPCHK(hipHostMalloc(&v, STAGE_BYTES, hipHostMallocDefault));
+        stage[b] = static_cast<char*>(v);
+        HIPCHK(hipEventCreateWithFlags(&stageFree[b], hipEventDisableTiming));
+    } else {
+        HIPCHK(hipEventSynchronize(stageFree[b]));
+    }
+    *buf = stage[b];
+    return MG_OK;
+}
+int HIPFusedInference::stageSent() {
+    HIPCHK(hipEventRecord(stageFree[stageAt], stream));
+    stageAt ^= 1;
+    return MG_OK;
+}
+
 int HIPFusedInference::setVec(int idx, float*& dst, const float* data, size_t n, size_t expect) {
     ARGCHK(n == expect, "SetWeight: wrong element count for a norm/bias slot");
     char* addr = nullptr;
     int rc = slotAddr(idx, &addr);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(stream));
-    HIPCHK(hipMemcpy(addr, data, expect * sizeof(float), hipMemcpyHostToDevice));
+    char* buf = nullptr;
+    rc = stageBuffer(&buf);
+    if (rc) return rc;
+    std::memcpy(buf, data, expect * sizeof(float));                  // (at most 64 KB)
+    HIPCHK(hipMemcpyAsync(addr, buf, expect * sizeof(float), hipMemcpyHostToDevice, stream));
+    rc = stageSent();
+    if (rc) return rc;
     dst = reinterpret_cast<float*>(addr);
     return MG_OK;
 }
 
-int HIPFusedInference::uploadMat(int idx, DevMat& m, int rows, int cols, const int8_t* q, const float* scales) {
-    HIPCHK(hipStreamSynchronize(stream));
+// Rows of a Q8 matrix from fp32 (src) or from quantized rows (q, scales).
+int HIPFusedInference::uploadMat(int idx, DevMat& m, int rows, int cols, const float* src, const int8_t* q, const float* scales) {
     invalidateGraphs();
     char* addr = nullptr;
     int rc = slotAddr(idx, &addr);
     if (rc) return rc;
     m = DevMat();
-    HIPCHK(hipMemcpy(addr, q, (size_t)rows * cols, hipMemcpyHostToDevice));
     char* sc = addr + alignUp256((size_t)rows * cols);
-    HIPCHK(hipMemcpy(sc, scales, (size_t)rows * 4, hipMemcpyHostToDevice));
+    const size_t per = STAGE_BYTES / ((size_t)cols + 4);             // rows of a piece: their bytes, then their scales
+    for (size_t r0 = 0; r0 < (size_t)rows; r0 += per) {
+        const size_t n = std::min(per, (size_t)rows - r0);
+        char* buf = nullptr;
+        rc = stageBuffer(&buf);
+        if (rc) return rc;
+        int8_t* bq = reinterpret_cast<int8_t*>(buf);
+        float* bs = reinterpret_cast<float*>(buf + (STAGE_BYTES - n * 4));
+        const size_t grain = std::max<size_t>(1, 65536 / (size_t)cols);
+        parallel_for(n, grain, [&](size_t a, size_t b) {
+            if (src) { quantize_q8_rows(src + r0 * cols, cols, quantRounding, bq, bs, a, b); return; }
+            std::memcpy(bq + a * cols, q + (r0 + a) * cols, (b - a) * cols);
+            std::memcpy(bs + a, scales + r0 + a, (b - a) * 4);
+        });
+        HIPCHK(hipMemcpyAsync(addr + r0 * cols, bq, n * cols, hipMemcpyHostToDevice, stream));
+        HIPCHK(hipMemcpyAsync(sc + r0 * 4, bs, n * 4, hipMemcpyHostToDevice, stream));
+        rc = stageSent();
+        if (rc) return rc;
+    }
     m.w = addr; m.scales = reinterpret_cast<float*>(sc);
     m.kind = WF_Q8; m.rows = rows; m.cols = cols;
     m.bytes = (size_t)rows * cols + (size_t)rows * 4;
@@ -293,15 +344,23 @@ int HIPFusedInference::uploadMatQ4(int idx, DevMat& m, int rows, int cols, const
     ARGCHK(cols % 32 == 0, "SetWeightQ4_0: cols must be a multiple of 32");
     size_t expect = (size_t)rows * (cols / 32) * 18;          // cuda_q4_0.go:16-19
     ARGCHK(nbytes == expect, "SetWeightQ4_0: byte count is not rows*(cols/32)*18");
-    HIPCHK(hipStreamSynchronize(stream));
     invalidateGraphs();
     char* addr = nullptr;
     int rc = slotAddr(idx, &addr);
     if (rc) return rc;
     m = DevMat();
-    std::vector<uint8_t> planar(expect);
-    repack_q4_0_host(raw, rows, cols, planar.data());
-    HIPCHK(hipMemcpy(addr, planar.data(), expect, hipMemcpyHostToDevice));
+    const size_t nb = expect / 18, per = STAGE_BYTES / 18;
+    for (size_t b0 = 0; b0 < nb; b0 += per) {
+        const size_t n = std::min(per, nb - b0);
+        char* buf = nullptr;
+        rc = stageBuffer(&buf);
+        if (rc) return rc;
+        parallel_for(n, 1 << 12, [&](size_t a, size_t b) { repack_q4_0_blocks(raw + b0 * 18, n, a, b, reinterpret_cast<uint8_t*>(buf)); });
+        HIPCHK(hipMemcpyAsync(addr + b0 * 16, buf, n * 16, hipMemcpyHostToDevice, stream));
+        HIPCHK(hipMemcpyAsync(addr + nb * 16 + b0 * 2, buf + n * 16, n * 2, hipMemcpyHostToDevice, stream));
+        rc = stageSent();
+        if (rc) return rc;
+    }
     m.w = addr; m.kind = WF_Q4P; m.rows = rows; m.cols = cols; m.bytes = expect;
     return MG_OK;
 }
@@ -313,10 +372,7 @@ int HIPFusedInference::SetWeight(int idx, const float* data, size_t n) {
     DevMat* m = matSlot(idx, &rows, &cols);
     if (m) {
         ARGCHK(n == (size_t)rows * cols, "SetWeight: wrong element count for a matrix slot");
-        std::vector<int8_t> q((size_t)rows * cols);
-        std::vector<float> sc(rows);
-        mg_quantize_q8(data, rows, cols, quantRounding, q.data(), sc.data());
-        return uploadMat(idx, *m, rows, cols, q.data(), sc.data());
+        return uploadMat(idx, *m, rows, cols, data, nullptr, nullptr);
     }
     if (idx == nLayers * 12) return setVec(idx, finalNorm, data, n, dim);
     LayerWeights& L = layers[idx / 12];
@@ -336,7 +392,7 @@ int HIPFusedInference::SetWeightQ8(int idx, const int8_t* q, const float* scales
     int rows = 0, cols = 0;
     DevMat* m = matSlot(idx, &rows, &cols);
     ARGCHK(m && q && scales, "SetWeightQ8: not a matrix slot or NULL data");
-    return uploadMat(idx, *m, rows, cols, q, scales);
+    return uploadMat(idx, *m, rows, cols, nullptr, q, scales);
 }
 
 int HIPFusedInference::SetWeightQ4_0(int idx, const uint8_t* q4Data, size_t nbytes) {

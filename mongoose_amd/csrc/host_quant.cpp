@@ -15,6 +15,9 @@
 #include <mutex>
 #include <thread>
 #include <vector>
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+#include <immintrin.h>
+#endif
 
 namespace mg {
 
@@ -117,9 +120,159 @@ void repack_q4_0_blocks(const uint8_t* raw, size_t nb, size_t b0, size_t b1, uin
     }
 }
 
-void repack_q4_0_host(const uint8_t* raw, int rows, int cols, uint8_t* planar) {
-    const size_t nb = (size_t)rows * (cols / 32);
-    parallel_for(nb, 1 << 13, [&](size_t a, size_t b) { repack_q4_0_blocks(raw, nb, a, b, planar); });
+// ---------------------------------------------------------------------------
+// The quantizers.  The plain loops say what they compute; where the CPU has AVX2 the same operations run eight at a time,
+// with the same bits: no operation is fused or reordered except the maximum of absolute values, which does not depend on
+// the order, and the conversions saturate as the plain ones do (below).  The plain loops do some 0.9 weights a nanosecond a
+// core; with AVX2 they keep up with the memory they read.
+// ---------------------------------------------------------------------------
+static void q8_row(const float* src, int c0, int cols, float s, float amax, int mode, int8_t* dst) {
+    if (mode == 0) {
+        const float inv = 1.0f / s;
+        for (int c = c0; c < cols; c++) {
+            const float t = src[c] * inv;
+            // Go's int(): truncate; NaN/overflow (only when 1/s overflowed) -> most negative
+            const bool inRange = t > -9.2233720368547758e18f && t < 9.2233720368547758e18f;
+            const long long v = inRange ? (long long)t : (-9223372036854775807LL - 1);
+            dst[c] = (int8_t)std::min(127LL, std::max(-128LL, v));
+        }
+    } else {
+        const float inv = 127.0f / amax;
+        for (int c = c0; c < cols; c++) {
+            float v = std::min(127.0f, std::max(-127.0f, src[c] * inv));
+            dst[c] = (int8_t)(v + (v > 0 ? 0.5f : -0.5f));
+        }
+    }
+}
+static float q8_absmax(const float* src, int c0, int cols, float amax) {
+    for (int c = c0; c < cols; c++) {
+        float v = std::fabs(src[c]);
+        if (v > amax) amax = v;
+    }
+    return amax;
+}
+static void q4_0_block(const float* x, uint8_t* y) {
+    float amax = 0.0f, vmax = 0.0f;
+    for (int j = 0; j < 32; j++) {
+        if (std::fabs(x[j]) > amax) { amax = std::fabs(x[j]); vmax = x[j]; }
+    }
+    const float d = vmax / -8.0f;
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    const uint16_t hd = mg_f32_to_f16(d);
+    std::memcpy(y, &hd, 2);
+    for (int j = 0; j < 16; j++) {
+        int lo = (int8_t)(x[j] * id + 8.5f);
+        int hi = (int8_t)(x[j + 16] * id + 8.5f);
+        y[2 + j] = (uint8_t)(std::min(lo, 15) | (std::min(hi, 15) << 4));
+    }
+}
+
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+#define MG_AVX2 __attribute__((target("avx2")))
+// max_ps takes its second operand when one is NaN: the running maximum, as `if (v > amax)` does
+MG_AVX2 static inline float hmax8(__m256 m) {
+    __m128 a = _mm_max_ps(_mm256_castps256_ps128(m), _mm256_extractf128_ps(m, 1));
+    a = _mm_max_ps(a, _mm_movehl_ps(a, a));
+    a = _mm_max_ss(a, _mm_shuffle_ps(a, a, 1));
+    return _mm_cvtss_f32(a);
+}
+MG_AVX2 static float q8_absmax_avx2(const float* src, int cols) {
+    const __m256 mask = _mm256_castsi256_ps(_mm256_set1_epi32(0x7fffffff));
+    __m256 m0 = _mm256_setzero_ps(), m1 = m0, m2 = m0, m3 = m0;
+    int c = 0;
+    for (; c + 32 <= cols; c += 32) {
+        m0 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(src + c), mask), m0);
+        m1 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(src + c + 8), mask), m1);
+        m2 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(src + c + 16), mask), m2);
+        m3 = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(src + c + 24), mask), m3);
+    }
+    return q8_absmax(src, c, cols, hmax8(_mm256_max_ps(_mm256_max_ps(m0, m1), _mm256_max_ps(m2, m3))));
+}
+// 32 values -> 32 int8.  cvttps gives INT_MIN for NaN and what does not fit, the packs saturate: -128, as the plain loop's
+// most negative value does.  (A finite value past 2^31 does not occur: |x * inv| is at most 127 but for rounding, or inv is
+// infinite.)
+MG_AVX2 static inline __m256i pack32(__m256i a, __m256i b, __m256i c, __m256i d) {
+    const __m256i p = _mm256_packs_epi16(_mm256_packs_epi32(a, b), _mm256_packs_epi32(c, d));
+    return _mm256_permutevar8x32_epi32(p, _mm256_setr_epi32(0, 4, 1, 5, 2, 6, 3, 7));
+}
+MG_AVX2 static void q8_row_avx2(const float* src, int cols, float s, float amax, int mode, int8_t* dst) {
+    int c = 0;
+    const __m256 inv = _mm256_set1_ps(mode == 0 ? 1.0f / s : 127.0f / amax);
+    if (mode == 0) {
+        for (; c + 32 <= cols; c += 32) {
+            __m256i v[4];
+            for (int k = 0; k < 4; k++) v[k] = _mm256_cvttps_epi32(_mm256_mul_ps(_mm256_loadu_ps(src + c + 8 * k), inv));
+            _mm256_storeu_si256(reinterpret_cast<__m256i*>(dst + c), pack32(v[0], v[1], v[2], v[3]));
+        }
+    } else {
+        const __m256 lo = _mm256_set1_ps(-127.0f), hi = _mm256_set1_ps(127.0f), up = _mm256_set1_ps(0.5f), dn = _mm256_set1_ps(-0.5f), z = _mm256_setzero_ps();
+        for (; c + 32 <= cols; c += 32) {
+            __m256i v[4];
+            for (int k = 0; k < 4; k++) {
+                const __m256 t = _mm256_min_ps(_mm256_max_ps(_mm256_mul_ps(_mm256_loadu_ps(src + c + 8 * k), inv), lo), hi);
+                v[k] = _mm256_cvttps_epi32(_mm256_add_ps(t, _mm256_blendv_ps(dn, up, _mm256_cmp_ps(t, z, _CMP_GT_OQ))));
+            }
+            _mm256_storeu_si256(reinterpret_cast<__m256i*>(dst + c), pack32(v[0], v[1], v[2], v[3]));
+        }
+    }
+    q8_row(src, c, cols, s, amax, mode, dst);
+}
+MG_AVX2 static void q4_0_block_avx2(const float* x, uint8_t* y) {
+    const __m256 mask = _mm256_castsi256_ps(_mm256_set1_epi32(0x7fffffff));
+    __m256 v[4], a[4], m = _mm256_setzero_ps();
+    for (int k = 0; k < 4; k++) {
+        v[k] = _mm256_loadu_ps(x + 8 * k);
+        a[k] = _mm256_and_ps(v[k], mask);
+        m = _mm256_max_ps(a[k], m);
+    }
+    const float amax = hmax8(m);
+    const __m256 am = _mm256_set1_ps(amax);
+    unsigned eq = 0;                               // the first value of that size gives the sign
+    for (int k = 0; k < 4; k++) eq |= (unsigned)_mm256_movemask_ps(_mm256_cmp_ps(a[k], am, _CMP_EQ_OQ)) << (8 * k);
+    const float vmax = amax > 0.0f ? x[__builtin_ctz(eq)] : 0.0f;
+    const float d = vmax / -8.0f;
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    const uint16_t hd = mg_f32_to_f16(d);
+    std::memcpy(y, &hd, 2);
+    const __m256 idv = _mm256_set1_ps(id), off = _mm256_set1_ps(8.5f);
+    const __m256i fifteen = _mm256_set1_epi32(15);
+    __m256i n[4];
+    for (int k = 0; k < 4; k++) {
+        n[k] = _mm256_cvttps_epi32(_mm256_add_ps(_mm256_mul_ps(v[k], idv), off));
+        n[k] = _mm256_min_epi32(_mm256_srai_epi32(_mm256_slli_epi32(n[k], 24), 24), fifteen);      // (int8_t), then at most 15
+    }
+    const __m256i b0 = _mm256_and_si256(_mm256_or_si256(n[0], _mm256_slli_epi32(n[2], 4)), _mm256_set1_epi32(255));
+    const __m256i b1 = _mm256_and_si256(_mm256_or_si256(n[1], _mm256_slli_epi32(n[3], 4)), _mm256_set1_epi32(255));
+    const __m256i p = _mm256_permute4x64_epi64(_mm256_packus_epi32(b0, b1), 0xd8);
+    _mm_storeu_si128(reinterpret_cast<__m128i*>(y + 2), _mm_packus_epi16(_mm256_castsi256_si128(p), _mm256_extracti128_si256(p, 1)));
+}
+static bool have_avx2() { static const bool h = __builtin_cpu_supports("avx2"); return h; }
+#else
+static bool have_avx2() { return false; }
+static float q8_absmax_avx2(const float* src, int cols) { return q8_absmax(src, 0, cols, 0.f); }
+static void q8_row_avx2(const float* src, int cols, float s, float amax, int mode, int8_t* dst) { q8_row(src, 0, cols, s, amax, mode, dst); }
+static void q4_0_block_avx2(const float* x, uint8_t* y) { q4_0_block(x, y); }
+#endif
+
+void quantize_q8_rows(const float* w, int cols, int mode, int8_t* q, float* scales, size_t r0, size_t r1) {
+    const bool wide = have_avx2();
+    for (size_t r = r0; r < r1; r++) {
+        const float* src = w + r * (size_t)cols;
+        int8_t* dst = q + r * (size_t)cols;
+        const float amax = wide ? q8_absmax_avx2(src, cols) : q8_absmax(src, 0, cols, 0.0f);
+        const float s = amax / 127.0f;
+        scales[r] = s;
+        if (!(s > 0.0f)) { std::memset(dst, 0, (size_t)cols); continue; }
+        if (wide) q8_row_avx2(src, cols, s, amax, mode, dst);
+        else q8_row(src, 0, cols, s, amax, mode, dst);
+    }
+}
+void quantize_q4_0_blocks(const float* w, size_t b0, size_t b1, uint8_t* blocks) {
+    const bool wide = have_avx2();
+    for (size_t b = b0; b < b1; b++) {
+        if (wide) q4_0_block_avx2(w + b * 32, blocks + b * 18);
+        else q4_0_block(w + b * 32, blocks + b * 18);
+    }
 }
 
 }  // namespace mg
@@ -174,60 +327,13 @@ float mg_f16_to_f32(uint16_t h) {
 // quantizeQ8, cuda_fused_infer.go:363-390 (mode 0), or the Metal loader's
 // rounding, metal_impl_darwin.m:5765-5780 (mode 1).  scale = absmax/127.
 void mg_quantize_q8(const float* w, int rows, int cols, int mode, int8_t* q, float* scales) {
-    mg::parallel_for((size_t)rows, 16, [&](size_t r0, size_t r1) {
-        for (size_t r = r0; r < r1; r++) {
-            const float* src = w + r * (size_t)cols;
-            int8_t* dst = q + r * (size_t)cols;
-            float amax = 0.0f;
-            for (int c = 0; c < cols; c++) {
-                float v = std::fabs(src[c]);
-                if (v > amax) amax = v;
-            }
-            const float s = amax / 127.0f;
-            scales[r] = s;
-            if (!(s > 0.0f)) { std::memset(dst, 0, (size_t)cols); continue; }
-            if (mode == 0) {
-                const float inv = 1.0f / s;
-                for (int c = 0; c < cols; c++) {
-                    const float t = src[c] * inv;
-                    // Go's int(): truncate; NaN/overflow (only when 1/s overflowed) -> most negative
-                    const bool inRange = t > -9.2233720368547758e18f && t < 9.2233720368547758e18f;
-                    const long long v = inRange ? (long long)t : (-9223372036854775807LL - 1);
-                    dst[c] = (int8_t)std::min(127LL, std::max(-128LL, v));
-                }
-            } else {
-                const float inv = 127.0f / amax;
-                for (int c = 0; c < cols; c++) {
-                    float v = std::min(127.0f, std::max(-127.0f, src[c] * inv));
-                    dst[c] = (int8_t)(v + (v > 0 ? 0.5f : -0.5f));
-                }
-            }
-        }
-    });
+    mg::parallel_for((size_t)rows, 16, [&](size_t r0, size_t r1) { mg::quantize_q8_rows(w, cols, mode, q, scales, r0, r1); });
 }
 
 // GGML quantize_row_q4_0 (the block format cuda_q4_0.go:13-17 uploads).
 void mg_quantize_q4_0(const float* w, int rows, int cols, uint8_t* blocks) {
     const size_t nb = (size_t)rows * (cols / 32);
-    mg::parallel_for(nb, 1 << 12, [&](size_t b0, size_t b1) {
-        for (size_t b = b0; b < b1; b++) {
-            const float* x = w + b * 32;
-            uint8_t* y = blocks + b * 18;
-            float amax = 0.0f, vmax = 0.0f;
-            for (int j = 0; j < 32; j++) {
-                if (std::fabs(x[j]) > amax) { amax = std::fabs(x[j]); vmax = x[j]; }
-            }
-            const float d = vmax / -8.0f;
-            const float id = d != 0.0f ? 1.0f / d : 0.0f;
-            const uint16_t hd = mg_f32_to_f16(d);
-            std::memcpy(y, &hd, 2);
-            for (int j = 0; j < 16; j++) {
-                int lo = (int8_t)(x[j] * id + 8.5f);
-                int hi = (int8_t)(x[j + 16] * id + 8.5f);
-                y[2 + j] = (uint8_t)(std::min(lo, 15) | (std::min(hi, 15) << 4));
-            }
-        }
-    });
+    mg::parallel_for(nb, 1 << 12, [&](size_t b0, size_t b1) { mg::quantize_q4_0_blocks(w, b0, b1, blocks); });
 }
 
 // ---------------------------------------------------------------------------
