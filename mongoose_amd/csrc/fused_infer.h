@@ -131,6 +131,8 @@ public:
     int hiddenIdx = 0;
     int enqueueLayer(const LayerWeights& L, int layer, const StepState* st, int posImm);
     int enqueueFinal(bool withArgmax);
+    int publish(const float* src, int n, const int* ints, int nInts);      // results on their way to hOut
+    int collect(float* out, int n, int* ints, int nInts);                  // ... waited for and copied to the caller
     float* logits = nullptr;
     float* finalNorm = nullptr;
     DevMat lmHead;
@@ -140,9 +142,10 @@ private:
     bool built = false;
     int invalidateGraphs();
     int uploadMat(int idx, DevMat& m, int rows, int cols, const float* src, const int8_t* q, const float* scales);
-    static constexpr size_t STAGE_BYTES = (size_t)4 << 20;
-    char* stage[2] = {nullptr, nullptr};             // pinned, made by the first upload
-    hipEvent_t stageFree[2] = {nullptr, nullptr};    // the copies out of them have ended
+    static constexpr size_t STAGE_BYTES = (size_t)2 << 20;
+    static constexpr int STAGES = 4;
+    char* stage[STAGES] = {};             // pinned, made by the first uploads
+    hipEvent_t stageFree[STAGES] = {};    // the copies out of them have ended
     int stageAt = 0;
     int stageBuffer(char** buf);                     // the buffer to fill next, once it is free
     int stageSent();                                 // its copies are queued
@@ -229,8 +232,6 @@ private:
     FlowTail* dFlowTail = nullptr;
     int enqueueTokensFlow(int nTokens, int pos = 0, int token = -1, int nPrompt = 0);
     int flowClean = 0;              // halves of the exchange area known to be as a reset leaves them (bits 0 and 1)
-    int publish(const float* src, int n, const int* ints, int nInts);      // results on their way to hOut
-    int collect(float* out, int n, int* ints, int nInts);                  // ... waited for and copied to the caller
     unsigned* hOut = nullptr;       // pinned: error word, flags of the slices from word 64, ints and floats at the offsets below
     int hOutInts = 0, hOutFloats = 0;
     unsigned hOutSeq = 0;

@@ -223,7 +223,7 @@ HIPFusedInference::~HIPFusedInference() {
     if (hGate) (void)hipHostFree(hGate);
     if (hOut) (void)hipHostFree(hOut);
     if (hIn) (void)hipHostFree(hIn);
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < STAGES; b++) {
         if (stage[b]) (void)hipHostFree(stage[b]);
         if (stageFree[b]) (void)hipEventDestroy(stageFree[b]);
     }
@@ -267,11 +267,11 @@ DevMat* HIPFusedInference::matSlot(int idx, int* rows, int* cols) {
 }
 
 // ---- uploads ----
-// A matrix goes to the device in pieces of STAGE_BYTES through two page-locked buffers of the context: the worker threads
-// fill one (copy, quantize or regroup) while the other is on its way.  The copies are queued on the context's stream --
+// A matrix goes to the device in pieces of STAGE_BYTES through a ring of page-locked buffers of the context: the worker
+// threads fill one (copy, quantize or regroup) while those before it are on their way.  The copies are queued on the context's stream --
 // behind whatever still reads the slot -- and the call returns once the last piece has been taken from the caller's memory.
 // (Quantizing a matrix into fresh memory and copying it from there, pageable, waiting for each: 13.5 ms for 88 million
-// weights of the 0.5B shape, 4.0 ms now.)
+// weights of the 0.5B shape, 3.1 to 3.7 ms now, depending on the host.)
 int HIPFusedInference::stageBuffer(char** buf) {
     const int b = stageAt;
     if (!stage[b]) {
@@ -287,7 +287,7 @@ int HIPFusedInference::stageBuffer(char** buf) {
 }
 int HIPFusedInference::stageSent() {
     HIPCHK(hipEventRecord(stageFree[stageAt], stream));
-    stageAt ^= 1;
+    stageAt = (stageAt + 1) % STAGES;
     return MG_OK;
 }
 
@@ -300,7 +300,7 @@ int HIPFusedInference::setVec(int idx, float*& dst, const float* data, size_t n,
     rc = stageBuffer(&buf);
     if (rc) return rc;
     std::memcpy(buf, data, expect * sizeof(float));                  // (at most 64 KB)
-    HIPCHK(hipMemcpyAsync(addr, buf, expect * sizeof(float), hipMemcpyHostToDevice, stream));
+    HIPCHK(launch_host_pieces(HostPieces{{buf}, {addr}, {expect * sizeof(float)}, 1}, stream));
     rc = stageSent();
     if (rc) return rc;
     dst = reinterpret_cast<float*>(addr);
@@ -315,22 +315,21 @@ int HIPFusedInference::uploadMat(int idx, DevMat& m, int rows, int cols, const f
     if (rc) return rc;
     m = DevMat();
     char* sc = addr + alignUp256((size_t)rows * cols);
-    const size_t per = STAGE_BYTES / ((size_t)cols + 4);             // rows of a piece: their bytes, then their scales
+    const size_t per = (STAGE_BYTES / ((size_t)cols + 4)) & ~(size_t)15;      // rows of a piece: their bytes, then their scales (16-byte aligned)
     for (size_t r0 = 0; r0 < (size_t)rows; r0 += per) {
         const size_t n = std::min(per, (size_t)rows - r0);
         char* buf = nullptr;
         rc = stageBuffer(&buf);
         if (rc) return rc;
         int8_t* bq = reinterpret_cast<int8_t*>(buf);
-        float* bs = reinterpret_cast<float*>(buf + (STAGE_BYTES - n * 4));
-        const size_t grain = std::max<size_t>(1, 65536 / (size_t)cols);
+        float* bs = reinterpret_cast<float*>(buf + ((STAGE_BYTES - n * 4) & ~(size_t)15));
+        const size_t grain = std::max<size_t>(1, 16384 / (size_t)cols);
         parallel_for(n, grain, [&](size_t a, size_t b) {
             if (src) { quantize_q8_rows(src + r0 * cols, cols, quantRounding, bq, bs, a, b); return; }
             std::memcpy(bq + a * cols, q + (r0 + a) * cols, (b - a) * cols);
             std::memcpy(bs + a, scales + r0 + a, (b - a) * 4);
         });
-        HIPCHK(hipMemcpyAsync(addr + r0 * cols, bq, n * cols, hipMemcpyHostToDevice, stream));
-        HIPCHK(hipMemcpyAsync(sc + r0 * 4, bs, n * 4, hipMemcpyHostToDevice, stream));
+        HIPCHK(launch_host_pieces(HostPieces{{bq, bs}, {addr + r0 * cols, sc + r0 * 4}, {n * cols, n * 4}, 2}, stream));
         rc = stageSent();
         if (rc) return rc;
     }
@@ -349,15 +348,14 @@ int HIPFusedInference::uploadMatQ4(int idx, DevMat& m, int rows, int cols, const
     int rc = slotAddr(idx, &addr);
     if (rc) return rc;
     m = DevMat();
-    const size_t nb = expect / 18, per = STAGE_BYTES / 18;
+    const size_t nb = expect / 18, per = (STAGE_BYTES / 18) & ~(size_t)7;      // (16-byte aligned pieces of both planes)
     for (size_t b0 = 0; b0 < nb; b0 += per) {
         const size_t n = std::min(per, nb - b0);
         char* buf = nullptr;
         rc = stageBuffer(&buf);
         if (rc) return rc;
-        parallel_for(n, 1 << 12, [&](size_t a, size_t b) { repack_q4_0_blocks(raw + b0 * 18, n, a, b, reinterpret_cast<uint8_t*>(buf)); });
-        HIPCHK(hipMemcpyAsync(addr + b0 * 16, buf, n * 16, hipMemcpyHostToDevice, stream));
-        HIPCHK(hipMemcpyAsync(addr + nb * 16 + b0 * 2, buf + n * 16, n * 2, hipMemcpyHostToDevice, stream));
+        parallel_for(n, 1 << 11, [&](size_t a, size_t b) { repack_q4_0_blocks(raw + b0 * 18, n, a, b, reinterpret_cast<uint8_t*>(buf)); });
+        HIPCHK(launch_host_pieces(HostPieces{{buf, buf + n * 16}, {addr + b0 * 16, addr + nb * 16 + b0 * 2}, {n * 16, n * 2}, 2}, stream));
         rc = stageSent();
         if (rc) return rc;
     }
@@ -904,9 +902,16 @@ int HIPFusedInference::ensureFlow() {
             T.ropeCur = ropeCur;
             T.vocab = vocabSize;
         }
-        HIPCHK(hipStreamSynchronize(stream));
-        HIPCHK(hipMemcpy(dFlowLayers, t.data(), sizeof(FlowLayer) * (size_t)nLayers, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(dFlowTail, &T, sizeof(FlowTail), hipMemcpyHostToDevice));
+        char* buf = nullptr;
+        int rc = stageBuffer(&buf);
+        if (rc) return rc;
+        const size_t tb = sizeof(FlowLayer) * (size_t)nLayers, at = alignUp256(tb);
+        if (at + sizeof(T) > STAGE_BYTES) { set_error("persistent launch: too many layers"); return MG_E_STATE; }
+        std::memcpy(buf, t.data(), tb);
+        std::memcpy(buf + at, &T, sizeof(T));
+        HIPCHK(launch_host_pieces(HostPieces{{buf, buf + at}, {dFlowLayers, dFlowTail}, {tb, sizeof(T)}, 2}, stream));
+        rc = stageSent();
+        if (rc) return rc;
         flowTableDirty = false;
     }
     return MG_OK;

@@ -7,8 +7,9 @@
 namespace mg {
 
 // fn(job) for job in [0, njobs) on the library's worker threads (up to 16 with the caller); returns when
-// all are done.  One region at a time; fn must not start another.
-void parallel_jobs(size_t njobs, const std::function<void(size_t)>& fn);
+// all are done.  One region at a time; fn must not start another.  meanwhile: what the caller does once the workers have
+// been set going, before it takes jobs itself.
+void parallel_jobs(size_t njobs, const std::function<void(size_t)>& fn, const std::function<void()>& meanwhile = nullptr);
 // fn(begin, end) over [0, n) in pieces of `grain`, through parallel_jobs.
 void parallel_for(size_t n, size_t grain, const std::function<void(size_t, size_t)>& fn);
 

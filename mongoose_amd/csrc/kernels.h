@@ -184,6 +184,10 @@ constexpr int PUBLISH_MAX_SLICES = 32;
 inline int publish_slice_floats(int n) { const int per = (n + PUBLISH_MAX_SLICES - 1) / PUBLISH_MAX_SLICES; return per < 1024 ? 1024 : (per + 255) / 256 * 256; }
 inline int publish_slices(int n) { return n > 0 ? (n + publish_slice_floats(n) - 1) / publish_slice_floats(n) : 1; }
 hipError_t launch_publish(const PublishParams& p, hipStream_t s);
+// Page-locked host memory -> device memory, up to three pieces in one launch (16-byte aligned on both sides; a length need
+// not be).
+struct HostPieces { const void* src[3]; void* dst[3]; size_t bytes[3]; int n; };
+hipError_t launch_host_pieces(const HostPieces& p, hipStream_t s);
 // n words of page-locked host memory -> device memory.
 hipError_t launch_take_words(const unsigned* src, unsigned* dst, int n, hipStream_t s);
 // The last row of a prefill -> the hidden buffer, and the step state for its lm_head.

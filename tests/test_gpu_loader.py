@@ -125,3 +125,16 @@ def test_stream_object_outliving_its_context_is_inert(hip):
     rc = st.StreamForwardToken(0, h, 1, [None] * 12, [0] * 7, None)
     assert rc == -4 and "destroyed" in E.last_error()
     st.Close()
+
+
+@pytest.mark.parametrize("fmt,vocab", [("q8", 33), ("q8", 41001), ("q4_0", 35), ("q4_0", 67003)])
+def test_matrix_in_several_pieces(hip, fmt, vocab):
+    """Matrices larger than a staging buffer, and lengths that are no multiple of 16 bytes: every row of the lm_head arrives."""
+    s = configs.TOY._replace(name="pieces", nLayers=1, dim=64, nHeads=1, nKVHeads=1, ffnDim=160, vocab=vocab)
+    m = H.Model(s, seed=5, maxSeq=4, eng=hip, threads=4, fmt=fmt)
+    got = np.empty(vocab, np.float32)
+    rc, nxt = m.hip.DecodeToken(7, 0, got)
+    assert rc == 0, E.last_error()
+    want, ref, _ = m.orc.decode_token(7, 0, shadow=True)
+    assert np.abs(got - ref).max() < 1e-4 * np.abs(ref).max() and nxt == want
+    m.close()
