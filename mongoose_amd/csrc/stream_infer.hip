@@ -1,16 +1,21 @@
 // stream_infer.hip -- HIPStreamInfer: decode with layer weights streamed from
 // host memory, for models larger than device memory.  Counterpart of
-// CUDAStreamInfer (cuda_fused_stream.go:98-726): two device weight sets, two
+// CUDAStreamInfer (cuda_fused_stream.go:98-726): three device weight sets, three
 // pinned staging buffers, and a three-way overlap per layer of
-//   host copy (layer i+2 -> pinned)  ||  DMA (layer i+1 -> device)  ||  compute (layer i).
+//   host copy (layer i+2 -> pinned)  ||  copy (layer i+1 -> device)  ||  compute (layer i).
 // The layer arithmetic is the resident path's (stepLayer :277-356 = the
 // 17-op body plus the three bias adds at :319-321).
 //
-// Differences by design: one DMA per layer instead of twelve (the staging
+// Differences by design: one copy launch per layer instead of twelve (the staging
 // buffer already has the device layout), and the Q4_0 rows are regrouped into
 // the split nibble/scale layout while they are being copied into the pinned
 // buffer, so the fast matvec kernel reads them with aligned 16-byte loads at
 // no extra pass over the data.
+//
+// Bound by the link: 16 workgroups read the page-locked blob at 55 GB/s (launch_host_pieces), and everything else hides
+// behind that: an 8.4 MB layer of the 0.5B shape crosses in 155 us, is staged in 60 and computed in 60.  Two copies are
+// queued ahead of the one that the host waits for before it fills that one's pinned buffer again.  Only the first
+// layer's staging is in nobody's shadow, so it goes out in three parts, each as soon as it is staged.
 #include "fused_infer.h"
 #include "../../include/mongoose_hip.h"
 #include "host_util.h"
@@ -41,12 +46,14 @@ public:
     size_t off[12];
     size_t nbytes[12];
     size_t layerSize = 0;
-    char* dev[2] = {nullptr, nullptr};
-    char* pinned[2] = {nullptr, nullptr};
+    static constexpr int SETS = 3;
+    char* dev[SETS] = {};
+    char* pinned[SETS] = {};
+    char* pinnedHidden = nullptr;            // the token's embedding on its way in
     hipStream_t uploadStream = nullptr;
-    hipEvent_t uploadDone[2] = {nullptr, nullptr};
-    hipEvent_t computeDone[2] = {nullptr, nullptr};
-    LayerWeights view[2];
+    hipEvent_t uploadDone[SETS] = {};      // of the copy out of a pinned buffer
+    hipEvent_t computeDone[SETS] = {};
+    LayerWeights view[SETS];
 
     ~HIPStreamInfer() {
         if (f) {                                   // still alive: no longer tell it about this object
@@ -55,11 +62,11 @@ public:
         }
         if (f && f->stream) (void)hipStreamSynchronize(f->stream);
         if (uploadStream) { (void)hipStreamSynchronize(uploadStream); (void)hipStreamDestroy(uploadStream); }
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < SETS; i++) {
             if (dev[i]) (void)hipFree(dev[i]);
+            if (computeDone[i]) (void)hipEventDestroy(computeDone[i]);
             if (pinned[i]) (void)hipHostFree(pinned[i]);
             if (uploadDone[i]) (void)hipEventDestroy(uploadDone[i]);
-            if (computeDone[i]) (void)hipEventDestroy(computeDone[i]);
         }
     }
 
@@ -86,14 +93,18 @@ public:
         }
         layerSize = o;
         SHIPCHK(hipStreamCreateWithFlags(&uploadStream, hipStreamNonBlocking));
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < SETS; i++) {
+            void* p = nullptr;
+            SHIPCHK(hipHostMalloc(&p, layerSize + (i == 0 ? alignUp((size_t)f->dim * 4) : 0), hipHostMallocDefault));     // cuda_fused_stream.go:170-180
+            pinned[i] = static_cast<char*>(p);
+            std::memset(pinned[i], 0, layerSize);
+            if (i == 0) pinnedHidden = pinned[0] + layerSize;
+            SHIPCHK(hipEventCreateWithFlags(&uploadDone[i], hipEventDisableTiming));
+        }
+        for (int i = 0; i < SETS; i++) {
             void* p = nullptr;
             SHIPCHK(hipMalloc(&p, layerSize));
             dev[i] = static_cast<char*>(p);
-            SHIPCHK(hipHostMalloc(&p, layerSize, hipHostMallocDefault));     // cuda_fused_stream.go:170-180
-            pinned[i] = static_cast<char*>(p);
-            std::memset(pinned[i], 0, layerSize);
-            SHIPCHK(hipEventCreateWithFlags(&uploadDone[i], hipEventDisableTiming));
             SHIPCHK(hipEventCreateWithFlags(&computeDone[i], hipEventDisableTiming));
             LayerWeights& L = view[i];
             char* b = dev[i];
@@ -113,16 +124,17 @@ public:
         return MG_OK;
     }
 
-    // stageLayerToPinned, cuda_fused_stream.go:200-247 (NULL bias -> zeros).  The seven matrices are cut
-    // into pieces of 8192 blocks and regrouped by all worker threads in one parallel region.
-    int stage(int set, const void* const* ptrs, const int32_t* sizes) {
+    // stageLayerToPinned, cuda_fused_stream.go:200-247 (NULL bias -> zeros), slots [k0, k1) of a layer.  The matrices are
+    // cut into pieces of 4096 blocks and regrouped by all worker threads in one parallel region, while the caller queues launches.
+    int stage(int set, const void* const* ptrs, const int32_t* sizes, int k0, int k1, const std::function<void()>& meanwhile = nullptr) {
         static const int matIdx[7] = {1, 2, 3, 7, 9, 10, 11};        // order of layerSizes[i*7+m] (:571-598)
-        constexpr size_t PIECE = 8192;
+        constexpr size_t PIECE = 4096;
         char* dst = pinned[set];
         struct Job { const uint8_t* src; uint8_t* out; size_t nb, b0, b1; };
         std::vector<Job> jobs;
         for (int m = 0; m < 7; m++) {
             int k = matIdx[m];
+            if (k < k0 || k >= k1) continue;
             if (!ptrs[k]) { set_error("StreamForwardToken: NULL matrix pointer"); return MG_E_ARG; }
             if ((size_t)sizes[m] != nbytes[k]) { set_error("StreamForwardToken: layerSizes entry is not rows*(cols/32)*18"); return MG_E_ARG; }
             int r, c;
@@ -135,15 +147,24 @@ public:
         parallel_jobs(jobs.size(), [&](size_t j) {
             const Job& jb = jobs[j];
             repack_q4_0_blocks(jb.src, jb.nb, jb.b0, jb.b1, jb.out);
-        });
+        }, meanwhile);
         for (int k : {0, 8}) {
+            if (k < k0 || k >= k1) continue;
             if (!ptrs[k]) { set_error("StreamForwardToken: NULL norm pointer"); return MG_E_ARG; }
             std::memcpy(dst + off[k], ptrs[k], nbytes[k]);
         }
         for (int k : {4, 5, 6}) {
+            if (k < k0 || k >= k1) continue;
             if (ptrs[k]) std::memcpy(dst + off[k], ptrs[k], nbytes[k]);
             else std::memset(dst + off[k], 0, nbytes[k]);
         }
+        return MG_OK;
+    }
+    // ... and slots [k0, k1) of staged layer l on their way to the device
+    int upload(int l, int k0, int k1) {
+        const size_t a = off[k0], b = k1 < 12 ? off[k1] : layerSize;
+        SHIPCHK(launch_host_pieces(HostPieces{{pinned[l % SETS] + a}, {dev[l % SETS] + a}, {b - a}, 1}, uploadStream));
+        if (k1 == 12) SHIPCHK(hipEventRecord(uploadDone[l % SETS], uploadStream));
         return MG_OK;
     }
 
@@ -156,46 +177,56 @@ public:
         for (int l = 0; l < nLayers; l++)
             if (!f->kCache[l]) { set_error("StreamForwardToken: KV cache missing, call SetLayerRange"); return MG_E_STATE; }
         hipStream_t cs = f->stream;
+        // (every call of this object waits for its own end; what others have queued on the context's stream comes first)
+        std::memcpy(pinnedHidden, embHidden, (size_t)f->dim * 4);
+        SHIPCHK(launch_host_pieces(HostPieces{{pinnedHidden}, {f->hidden[f->hiddenIdx]}, {(size_t)f->dim * 4}, 1}, cs));
+        int rc = run(pos, nLayers, layerPtrs, layerSizes, logitsOut != nullptr);
+        if (rc == MG_OK && logitsOut) {                                    // stepFinal :469-484
+            rc = f->publish(f->logits, f->vocabSize, nullptr, 0);
+            return rc ? rc : f->collect(logitsOut, f->vocabSize, nullptr, 0);
+        }
+        SHIPCHK(hipStreamSynchronize(uploadStream));      // (before an error is reported too: the buffers are in use)
         SHIPCHK(hipStreamSynchronize(cs));
-        SHIPCHK(hipStreamSynchronize(uploadStream));
-        SHIPCHK(hipMemcpy(f->hidden[f->hiddenIdx], embHidden, (size_t)f->dim * 4, hipMemcpyHostToDevice));
+        return rc;
+    }
 
-        int rc = stage(0, layerPtrs, layerSizes);
-        if (rc) return rc;
-        SHIPCHK(hipMemcpyAsync(dev[0], pinned[0], layerSize, hipMemcpyHostToDevice, uploadStream));
-        SHIPCHK(hipEventRecord(uploadDone[0], uploadStream));
-        if (nLayers > 1) {
-            rc = stage(1, layerPtrs + 12, layerSizes + 7);
+    int run(int pos, int nLayers, const void* const* layerPtrs, const int32_t* layerSizes, bool head) {
+        hipStream_t cs = f->stream;
+        int rc = MG_OK;
+        constexpr int cut[4] = {0, 8, 11, 12};                             // norm1 .. Wo | norm2, gate, up | down
+        for (int k = 0; k < 3; k++) {
+            rc = stage(0, layerPtrs, layerSizes, cut[k], cut[k + 1]);
+            if (rc == MG_OK) rc = upload(0, cut[k], cut[k + 1]);
             if (rc) return rc;
         }
-        for (int i = 0; i < nLayers; i++) {
-            const int set = i & 1, other = set ^ 1;
-            if (i + 1 < nLayers) {
-                // device set `other` was last read by layer i-1
-                if (i >= 1) SHIPCHK(hipStreamWaitEvent(uploadStream, computeDone[other], 0));
-                SHIPCHK(hipMemcpyAsync(dev[other], pinned[other], layerSize, hipMemcpyHostToDevice, uploadStream));
-                SHIPCHK(hipEventRecord(uploadDone[other], uploadStream));
-            }
-            SHIPCHK(hipStreamWaitEvent(cs, uploadDone[set], 0));
-            rc = f->enqueueLayer(view[set], i, nullptr, pos);
+        if (nLayers > 1) {
+            rc = stage(1, layerPtrs + 12, layerSizes + 7, 0, 12);
+            if (rc == MG_OK) rc = upload(1, 0, 12);
             if (rc) return rc;
-            SHIPCHK(hipEventRecord(computeDone[set], cs));
-            if (i + 2 < nLayers) {
-                // pinned[set] is free once its DMA (layer i) has finished
-                SHIPCHK(hipEventSynchronize(uploadDone[set]));
-                rc = stage(set, layerPtrs + (size_t)(i + 2) * 12, layerSizes + (size_t)(i + 2) * 7);
+        }
+        auto compute = [&](int i) {
+            SHIPCHK(hipStreamWaitEvent(cs, uploadDone[i % SETS], 0));
+            const int crc = f->enqueueLayer(view[i % SETS], i, nullptr, pos);
+            if (crc) return crc;
+            SHIPCHK(hipEventRecord(computeDone[i % SETS], cs));
+            return (int)MG_OK;
+        };
+        for (int i = 0; i < nLayers; i++) {
+            const int n = i + 2, set = n % SETS;
+            int crc = MG_OK;
+            if (n >= nLayers) {
+                crc = compute(i);
+            } else {
+                if (n >= SETS) SHIPCHK(hipEventSynchronize(uploadDone[set]));                // layer n - 3 has left the pinned buffer
+                rc = stage(set, layerPtrs + (size_t)n * 12, layerSizes + (size_t)n * 7, 0, 12, [&] { crc = compute(i); });
+                if (rc) return rc;
+                if (n >= SETS) SHIPCHK(hipStreamWaitEvent(uploadStream, computeDone[set], 0));      // ... and the device's weight set
+                rc = upload(n, 0, 12);
                 if (rc) return rc;
             }
+            if (crc) return crc;
         }
-        if (logitsOut) {                                                   // stepFinal :469-484
-            rc = f->enqueueFinal(false);
-            if (rc) return rc;
-            SHIPCHK(hipStreamSynchronize(cs));
-            SHIPCHK(hipMemcpy(logitsOut, f->logits, (size_t)f->vocabSize * 4, hipMemcpyDeviceToHost));
-        }
-        SHIPCHK(hipStreamSynchronize(cs));
-        SHIPCHK(hipStreamSynchronize(uploadStream));
-        return MG_OK;
+        return head ? f->enqueueFinal(false) : MG_OK;
     }
 };
 
