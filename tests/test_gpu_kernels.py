@@ -354,3 +354,23 @@ def test_q4_0_matvec_dp4a_forms(hip, N, K):
     assert np.array_equal(gotB[0], got)
     for t in (dw, da, dscratch, dout, dout2, dq8, doutB):
         t.Release()
+
+
+@pytest.mark.parametrize("N,K,B", [(17, 512, 16), (4100, 2048, 4), (1700, 1024 + 32, 16), (2100, 1024 + 32, 17), (520, 2048, 32), (3017, 192, 33), (600, 4864, 50), (9000, 544, 97)])
+def test_q4_0_batch_tiles(hip, N, K, B):
+    """The matrix-instruction form at the edges of its tiles: remainders of rows, vectors and chunks of blocks."""
+    blocks = ob.quantize_q4_0(E.synth_normal(18, N * 19 + K, 0.02, (N, K)))
+    acts = rng.standard_normal(K * B).astype(np.float32)
+    acts[:32] = 0.0
+    dw, da = _up(hip, blocks), _up(hip, acts)
+    dq8, dout = hip.UploadRawBytes(np.zeros(K // 32 * 40 * B, np.uint8)), hip.FromHost(np.full(B * N, np.nan, np.float32), [B * N])
+    E.KQ8QuantizeActBatch(da, dq8, K, B)
+    E.KQ4_0MatvecDP4ABatch(dw, dq8, dout, N, K, B)
+    _check()
+    got = hip.ToHost(dout).reshape(B, N)
+    for b in {0, 1, min(15, B - 1), min(16, B - 1), B - 2, B - 1}:
+        ref = ob.q4_0_matvec_q8act(ob.q8_quantize_act(acts[b * K:(b + 1) * K]), blocks, N, K, shadow=True, threads=8)
+        assert H.rel_err(got[b], ref) < 1e-5, b
+    assert np.isfinite(got).all()
+    for t in (dw, da, dq8, dout):
+        t.Release()
