@@ -30,7 +30,7 @@ struct FewParams {
     unsigned short* nextHi;
     unsigned short* nextLo;
     int nextQ4;                      // weight format of the projection that reads them
-    float* nextSumSq;                // [tiles of the launch][sumStride]; few_rows_sum_parts(N, T, K) of them
+    float* nextSumSq;                // [tiles of the launch][sumStride]; few_rows_sum_parts(N, T, K, q4) of them
     // FEW_QKV
     void* Kc;
     void* Vc;
@@ -40,7 +40,7 @@ struct FewParams {
     // filled by the launcher
     int nTiles;
 };
-int few_rows_sum_parts(int N, int T, int K);
+int few_rows_sum_parts(int N, int T, int K, int q4);
 // K a multiple of 32, W and the planes 16-byte aligned; FEW_QKV: headDim 64 or 128, N multiples of it.
 hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s);
 

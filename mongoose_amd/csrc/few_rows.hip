@@ -435,26 +435,31 @@ static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
     return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1>(p, s);
 }
 
-// The tile of a launch (16 MT activation rows x 16 NB weight rows a workgroup).  A CU pulls some 53 bytes a nanosecond
-// through its load path here, whether they come from its L2 or from beyond it, and a round of workgroups pays 2.5 us of
-// start-up and end of its own: the tile with the shortest rounds * (start-up + bytes) is taken, with a workgroup on every CU
-// in mind.  (0.5B shape, 37 rows: gate | up in 304 workgroups of 48 x 16 + 16 rows 15.5 us, of 32 x 32 + 32 rows
-// 11.3 us, in 228 of 16 x 64 + 64 rows 10.5 us.)
+// The tile of a launch (16 MT activation rows x 16 NB weight rows a workgroup): the one with the shortest time by a model of
+// a workgroup's nanoseconds -- the bytes it pulls (a CU gets some 80 a nanosecond, whether they come from its L2 or from
+// beyond it), the weights it converts (no other workgroup's conversions serve it: a Q4_0 weight costs three int8 ones), the
+// sums it exchanges -- times the workgroups of the busiest CU, a quarter of which overlap evenly over the chip.  Short rows
+// go through two workgroups a CU at once; tiles of more than four blocks take too many registers for that (1.5).  The
+// constants are a fit to every tile of gate | up and of Wo + down at 64 to 512 rows of the three benchmark shapes, both
+// formats: what it picks is within 2 % of a layer of the best one at all of them.  (Bytes alone and 2.5 us a round of 256
+// workgroups: 301 rows of the 0.5B shape 88 -> 78 us a layer, Q4_0 111 -> 86; 1.1B Q4_0 238 -> 180.)
 struct FewTile { int mt, nb; };
-static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast) {
+static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4) {
     const int b16 = (T + 15) / 16;
     FewTile best{1, nbFirst};
     double least = 1e30;
     for (int nb = nbFirst; nb <= nbLast; nb *= 2)
         for (int mt = 1; mt <= 4 && mt <= b16 && mt * nb <= 8; mt++) {
-            const long long wgs = (long long)((rowsN + 16 * nb - 1) / (16 * nb)) * ((b16 + mt - 1) / mt);
-            const double bytes = (64.0 * mt + 16.0 * nb) * K;
-            const double cost = (double)((wgs + 255) / 256) * (2500.0 + bytes / 53.0) + bytes * (double)wgs * 1e-9;
+            const double wgs = (double)((rowsN + 16 * nb - 1) / (16 * nb)) * ((b16 + mt - 1) / mt);
+            const double bytes = (64.0 * mt + (q4 ? 9.0 : 16.0) * nb) * K;
+            double each = bytes / 80.0 + (q4 ? 0.74 : 0.225) * nb * K + 25.0 * mt * nb;
+            if (K <= 64 * 2 * FR_WAVES && mt * nb > 4) each *= 1.5;
+            const double cost = (0.75 * ceil(wgs / 256.0) + 0.25 * wgs / 256.0) * each;
             if (cost < least) { least = cost; best = FewTile{mt, nb}; }
         }
     return best;
 }
-int few_rows_sum_parts(int N, int T, int K) { const int b = few_tile(N, T, K, 1, 4).nb; return (N + 16 * b - 1) / (16 * b); }
+int few_rows_sum_parts(int N, int T, int K, int q4) { const int b = few_tile(N, T, K, 1, 4, q4).nb; return (N + 16 * b - 1) / (16 * b); }
 
 template <int MODE, int MT, int NB>
 static hipError_t launch_few_fmt(const FewParams& p, hipStream_t s) {
@@ -477,14 +482,14 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
     if (p.K <= 0 || p.K % 32 || !p.Ahi || !p.Alo || p.seg[0].N <= 0) return hipErrorInvalidValue;
     const int N = p.seg[0].N;
     if (mode == FEW_STORE || mode == FEW_RESID) {
-        const FewTile t = few_tile(N, p.T, p.K, 1, 4);
+        const FewTile t = few_tile(N, p.T, p.K, 1, 4, p.q4);
         p.nTiles = (N + 16 * t.nb - 1) / (16 * t.nb);
         if (mode == FEW_STORE) return t.nb == 1 ? launch_few_mt<FEW_STORE, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_STORE, 2>(t.mt, p, s) : launch_few_mt<FEW_STORE, 4>(t.mt, p, s);
         return t.nb == 1 ? launch_few_mt<FEW_RESID, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_RESID, 2>(t.mt, p, s) : launch_few_mt<FEW_RESID, 4>(t.mt, p, s);
     }
     if (mode == FEW_SWIGLU) {
         if (p.seg[1].N != N || !p.nextHi || !p.nextLo) return hipErrorInvalidValue;
-        const FewTile t = few_tile(2 * N, p.T, p.K, 2, 8);
+        const FewTile t = few_tile(2 * N, p.T, p.K, 2, 8, p.q4);
         p.nTiles = (N + 8 * t.nb - 1) / (8 * t.nb);
         return t.nb == 2 ? launch_few_mt<FEW_SWIGLU, 2>(t.mt, p, s) : t.nb == 4 ? launch_few_mt<FEW_SWIGLU, 4>(t.mt, p, s) : launch_few_mt<FEW_SWIGLU, 8>(t.mt, p, s);
     }
@@ -492,7 +497,7 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
         if ((p.headDim != 64 && p.headDim != 128) || N % p.headDim || p.seg[1].N <= 0 || p.seg[1].N % p.headDim ||
             p.seg[2].N != p.seg[1].N || !p.Kc || !p.Vc) return hipErrorInvalidValue;
         p.nTiles = (N + 2 * p.seg[1].N) / 32;
-        return launch_few_mt<FEW_QKV, 2>(few_tile(N + 2 * p.seg[1].N, p.T, p.K, 2, 2).mt, p, s);
+        return launch_few_mt<FEW_QKV, 2>(few_tile(N + 2 * p.seg[1].N, p.T, p.K, 2, 2, p.q4).mt, p, s);
     }
     return hipErrorInvalidValue;
 }

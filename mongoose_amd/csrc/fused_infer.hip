@@ -1811,7 +1811,6 @@ int HIPFusedInference::enqueuePrefillFew(int T, int pos0) {
     HIPCHK(launch_embed_split(table ? embedKind : (lmHead.kind == WF_Q8 ? 0 : 3), table ? embedTable : lmHead.w, table ? nullptr : lmHead.scales,
                               pfTokens, pfX, layers[0].norm1, hi, lo, pfSumSq, T, dim, vocabSize, layers[0].wq.kind == WF_Q4P, stream));
     int parts = 1;
-    const int woParts = few_rows_sum_parts(dim, T, dim), downParts = few_rows_sum_parts(dim, T, ffnDim);
     auto seg = [](const DevMat& m, const float* bias, float* y) {
         return FewSeg{static_cast<const signed char*>(m.w), m.scales, bias, y, m.rows};
     };
@@ -1831,7 +1830,7 @@ int HIPFusedInference::enqueuePrefillFew(int T, int pos0) {
         r.q4 = L.wo.kind == WF_Q4P; r.seg[0] = seg(L.wo, nullptr, pfX);
         r.nextGain = L.norm2; r.nextHi = hi; r.nextLo = lo; r.nextSumSq = pfSumSq; r.nextQ4 = L.gate.kind == WF_Q4P;
         HIPCHK(launch_few_rows(FEW_RESID, r, stream));
-        parts = woParts;
+        parts = few_rows_sum_parts(dim, T, dim, r.q4);
         FewParams g{};
         g.T = T; g.K = dim; g.Ahi = hi; g.Alo = lo; g.eps = eps;
         g.sumSq = pfSumSq; g.sumParts = parts; g.sumStride = T;
@@ -1842,7 +1841,7 @@ int HIPFusedInference::enqueuePrefillFew(int T, int pos0) {
         if (l + 1 < nLayers) { r.nextGain = layers[l + 1].norm1; r.nextQ4 = layers[l + 1].wq.kind == WF_Q4P; }
         else { r.nextGain = nullptr; r.nextHi = nullptr; r.nextLo = nullptr; r.nextSumSq = nullptr; }
         HIPCHK(launch_few_rows(FEW_RESID, r, stream));
-        parts = downParts;
+        parts = few_rows_sum_parts(dim, T, ffnDim, r.q4);
     }
     return MG_OK;
 }
