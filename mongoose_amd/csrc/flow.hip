@@ -996,13 +996,14 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                     // matrices fit the L2s (1.1B shape: 0.465 -> 0.436 ms a token; the down projection on top overflows the L2s:
                     // 0.470), else half of the first round of rows, which is what a phase waits for before it streams (8B shape
                     // with both: 1.845 -> 1.790; the whole first round 1.804, a quarter 1.800).
-                    // Only while at least half the launch is idle (short contexts), and only without dedicated prefetchers.
+                    // Only while at least a third of the launch is idle (1.1B shape at 600 positions, 96 of 256 idle: 477 -> 457 us a token; a
+                    // half before, an eighth gives no more), and only without dedicated prefetchers.
                     if (!hasPrefetchers && (p.idleWoRows > 0 || p.idleGateUpRows > 0)) {
                         const int live = nsplit < G.smax ? nsplit : G.smax;
                         int nBusy = unit * live;
                         if (grouped && nBusy < nHeadsV) nBusy = nHeadsV;
                         nBusy = (nBusy + 7) & ~7;
-                        if ((int)blockIdx.x >= nBusy && 2 * ((int)gridDim.x - nBusy) >= (int)gridDim.x) {
+                        if ((int)blockIdx.x >= nBusy && 3 * ((int)gridDim.x - nBusy) >= (int)gridDim.x) {
                             Prefetcher pf{(int)blockIdx.x & 7, ((int)blockIdx.x - nBusy) >> 3, ((int)gridDim.x - nBusy) >> 3, tid, pfScrap};
                             const size_t rbD = Q4 ? dim >> 1 : dim, rdD = dim >> 4;
                             // (a workgroup without q | k | v rows gets here at the top of the layer; holding it back until q | k | v is
@@ -1878,8 +1879,10 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
 }
 
 __global__ void flow_reset_kernel(uint4* x, size_t n4, const float* hiddenIn, float* hidden, int dim) {
-    if (hiddenIn && blockIdx.x == 0)
-        for (int i = threadIdx.x; i < dim; i += blockDim.x) hidden[i] = hiddenIn[i];
+    // (hiddenIn is page-locked host memory, a microsecond and a half away: one load a thread)
+    if (hiddenIn)
+        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim / 4; i += gridDim.x * blockDim.x)
+            reinterpret_cast<float4*>(hidden)[i] = reinterpret_cast<const float4*>(hiddenIn)[i];
     const uint4 sent = make_uint4(XSENT, XSENT, XSENT, XSENT);
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) x[i] = sent;
 }
