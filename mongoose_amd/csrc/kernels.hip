@@ -130,11 +130,9 @@ template <> struct Fmt<WF_Q4RAW> {
     struct Chunk { int2 w; unsigned short d; };
     __device__ static Chunk load(const Row& r, int c) {
         const unsigned short* b = r.b + (size_t)(c >> 1) * 9;
-        const unsigned short* h = b + 1 + (c & 1) * 4;
         Chunk ck;
         ck.d = b[0];
-        ck.w.x = (int)((unsigned)h[0] | ((unsigned)h[1] << 16));
-        ck.w.y = (int)((unsigned)h[2] | ((unsigned)h[3] << 16));
+        __builtin_memcpy(&ck.w, b + 1 + (c & 1) * 4, 8);        // (one load; it need not be aligned)
         return ck;
     }
     __device__ static float dot(const Chunk& ck, const float4 (&av)[4], float asum, float acc) {
@@ -676,6 +674,26 @@ __global__ __launch_bounds__(WG) void matvec_rows_q4_kernel(MvParams p) {
 MvConfig pick_config(int wf, int epi, int totalRows, int K) {
     const int nch = K / 16;
     MvConfig c;
+    if (epi == EPI_STORE) {
+        // The per-op matvecs.  Tall matrices: a workgroup pays for staging the vector once, so 512 to 1024 of them with
+        // several groups each, four rows a group where rows are short (32000 x 2048 18.9 -> 15.1 us, 50000 x 512 15.1 ->
+        // 11.1, 8039 x 896 5.7 -> 4.8), one where they are long (14336 x 4096 18.0 -> 13.7; raw Q4_0 blocks want four there
+        // too, 19.1 -> 14.0).  Few rows: a row to a workgroup's four waves (256 x 2048 3.34 -> 2.89 us), or one row a wave
+        // (1536 x 2688 4.88 -> 4.39).
+        c.grid = 0;
+        c.ks = 1;
+        if (totalRows > 6000) {
+            c.nr = (K <= 2048 || wf == WF_Q4RAW) ? 4 : 1;
+            c.grid = wf == WF_Q8 && K <= 2048 ? (K <= 1024 ? 768 : 512) : 1024;      // (whole workgroups a CU, not even shares: 15.5 us)
+        } else if (nch > 64 && totalRows <= 512) {
+            c.nr = 1; c.ks = 4;
+        } else if (nch >= 250 && totalRows <= 2048) {
+            c.nr = 4; c.ks = 4;
+        } else {
+            c.nr = totalRows <= (nch > 128 ? 2048 : 1024) ? 1 : 2;
+        }
+        return c;
+    }
     c.ks = (nch > 128 && totalRows <= 2048) ? 4 : 1;
     if (epi == EPI_QKV) {
         c.nr = 2;
