@@ -1348,7 +1348,13 @@ EmbedRef HIPFusedInference::embedRef() const {
     return e;
 }
 int HIPFusedInference::primeGraph() {
-    // (a captured token leaves the exchange area reset for its successor; the first one finds it so from setState)
+    // A captured token resets nothing before it reads: it finds its half of the exchange area as the token before it left
+    // it.  The first one of a run finds it so from here, whatever ran before (setState has done it already where that was
+    // called; a prefill does not touch the area, and eager launches leave a half of it written).
+    if (graphsUseFlow && flowClean != 3) {
+        HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
+        flowClean = 3;
+    }
     return enqueueEmbed();
 }
 

@@ -446,6 +446,45 @@ def test_runs_of_tokens_in_one_launch(hip, fmt):
     m.close()
 
 
+@pytest.mark.parametrize("how", ["decode", "partial", "run"])
+@pytest.mark.parametrize("graphs", ["mixed-formats", "no-tail", "one-token"])
+def test_token_graphs_after_eager_launches(hip, graphs, how):
+    """GeneratePrefill through graph replays finds the exchange area as a reset leaves it, whatever ran before it: an eager
+    token, layers alone, or another run that ended in the half the first replay starts in (same prompt length, an even
+    count of tokens).  Against the same call on a fresh context.  The three ways into graph replays with the launch in use:
+    an lm_head of another format than the layers, the tail switched off, one token a launch."""
+    s = H.with_layers(configs.TOY, 3)
+    fresh, used = (H.Model(s, seed=61, maxSeq=60, eng=hip, oracle=False, fmt="q4_0" if graphs == "mixed-formats" else "q8") for _ in range(2))
+    for m in (fresh, used):
+        if graphs == "mixed-formats":
+            idx = s.nLayers * 12 + 1
+            q, sc = E.quantize_q8(H.gen_slot(s, 61, idx), 0)
+            assert m.hip.SetWeightQ8(idx, q, sc) == 0, E.last_error()
+        elif graphs == "no-tail":
+            assert m.hip.SetFlowTail(False) == 0
+        else:
+            assert m.hip.SetTokensPerLaunch(1) == 0
+        assert m.hip.FlowTailInUse() == (graphs == "one-token")
+    prompt = fresh.prompt(9)
+    rc, ref = fresh.hip.GeneratePrefill(prompt, 12)
+    assert rc == 0, E.last_error()
+    hidden = E.synth_normal(61, 5, 1.0, (s.dim,))
+    for pos in (3, 8, 9):                                   # both halves
+        if how == "decode":
+            rc, _ = used.hip.DecodeToken(int(prompt[0]), pos)
+        elif how == "partial":
+            rc = used.hip.PartialStep(hidden, pos, 0, s.nLayers, None, None)
+        else:
+            rc, _ = used.hip.GeneratePrefill(used.prompt(9)[::-1].copy(), 12)
+        assert rc == 0, E.last_error()
+        assert used.hip.ResetKV() == 0
+        rc, t = used.hip.GeneratePrefill(prompt, 12)
+        assert rc == 0, E.last_error()
+        assert t.tolist() == ref.tolist(), (pos, H.first_divergence(t, ref))
+    fresh.close()
+    used.close()
+
+
 def test_new_context_uses_the_launch_and_trace(hip):
     s = H.with_layers(configs.TOY, 8)
     m = H.Model(s, seed=5, maxSeq=40, eng=hip, threads=8)
