@@ -13,6 +13,7 @@
 #include "kernels.h"
 #include "prefill.h"
 #include "few_rows.h"
+#include "few_rules.h"
 #include "device_util.h"
 
 namespace mg {
@@ -113,12 +114,13 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
     const int N = sg.N;
 
     const int chunks = K >> 6, planeChunks = (K + 63) >> 6;           // whole chunks; a last half one is multiplied after them
+    const int lastChunk = few_last_chunk(K);
     // A lane's weights of a chunk: row fr of the block, 16 of its 64 bytes (Q4_0: 8 bytes of each of two blocks).  Loaded
     // like that a quarter wave touches 16 rows; so lane 16 Q + R loads piece R % 4 of row 4 Q + R / 4 instead (whole
     // rows of 64 bytes) and the pieces change lanes (ds_bpermute).
     const signed char* wP[NB];
     const unsigned short* dP[NB];
-    const int ldRow = 4 * fq + (fr >> 2), ldPiece = fr & 3;
+    const int ldRow = few_load_row(fq, fr), ldPiece = few_piece(fr, K);
     const int from = 4 * (16 * (fr >> 2) + 4 * (fr & 3) + (Q4 ? fq & 1 : fq));      // (bytes: ds_bpermute's lane address)
     auto blockRow = [&](int b, int i) __attribute__((always_inline)) {
         return min((MODE == FEW_SWIGLU ? r0 + (b % (NB / 2 > 0 ? NB / 2 : 1)) * 16 : r0 + b * blk) + i, N - 1);
@@ -126,8 +128,8 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const signed char* W = (MODE == FEW_SWIGLU && b >= NB / 2) ? p.seg[1].W : sg.W;
-        wP[b] = Q4 ? W + (size_t)blockRow(b, ldRow) * (K >> 1) + ldPiece * 8 : W + (size_t)blockRow(b, ldRow) * K + ldPiece * 16;
-        dP[b] = Q4 ? reinterpret_cast<const unsigned short*>(W + (size_t)N * (K >> 1)) + (size_t)blockRow(b, fr) * (K >> 5) : nullptr;
+        wP[b] = W + few_piece_at(blockRow(b, ldRow), ldPiece, K, Q4);
+        dP[b] = Q4 ? reinterpret_cast<const unsigned short*>(W + (size_t)N * (K >> 1)) + few_scales_at(blockRow(b, fr), K) : nullptr;
     }
     const size_t aBlk = (size_t)planeChunks * 1024;                   // elements from one 16-row block to the next
     const unsigned short* aH[MT];
@@ -187,15 +189,15 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
     int4 vw[D][NB];
     unsigned vd[D][NB];
     auto load = [&](int c, uint4 (&h)[MT][2], uint4 (&l)[MT][2], int4 (&w)[NB], unsigned (&d)[NB]) __attribute__((always_inline)) {
-        const int cc = max(min(c, chunks - 1), 0);
+        const int cc = min(c, lastChunk);
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             if (Q4) {
-                const int2 x = *reinterpret_cast<const int2*>(wP[b] + cc * 32);
+                const int2 x = *reinterpret_cast<const int2*>(wP[b] + cc * few_chunk_bytes(1));
                 w[b] = make_int4(x.x, x.y, 0, 0);
                 d[b] = (unsigned)dP[b][cc * 2] | ((unsigned)dP[b][cc * 2 + 1] << 16);
             } else {
-                w[b] = *reinterpret_cast<const int4*>(wP[b] + cc * 64);
+                w[b] = *reinterpret_cast<const int4*>(wP[b] + cc * few_chunk_bytes(0));
             }
         }
         // (every load is unconditional: one under a branch, even a branch that is always taken, makes the compiler's waits
@@ -276,7 +278,7 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
             if (Q4) {
                 const signed char* W = (MODE == FEW_SWIGLU && b >= NB / 2) ? p.seg[1].W : sg.W;
                 f[b] = frag_nib(*reinterpret_cast<const int2*>(W + (size_t)blockRow(b, fr) * (K >> 1) + chunks * 32 + (fq & 1) * 8), fq >= 2 ? 4u : 0u);
-                dd[b] = half_bits_to_float(dP[b][chunks * 2]);
+                dd[b] = half_bits_to_float(dP[b][chunks * 2 + few_own_scale(K)]);
             } else {
                 const signed char* W = (MODE == FEW_SWIGLU && b >= NB / 2) ? p.seg[1].W : sg.W;
                 const int2 x = *reinterpret_cast<const int2*>(W + (size_t)blockRow(b, fr) * K + chunks * 64 + 8 * fq);

@@ -14,12 +14,13 @@ SMALL = configs.TOY._replace(name="small", nLayers=2, dim=448, nHeads=7, nKVHead
 
 
 WIDE = configs.TOY._replace(name="wide", nLayers=2, dim=512, ffnDim=9728, vocab=300)
+NARROW = SMALL._replace(name="narrow", ffnDim=32)          # the down projection's rows are one half chunk, one Q4_0 block
 
 
 @pytest.mark.parametrize("shape,fmt,kv_f16,pos0,rows", [
     (WIDE, "q8", False, 9, 37), (WIDE, "q4_0", False, 0, 64), (SMALL, "q8", False, 0, 1), (SMALL, "q8", False, 0, 16), (SMALL, "q8", False, 3, 17), (SMALL, "q8", False, 130, 64),
     (SMALL, "q4_0", False, 5, 33), (SMALL, "q4_0", True, 0, 48), (ODD, "q8", False, 100, 15), (ODD, "q8", True, 17, 63),
-    (ODD, "q4_0", False, 250, 31)])
+    (ODD, "q4_0", False, 250, 31), (NARROW, "q8", False, 0, 17), (NARROW, "q4_0", False, 2, 33)])
 def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
     m = H.Model(shape, seed=rows, maxSeq=pos0 + rows + 3, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
     toks = m.prompt(pos0 + rows + 1)
@@ -46,7 +47,7 @@ def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
 
 
 @pytest.mark.parametrize("rows,n,k,accumulate", [(1, 16, 32, 0), (17, 33, 96, 1), (64, 300, 1056, 0), (77, 129, 2080, 1), (130, 1000, 4864, 0),
-                                                 (513, 2900, 64, 0), (48, 9000, 64, 0), (300, 5632, 160, 1)])
+                                                 (513, 2900, 64, 0), (48, 9000, 64, 0), (300, 5632, 160, 1), (17, 33, 32, 1), (200, 1000, 32, 0)])
 def test_few_row_gemm_matches_float64(hip, rows, n, k, accumulate):
     rng = np.random.default_rng(rows)
     a = rng.standard_normal((rows, k), dtype=np.float32)
