@@ -110,12 +110,13 @@ public:
     // Persistent launches of several contexts on one device take turns (fused_infer.hip).
     int takeFlowTurn();                     // under flowTurnMutex(), before the launch
     std::mutex& flowTurnMutex() const;
+    std::unique_lock<std::mutex> captureLock() const;
     int launchFlowGraph(hipGraphExec_t ex);
     int launchTokenGraph(hipGraphExec_t ex);
     void leaveFlowTurns();
     int flowDevice = 0;
     hipEvent_t flowTurnEvent = nullptr;     // created with the launch's buffers
-    bool capturing = false;                 // a graph capture of this context is under way (holds flowTurnMutex())
+    bool capturing = false;                 // a graph capture of this context is under way (holds captureLock())
 
     // shape
     int dim, kvDim, headDim, nHeads, nKVHeads, ffnDim, vocabSize, nLayers, maxSeq;

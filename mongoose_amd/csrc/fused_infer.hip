@@ -721,6 +721,13 @@ int HIPFusedInference::takeFlowTurn() {
 }
 std::mutex& HIPFusedInference::flowTurnMutex() const { return g_flowTurns[flowDevice].m; }
 
+// Held while a graph is captured: a context that takes the turn records an event on the stream of the one that launched
+// last, and an event must not be recorded on a stream that is being captured.  That one may have changed to other launches
+// since, so what counts is that this context has ever been in the turns, not whether this capture uses the launch.
+std::unique_lock<std::mutex> HIPFusedInference::captureLock() const {
+    return flowTurnEvent ? std::unique_lock<std::mutex>(flowTurnMutex()) : std::unique_lock<std::mutex>();
+}
+
 // A replay of a captured graph that holds the persistent launch.
 int HIPFusedInference::launchFlowGraph(hipGraphExec_t ex) {
     std::lock_guard<std::mutex> lk(flowTurnMutex());
@@ -1436,9 +1443,7 @@ int HIPFusedInference::GraphCapture() {
     if (flow) { rc = ensureFlow(); if (rc) return rc; }     // allocations and uploads come before the capture
     HIPCHK(hipStreamSynchronize(stream));
     statePosHost = -1;                              // a captured launch is replayed at any position: the variant that covers all
-    // (no other context may record its turn's event on a stream that is being captured)
-    std::unique_lock<std::mutex> lk;
-    if (flow) lk = std::unique_lock<std::mutex>(flowTurnMutex());
+    const auto lk = captureLock();
     for (int which = 0; which < 2; which++) {
         HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
         fuseEmbed = capturing = true;
@@ -1471,8 +1476,7 @@ int HIPFusedInference::LayerGraphCapture(LayerGraph& lg) {
     if (flow) { int rc = ensureFlow(); if (rc) return rc; }          // allocations and uploads come before the capture
     HIPCHK(hipStreamSynchronize(stream));
     statePosHost = -1;                              // (replayed at any position)
-    std::unique_lock<std::mutex> lk;                // (as in GraphCapture)
-    if (flow) lk = std::unique_lock<std::mutex>(flowTurnMutex());
+    const auto lk = captureLock();
     HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
     int rc = MG_OK;
     capturing = true;
