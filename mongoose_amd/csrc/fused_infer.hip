@@ -1119,9 +1119,14 @@ int HIPFusedInference::decodeRun(int nTokens, bool useGraph) {
         return rc;
     }
     for (int i = 0; i < nTokens; i++) {
-        statePosHost = -1;                          // (advanced on the device by launches that do not tell the host)
-        if (useGraph) { int rc = launchTokenGraph(execFull); if (rc) return rc; }
-        else { int rc = enqueueToken(true); if (rc) return rc; }
+        if (useGraph) {
+            statePosHost = -1;                      // (advanced on the device by launches that do not tell the host)
+            int rc = launchTokenGraph(execFull);
+            if (rc) return rc;
+        } else {
+            int rc = enqueueToken(true);
+            if (rc) return rc;
+        }
     }
     return MG_OK;
 }
@@ -1373,6 +1378,7 @@ int HIPFusedInference::enqueueToken(bool withHead) {
     int rc = fuseEmbed ? MG_OK : enqueueEmbed();
     if (rc) return rc;
     const bool flow = flowEligible(0, nLayers);
+    const int clean = flowClean;
     if (flow) {
         rc = ensureFlow();
         if (rc == 0) rc = enqueueLayersFlow(0, nLayers, dState, 0, !fuseEmbed);
@@ -1388,7 +1394,10 @@ int HIPFusedInference::enqueueToken(bool withHead) {
     HIPCHK(launch_advance_prompt(dState, dPrompt, ropeRef(), embedRef(), stream));
     // no lm_head launch to leave the exchange area reset for the next launch: a captured prompt step does it itself,
     // and so does any prompt step where whole tokens run in the launch (they expect to find it so)
-    if (flow && (fuseEmbed || flowTailEligible())) HIPCHK(launch_flow_reset(flowXchg, flowGeo, 0, nLayers, nullptr, nullptr, 0, stream));
+    if (flow && (fuseEmbed || flowTailEligible())) {
+        HIPCHK(launch_flow_reset(flowXchg, flowGeo, 0, nLayers, nullptr, nullptr, 0, stream));
+        if (!capturing) flowClean = clean;          // (the layers' launch wrote the first half only)
+    }
     return MG_OK;
 }
 

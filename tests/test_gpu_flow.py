@@ -485,6 +485,31 @@ def test_token_graphs_after_eager_launches(hip, graphs, how):
     used.close()
 
 
+def _kernels(call):
+    """Names of the kernels a call launches."""
+    import torch
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events()]
+
+
+def test_eager_tokens_reset_the_exchange_area_once_a_run(hip):
+    """A token inside the launch leaves the half of its successor reset: launched one by one from the host (useGraph=False) the
+    tokens of a run need the reset in front of it only, and each prompt step the two of its own half."""
+    s = H.with_layers(configs.TOY, 2)
+    m = H.Model(s, seed=62, maxSeq=40, eng=hip, oracle=False)
+    prompt = m.prompt(5)
+    rc, want = m.hip.Generate(prompt, 16, useGraph=True)
+    assert rc == 0, E.last_error()
+    got = []
+    names = _kernels(lambda: got.append(m.hip.Generate(prompt, 16, useGraph=False)))
+    assert got[0][0] == 0 and got[0][1].tolist() == want.tolist()
+    assert sum("flow_layers_kernel" in n for n in names) == 4 + 16
+    assert sum("flow_reset_kernel" in n for n in names) == 1 + 2 * 4
+    m.close()
+
+
 def test_new_context_uses_the_launch_and_trace(hip):
     s = H.with_layers(configs.TOY, 8)
     m = H.Model(s, seed=5, maxSeq=40, eng=hip, threads=8)
