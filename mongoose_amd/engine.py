@@ -20,30 +20,35 @@ import numpy as np
 
 from .lib import lib, last_error
 
-# Address of an array's data.  `a.ctypes.data` builds an interface object, 0.9 us a time (a streamed token of 24 layers takes
-# 290 of them); the array object itself holds the address in a fixed place, found here by looking for a known one.
-_word = ctypes.c_size_t.from_address
+# Host buffers as typed pointers.  A ctypes object over the array's buffer, passed by reference, takes 0.3 us; the pointer
+# object of `a.ctypes.data_as` takes 2 (a streamed token of 24 layers takes 290 addresses).  Arrays that the buffer protocol
+# does not hand out for writing -- read-only, strided, empty ones -- go the long way.
+def _typed(ctype):
+    pointer = ctypes.POINTER(ctype)
+
+    def ref(a):
+        if a is None:
+            return None
+        try:
+            return ctypes.byref(ctype.from_buffer(a))
+        except (TypeError, ValueError):
+            return a.ctypes.data_as(pointer)
+
+    return ref
 
 
-def _find_data_word():
-    probe = np.zeros(8, np.uint8)
-    for at in range(16, min(probe.__sizeof__(), 64) - 7, 8):
-        if _word(id(probe) + at).value == probe.ctypes.data:
-            other = np.zeros(3, np.float32)
-            return at if _word(id(other) + at).value == other.ctypes.data else None
-    return None
+_fp, _ip = _typed(ctypes.c_float), _typed(ctypes.c_int)
+_i8p, _u8p, _u16p, _i64p = _typed(ctypes.c_int8), _typed(ctypes.c_uint8), _typed(ctypes.c_uint16), _typed(ctypes.c_longlong)
 
 
-_DATA_WORD = _find_data_word()
-
-
-def _fp(a):
-    if a is None:
-        return None
-    return _word(id(a) + _DATA_WORD).value if type(a) is np.ndarray and _DATA_WORD else a.ctypes.data
-
-
-_ip = _fp
+def _addresses(arrays):
+    """Addresses of C-contiguous buffers (None: a NULL pointer) and what has to be kept alive while they are used."""
+    addressof, over = ctypes.addressof, ctypes.c_char.from_buffer
+    try:
+        return [None if a is None else addressof(over(a)) for a in arrays], arrays
+    except (TypeError, ValueError):
+        keep = [None if a is None else np.ascontiguousarray(a) for a in arrays]
+        return [None if a is None else a.ctypes.data for a in keep], keep
 
 
 def _as_f32(a):
@@ -352,7 +357,7 @@ def quantize_q8(w, mode=0):
     rows, cols = w.shape
     q = np.empty((rows, cols), dtype=np.int8)
     s = np.empty(rows, dtype=np.float32)
-    lib.mg_quantize_q8(_fp(w), rows, cols, mode, _fp(q), _fp(s))
+    lib.mg_quantize_q8(_fp(w), rows, cols, mode, _i8p(q), _fp(s))
     return q, s
 
 
@@ -360,7 +365,7 @@ def quantize_q4_0(w):
     w = _as_f32(w)
     rows, cols = w.shape
     out = np.empty(rows * (cols // 32) * 18, dtype=np.uint8)
-    lib.mg_quantize_q4_0(_fp(w), rows, cols, _fp(out))
+    lib.mg_quantize_q4_0(_fp(w), rows, cols, _u8p(out))
     return out
 
 
@@ -436,18 +441,18 @@ class HIPFusedInference:
     def SetWeightQ8(self, idx, q, scales):
         q = np.ascontiguousarray(q, dtype=np.int8)
         s = _as_f32(scales)
-        return lib.mg_set_weight_q8(self._h, idx, _fp(q), _fp(s))
+        return lib.mg_set_weight_q8(self._h, idx, _i8p(q), _fp(s))
 
     def SetWeightQ4_0(self, idx, q4Data):
         a = np.ascontiguousarray(q4Data, dtype=np.uint8).ravel()
-        return lib.mg_set_weight_q4_0(self._h, idx, _fp(a), a.size)
+        return lib.mg_set_weight_q4_0(self._h, idx, _u8p(a), a.size)
 
     def SetQuantRounding(self, mode):
         return lib.mg_set_quant_rounding(self._h, mode)
 
     def SetEmbeddingF16(self, table):
         a = np.ascontiguousarray(table).view(np.uint16)
-        return lib.mg_set_embedding_f16(self._h, _fp(a))
+        return lib.mg_set_embedding_f16(self._h, _u16p(a))
 
     def SetEmbeddingF32(self, table):
         a = _as_f32(table)
@@ -645,7 +650,7 @@ class HIPFusedInference:
         if rc != 0 or not read:
             return rc, None
         buf = np.zeros(int(dims[0]) * int(dims[1]) * int(dims[2]), dtype=np.int64)
-        rc = lib.mg_flow_trace(self._h, 1, _fp(buf), buf.size, _ip(dims))
+        rc = lib.mg_flow_trace(self._h, 1, _i64p(buf), buf.size, _ip(dims))
         return rc, buf.reshape(int(dims[0]), int(dims[1]), int(dims[2]))
 
     def FlowInUse(self):
@@ -678,7 +683,7 @@ class HIPFusedInference:
         if rc != 0:
             return rc, None
         buf = np.zeros(int(dims[0]) * int(dims[1]), dtype=np.int64)
-        rc = lib.mg_flow_tail_trace(self._h, _fp(buf), buf.size, _ip(dims))
+        rc = lib.mg_flow_tail_trace(self._h, _i64p(buf), buf.size, _ip(dims))
         return rc, buf.reshape(int(dims[0]), int(dims[1]))
 
     def SetFlowWaitLimit(self, ticks):
@@ -727,12 +732,12 @@ class HIPStreamInfer:
 
     def StreamForwardToken(self, pos, embHidden, nLayers, layerPtrs, layerSizes, logitsOut):
         """layerPtrs: list of nLayers*12 numpy arrays or None; layerSizes: nLayers*7 ints."""
-        keep = [np.ascontiguousarray(a) if a is not None else None for a in layerPtrs]
-        arr = (ctypes.c_void_p * len(keep))(*map(_fp, keep))
+        at, keep = _addresses(layerPtrs)                   # (the arrays, or copies of them, live until the call is over)
+        arr = (ctypes.c_void_p * len(keep))(*at)
         sizes = np.ascontiguousarray(layerSizes, dtype=np.int32)
         h = _as_f32(embHidden)
         return lib.mg_stream_forward_token(self._h, pos, _fp(h), nLayers, arr,
-                                           _fp(sizes), _fp(logitsOut))
+                                           _ip(sizes), _fp(logitsOut))
 
 
 def KQ8GemmNoAlloc(act, w, scales, bias, out, T, N, K, accumulate):

@@ -5,7 +5,8 @@ raises.  Build it with ``python -m mongoose_amd.build``.
 """
 import ctypes
 import os
-from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_size_t, c_uint16, c_uint64, c_void_p
+from ctypes import (POINTER, c_char_p, c_double, c_float, c_int, c_int8, c_longlong, c_size_t, c_uint8, c_uint16,
+                    c_uint64, c_void_p)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libmongoose_hip.so")
@@ -17,9 +18,9 @@ if not os.path.exists(LIB_PATH):
 
 lib = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_GLOBAL)
 
-# Host buffers are passed by address (an int, or any ctypes pointer): making a typed pointer object of a numpy array takes
-# longer than a small call of the library.
-_f = _i = c_void_p
+# Host buffers: typed pointers, so that one of another type is refused.
+_f, _i = POINTER(c_float), POINTER(c_int)
+_i8, _u8, _u16, _i64 = POINTER(c_int8), POINTER(c_uint8), POINTER(c_uint16), POINTER(c_longlong)
 
 
 def _sig(name, restype, *argtypes):
@@ -81,11 +82,11 @@ _sig("mg_destroy", None, c_void_p)
 _sig("mg_last_error", c_char_p)
 _sig("mg_num_weights", c_int, c_void_p)
 _sig("mg_set_weight", c_int, c_void_p, c_int, _f, c_size_t)
-_sig("mg_set_weight_q8", c_int, c_void_p, c_int, c_void_p, _f)
-_sig("mg_set_weight_q4_0", c_int, c_void_p, c_int, c_void_p, c_size_t)
+_sig("mg_set_weight_q8", c_int, c_void_p, c_int, _i8, _f)
+_sig("mg_set_weight_q4_0", c_int, c_void_p, c_int, _u8, c_size_t)
 _sig("mg_set_q4_act_quant", c_int, c_void_p, c_int)
 _sig("mg_set_quant_rounding", c_int, c_void_p, c_int)
-_sig("mg_set_embedding_f16", c_int, c_void_p, c_void_p)
+_sig("mg_set_embedding_f16", c_int, c_void_p, _u16)
 _sig("mg_set_embedding_f32", c_int, c_void_p, _f)
 _sig("mg_set_layer_range", c_int, c_void_p, c_int, c_int)
 _sig("mg_reset_kv", c_int, c_void_p)
@@ -96,7 +97,7 @@ _sig("mg_export_hidden", c_int, c_void_p, _f)
 _sig("mg_set_exec_mode", c_int, c_void_p, c_int)
 _sig("mg_queue_hidden_to_l3", c_int, c_void_p)
 _sig("mg_wait_l3", c_int, c_void_p)
-_sig("mg_get_l3_hidden", POINTER(c_float), c_void_p)
+_sig("mg_get_l3_hidden", _f, c_void_p)
 _sig("mg_signal_mailbox", c_int, c_void_p)
 _sig("mg_wait_mailbox", c_int, c_void_p, c_int)
 _sig("mg_swap_hidden_buffer", c_int, c_void_p)
@@ -126,18 +127,18 @@ _sig("mg_set_flow_tail", c_int, c_void_p, c_int)
 _sig("mg_set_flow_generic", c_int, c_void_p, c_int)
 _sig("mg_set_tokens_per_launch", c_int, c_void_p, c_int)
 _sig("mg_tokens_per_launch", c_int, c_void_p)
-_sig("mg_flow_tail_trace", c_int, c_void_p, c_void_p, c_size_t, _i)
-_sig("mg_flow_set_wait_limit", c_int, c_void_p, ctypes.c_longlong)
-_sig("mg_flow_trace", c_int, c_void_p, c_int, c_void_p, c_size_t, _i)
+_sig("mg_flow_tail_trace", c_int, c_void_p, _i64, c_size_t, _i)
+_sig("mg_flow_set_wait_limit", c_int, c_void_p, c_longlong)
+_sig("mg_flow_trace", c_int, c_void_p, c_int, _i64, c_size_t, _i)
 _sig("mg_weight_bytes_per_token", c_uint64, c_void_p)
 _sig("mg_kv_bytes_at", c_uint64, c_void_p, c_int)
 _sig("mg_stream_build", c_void_p, c_void_p)
 _sig("mg_stream_destroy", None, c_void_p)
-_sig("mg_stream_forward_token", c_int, c_void_p, c_int, _f, c_int, POINTER(c_void_p), c_void_p, _f)
+_sig("mg_stream_forward_token", c_int, c_void_p, c_int, _f, c_int, POINTER(c_void_p), _i, _f)
 
 # host helpers
-_sig("mg_quantize_q8", None, _f, c_int, c_int, c_int, c_void_p, _f)
-_sig("mg_quantize_q4_0", None, _f, c_int, c_int, c_void_p)
+_sig("mg_quantize_q8", None, _f, c_int, c_int, c_int, _i8, _f)
+_sig("mg_quantize_q4_0", None, _f, c_int, c_int, _u8)
 _sig("mg_f32_to_f16", c_uint16, c_float)
 _sig("mg_f16_to_f32", c_float, c_uint16)
 _sig("mg_synth_normal", None, c_uint64, c_uint64, c_float, _f, c_size_t)

@@ -1,11 +1,13 @@
 """CPU-side checks of the product: the C ABI library loads and exports every
 symbol the header declares, and its host-side quantizers / fp16 conversion /
 synthetic generator agree bit for bit with the oracle (no GPU needed)."""
+import ctypes
 import os
 import re
 import subprocess
 
 import numpy as np
+import pytest
 
 from mongoose_amd import engine as E
 from mongoose_amd.lib import LIB_PATH, lib
@@ -108,3 +110,37 @@ def test_host_worker_pool_is_safe_under_concurrent_callers():
     for t in ths:
         t.join()
     assert not bad, bad[:5]
+
+
+def test_buffers_of_another_type_are_refused():
+    """A pointer to ints where the library takes floats is an error of the call, not an address to read from."""
+    w, q, sc = np.ones((1, 32), np.float32), np.empty((1, 32), np.int8), np.empty(1, np.float32)
+    f, i8 = (lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_float))), (lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_int8)))
+    lib.mg_quantize_q8(f(w), 1, 32, 0, i8(q), f(sc))
+    assert (q == 127).all()
+    for bad in ((i8(q), i8(q), f(sc)), (f(w), f(sc), f(sc)), (w.ctypes.data, i8(q), f(sc))):
+        with pytest.raises(ctypes.ArgumentError):
+            lib.mg_quantize_q8(bad[0], 1, 32, 0, bad[1], bad[2])
+
+
+def test_buffers_reach_the_library_whatever_their_kind():
+    """Writable, read-only, strided and Fortran-ordered arrays: the same bytes, and the address of a copy only where one has
+    to be made."""
+    a = np.arange(96, dtype=np.float32).reshape(3, 32) - 40
+    want = E.quantize_q8(a)
+    ro = a.copy()
+    ro.flags.writeable = False
+    for v in (ro, np.asfortranarray(a), np.repeat(a, 2, axis=1)[:, ::2]):
+        got = E.quantize_q8(v)
+        assert (got[0] == want[0]).all() and (got[1] == want[1]).all()
+
+    def read(at, n):
+        return bytes((ctypes.c_char * n).from_address(at))
+
+    at, keep = E._addresses([a, None, ro[1:]])
+    assert at == [a.ctypes.data, None, ro[1:].ctypes.data] and keep[1] is None
+    at, keep = E._addresses([a, None])
+    assert at == [a.ctypes.data, None]
+    at, keep = E._addresses([a.T, a])
+    assert at[1] == a.ctypes.data and read(at[0], a.nbytes) == np.ascontiguousarray(a.T).tobytes()
+    assert E._fp(np.empty(0, np.float32)) is not None and E._fp(None) is None
