@@ -1,6 +1,8 @@
-// few_rules.h -- where the few-row kernels (few_rows.hip) read a weight matrix, in plain C++: the kernels use these
-// functions, and so does the host test that walks them over whole matrices.
+// few_rules.h -- where the few-row kernels (few_rows.hip) read a weight matrix and which prefills take them, in plain C++:
+// the kernels and the dispatch use these functions, and so do the host tests that walk them over whole matrices and over
+// what was measured.
 #pragma once
+#include <cmath>
 #include <cstddef>
 
 namespace mg {
@@ -21,5 +23,35 @@ constexpr int few_last_chunk(int K) { return K < 64 ? 0 : (K >> 6) - 1; }
 // which the last row does not have.  few_own_scale: where the row's first scale then lies.
 constexpr int few_own_scale(int K) { return K < 64 ? 1 : 0; }
 constexpr long long few_scales_at(int row, int K) { return (long long)row * (K >> 5) - few_own_scale(K); }
+
+// ---- which prefills take the few-row kernels, and which the tiled GEMMs (prefill.hip) ----
+// Rows up to which some prefill takes them.  The tiled GEMMs want work for every CU, so the line falls with the weights of a
+// layer.  Microseconds a layer, few-row / tiled, Q8 and Q4_0, nothing cached: 0.5B shape (15 million weights) 36 / 69 and
+// 39 / 77 at 37 rows, 103 / 119 and 118 / 141 at 506, 138 / 136 and 156 / 154 at 625; 1.1B (44) 147 / 164 and 182 / 203 at
+// 294, 161 / 173 and 203 / 211 at 346, 183 / 191 and 239 / 219 at 415; 8B (218) 236 / 243 and 286 / 297 at 124.
+inline int few_rows_most(int dim, int kvDim, int ffn) {
+    const double millions = ((double)dim * (2.0 * dim + 2.0 * kvDim) + 3.0 * dim * ffn) * 1e-6;
+    const int n = (int)(2300.0 / std::sqrt(millions));
+    return n < 1500 ? n : 1500;
+}
+// T rows behind pos0 cached ones.
+//   * The largest Q8 layers, past 128 rows: a third block of 64 rows through every few-row tile costs more than the half-filled second
+//     tile of 128 rows does (dim 4096: ffn 11008 at 137 rows 299 / 322, 12288 at 132 300 / 291; 3584 x 14336 at 152 296 / 270;
+//     4096 x 14336 at 132 315 / 275).  Q4_0 layers, whose conversions weigh more in the tiled GEMMs, keep the line above
+//     (380 / 367 there, 352 / 347 at 3584 x 14336, 303 / 340 at 4096 x 11008); so do layers whose attention is one round
+//     (below) behind a long cache (3584 x 14336, 28 heads, 144 rows: 270 / 262, behind 3,000 333 / 391).
+//   * Cached rows: the few-row attention takes a workgroup a query head and 16 rows, 256 at a time, and each such round reads the
+//     cache once; the tiled one splits the cache rows in a pass of its own and reads them once for 128 rows.  One or two
+//     rounds cost less than that for every cached row (heads of 64: 0.011 us a round against 0.026; of 128: 0.020 against
+//     0.042), so the line does not move: 8B at 128 rows behind 12,000 472 / 757, 1.1B at 256 391 / 447.  With three rounds the
+//     projections' lead is used up after 400 (at the line) to 3,000 rows (at three quarters of it): 0.5B at 590 rows 133 / 136
+//     with nothing cached, 154 / 150 behind 600, 331 / 283 behind 6,000; 1.1B at 301 167 / 184 behind 600, 247 / 246
+//     behind 3,000, 350 / 324 behind 6,000; the toy shape at 1,034 107 / 123 and, behind 3,000, 208 / 202.
+inline bool few_rows_pay(int T, int pos0, int dim, int kvDim, int ffn, int nHeads, bool q4) {
+    const int most = few_rows_most(dim, kvDim, ffn);
+    const int rounds = (int)(((long long)nHeads * ((T + 15) / 16) + 255) / 256);
+    if (T > most || (!q4 && T > 128 && 3.0 * dim * ffn > 145e6 && (rounds > 1 || pos0 < 800))) return false;
+    return rounds <= 2 || T <= most * (1.05 - pos0 / 8000.0);
+}
 
 }  // namespace mg

@@ -6,6 +6,7 @@
 #pragma once
 #include "kernels.h"
 #include "flow.h"
+#include "few_rules.h"
 
 #include <algorithm>
 #include <cmath>
@@ -165,14 +166,6 @@ private:
     float* pfPartial = nullptr;
     int ensurePrefill(int rows, int kvRows);
     float* pfSumSq = nullptr;               // few-row path: partial sums of squares of the rows
-    // Rows up to which a prefill takes the few-row kernels.  The tiled GEMMs want work for every CU, so the line falls with
-    // the weights of a layer.  Microseconds a layer, few-row / tiled, measured, Q8 and Q4_0: 0.5B shape (15 million) 35 / 69
-    // at 32 rows, 104 / 120 at 512, 140 / 137 and 158 / 153 at 640; 1.1B (44) 160 / 178 and 184 / 203 at 301, 214 / 205 and
-    // 257 / 224 at 448; 8B (218) 243 / 248 and 298 / 304 at 128, 356 / 310 and 441 / 374 at 192.
-    int fewRowsLimit() const {
-        const double w = ((double)dim * (2.0 * dim + 2.0 * kvDim) + 3.0 * dim * ffnDim) * 1e-6;
-        return std::min(1500, (int)(2300.0 / std::sqrt(w)));
-    }
     int enqueuePrefillFew(int T, int pos0);
     int enqueuePrefillTiles(int T, int pos0);
     std::vector<Slab> layerSlabs, kvSlabs;

@@ -1740,7 +1740,7 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     prefillCap = 0;
     const size_t T = ((size_t)rows + 127) / 128 * 128;
     const size_t plane = split_plane_elems((int)T, ffnDim > dim ? ffnDim : dim) * 2;
-    const size_t sums = (size_t)(dim / 16 + 1) * std::min<size_t>(T, (size_t)fewRowsLimit());
+    const size_t sums = (size_t)(dim / 16 + 1) * std::min<size_t>(T, (size_t)few_rows_most(dim, kvDim, ffnDim));
     size_t bytes = alignUp256(sums * 4) + 2 * alignUp256(T * dim * 4) + 2 * alignUp256(T * kvDim * 4) +
                    2 * alignUp256(T * ffnDim * 4) + 4 * alignUp256(plane) + alignUp256(gemm_partial_floats() * 4) + 16 * 256;
     int rc = prefillSlab.init(bytes);
@@ -1881,7 +1881,7 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
     rc = ensurePrefill(nTokens, pos0 + nTokens);
     if (rc) return rc;
     const int T = nTokens;
-    const bool few = T <= fewRowsLimit();
+    const bool few = few_rows_pay(T, pos0, dim, kvDim, ffnDim, nHeads, layers[0].gate.kind == WF_Q4P);
     std::memcpy(hIn, tokens, sizeof(int) * (size_t)T);              // (the embedding rows' launch reads them there)
     pfTokens = reinterpret_cast<const int*>(hIn);
     if (elapsedMs) HIPCHK(hipEventRecord(ev0, stream));

@@ -1,4 +1,4 @@
-"""Where the few-row kernels read a weight matrix (few_rules.h), compiled for the host and walked over whole matrices."""
+"""Where the few-row kernels read a weight matrix and which prefills take them (few_rules.h), compiled for the host."""
 import os
 import subprocess
 
@@ -45,3 +45,21 @@ int main() {
 }
 """ % q4)
     assert out == "ok\n", out
+
+
+QWEN, TINY, LLAMA, TOY = (896, 128, 4864, 14), (2048, 256, 5632, 32), (4096, 1024, 14336, 32), (512, 128, 1376, 8)
+
+
+# (shape, Q4_0, rows, cached rows, microseconds a layer few-row and tiled) as measured where the two differ by more than 4 %
+@pytest.mark.parametrize("shape,q4,rows,pos0,few,tiled", [
+    (TOY, 0, 646, 0, 73, 101), (TOY, 0, 970, 12000, 361, 438), (TOY, 0, 1293, 3000, 225, 214), (TOY, 0, 1380, 6000, 334, 304),
+    (QWEN, 0, 37, 200, 38, 74), (QWEN, 0, 512, 6000, 234, 269), (QWEN, 0, 590, 3000, 233, 208), (QWEN, 1, 301, 12000, 346, 418),
+    (QWEN, 1, 590, 1500, 198, 189), (TINY, 0, 301, 600, 167, 184), (TINY, 0, 301, 6000, 350, 324), (TINY, 0, 256, 12000, 391, 447),
+    (TINY, 1, 340, 3000, 303, 285), (TINY, 1, 448, 0, 257, 224), (LLAMA, 0, 64, 12000, 407, 701), (LLAMA, 0, 128, 12000, 472, 757),
+    (LLAMA, 0, 132, 0, 315, 275), (LLAMA, 0, 150, 6000, 564, 542), (LLAMA, 1, 128, 0, 280, 298), (LLAMA, 1, 192, 0, 441, 374),
+    ((4096, 4096, 11008, 32), 0, 137, 0, 299, 322), ((3584, 512, 14336, 28), 0, 152, 0, 296, 270),
+    ((3584, 512, 14336, 28), 0, 144, 3000, 333, 391), ((3584, 512, 14336, 28), 0, 152, 3000, 418, 395)])
+def test_the_faster_path_is_taken(tmp_path, shape, q4, rows, pos0, few, tiled):
+    out = _run(tmp_path, '#include "few_rules.h"\n#include <cstdio>\nint main() { std::puts(mg::few_rows_pay(%d, %d, %d, %d, %d, %d, %d != 0) ? "few" : "tiled"); }'
+               % (rows, pos0, *shape, q4))
+    assert out.strip() == ("few" if few < tiled else "tiled")
