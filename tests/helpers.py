@@ -138,6 +138,15 @@ def oracle_generate(m, prompt, nDecode, want=None, shadow=False):
     return np.array(toks, np.int32), rec
 
 
+def launched(call):
+    """Names of the kernels that a call launches."""
+    import torch
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events()]
+
+
 def first_divergence(a, b):
     """Index of the first position where two token sequences differ, or None."""
     n = min(len(a), len(b))

@@ -485,15 +485,6 @@ def test_token_graphs_after_eager_launches(hip, graphs, how):
     used.close()
 
 
-def _kernels(call):
-    """Names of the kernels a call launches."""
-    import torch
-    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
-        call()
-        torch.cuda.synchronize()
-    return [e.name for e in prof.events()]
-
-
 def test_eager_tokens_reset_the_exchange_area_once_a_run(hip):
     """A token inside the launch leaves the half of its successor reset: launched one by one from the host (useGraph=False) the
     tokens of a run need the reset in front of it only, and each prompt step the two of its own half."""
@@ -503,7 +494,7 @@ def test_eager_tokens_reset_the_exchange_area_once_a_run(hip):
     rc, want = m.hip.Generate(prompt, 16, useGraph=True)
     assert rc == 0, E.last_error()
     got = []
-    names = _kernels(lambda: got.append(m.hip.Generate(prompt, 16, useGraph=False)))
+    names = H.launched(lambda: got.append(m.hip.Generate(prompt, 16, useGraph=False)))
     assert got[0][0] == 0 and got[0][1].tolist() == want.tolist()
     assert sum("flow_layers_kernel" in n for n in names) == 4 + 16
     assert sum("flow_reset_kernel" in n for n in names) == 1 + 2 * 4

@@ -1,4 +1,5 @@
-"""Batched prefill (MFMA GEMM path) against the token-by-token decode step.
+"""Batched prefill, on the few-row kernels (few_rows.hip: what most prompts here take) and on the tiled GEMMs (prefill.hip:
+the longer ones, the `tiled` tests), against the token-by-token decode step.
 
 The reference has no batched prompt path: its semantics for a prompt are the
 decode step applied position by position, which is what the oracle does here.
@@ -27,10 +28,26 @@ def _up(eng, a):
 @pytest.mark.parametrize("T,N,K,acc,bias", [
     (1, 128, 32, False, False), (5, 100, 64, False, True), (130, 300, 896, True, False),
     (128, 128, 4864, False, False), (257, 1376, 512, True, True), (512, 1024, 4096, False, False),
-    # enough 256 x 256 tiles for the direct-to-LDS ring kernel: accumulate form, bias form, odd count of 32-wide K steps
+    # wide matrices: accumulate form, bias form, odd count of 32-wide K steps
     (512, 12288, 64, True, False), (300, 12800, 96, False, True),
 ])
 def test_q8_gemm_against_float64(hip, T, N, K, acc, bias):
+    _gemm_against_float64(hip, T, N, K, acc, bias)
+
+
+@pytest.mark.parametrize("T,N,K,acc,bias,kernel", [
+    # past the few-row kernel's line: the small tiles; 256 x 256 tiles with K not a multiple of 128, and through the
+    # direct-to-LDS ring (accumulate and bias forms of each; the last row and column tiles partly empty)
+    (513, 2925, 32, True, False, "gemm_q8_bf16x2_kernel<0, 64, 128, 256, 1>"), (520, 3001, 96, False, True, "gemm_q8_bf16x2_kernel<0, 64, 128, 256, 0>"),
+    (600, 17408, 64, True, False, "gemm_q8_bf16x2_kernel<0, 256, 256, 1024, 1>"), (550, 17300, 96, False, True, "gemm_q8_bf16x2_kernel<0, 256, 256, 1024, 0>"),
+    (600, 17400, 128, True, True, "gemm_q8_ring_kernel<1>"), (530, 17408, 384, False, True, "gemm_q8_ring_kernel<0>"),
+])
+def test_q8_gemm_tiled_against_float64(hip, T, N, K, acc, bias, kernel):
+    names = H.launched(lambda: _gemm_against_float64(hip, T, N, K, acc, bias))
+    assert any(kernel in n for n in names) and not any("few_rows" in n for n in names), names
+
+
+def _gemm_against_float64(hip, T, N, K, acc, bias):
     print(f"q8 gemm T={T} N={N} K={K} acc={acc} bias={bias}", flush=True)
     w = E.synth_normal(9, T * 7 + N, 0.02, (N, K))
     q, s = ob.quantize_q8(w)
@@ -130,14 +147,14 @@ def test_prefill_toy_matches_decode(hip):
 
 
 def test_prefill_qwen_shape_with_bias(hip):
-    """Qwen2.5-0.5B shape (GQA 14/2, head 64, QKV bias), 3 layers, 200-token prompt (two row tiles)."""
+    """Qwen2.5-0.5B shape (GQA 14/2, head 64, QKV bias), 3 layers, 200-token prompt (few-row kernels, 13 row blocks)."""
     s = H.with_layers(configs.QWEN, 3)
     m, _, _ = _prefill_case(hip, s, seed=3, nPrompt=200, nDecode=8, maxSeq=256)
     m.close()
 
 
 def test_prefill_llama3_shape_one_layer(hip):
-    """Llama-3-8B shape (head 128, GQA 32/8), 1 layer, 160-token prompt."""
+    """Llama-3-8B shape (head 128, GQA 32/8), 1 layer, 160-token prompt (tiled GEMMs: past 128 rows)."""
     s = H.with_layers(configs.LLAMA3_8B, 1)
     m, _, _ = _prefill_case(hip, s, seed=4, nPrompt=160, nDecode=4, maxSeq=192)
     m.close()
@@ -154,9 +171,8 @@ def test_prefill_llama3_shape_two_row_tiles(hip):
 
 
 def test_prefill_wide_ffn_with_a_partial_column_tile(hip):
-    """An FFN of 80.5 tiles of 128 columns at 300 rows: the gate|up GEMM runs unsplit on the 256 x 256 tiles and forms
-    silu(gate)*up itself.  Whole tiles leave through LDS as 128-byte rows (row blocks past the planes' 384 rows are
-    skipped), the last tile has 64 columns and stores element by element; the down projection then reads both."""
+    """An FFN of 80.5 tiles of 128 columns at 300 rows, on the few-row kernels (the tiled GEMMs' partial gate|up tile:
+    test_tiled_prefill)."""
     s = configs.Shape("ffn-edge", 1, 256, 4, 2, 64, 10304, 512, 1e-5, 1e4, False, True, "q8")
     m, _, _ = _prefill_case(hip, s, seed=21, nPrompt=300, nDecode=2, maxSeq=320)
     m.close()
@@ -208,14 +224,69 @@ def test_prefill_errors(hip):
 
 
 def test_prefill_qwen_q4_0_shape(hip):
-    """Qwen shape with GGUF Q4_0 weights and an fp16 embedding table, 2 layers, 150-token prompt (large-tile path)."""
+    """Qwen shape with GGUF Q4_0 weights and an fp16 embedding table, 2 layers, 150-token prompt."""
     s = H.with_layers(configs.QWEN_Q4, 2)
     m, _, _ = _prefill_case(hip, s, seed=5, nPrompt=150, nDecode=6, maxSeq=192)
     m.close()
 
 
 def test_prefill_q4_0_short_prompt_and_k_tail(hip):
-    """Toy shape in Q4_0 (ffn 1376: a K of 43 blocks, odd, so the last K step is half empty), 40-token prompt (small tiles)."""
+    """Toy shape in Q4_0 (ffn 1376: a K of 43 blocks, odd, so the last K step is half empty), 40-token prompt."""
     s = configs.TOY._replace(fmt="q4_0", name="toy-q4")
     m, _, _ = _prefill_case(hip, s, seed=6, nPrompt=40, nDecode=6, maxSeq=64)
+    m.close()
+
+
+EDGE = configs.Shape("ffn-edge", 1, 256, 4, 2, 64, 10304, 512, 1e-5, 1e4, True, True, "q8")
+ODD = configs.Shape("odd", 2, 384, 3, 1, 128, 1408, 300, 1e-6, 1e4, True, True, "q8")
+MINI = configs.Shape("l3-mini", 2, 512, 4, 1, 128, 1024, 512, 1e-5, 5e5, True, True, "q8")
+
+
+@pytest.mark.parametrize("s,fmt,kv_f16,pos0,rows,kernels", [
+    # an FFN of 80.5 tiles of 128 columns: the gate|up GEMM runs unsplit on the 256 x 256 tiles and forms silu(gate)*up
+    # itself.  Whole tiles leave through LDS as 128-byte rows (row blocks past the planes' 896 rows are skipped), the last
+    # tile has 64 columns and stores element by element; the down projection then reads both.  Biases without a K split
+    (EDGE, "q8", False, 0, 820, ["gemm_q8_ring_kernel<3>", "rope_store_rows"]),
+    # ... and in Q4_0, whose gate and up leave the GEMM apart
+    (EDGE, "q4_0", False, 7, 820, ["gemm_q8_bf16x2_kernel<1, 128, 256, 512, 0>", "swiglu_split_kernel"]),
+    # K split: biases, RoPE and fp16 K/V rows in the kernel that sums the splits
+    (H.with_layers(configs.QWEN, 2), "q8", True, 0, 600, ["gemm_q8_bf16x2_kernel<0, 64, 128, 256, 2>", "gemm_reduce_qkv_rope"]),
+    # Q4_0 gate|up with the SwiGLU in the epilogue of the tiles in between; an fp16 embedding table
+    (H.with_layers(configs.QWEN_Q4, 2), "q4_0", False, 33, 600, ["gemm_q8_bf16x2_kernel<1, 128, 256, 512, 3>", "gemm_reduce_norm_split"]),
+    # heads of 128 in groups of 3, widths that end inside a tile: SwiGLU in the small tiles' epilogue, K/V rows of 128
+    (ODD, "q8", False, 0, 1505, ["gemm_q8_bf16x2_kernel<0, 64, 128, 256, 3>", "rope_store_rows"]),
+    (ODD, "q4_0", True, 3, 1505, ["gemm_q8_bf16x2_kernel<1, 64, 128, 256, 1>", "rope_store_rows"]),
+    (MINI, "q8", True, 0, 1510, ["gemm_reduce_swiglu_split", "gemm_reduce_qkv_rope"]),
+    # a K of 43 blocks: the last K step is half empty
+    (configs.TOY, "q4_0", False, 0, 1390, ["gemm_q8_bf16x2_kernel<1, 64, 128, 256, 2>", "gemm_reduce_swiglu_split"]),
+    # large matrices: the ring kernel with K splits; Q4_0 on the large tiles with and without, fp16 K/V rows
+    (H.with_layers(configs.TINYLLAMA, 1)._replace(vocab=2000), "q8", False, 0, 350, ["gemm_q8_ring_kernel<2>"]),
+    (H.with_layers(configs.LLAMA3_8B, 1)._replace(vocab=2000), "q4_0", True, 0, 170, ["gemm_q8_bf16x2_kernel<1, 128, 256, 512, 2>", "swiglu_split_kernel"]),
+    # behind cached rows, three rounds of attention workgroups: a prefill that takes the few-row kernels with nothing cached
+    (H.with_layers(configs.TOY, 1), "q8", False, 3000, 1050, ["gemm_q8_bf16x2_kernel"]),
+], ids=lambda v: getattr(v, "name", None))
+def test_tiled_prefill(hip, s, fmt, kv_f16, pos0, rows, kernels):
+    """The tiled GEMMs against the oracle: the last row's logits, and those of a token behind it, which reads every K/V row.
+    The bars: a product's two bf16 terms leave 2^-16 of an activation, some 1e-5 of the logits over these layers, ten times
+    that is asked for; fp16 rows round at 2^-11 of a value, averaged over the rows, and keep the logit bar."""
+    m = H.Model(s, seed=rows, maxSeq=pos0 + rows + 2, eng=hip, threads=16, fmt=fmt, kv_f16=kv_f16)
+    toks = m.prompt(pos0 + rows + 1)
+    want = []
+    m.orc.reset_kv()
+    for pos, tok in enumerate(toks):
+        _, logits, _ = m.orc.decode_token(int(tok), pos, shadow=True, want_layers=False)
+        if pos >= pos0 + rows - 1:
+            want.append(logits.copy())
+    for p in range(0, pos0, 1000):
+        assert m.hip.Prefill(toks[p:min(pos0, p + 1000)], p)[0] == 0, E.last_error()
+    got = []
+    names = H.launched(lambda: got.append(m.hip.Prefill(toks[pos0:pos0 + rows], pos0, wantLogits=True)))
+    rc, nxt, logits, _ = got[0]
+    assert rc == 0, E.last_error()
+    assert not any("few_" in n for n in names) and all(any(k in n for n in names) for k in kernels), sorted(set(names))
+    bar = 1e-3 if kv_f16 else 1e-4
+    assert H.rel_err(logits, want[0]) < bar and nxt == int(np.argmax(want[0]))
+    after = np.empty(s.vocab, np.float32)
+    rc, _ = m.hip.DecodeToken(int(toks[-1]), pos0 + rows, after)
+    assert rc == 0 and H.rel_err(after, want[1]) < bar
     m.close()
