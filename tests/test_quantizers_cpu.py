@@ -74,7 +74,11 @@ extern "C" void q4(int isa, const float* w, size_t nb, uint8_t* out) {
     so = d / "v.so"
     subprocess.run(["g++", "-O3", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", "-w", "-I", os.path.join(ROOT, "mongoose_amd", "csrc"),
                     str(d / "v.cpp"), "-o", str(so), "-lpthread"], check=True)
-    return ctypes.CDLL(str(so))
+    v = ctypes.CDLL(str(so))
+    f, i8, u8 = ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_int8), ctypes.POINTER(ctypes.c_uint8)
+    v.q8.argtypes = [ctypes.c_int, f, ctypes.c_int, ctypes.c_int, ctypes.c_int, i8, f]
+    v.q4.argtypes = [ctypes.c_int, f, ctypes.c_size_t, u8]
+    return v
 
 
 @pytest.mark.parametrize("isa", [0, 1, 2], ids=["plain", "avx2", "avx512"])
@@ -91,7 +95,7 @@ def test_every_instruction_set(variants, isa, monkeypatch):
 
     def q4(w):
         out = np.empty(w.size // 32 * 18, np.uint8)
-        variants.q4(isa, E._fp(w), ctypes.c_size_t(w.size // 32), E._u8p(out))
+        variants.q4(isa, E._fp(w), w.size // 32, E._u8p(out))
         return out
 
     monkeypatch.setattr(E, "quantize_q8", q8)
