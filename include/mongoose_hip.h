@@ -259,7 +259,7 @@ int mg_hidden_idx(mg_ctx* ctx);
  * also fetch the following matrices into L2 with its idle workgroups (for a GPU
  * shared with other work); 3 = all layers of a step in ONE persistent launch whose
  * workgroups hand their vectors over through device memory, wherever the model allows it
- * (all matrices of the layers Q8, or all Q4_0; fp32 KV rows, heads of 64 or 128, a context of at most
+ * (all matrices of the layers Q8, or all Q4_0; heads of 64 or 128, a context of at most
  * 128 x floor(CUs / nKVHeads) positions -- an attention workgroup per query head and 128 positions where
  * that covers the context, else per KV head -- with at most 8 query heads a KV head; otherwise as mode 1).
  * In mode 3, 32 of the launch's workgroups compute nothing and instead read the weights that the others
@@ -267,10 +267,10 @@ int mg_hidden_idx(mg_ctx* ctx);
  * 4 = mode 3 with every workgroup computing (bit-identical results; for comparison).
  * A new context is in mode 3 (measured against mode 1: 0.5B shape 56 % more tokens per second, 1.1B
  * shape 59 %, 8B shape 20 %, also at contexts of thousands of positions).
- * On every device one context at a time owns the persistent launch -- the first that needs it, until it is
- * destroyed or set to another mode (mg_flow_in_use).  Other contexts' launches take turns with the owner's (two at
- * once could each hold part of the CUs and wait for workgroups that cannot start): one queued behind another
- * context's waits on the device for what that context has queued so far.
+ * On every device the contexts' persistent launches take turns (two at once could each hold part of the CUs and wait
+ * for workgroups that cannot start): one queued behind another context's waits on the device for what that context has
+ * queued so far.  mg_flow_in_use reports one of them as the launch's owner -- the first that asks, until it is destroyed,
+ * set to another mode or has had a wait run out; the others' launches are the same.
  * The persistent launch needs all its workgroups resident at once: on a GPU shared with
  * other kernels its waits can run into their time limit; the call then returns MG_E_HIP,
  * and the context continues with the fused launches.  All modes give the same results to
@@ -359,7 +359,8 @@ int mg_profile_decode(mg_ctx* ctx, int token, int pos, int steps, unsigned class
  * prompt.  The reference has no batched prompt path: a caller feeds the prompt
  * through PartialStep one position at a time (cuda_fused_infer.go:392), and it has
  * GEMM-shaped launches only on its training path (cuda.go:230 MatMul via cuBLAS);
- * here the seven projections of a layer over nTokens rows are MFMA GEMMs that
+ * here the seven projections of a layer over nTokens rows are MFMA GEMMs (kernels
+ * for a handful of rows and tiled ones, chosen by rows, cached rows and layer size) that
  * read the int8 weights exactly (int8 is exact in bf16) against activations
  * split into two bf16 terms, so the result stays within ~1e-5 of the
  * token-by-token path.  Q4_0 weights are multiplied block by block (nibble - 8

@@ -443,7 +443,7 @@ static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
 // sums it exchanges -- times the workgroups of the busiest CU, a quarter of which overlap evenly over the chip.  Short rows
 // go through two workgroups a CU at once; tiles of more than four blocks take too many registers for that (1.5).  The
 // constants are a fit to every tile of gate | up and of Wo + down at 64 to 512 rows of the three benchmark shapes, both
-// formats: what it picks is within 2 % of a layer of the best one at all of them.  (Bytes alone and 2.5 us a round of 256
+// formats: what it picks is within 3 % of a layer of the best one at all of them, and at 16 and 37 rows.  (Bytes alone and 2.5 us a round of 256
 // workgroups: 301 rows of the 0.5B shape 88 -> 78 us a layer, Q4_0 111 -> 86; 1.1B Q4_0 238 -> 180.)
 struct FewTile { int mt, nb; };
 static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4) {

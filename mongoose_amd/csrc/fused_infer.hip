@@ -1056,8 +1056,10 @@ int HIPFusedInference::SetTokensPerLaunch(int n) {
     return MG_OK;
 }
 
-// Sets the device-resident step state; where the persistent launch runs whole tokens, also leaves its exchange area
-// reset (a token expects the half of its position's parity so, and resets the other for its successor).
+// Sets the device-resident step state; where the persistent launch is set up, also leaves its exchange area reset (a token
+// expects the half of its position's parity so, and resets the other for its successor).  What changes the state without
+// this -- a prefill's tail, a layer graph's launch -- leaves the area to flowClean: enqueueLayersFlow and primeGraph reset
+// it where it is not known to be so.
 int HIPFusedInference::setState(int pos, int token, int count, int nPrompt) {
     HIPCHK(launch_set_state(dState, pos, token, count, nPrompt, ropeRef(), stream));
     statePosHost = pos;
@@ -1378,9 +1380,10 @@ int HIPFusedInference::enqueueToken(bool withHead) {
     int rc = fuseEmbed ? MG_OK : enqueueEmbed();
     if (rc) return rc;
     const bool flow = flowEligible(0, nLayers);
-    const int clean = flowClean;
+    int clean = 0;
     if (flow) {
         rc = ensureFlow();
+        clean = flowClean;
         if (rc == 0) rc = enqueueLayersFlow(0, nLayers, dState, 0, !fuseEmbed);
         if (rc) return rc;
     } else {

@@ -14,7 +14,10 @@
 //
 // Bound by the link: 16 workgroups read the page-locked blob at 55 GB/s (launch_host_pieces), and everything else hides
 // behind that: an 8.4 MB layer of the 0.5B shape crosses in 155 us, is staged in 60 and computed in 60.  Two copies are
-// queued ahead of the one that the host waits for before it fills that one's pinned buffer again.  Only the first
+// queued ahead of the one that the host waits for before it fills that one's pinned buffer again.  The third device set is
+// there for the copy stream: with two, the copy of layer i + 2 has to wait for the event of layer i's computation, which is
+// long over when its turn comes, but not when it is queued, and every such wait leaves a gap (4.36 -> 4.42 ms a token of the
+// 0.5B shape; with the host waiting instead 4.47 to 4.72).  Only the first
 // layer's staging is in nobody's shadow, so it goes out in three parts, each as soon as it is staged.
 #include "fused_infer.h"
 #include "../../include/mongoose_hip.h"

@@ -540,7 +540,7 @@ def test_one_context_a_device_owns_the_launch(hip):
     assert _in_use(a.hip) and not _in_use(b.hip)
     rc, ta = a.hip.Generate(prompt, 8)
     assert rc == 0, E.last_error()
-    rc, tb = b.hip.Generate(prompt, 8)                 # the fused launches
+    rc, tb = b.hip.Generate(prompt, 8)                 # the same launch, in its turn
     assert rc == 0, E.last_error()
     assert ta.tolist() == tb.tolist()
     assert a.hip.SetExecMode(1) == 0                   # gives the launch up
