@@ -12,15 +12,18 @@ steps are the W prompt positions; the K timed steps are the K decode positions
 after them.  Weights are synthetic (seeded N(0, 0.02), quantized on the host by
 the library's own loader) and resident in HBM before the timed region starts.
 
-Prints ONE JSON line: the throughput of the headline configuration, the roofline of
+Prints ONE JSON line, short enough (under 8,000 characters) for whoever keeps only the end of
+a log: the throughput of the headline configuration, the roofline of
 the kernel that takes most of the step's time (HIP events around its launches inside
-the step), a per-launch table, the lm_head matvec's own bandwidth (the second half of
+the step), its phases, the lm_head matvec's own bandwidth (the second half of
 the metric), the CPU oracle timed on this box's host cores as a baseline, and -- under
-"configs" -- the same measurements for the other benchmark configurations (toy,
+"configs" -- the step times of the other benchmark configurations (toy,
 TinyLlama-1.1B shape, Qwen2.5-0.5B Q4_0 with a leg through the weight-streaming front end,
 Llama-3-8B shape at a short context, at ~4k context with fp32 and with fp16 K/V rows, and
 its 512-token batched prefill), each with its greedy tokens checked against the oracle
 on a bounded sample (the ~4k-context runs against the fused launches on the same positions).
+--details PATH writes everything measured, per-launch and per-phase tables of every configuration
+among it, to a file (22,000 characters).
 """
 import argparse
 import json
@@ -516,8 +519,25 @@ def stream_leg(E, np, configs, f, s, seed, n):
     return {"tokens": n, "ms_per_token": round(el / n * 1e3, 3),
             "tok_per_s": round(n / el, 1), "host_to_device_bytes_per_token": int(layer_bytes),
             "host_to_device_GBps": round(layer_bytes * n / el / 1e9, 2),
-            "note": "host wall clock; every token stages all layers from pageable host memory through two pinned "
-                    "buffers into two device sets (copy of layer l+1 overlaps compute of layer l); logits read back each token"}
+            "note": "host wall clock; every token stages all layers from pageable host memory through three pinned "
+                    "buffers into three device sets (copy of layer l+1 overlaps compute of layer l); logits read back each token"}
+
+
+def digest(out):
+    """The printed form of a record: the headline configuration without the fused launches' table, the others by their step
+    times."""
+    d = {k: v for k, v in out.items() if k != "kernels_fused_launches" and not (v is None and k in ("prefill", "stream", "flow_trace"))}
+    if d.get("configs"):
+        run_keys = ("start_position", "steps", "ms_per_step", "tok_per_s", "step_roofline_frac", "fused_launches_ms_per_step",
+                    "graph_replay_one_token_a_launch_ms_per_step", "tokens_match_fused_launches")
+        leg_keys = ("tokens", "ms", "tok_per_s", "mfma_frac_of_bf16_peak", "ms_per_token", "host_to_device_GBps")
+
+        def pick(x, keys):
+            return {k: x[k] for k in keys if k in x}
+        d["configs"] = {n: {"runs": [pick(r, run_keys) for r in c["runs"]], **pick(c, ("tokens_match", "tokens_checked")),
+                            **{leg: pick(c[leg], leg_keys) for leg in ("prefill", "stream") if c.get(leg)}}
+                        for n, c in d["configs"].items()}
+    return d
 
 
 def main():
@@ -559,6 +579,7 @@ def main():
     ap.add_argument("--no-live-pmc", action="store_true",
                     help="do not run the two rocprofv3 --pmc passes that measure the launch's HBM traffic (the figures recorded "
                          "from profiles/ are reported instead)")
+    ap.add_argument("--details", metavar="PATH", help="write everything measured to this file (the printed line is a digest)")
     ap.add_argument("--no-configs", action="store_true",
                     help="only the configuration named by --config (no 'configs' object with the other benchmark configurations)")
     args = ap.parse_args()
@@ -736,7 +757,10 @@ def main():
         "cpu_baseline": cpu, "prefill": res.get("prefill"), "stream": stream, "flow_trace": flow_trace, "configs": others,
         "load_s": res["load_s"], "device": eng.Name(),
     }
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as fh:
+            json.dump(out, fh)
+    print(json.dumps(digest(out)))
 
 
 if __name__ == "__main__":

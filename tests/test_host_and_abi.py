@@ -144,3 +144,24 @@ def test_buffers_reach_the_library_whatever_their_kind():
     at, keep = E._addresses([a.T, a])
     assert at[1] == a.ctypes.data and read(at[0], a.nbytes) == np.ascontiguousarray(a.T).tobytes()
     assert E._fp(np.empty(0, np.float32)) is not None and E._fp(None) is None
+
+
+def test_the_benchmark_line_stays_short():
+    """A record of every configuration, tables and all, is printed as one line of at most 8,000 characters that still has
+    what the line is for."""
+    import json
+    import bench
+    table = [{"launch": "norm2+gate|up+SwiGLU (a launch of the fused path)", "cls": 4, "per_token": 24, "avg_us": 7.123, "share_of_step": 0.2, "bytes": 8755200, "GBps": 1234.5}] * 8
+    run = {"start_position": 4000, "steps": 200, "ms_per_step": 0.31234, "tok_per_s": 3201.5, "step_bytes": 8568968192, "step_GBps": 4546.1,
+           "step_roofline_frac": 0.5683, "launches": 4, "graph_replay_one_token_a_launch_ms_per_step": 1.89466, "fused_launches_ms_per_step": 2.50344,
+           "in_launch_phases": {"phases": table}, "kernels": table, "kernels_fused_launches": table, "tokens_match_fused_launches": True}
+    leg = {"tokens": 512, "ms": 15.222, "ms_per_token": 4.303, "host_to_device_GBps": 46.84, "note": "n" * 300}
+    conf = {"exec": "e" * 70, "runs": [run, run], "tokens_match": True, "tokens_checked": 48, "tokens_checked_at": "p" * 80, "prefill": leg, "stream": leg}
+    out = {"metric": "m", "value": 3201.5, "ms_per_step": 0.31234, "vs_baseline": None, "config": {"workload": "w" * 200}, "roofline": {"kernel": "k" * 700},
+           "matvec": {"kernel": "k" * 500}, "kernels": table[:1], "kernels_fused_launches": table, "in_launch_phases": {"phases": table},
+           "cpu_baseline": {"sample": "s" * 200}, "prefill": None, "stream": None, "flow_trace": None, "configs": {f"configuration-{i}": conf for i in range(5)}}
+    assert len(json.dumps(out)) > 20000
+    d = json.loads(json.dumps(bench.digest(out)))
+    assert len(json.dumps(d)) < 8000
+    assert d["value"] == 3201.5 and d["vs_baseline"] is None and d["roofline"] == out["roofline"]
+    assert all(c["runs"][0]["ms_per_step"] == 0.31234 and c["tokens_match"] and c["prefill"]["ms"] == 15.222 for c in d["configs"].values())
