@@ -4,8 +4,8 @@
 
 namespace mg {
 
-// One launch over a tile of 16 or 32 weight rows x 16, 32 or 64 activation rows a workgroup; what follows the product is
-// the epilogue of the mode.
+// One launch, tiles of 16 to 128 weight rows x 16 to 64 activation rows a workgroup (few_tile chooses); what follows the
+// product is the epilogue of the mode.
 enum FewMode {
     FEW_STORE = 0,   // Y (+)= v * scale + bias
     FEW_RESID = 1,   // Y += v * scale + bias; optionally the next projection's split of Y * nextGain and the rows' sums of squares
