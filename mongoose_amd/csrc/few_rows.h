@@ -17,6 +17,7 @@ struct FewParams {
     FewSeg seg[3];
     const unsigned short* Ahi;       // split activations in the order few_rows.hip describes (for this launch's weight format)
     const unsigned short* Alo;
+    const unsigned short* Ax;        // third terms (NULL: two terms); not with FEW_STORE
     int T, K;
     int q4;                          // weights: 0 = int8 rows with scales, 1 = Q4_0 in the split layout
     int accumulate;                  // FEW_STORE: Y += instead of Y =
@@ -29,8 +30,9 @@ struct FewParams {
     const float* nextGain;
     unsigned short* nextHi;
     unsigned short* nextLo;
+    unsigned short* nextX;           // with Ax
     int nextQ4;                      // weight format of the projection that reads them
-    float* nextSumSq;                // [tiles of the launch][sumStride]; few_rows_sum_parts(N, T, K, q4) of them
+    float* nextSumSq;                // [tiles of the launch][sumStride]; few_rows_sum_parts of them
     // FEW_QKV
     void* Kc;
     void* Vc;
@@ -40,21 +42,22 @@ struct FewParams {
     // filled by the launcher
     int nTiles;
 };
-int few_rows_sum_parts(int N, int T, int K, int q4);
+int few_rows_sum_parts(int N, int T, int K, int q4, int terms);
 // K a multiple of 32, W and the planes 16-byte aligned; FEW_QKV: headDim 64 or 128, N multiples of it.
 hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s);
 
 // Rows of the embedding table (kinds as launch_embed_rows) into x, their split times `gain` and their sums of squares
-// (one part).  tokens may be pinned host memory.
+// (one part).  tokens may be pinned host memory.  ext (here and below): the plane of the third terms, or NULL.
 hipError_t launch_embed_split(int kind, const void* table, const float* scales, const int* tokens, float* x, const float* gain,
-                              unsigned short* hi, unsigned short* lo, float* sumSq, int T, int dim, int vocab, int q4, hipStream_t s);
+                              unsigned short* hi, unsigned short* lo, unsigned short* ext, float* sumSq, int T, int dim, int vocab, int q4,
+                              hipStream_t s);
 // Rows of fp32 activations split for a launch over weights of format q4.
 hipError_t launch_few_split(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4, hipStream_t s);
 
 // Causal attention of T query rows (rotated) at positions pos0 .. over the cache rows [0, pos0 + T), all products and sums
 // in fp32; the result goes out as the split the output projection reads.
 hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
-                                int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4,
+                                unsigned short* ext, int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4,
                                 hipStream_t s);
 
 }  // namespace mg

@@ -24,6 +24,7 @@ typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 constexpr int FR_WAVES = 8, FR_WG = 64 * FR_WAVES;
+constexpr int FEW_MT3 = 2;                 // row blocks of a tile with three terms (registers)
 
 // two floats -> two bf16, round to nearest even
 __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
@@ -65,6 +66,17 @@ __device__ __forceinline__ size_t few_index(int t, int k, int K, int q4) {
     return ((size_t)(t >> 4) * ((K + 63) >> 6) + (k >> 6)) * 1024 + s * 512 + (q * 16 + (t & 15)) * 8 + (k & 7);
 }
 
+// A value's terms to element o of the planes: hi + lo, and what those leave of it in a third one.
+template <bool THIRD>
+__device__ __forceinline__ void put_split(unsigned short* hi, unsigned short* lo, unsigned short* ext, size_t o, float a) {
+    const unsigned short h = bf16_one(a);
+    const float r = a - bf16_value(h);
+    const unsigned short l = bf16_one(r);
+    hi[o] = h;
+    lo[o] = l;
+    if (THIRD) ext[o] = bf16_one(r - bf16_value(l));
+}
+
 // ---------------------------------------------------------------------------
 // Y[T,N] = (Ahi + Alo)[T,K] . W[N,K]^T with the mode's epilogue.  A workgroup = 8 waves that split K: wave w takes the
 // 64-k chunks w, w + 8, ...; a chunk of 16 weight rows is one 16-byte load a lane (Q4_0: two of 8 bytes), a chunk of 16
@@ -76,9 +88,11 @@ __device__ __forceinline__ size_t few_index(int t, int k, int K, int q4) {
 // each of the two Q4_0 blocks -- any order serves as long as both operands have the same.
 // ---------------------------------------------------------------------------
 //   LOOP = 0: K of at most 16 chunks, two a wave: both are requested at once, no ring.
-template <int MODE, int MT, int NB, int Q4, int LOOP>
+//   TERMS: bf16 terms of an activation, one plane each: 2 (2^-16 of the value left over), or 3 -- all 24 bits of an fp32 value,
+//   so that the products are those of the decode step and only the order of the fp32 sums differs.
+template <int MODE, int MT, int NB, int Q4, int LOOP, int TERMS>
 __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
-    constexpr int D = !LOOP || MT * NB >= 6 || MT == 4 ? 2 : (MT * NB >= 3 ? 3 : 4);
+    constexpr int D = !LOOP || MT * NB >= 6 || MT == 4 || (TERMS == 3 && MT * NB >= 4) ? 2 : (MT * NB >= 3 ? 3 : 4);
     constexpr int NCOL = 16 * NB, MROW = 16 * MT, LST = MROW + 4;
     static_assert(NCOL * (MROW / 4) <= FR_WG, "four results a thread");
     extern __shared__ __attribute__((aligned(16))) float part[];      // [wave][column][LST]: the waves' sums
@@ -132,13 +146,13 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
         dP[b] = Q4 ? reinterpret_cast<const unsigned short*>(W + (size_t)N * (K >> 1)) + few_scales_at(blockRow(b, fr), K) : nullptr;
     }
     const size_t aBlk = (size_t)planeChunks * 1024;                   // elements from one 16-row block to the next
-    const unsigned short* aH[MT];
-    const unsigned short* aL[MT];
+    const unsigned short* aP[TERMS][MT];
 #pragma unroll
     for (int i = 0; i < MT; i++) {                                    // (blocks past the last row repeat the last one)
         const size_t o = (size_t)min((m0 >> 4) + i, (T - 1) >> 4) * aBlk + lane * 8;
-        aH[i] = p.Ahi + o;
-        aL[i] = p.Alo + o;
+        aP[0][i] = p.Ahi + o;
+        aP[1][i] = p.Alo + o;
+        if constexpr (TERMS == 3) aP[2][i] = p.Ax + o;
     }
 
     // What the epilogue needs is requested before the products' operands: the rows' sums of squares (for the RMS factor;
@@ -177,18 +191,23 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
         }
     }
 
-    float4_t acc[MT][NB];
+    // (three terms: the lower two have sums of their own, so that a sum is rounded once a step, not three times)
+    constexpr bool SUMS2 = TERMS == 3 && !Q4;
+    float4_t acc[MT][NB], acc2[SUMS2 ? MT : 1][SUMS2 ? NB : 1];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int b = 0; b < NB; b++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[i][b][e] = 0.f;
+            for (int e = 0; e < 4; e++) {
+                acc[i][b][e] = 0.f;
+                if constexpr (SUMS2) acc2[i][b][e] = 0.f;
+            }
 
-    uint4 vh[D][MT][2], vl[D][MT][2];
+    uint4 va[D][TERMS][MT][2];
     int4 vw[D][NB];
     unsigned vd[D][NB];
-    auto load = [&](int c, uint4 (&h)[MT][2], uint4 (&l)[MT][2], int4 (&w)[NB], unsigned (&d)[NB]) __attribute__((always_inline)) {
+    auto load = [&](int c, uint4 (&a)[TERMS][MT][2], int4 (&w)[NB], unsigned (&d)[NB]) __attribute__((always_inline)) {
         const int cc = min(c, lastChunk);
 #pragma unroll
         for (int b = 0; b < NB; b++) {
@@ -205,31 +224,32 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int s = 0; s < 2; s++) {
-                h[i][s] = *reinterpret_cast<const uint4*>(aH[i] + cc * 1024 + s * 512);
-                l[i][s] = *reinterpret_cast<const uint4*>(aL[i] + cc * 1024 + s * 512);
-            }
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int t = 0; t < TERMS; t++) a[t][i][s] = *reinterpret_cast<const uint4*>(aP[t][i] + cc * 1024 + s * 512);
         asm volatile("" ::: "memory");                                // (the loads stay here, ahead of the products before them)
     };
     // a 32-k step: weight fragments f (Q4_0: block scales d) against activation blocks
-    auto product = [&](const bf16x8_t (&f)[NB], const float (&d)[NB], int i, uint4 h, uint4 l) __attribute__((always_inline)) {
-        const bf16x8_t ah = __builtin_bit_cast(bf16x8_t, h), al = __builtin_bit_cast(bf16x8_t, l);
+    auto product = [&](const bf16x8_t (&f)[NB], const float (&d)[NB], int i, const uint4 (&a)[TERMS]) __attribute__((always_inline)) {
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             if (Q4) {
                 // a Q4_0 block's sum, then its fp16 scale (not foldable into a bf16 weight without loss)
                 float4_t t = {0.f, 0.f, 0.f, 0.f};
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, f[b], t, 0, 0, 0);
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, f[b], t, 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < TERMS; k++) t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[k]), f[b], t, 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < 4; e++) acc[i][b][e] = fmaf(d[b], t[e], acc[i][b][e]);
             } else {
-                acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, f[b], acc[i][b], 0, 0, 0);
-                acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, f[b], acc[i][b], 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < TERMS; k++) {
+                    float4_t& sum = SUMS2 && k > 0 ? acc2[SUMS2 ? i : 0][SUMS2 ? b : 0] : acc[i][b];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[k]), f[b], sum, 0, 0, 0);
+                }
             }
         }
     };
-    auto multiply = [&](const uint4 (&h)[MT][2], const uint4 (&l)[MT][2], const int4 (&w)[NB], const unsigned (&d)[NB]) __attribute__((always_inline)) {
+    auto multiply = [&](const uint4 (&a)[TERMS][MT][2], const int4 (&w)[NB], const unsigned (&d)[NB]) __attribute__((always_inline)) {
         int4 x[NB];                                                   // this lane's own pieces
 #pragma unroll
         for (int b = 0; b < NB; b++) {
@@ -249,23 +269,28 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
                 dd[b] = Q4 ? half_bits_to_float((unsigned short)(s ? d[b] >> 16 : d[b] & 0xffffu)) : 1.0f;
             }
 #pragma unroll
-            for (int i = 0; i < MT; i++) product(f, dd, i, h[i][s], l[i][s]);
+            for (int i = 0; i < MT; i++) {
+                uint4 at[TERMS];
+#pragma unroll
+                for (int t = 0; t < TERMS; t++) at[t] = a[t][i][s];
+                product(f, dd, i, at);
+            }
         }
     };
     if (!LOOP) {
-        load(wave, vh[0], vl[0], vw[0], vd[0]);
-        load(wave + FR_WAVES, vh[1], vl[1], vw[1], vd[1]);
-        if (wave < chunks) multiply(vh[0], vl[0], vw[0], vd[0]);
-        if (wave + FR_WAVES < chunks) multiply(vh[1], vl[1], vw[1], vd[1]);
+        load(wave, va[0], vw[0], vd[0]);
+        load(wave + FR_WAVES, va[1], vw[1], vd[1]);
+        if (wave < chunks) multiply(va[0], vw[0], vd[0]);
+        if (wave + FR_WAVES < chunks) multiply(va[1], vw[1], vd[1]);
     } else {
 #pragma unroll
-        for (int j = 0; j < D - 1; j++) load(wave + j * FR_WAVES, vh[j], vl[j], vw[j], vd[j]);
+        for (int j = 0; j < D - 1; j++) load(wave + j * FR_WAVES, va[j], vw[j], vd[j]);
         for (int c = wave; c < chunks; c += D * FR_WAVES) {
 #pragma unroll
             for (int j = 0; j < D; j++) {
                 constexpr int DM = D - 1;
-                load(c + (j + DM) * FR_WAVES, vh[(j + DM) % D], vl[(j + DM) % D], vw[(j + DM) % D], vd[(j + DM) % D]);
-                if (c + j * FR_WAVES < chunks) multiply(vh[j], vl[j], vw[j], vd[j]);
+                load(c + (j + DM) * FR_WAVES, va[(j + DM) % D], vw[(j + DM) % D], vd[(j + DM) % D]);
+                if (c + j * FR_WAVES < chunks) multiply(va[j], vw[j], vd[j]);
             }
         }
     }
@@ -288,16 +313,23 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
         }
         const int at = chunks * 1024 + (Q4 ? 0 : (fq & 1) * 512 + ((fq >> 1) * 16 + fr) * 8 - lane * 8);      // k = 8 q .. 8 q + 7
 #pragma unroll
-        for (int i = 0; i < MT; i++)
-            product(f, dd, i, *reinterpret_cast<const uint4*>(aH[i] + at), *reinterpret_cast<const uint4*>(aL[i] + at));
+        for (int i = 0; i < MT; i++) {
+            uint4 a[TERMS];
+#pragma unroll
+            for (int t = 0; t < TERMS; t++) a[t] = *reinterpret_cast<const uint4*>(aP[t][i] + at);
+            product(f, dd, i, a);
+        }
     }
 
     // C layout: lane holds column fr, rows 4 fq .. 4 fq + 3 of a block
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int b = 0; b < NB; b++)
-            *reinterpret_cast<float4_t*>(&part[(wave * NCOL + b * 16 + fr) * LST + i * 16 + 4 * fq]) = acc[i][b];
+        for (int b = 0; b < NB; b++) {
+            float4_t v = acc[i][b];
+            if constexpr (SUMS2) v += acc2[i][b];
+            *reinterpret_cast<float4_t*>(&part[(wave * NCOL + b * 16 + fr) * LST + i * 16 + 4 * fq]) = v;
+        }
     {
         float sq = (sqv[0] + sqv[1]) + (sqv[2] + sqv[3]);
         if (p.sumSq)
@@ -347,10 +379,7 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
                 q2[e] = x * x;
                 if (p.nextHi) {
                     const float a = x * gain;
-                    const unsigned short h = bf16_one(a);
-                    const size_t o = few_index(m, row, N, p.nextQ4);
-                    p.nextHi[o] = h;
-                    p.nextLo[o] = bf16_one(a - bf16_value(h));
+                    put_split<TERMS == 3>(p.nextHi, p.nextLo, p.nextX, few_index(m, row, N, p.nextQ4), a);
                 }
             }
         }
@@ -388,10 +417,7 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
             if (!isUp && okN && m < T) {
                 const float g = v[e];
                 const float a = g * (1.0f / (1.0f + expf(-g))) * u;          // mongoose.cu:949-956
-                const unsigned short h = bf16_one(a);
-                const size_t o = few_index(m, row, N, p.nextQ4);
-                p.nextHi[o] = h;
-                p.nextLo[o] = bf16_one(a - bf16_value(h));
+                put_split<TERMS == 3>(p.nextHi, p.nextLo, p.nextX, few_index(m, row, N, p.nextQ4), a);
             }
         }
     } else {
@@ -414,13 +440,13 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
     }
 }
 
-template <int MODE, int MT, int NB, int Q4, int LOOP>
+template <int MODE, int MT, int NB, int Q4, int LOOP, int TERMS>
 static hipError_t launch_few_l(const FewParams& p, hipStream_t s) {
     constexpr int bytes = FR_WAVES * 16 * NB * (16 * MT + 4) * 4;
     if (bytes > 48 * 1024) {
         static bool raised = false;                                    // (more than the default cap on dynamic LDS)
         if (!raised) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_rows_kernel<MODE, MT, NB, Q4, LOOP>),
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_rows_kernel<MODE, MT, NB, Q4, LOOP, TERMS>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
             if (e != hipSuccess) return e;
             raised = true;
@@ -428,13 +454,16 @@ static hipError_t launch_few_l(const FewParams& p, hipStream_t s) {
     }
     const int numM = (p.T + 16 * MT - 1) / (16 * MT);
     const unsigned grid = (unsigned)((p.nTiles + 7) / 8 * 8) * (unsigned)numM;
-    hipLaunchKernelGGL((few_rows_kernel<MODE, MT, NB, Q4, LOOP>), dim3(grid), dim3(FR_WG), bytes, s, p);
+    hipLaunchKernelGGL((few_rows_kernel<MODE, MT, NB, Q4, LOOP, TERMS>), dim3(grid), dim3(FR_WG), bytes, s, p);
     return hipGetLastError();
 }
 
 template <int MODE, int MT, int NB, int Q4>
 static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
-    return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1>(p, s);
+    if constexpr (MODE != FEW_STORE && MT <= FEW_MT3)
+        if (p.Ax) return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0, 3>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1, 3>(p, s);
+    if (p.Ax) return hipErrorInvalidValue;
+    return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0, 2>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1, 2>(p, s);
 }
 
 // The tile of a launch (16 MT activation rows x 16 NB weight rows a workgroup): the one with the shortest time by a model of
@@ -446,14 +475,15 @@ static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
 // formats: what it picks is within 3 % of a layer of the best one at all of them, and at 16 and 37 rows.  (Bytes alone and 2.5 us a round of 256
 // workgroups: 301 rows of the 0.5B shape 88 -> 78 us a layer, Q4_0 111 -> 86; 1.1B Q4_0 238 -> 180.)
 struct FewTile { int mt, nb; };
-static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4) {
+// With three terms an activation row is half as many bytes again, and a tile has at most FEW_MT3 row blocks.
+static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4, int terms) {
     const int b16 = (T + 15) / 16;
     FewTile best{1, nbFirst};
     double least = 1e30;
     for (int nb = nbFirst; nb <= nbLast; nb *= 2)
-        for (int mt = 1; mt <= 4 && mt <= b16 && mt * nb <= 8; mt++) {
+        for (int mt = 1; mt <= (terms == 3 ? FEW_MT3 : 4) && mt <= b16 && mt * nb <= 8; mt++) {
             const double wgs = (double)((rowsN + 16 * nb - 1) / (16 * nb)) * ((b16 + mt - 1) / mt);
-            const double bytes = (64.0 * mt + (q4 ? 9.0 : 16.0) * nb) * K;
+            const double bytes = (32.0 * terms * mt + (q4 ? 9.0 : 16.0) * nb) * K;
             double each = bytes / 80.0 + (q4 ? 0.74 : 0.225) * nb * K + 25.0 * mt * nb;
             if (K <= 64 * 2 * FR_WAVES && mt * nb > 4) each *= 1.5;
             const double cost = (0.75 * ceil(wgs / 256.0) + 0.25 * wgs / 256.0) * each;
@@ -461,7 +491,10 @@ static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4
         }
     return best;
 }
-int few_rows_sum_parts(int N, int T, int K, int q4) { const int b = few_tile(N, T, K, 1, 4, q4).nb; return (N + 16 * b - 1) / (16 * b); }
+int few_rows_sum_parts(int N, int T, int K, int q4, int terms) {
+    const int b = few_tile(N, T, K, 1, 4, q4, terms).nb;
+    return (N + 16 * b - 1) / (16 * b);
+}
 
 template <int MODE, int MT, int NB>
 static hipError_t launch_few_fmt(const FewParams& p, hipStream_t s) {
@@ -482,16 +515,18 @@ static hipError_t launch_few_mt(int mt, const FewParams& p, hipStream_t s) {
 hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
     if (p.T <= 0) return hipSuccess;
     if (p.K <= 0 || p.K % 32 || !p.Ahi || !p.Alo || p.seg[0].N <= 0) return hipErrorInvalidValue;
+    const int terms = p.Ax ? 3 : 2;
+    if (terms == 3 && (mode == FEW_STORE || (p.nextHi && !p.nextX))) return hipErrorInvalidValue;
     const int N = p.seg[0].N;
     if (mode == FEW_STORE || mode == FEW_RESID) {
-        const FewTile t = few_tile(N, p.T, p.K, 1, 4, p.q4);
+        const FewTile t = few_tile(N, p.T, p.K, 1, 4, p.q4, terms);
         p.nTiles = (N + 16 * t.nb - 1) / (16 * t.nb);
         if (mode == FEW_STORE) return t.nb == 1 ? launch_few_mt<FEW_STORE, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_STORE, 2>(t.mt, p, s) : launch_few_mt<FEW_STORE, 4>(t.mt, p, s);
         return t.nb == 1 ? launch_few_mt<FEW_RESID, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_RESID, 2>(t.mt, p, s) : launch_few_mt<FEW_RESID, 4>(t.mt, p, s);
     }
     if (mode == FEW_SWIGLU) {
         if (p.seg[1].N != N || !p.nextHi || !p.nextLo) return hipErrorInvalidValue;
-        const FewTile t = few_tile(2 * N, p.T, p.K, 2, 8, p.q4);
+        const FewTile t = few_tile(2 * N, p.T, p.K, 2, 8, p.q4, terms);
         p.nTiles = (N + 8 * t.nb - 1) / (8 * t.nb);
         return t.nb == 2 ? launch_few_mt<FEW_SWIGLU, 2>(t.mt, p, s) : t.nb == 4 ? launch_few_mt<FEW_SWIGLU, 4>(t.mt, p, s) : launch_few_mt<FEW_SWIGLU, 8>(t.mt, p, s);
     }
@@ -499,7 +534,7 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
         if ((p.headDim != 64 && p.headDim != 128) || N % p.headDim || p.seg[1].N <= 0 || p.seg[1].N % p.headDim ||
             p.seg[2].N != p.seg[1].N || !p.Kc || !p.Vc) return hipErrorInvalidValue;
         p.nTiles = (N + 2 * p.seg[1].N) / 32;
-        return launch_few_mt<FEW_QKV, 2>(few_tile(N + 2 * p.seg[1].N, p.T, p.K, 2, 2, p.q4).mt, p, s);
+        return launch_few_mt<FEW_QKV, 2>(few_tile(N + 2 * p.seg[1].N, p.T, p.K, 2, 2, p.q4, terms).mt, p, s);
     }
     return hipErrorInvalidValue;
 }
@@ -508,7 +543,7 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
 // Embedding rows, their split times the first gain, their sums of squares: one workgroup a row.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(WG) void embed_split_kernel(int kind, const void* table, const float* scales, const int* tokens, float* x,
-                                                         const float* gain, unsigned short* hi, unsigned short* lo, float* sumSq,
+                                                         const float* gain, unsigned short* hi, unsigned short* lo, unsigned short* ext, float* sumSq,
                                                          int dim, int vocab, int q4) {
     __shared__ float red[4];
     const int t = blockIdx.x;
@@ -520,18 +555,18 @@ __global__ __launch_bounds__(WG) void embed_split_kernel(int kind, const void* t
         x[(size_t)t * dim + i] = v;
         ss += v * v;
         const float a = v * gain[i];
-        const unsigned short h = bf16_one(a);
         const size_t o = few_index(t, i, dim, q4);
-        hi[o] = h;
-        lo[o] = bf16_one(a - bf16_value(h));
+        if (ext) put_split<true>(hi, lo, ext, o, a);
+        else put_split<false>(hi, lo, ext, o, a);
     }
     ss = block_sum(ss, red);
     if (threadIdx.x == 0) sumSq[t] = ss;
 }
 hipError_t launch_embed_split(int kind, const void* table, const float* scales, const int* tokens, float* x, const float* gain,
-                              unsigned short* hi, unsigned short* lo, float* sumSq, int T, int dim, int vocab, int q4, hipStream_t s) {
+                              unsigned short* hi, unsigned short* lo, unsigned short* ext, float* sumSq, int T, int dim, int vocab, int q4,
+                              hipStream_t s) {
     if (T <= 0) return hipSuccess;
-    hipLaunchKernelGGL(embed_split_kernel, dim3((unsigned)T), dim3(WG), 0, s, kind, table, scales, tokens, x, gain, hi, lo, sumSq, dim, vocab, q4);
+    hipLaunchKernelGGL(embed_split_kernel, dim3((unsigned)T), dim3(WG), 0, s, kind, table, scales, tokens, x, gain, hi, lo, ext, sumSq, dim, vocab, q4);
     return hipGetLastError();
 }
 
@@ -588,7 +623,7 @@ __device__ __forceinline__ float4 ld_row4(const void* base, size_t i) {
 
 template <int HD, bool KVH>
 __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, const void* Kc, const void* Vc, unsigned short* hi,
-                                                             unsigned short* lo, int T, int pos0, int dim, int kvDim, int nHeads,
+                                                             unsigned short* lo, unsigned short* ext, int T, int pos0, int dim, int kvDim, int nHeads,
                                                              int nKVHeads, int q4) {
     constexpr int KF = HD / 16, VF = HD / 16;              // K: float4 a lane and row (HD/4 elements); V: elements a lane and row
     constexpr int OST = 17;
@@ -707,16 +742,15 @@ __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, co
             den = fmaf(g, wl[w][qq], den);
         }
         const float a = num / den;
-        const unsigned short h = bf16_one(a);
         const size_t ix = few_index(q0 + qq, head * HD + d, dim, q4);
-        hi[ix] = h;
-        lo[ix] = bf16_one(a - bf16_value(h));
+        if (ext) put_split<true>(hi, lo, ext, ix, a);
+        else put_split<false>(hi, lo, ext, ix, a);
     }
 }
 
 template <int HD, bool KVH>
 static hipError_t launch_few_attn_t(unsigned grid, hipStream_t s, const float* q, const void* Kc, const void* Vc, unsigned short* hi,
-                                    unsigned short* lo, int T, int pos0, int dim, int kvDim, int nHeads, int nKVHeads, int q4) {
+                                    unsigned short* lo, unsigned short* ext, int T, int pos0, int dim, int kvDim, int nHeads, int nKVHeads, int q4) {
     constexpr int bytes = FR_WAVES * HD * 17 * 4;
     if (bytes > 48 * 1024) {
         static bool raised = false;
@@ -727,20 +761,20 @@ static hipError_t launch_few_attn_t(unsigned grid, hipStream_t s, const float* q
             raised = true;
         }
     }
-    hipLaunchKernelGGL((few_attention_kernel<HD, KVH>), dim3(grid), dim3(FR_WG), bytes, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    hipLaunchKernelGGL((few_attention_kernel<HD, KVH>), dim3(grid), dim3(FR_WG), bytes, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
     return hipGetLastError();
 }
 
 hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
-                                int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4, hipStream_t s) {
+                                unsigned short* ext, int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4, hipStream_t s) {
     if (T <= 0) return hipSuccess;
     if (nKVHeads <= 0 || nHeads % nKVHeads || pos0 < 0 || pos0 + T > rowLimit || dim != nHeads * headDim || kvDim != nKVHeads * headDim ||
         (headDim != 64 && headDim != 128) || !hi || !lo) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)nHeads * (unsigned)((T + 15) / 16);
-    if (headDim == 64) return kvHalf ? launch_few_attn_t<64, true>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
-                                     : launch_few_attn_t<64, false>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
-    return kvHalf ? launch_few_attn_t<128, true>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
-                  : launch_few_attn_t<128, false>(grid, s, q, Kc, Vc, hi, lo, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    if (headDim == 64) return kvHalf ? launch_few_attn_t<64, true>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
+                                     : launch_few_attn_t<64, false>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    return kvHalf ? launch_few_attn_t<128, true>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
+                  : launch_few_attn_t<128, false>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
 }
 
 }  // namespace mg

@@ -166,7 +166,16 @@ private:
     float* pfPartial = nullptr;
     int ensurePrefill(int rows, int kvRows);
     float* pfSumSq = nullptr;               // few-row path: partial sums of squares of the rows
-    int enqueuePrefillFew(int T, int pos0);
+    // Buffers of the few-row path; the third planes: NULL, or the third terms of the activations (few_rows.h).
+    struct FewScratch { float *x, *q, *sumSq; unsigned short *a[3], *b[3]; };
+    int enqueuePrefillFew(const int* tokens, int T, int pos0, const FewScratch& S, bool cachesOnly);
+    static constexpr int PROMPT_ROWS = 128;      // prompt positions that go through the layers together
+    static constexpr int PROMPT_ROWS_FROM = 3;   // ... from as many on (below, Generate has them as tokens of its launches)
+    Slab promptSlab;
+    FewScratch promptScratch{};
+    int promptCap = 0;              // rows promptSlab holds
+    int ensurePrompt(int rows);
+    int enqueuePrompt(const int* tokens, int n);    // the cache rows of positions 0 .. n - 1 (tokens: page-locked)
     int enqueuePrefillTiles(int T, int pos0);
     std::vector<Slab> layerSlabs, kvSlabs;
     size_t slotOff[12] = {0};

@@ -46,6 +46,39 @@ def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
     m.close()
 
 
+@pytest.mark.parametrize("shape,fmt,kv_f16,n", [
+    (SMALL, "q8", False, 3), (SMALL, "q8", False, 4), (SMALL, "q8", False, 17), (SMALL, "q8", False, 18), (SMALL, "q4_0", True, 34),
+    (ODD, "q8", False, 16), (ODD, "q4_0", False, 66), (NARROW, "q8", False, 19), (NARROW, "q4_0", False, 34), (WIDE, "q8", False, 49),
+    (SMALL, "q8", False, 130), (ODD, "q8", True, 129), (SMALL, "q4_0", False, 258)])
+def test_prompts_of_generate_match_token_by_token(hip, shape, fmt, kv_f16, n):
+    """Generate takes a prompt's positions through the layers together (from three on, 128 at a time): the token it chooses and
+    the logits of the step after, which reads every cache row, against the same tokens one by one.  Bar: the products are the
+    same (three bf16 terms are an fp32 value), so what differs are the roundings of fp32 sums: 2^-24 of a partial sum each,
+    some 20 that matter in each of 7 products and 4 norms of 2 layers, at random: 2^-24 sqrt(20 * 11 * 2) = 1.3e-6, and
+    4e-6 for the largest of the logits.  Two terms would be off by 2^-18 a value: 1e-5 and more."""
+    m = H.Model(shape, seed=n, maxSeq=n + 3, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
+    toks = m.prompt(n)
+    for pos in range(n):
+        rc, want = m.hip.DecodeToken(int(toks[pos]), pos)
+        assert rc == 0, E.last_error()
+    ref, got = np.empty((2, shape.vocab), np.float32)
+    rc, _ = m.hip.DecodeToken(want, n, ref)
+    assert rc == 0
+    assert m.hip.ResetKV() == 0
+    out = []
+    names = H.launched(lambda: out.append(m.hip.Generate(toks, 2)))
+    rc, t = out[0]
+    assert rc == 0 and int(t[0]) == want, E.last_error()
+    assert any("few_rows_kernel" in k for k in names) == (n > 3) and any("flow_layers_kernel" in k for k in names)
+    rc, _ = m.hip.DecodeToken(want, n, got)
+    assert rc == 0 and H.rel_err(got, ref) < (1e-3 if kv_f16 else 4e-6)
+    rc, t = m.hip.Generate(toks[::-1].copy(), 2)            # another prompt into the same buffers, and the first again
+    assert rc == 0
+    rc, t = m.hip.Generate(toks, 1)
+    assert rc == 0 and int(t[0]) == want
+    m.close()
+
+
 @pytest.mark.parametrize("rows,n,k,accumulate", [(1, 16, 32, 0), (17, 33, 96, 1), (64, 300, 1056, 0), (77, 129, 2080, 1), (130, 1000, 4864, 0),
                                                  (513, 2900, 64, 0), (48, 9000, 64, 0), (300, 5632, 160, 1), (17, 33, 32, 1), (200, 1000, 32, 0)])
 def test_few_row_gemm_matches_float64(hip, rows, n, k, accumulate):
