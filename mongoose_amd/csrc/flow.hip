@@ -552,6 +552,12 @@ struct Prefetcher {
         if (!base || rank != 0) return;
         span(static_cast<const char*>(base), 0, bytes);
     }
+    // an array that every workgroup of the XCD reads and that is too large for one prefetcher: 8 KB to each in turn
+    __device__ __forceinline__ void shared(const void* base, size_t bytes) {
+        bytes &= ~(size_t)15;
+        for (size_t o = ((size_t)rank * FWG + tid) * 16; o < bytes; o += (size_t)nRank * FWG * 16)
+            __builtin_amdgcn_global_load_lds(reinterpret_cast<const int4*>(static_cast<const char*>(base) + o), scrap, 16, 0, 0);
+    }
     // everything requested so far has landed (in the L2 on its way): nothing of it can arrive in the scrap area later
     __device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 };
@@ -646,7 +652,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     // Measured per variant, ms a token with / without: 0.5B Q8 0.3141 / 0.3230, 8B 1.558 / 1.561 (fp16 rows at 4,000
     // positions 1.841 / 1.847), 0.5B Q4_0 0.3235 / 0.3230, 1.1B 0.378 / 0.372 -- the last two keep them in registers.
     constexpr bool FXF = FX && (((FIX & 7) == 1 && !Q4) || (FIX & 7) == 3);
-    constexpr bool FXD = FX && (FIX & 7) == 1;        // (0.5B Q4_0 0.3267 -> 0.3204 ms a token, Q8 0.3141 -> 0.3138; the others gain nothing)
+    // (0.5B Q4_0 0.3267 -> 0.3204 ms a token, Q8 0.3141 -> 0.3138; 1.1B 0.366 -> 0.364, at 600 positions 0.433 -> 0.430; 8B gains nothing)
+    constexpr bool FXD = FX && ((FIX & 7) == 1 || (FIX & 7) == 2);
     // whether workgroups past the computing ones prefetch (then none prefetches while idle during the attention): of the
     // two roles a known shape has one, the other's code is not in its variant
     const bool hasPrefetchers = FXD ? FS.dedicated != 0 : nC != (int)gridDim.x;
@@ -768,13 +775,16 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                     if (!Q4) { pf.whole(L.sq(), (size_t)dim * 4); pf.whole(L.sk(), (size_t)kvDim * 4); pf.whole(L.sv(), (size_t)kvDim * 4); }
                     pf.whole(L.bq(), (size_t)dim * 4); pf.whole(L.bk(), (size_t)kvDim * 4); pf.whole(L.bv(), (size_t)kvDim * 4);
                     pf.whole(L.g1(), (size_t)dim * 4);
+                    // the K / V rows of the earlier positions (the attention workgroups of every XCD read them; the row of the
+                    // current position comes through the exchange area), while both fit half an L2.  Shared out among the XCD's
+                    // prefetchers: by one alone, at what a CU pulls, they hold up the weights behind them from a hundred positions
+                    // on (0.5B shape, 24 layers with a small lm_head, one / shared: Q8 285 / 277 us a token at 130 positions, 307 /
+                    // 288 at 330, 334 / 309 at 530; Q4_0 352 / 297 at 330, 400 / 314 at 530; past 512 KB, which was the limit,
+                    // 363 / 352 at 1,130).
+                    const size_t kvBytes = (size_t)pos * kvDim * (kvHalfV ? 2 : 4);
+                    if (kvBytes <= ((size_t)1 << 20)) { pf.shared(L.Kc(), kvBytes); pf.shared(L.Vc(), kvBytes); }
                     pf.rows(L.wo(), rbD, dim, 8);
                     if (Q4) pf.rows(L.so(), rdD, dim, 8); else pf.whole(L.so(), (size_t)dim * 4);
-                    // the K / V rows of the earlier positions (the attention workgroups of every XCD read them; the row of the
-                    // current position comes through the exchange area), while they are a small part of an L2: 0.5B shape at
-                    // positions 16 .. 216 0.3766 -> 0.3710 ms a token
-                    const size_t kvBytes = (size_t)pos * kvDim * (kvHalfV ? 2 : 4);
-                    if (kvBytes <= ((size_t)512 << 10)) { pf.whole(L.Kc(), kvBytes); pf.whole(L.Vc(), kvBytes); }
                 }
                 release(G.offM);               // ... past its gate | up: gate | up of this one
                 pf.rows(L.gate(), rbD, ffn, 8);
@@ -1846,7 +1856,7 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         for (int k = 1; k <= 3 && !fix; k++) {
             const FlowFixedShape fs = flow_fixed_shape(k);
             if (p.dim == fs.dim && p.kvDim == fs.kvDim && p.ffn == fs.ffn && p.nHeads == fs.nHeads && p.nKVHeads == fs.nKVHeads &&
-                p.headDim == fs.headDim && (p.downSplit != 0) == (fs.downSplit != 0) && (k != 1 || (nC != grid) == (fs.dedicated != 0))) fix = k;
+                p.headDim == fs.headDim && (p.downSplit != 0) == (fs.downSplit != 0) && (k == 3 || (nC != grid) == (fs.dedicated != 0))) fix = k;
         }
 #define FLOW_LAUNCH_F(HDv, CBv, RGv, GQv, Q4v, FXv) do { \
         if (p.trace) hipLaunchKernelGGL((flow_layers_kernel<HDv, CBv, RGv, GQv, Q4v, true, FXv>), dim3(grid), dim3(FWG), lds, s, p); \
