@@ -193,6 +193,10 @@ void mongoose_kv_cache_write(float* cache, const float* src, int pos, int kvDim,
 void mongoose_decode_attention(const float* Q, const float* K, const float* V, float* out, int cacheLen, int dim, int kvDim,
                                int nHeads, int nKVHeads, void* stream) {
     if (cacheLen <= 0 || nHeads <= 0) return;
+    // No room for partial results here, so the context is not split.  Four workgroups a query head share out its columns while
+    // that is at most a workgroup for every CU (kernels.hip); with more heads the K rows they read again cost more than the
+    // idle CUs do, and a workgroup takes a head.
+    if (nHeads <= 64) { note(mg::launch_attention_columns(Q, K, V, out, cacheLen, kvDim, nHeads, nKVHeads, dim / nHeads, S(stream))); return; }
     mg::AttnParams p{};
     p.q = Q; p.Kc = K; p.Vc = V;
     p.posImm = cacheLen - 1;
@@ -200,10 +204,7 @@ void mongoose_decode_attention(const float* Q, const float* K, const float* V, f
     p.kvDim = kvDim; p.nHeads = nHeads; p.nKVHeads = nKVHeads;
     p.headDim = dim / nHeads;                                    // mongoose.cu:939
     p.out = out; p.smax = 1; p.splitLen = 0;
-    // One query head a workgroup: there is no room for partial results here, so the context is not split, and a workgroup
-    // is bound by what one CU pulls (some 53 bytes a nanosecond); the heads of a group read the same rows, from the L2s.
-    // 32 heads of 64 on 4 K/V heads: 10.9 us at 1,200 rows, 33.9 with four heads a workgroup, 4.8 / 9.6 at 256.
-    p.headsPerWG = 1;
+    p.headsPerWG = 1;      // (the heads of a group read the same rows, from the L2s; four heads a workgroup take three times as long)
     note(mg::launch_attention(p, S(stream)));
 }
 void mongoose_silu_gate_mul(const float* gate, const float* up, float* out, int n, void* stream) {

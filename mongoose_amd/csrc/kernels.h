@@ -123,6 +123,10 @@ struct AttnParams {
     PfJob pf;             // pf.rows > 0: grid rows smax .. smax + pf.rows - 1 are prefetch helpers
 };
 hipError_t launch_attention(const AttnParams& p, hipStream_t s);
+// One query position over len fp32 cache rows without any scratch memory: four workgroups a query head, a quarter of its
+// output each.
+hipError_t launch_attention_columns(const float* q, const float* K, const float* V, float* out, int len, int kvDim, int nHeads, int nKVHeads,
+                                    int headDim, hipStream_t s);
 int attention_columns(int nHeads, int nKVHeads, int headsPerWG);
 
 hipError_t launch_rmsnorm_out(const float* in, float* out, const float* w, int seqLen, int dim, float eps, hipStream_t s);

@@ -1345,6 +1345,114 @@ hipError_t launch_attention(const AttnParams& p, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
+// The per-op decode attention: no room for partial results, so a context cannot be split over workgroups.  The columns of
+// the output can: CS workgroups a query head compute all of its scores and a CS-th of P.V each -- what bounds a workgroup is
+// the bytes its CU pulls (some 60 a nanosecond, whatever is requested ahead), and it then reads the K rows and a quarter of
+// the V rows instead of both whole.  32 heads of 64 on 4 K/V heads: 9.4 -> 7.2 us at 1,200 rows, 21.8 -> 16.8 at 3,000; 32 of
+// 128 on 8: 16.5 -> 12.0 and 35.5 -> 24.6; up to 256 rows both end within what a launch costs.
+// Layout as above (16 lanes a K row, 32 rows a load step); of a V row's part LV lanes, so a row group's lanes take RP rows
+// at once and keep the sums of theirs apart until the end.
+// ---------------------------------------------------------------------------
+template <int HD, int CS, int VU>
+__global__ __launch_bounds__(2 * WG) void attn_columns_kernel(const float* q, const float* Kc, const float* Vc, float* out, int len, int kvDim,
+                                                             int nHeads, int nKVHeads) {
+    constexpr int NWV = 2 * WG / 64, LPR = 16, NF = HD / 64, TG = 2 * WG / LPR, TILE = TG * VU;
+    constexpr int LV = HD / 4 / CS, RP = LPR / LV, NV = VU / RP;
+    static_assert(VU % RP == 0 && (LV == 4 || LV == 8), "whole steps");
+    __shared__ float wred[NWV], lbuf[NWV];
+    __shared__ float4 accbuf[NWV][LV];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    // the workgroups of neighbouring heads on one XCD (i mod 8), whose L2 then fetches the rows of few K/V heads (rows that come
+    // from beyond the L2s, 32 heads on 4, 1,200 rows: 12.1 us a launch with a workgroup a head, 10.1 with four, 9.1 so)
+    const int wgs = gridDim.x, at = wgs % 8 ? (int)blockIdx.x : (int)blockIdx.x % 8 * (wgs / 8) + (int)blockIdx.x / 8;
+    const int h = at / CS, part = at % CS;
+    const int kvOff = h / (nHeads / nKVHeads) * HD;
+    const int tg = tid / LPR, dl = tid % LPR, rp = dl / LV;
+    const float4* K4 = reinterpret_cast<const float4*>(Kc + kvOff) + dl;
+    const float4* V4 = reinterpret_cast<const float4*>(Vc + kvOff) + part * LV + dl % LV;
+    const size_t stride = (size_t)kvDim / 4;
+    float4 q4[NF];
+#pragma unroll
+    for (int j = 0; j < NF; j++) q4[j] = reinterpret_cast<const float4*>(q + (size_t)h * HD)[j * 16 + dl];
+    const float scale = 1.0f / sqrtf((float)HD);          // mongoose.cu:867 rsqrtf(headDim)
+    float m = -INFINITY, l = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int tile = 0; tile < len; tile += TILE) {
+        float4 k[VU][NF], v[NV];
+#pragma unroll
+        for (int u = 0; u < VU; u++)
+#pragma unroll
+            for (int j = 0; j < NF; j++) k[u][j] = K4[(size_t)min(tile + tg + u * TG, len - 1) * stride + j * 16];
+#pragma unroll
+        for (int i = 0; i < NV; i++) v[i] = V4[(size_t)min(tile + tg + (i * RP + rp) * TG, len - 1) * stride];
+        float sc[VU], tmax = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < VU; u++) {
+            float d = 0.f;
+#pragma unroll
+            for (int j = 0; j < NF; j++) {
+                d = fmaf(q4[j].x, k[u][j].x, d); d = fmaf(q4[j].y, k[u][j].y, d);
+                d = fmaf(q4[j].z, k[u][j].z, d); d = fmaf(q4[j].w, k[u][j].w, d);
+            }
+            sc[u] = tile + tg + u * TG < len ? row_sum16(d) * scale : -INFINITY;
+            tmax = fmaxf(tmax, sc[u]);
+        }
+        const float mNew = fmaxf(m, tg_max(tmax));          // the wave's maximum
+        const float mRef = mNew == -INFINITY ? 0.f : mNew;  // a wave none of whose rows exist yet
+        const float corr = exp_neg(m - mRef);
+        m = mNew;
+        acc.x *= corr; acc.y *= corr; acc.z *= corr; acc.w *= corr;
+        l *= corr;
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            float x = sc[i * RP];
+#pragma unroll
+            for (int r = 1; r < RP; r++) x = rp == r ? sc[i * RP + r] : x;
+            const float pv = exp_neg(x - mRef);             // masked rows: exp(-inf) = 0
+            l += pv;
+            acc.x = fmaf(pv, v[i].x, acc.x); acc.y = fmaf(pv, v[i].y, acc.y);
+            acc.z = fmaf(pv, v[i].z, acc.z); acc.w = fmaf(pv, v[i].w, acc.w);
+        }
+    }
+    // over the RP rows of a row group, then the wave's four row groups
+    auto rows = [](float x) __attribute__((always_inline)) {
+        if (RP == 4) x += dpp_f<0x124>(x);
+        x += dpp_f<0x128>(x);
+        return tg_sum(x);
+    };
+    acc.x = rows(acc.x); acc.y = rows(acc.y); acc.z = rows(acc.z); acc.w = rows(acc.w);
+    l = rows(l);
+    if ((tid & 63) < LV) accbuf[wave][tid & 63] = acc;
+    if ((tid & 63) == 0) { wred[wave] = m; lbuf[wave] = l; }
+    __syncthreads();
+    if (tid < LV) {
+        float M = wred[0];
+#pragma unroll
+        for (int w = 1; w < NWV; w++) M = fmaxf(M, wred[w]);
+        float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+        float den = 0.f;
+#pragma unroll
+        for (int w = 0; w < NWV; w++) {
+            const float g = exp_neg(wred[w] - M);           // a wave without rows: exp(-inf) = 0
+            const float4 a = accbuf[w][tid];
+            r.x = fmaf(g, a.x, r.x); r.y = fmaf(g, a.y, r.y); r.z = fmaf(g, a.z, r.z); r.w = fmaf(g, a.w, r.w);
+            den = fmaf(g, lbuf[w], den);
+        }
+        const float il = __builtin_amdgcn_rcpf(den);
+        reinterpret_cast<float4*>(out + (size_t)h * HD)[part * LV + tid] = make_float4(r.x * il, r.y * il, r.z * il, r.w * il);
+    }
+}
+
+hipError_t launch_attention_columns(const float* q, const float* K, const float* V, float* out, int len, int kvDim, int nHeads, int nKVHeads,
+                                    int headDim, hipStream_t s) {
+    if (len <= 0 || nHeads <= 0 || nKVHeads <= 0 || nHeads % nKVHeads != 0 || (headDim != 64 && headDim != 128)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)nHeads * 4);
+    if (headDim == 64) hipLaunchKernelGGL((attn_columns_kernel<64, 4, 8>), grid, dim3(2 * WG), 0, s, q, K, V, out, len, kvDim, nHeads, nKVHeads);
+    else hipLaunchKernelGGL((attn_columns_kernel<128, 4, 4>), grid, dim3(2 * WG), 0, s, q, K, V, out, len, kvDim, nHeads, nKVHeads);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Small per-op kernels (the reference's one-launch-per-op path)
 // ---------------------------------------------------------------------------
 // mongoose.cu:145-174, 372-404: out = rmsnorm(a (+ b), w), one workgroup a row; out may be a or b.

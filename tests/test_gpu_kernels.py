@@ -190,6 +190,30 @@ def test_decode_attention(hip, nH, nKV, hd, T):
             assert (got[h * hd:(h + 1) * hd] == Vc[0, (h // G) * hd:(h // G + 1) * hd]).all()
 
 
+@pytest.mark.parametrize("nH,nKV,hd,T", [(1, 1, 64, 1), (3, 3, 64, 31), (14, 2, 64, 33), (14, 2, 64, 255), (64, 8, 64, 256), (5, 1, 64, 257),
+                                         (65, 5, 64, 300), (8, 2, 128, 127), (8, 2, 128, 129), (64, 64, 128, 130), (66, 3, 128, 260), (4, 4, 64, 1025)])
+def test_decode_attention_by_columns(hip, nH, nKV, hd, T):
+    """Four workgroups a query head up to 64 heads, one beyond: around a tile (256 rows of 64, 128 of 128), with scores of some
+    +-60 (a maximum in any tile) and the lowest finite values among the keys.  The sum of T rounded products: 1e-5."""
+    dim, kvDim = nH * hd, nKV * hd
+    Q = (6 * rng.standard_normal(dim)).astype(np.float32)
+    Kc = (2 * rng.standard_normal((T, kvDim))).astype(np.float32)
+    Vc = rng.standard_normal((T, kvDim)).astype(np.float32)
+    if T > 2:
+        Kc[T // 2, :] = np.where(Q[:hd][None, :].repeat(nKV, 0).reshape(-1) > 0, -1e36, 1e36)      # head 0: a score of about -1e38
+        Kc[T // 2, hd:] = 0
+    dq, dk, dv, do = _up(hip, Q), _up(hip, Kc), _up(hip, Vc), hip.Zeros([dim])
+    E.KDecodeAttention(dq, dk, dv, do, T, dim, kvDim, nH, nKV)
+    _check()
+    ref = np.empty(dim)
+    for h in range(nH):
+        kv = slice(h // (nH // nKV) * hd, (h // (nH // nKV) + 1) * hd)
+        sc = Kc[:, kv].astype(np.float64) @ Q[h * hd:(h + 1) * hd] / np.sqrt(hd)
+        w = np.exp(sc - sc.max())
+        ref[h * hd:(h + 1) * hd] = (w / w.sum()) @ Vc[:, kv]
+    assert H.rel_err(hip.ToHost(do), ref) < 1e-5
+
+
 def test_elementwise_ops(hip):
     n = 4864
     g = (rng.standard_normal(n) * 3).astype(np.float32)
