@@ -139,14 +139,15 @@ void mongoose_dequant_q4_0(const void* w_q4_0, float* out, int rows, int cols, v
  * prefill.  The reference's nearest op is its dequantize-then-cuBLAS route
  * (mongoose_dequant_int8_to_fp32, mongoose.cu:1489, followed by MatMul,
  * cuda.go:230); here the int8 weights are read directly.  workspace: device
- * memory of at least 4 * roundup(T,128) * roundup(K,64) bytes for the two bf16
- * planes of the split activations.  K a multiple of 32; w and workspace
+ * memory of at least 4 * roundup(T,128) * roundup(K,64) bytes for the split
+ * activations (up to some hundred rows three planes of signed bytes and a scale
+ * a row and eighth of K, beyond two bf16 planes).  K a multiple of 32; w and workspace
  * 16-byte aligned. */
 void mongoose_q8_gemm(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
                       int K, int accumulate, void* workspace, size_t workspaceBytes, void* stream);
 /* No counterpart in the reference.  mongoose_q8_gemm for callers that cannot allocate and have no
  * workspace to hand over (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc): the two bf16 planes of the split activations are written into a static device array
+ * hipMalloc): the split activations are written into a static device array
  * of mg_q8_gemm_noalloc_max_bytes() = 8 MiB inside the library, so the call allocates nothing.
  * Limit: 4 * roundup(T,128) * roundup(K,64) <= 8 MiB (e.g. 512 x 4096, 128 x 16384); larger shapes
  * return MG_E_ARG with the sizes in mg_last_error().  Results are those of mongoose_q8_gemm bit

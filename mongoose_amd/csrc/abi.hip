@@ -14,7 +14,7 @@
 #include <string>
 #include <vector>
 
-// Scratch memory of mg_q8_gemm_noalloc: the two bf16 planes of the split activations live in this
+// Scratch memory of mg_q8_gemm_noalloc: the split activations live in this
 // array instead of a caller's workspace.  Every GPU the library runs on holds its own copy for the life
 // of the process.  In host code the name is only a handle: the device address is looked up once per
 // device (scratch_on_current_device) and that pointer is what kernels and copies are given.
@@ -225,23 +225,20 @@ void mongoose_dequant_q8_rowscale(const void* w, const float* scales, float* out
 void mongoose_dequant_q4_0(const void* w, float* out, int rows, int cols, void* stream) {
     note(mg::launch_dequant_q4_0(w, out, rows, cols, S(stream)));
 }
-// The two launches of the multi-row product: the activations' split into the planes at `ws` (`plane` bytes each), the
-// product.  The few-row kernel serves up to 512 rows, more where the matrix is narrow: the tiled kernel has no room for K
-// splits here and leaves most CUs idle until N / 128 x T / 64 tiles fill them.  Microseconds a call, few-row / tiled:
-// 5632 x 2048 14 / 38 at 77 rows, 43 / 53 at 450, 70 / 66 at 800; 896 x 4864 13 / 78 at 77, 77 / 84 at 1500; 9000 x 8192
-// 53 / 129 at 77, 204 / 236 at 450, 276 / 254 at 600.
+// The two launches of the multi-row product: the activations' digits (few_gemm.hip) or their split into the planes at `ws`
+// (`plane` bytes each), and the product.  The kernel for few rows serves up to 512, more where the matrix is narrow: the tiled
+// kernel has no room for K splits here and leaves most CUs idle until N / 128 x T / 64 tiles fill them.  Microseconds a call,
+// few rows / tiled: 5632 x 2048 54 / 58 at 513 rows, 74 / 68 at 800; 9000 x 8192 230 / 239 at 513, 400 / 317 at 800; 900 x
+// 2048 28 / 31 at 1000, 38 / 42 at 1500, 48 / 45 at 2000; 28672 x 4096 400 / 373 at 513.
 static hipError_t q8_gemm_launches(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
                                    int K, int accumulate, void* ws, size_t plane, hipStream_t s) {
     void* hi = ws;
     void* lo = static_cast<char*>(ws) + plane;
     if (T > 0 && N > 0 && (T <= 512 || (long long)T * N <= 1500000) && aligned16(act)) {
-        hipError_t e = mg::launch_few_split(act, static_cast<unsigned short*>(hi), static_cast<unsigned short*>(lo), T, K, 0, s);
-        if (e != hipSuccess) return e;
-        mg::FewParams f{};
-        f.seg[0] = mg::FewSeg{static_cast<const signed char*>(w), scales, bias, out, N};
-        f.T = T; f.K = K; f.accumulate = accumulate;
-        f.Ahi = static_cast<const unsigned short*>(hi); f.Alo = static_cast<const unsigned short*>(lo);
-        return mg::launch_few_rows(mg::FEW_STORE, f, s);
+        mg::FewGemmParams f{};
+        f.W = static_cast<const signed char*>(w); f.scales = scales; f.bias = bias; f.Y = out;
+        f.T = T; f.N = N; f.K = K; f.accumulate = accumulate;
+        return mg::launch_few_gemm(act, f, ws, s);
     }
     hipError_t e = mg::launch_split_rows(act, nullptr, 0.f, T, K, hi, lo, s);
     if (e != hipSuccess || T == 0 || N == 0) return e;

@@ -7,20 +7,18 @@ namespace mg {
 // One launch, tiles of 16 to 128 weight rows x 16 to 64 activation rows a workgroup (few_tile chooses); what follows the
 // product is the epilogue of the mode.
 enum FewMode {
-    FEW_STORE = 0,   // Y (+)= v * scale + bias
-    FEW_RESID = 1,   // Y += v * scale + bias; optionally the next projection's split of Y * nextGain and the rows' sums of squares
-    FEW_SWIGLU = 2,  // seg0 = gate, seg1 = up: silu(g) * u as the split of the down projection's input
-    FEW_QKV = 3,     // seg0 = q, seg1 = k, seg2 = v: bias, RoPE, q rows to seg0.Y, K / V rows into the caches at pos0 + row
+    FEW_RESID,       // Y += v * scale + bias; optionally the next projection's split of Y * nextGain and the rows' sums of squares
+    FEW_SWIGLU,    // seg0 = gate, seg1 = up: silu(g) * u as the split of the down projection's input
+    FEW_QKV,         // seg0 = q, seg1 = k, seg2 = v: bias, RoPE, q rows to seg0.Y, K / V rows into the caches at pos0 + row
 };
 struct FewSeg { const signed char* W; const float* scales; const float* bias; float* Y; int N; };
 struct FewParams {
     FewSeg seg[3];
     const unsigned short* Ahi;       // split activations in the order few_rows.hip describes (for this launch's weight format)
     const unsigned short* Alo;
-    const unsigned short* Ax;        // third terms (NULL: two terms); not with FEW_STORE
+    const unsigned short* Ax;        // third terms (NULL: two terms)
     int T, K;
     int q4;                          // weights: 0 = int8 rows with scales, 1 = Q4_0 in the split layout
-    int accumulate;                  // FEW_STORE: Y += instead of Y =
     // the rows' RMS factor, applied to the finished sums: sumSq holds sumParts partial sums of squares of every row,
     // sumStride floats apart (NULL: no factor)
     const float* sumSq;
@@ -51,8 +49,17 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s);
 hipError_t launch_embed_split(int kind, const void* table, const float* scales, const int* tokens, float* x, const float* gain,
                               unsigned short* hi, unsigned short* lo, unsigned short* ext, float* sumSq, int T, int dim, int vocab, int q4,
                               hipStream_t s);
-// Rows of fp32 activations split for a launch over weights of format q4.
-hipError_t launch_few_split(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4, hipStream_t s);
+// Several rows through one Q8 matrix on the integer matrix instruction (few_gemm.hip): Y[T,N] (+)= act[T,K] . W[N,K]^T *
+// scales[n] (+ bias[n]).  act, W and ws 16-byte aligned, K a multiple of 32; ws: few_gemm_bytes(T, K).
+struct FewGemmParams {
+    const signed char* W; const float* scales; const float* bias; float* Y;
+    int T, N, K, accumulate;
+    // filled by the launcher
+    const signed char* A; const float* aScales;
+    int nTiles;
+};
+size_t few_gemm_bytes(int T, int K);
+hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, hipStream_t s);
 
 // Causal attention of T query rows (rotated) at positions pos0 .. over the cache rows [0, pos0 + T), all products and sums
 // in fp32; the result goes out as the split the output projection reads.

@@ -1,5 +1,4 @@
-// few_rows.hip -- a layer over a handful of positions (short prompts, further turns of a conversation, small batches of
-// rows through one matrix).
+// few_rows.hip -- a layer over a handful of positions (short prompts, further turns of a conversation).
 //
 // Up to some hundred rows a projection is bound by its weight bytes and by launch latency, not by the matrix cores: what
 // counts is that every weight byte is requested once and early, by enough workgroups, and that a layer is few launches.
@@ -175,11 +174,10 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
     const int rowC = min(row, N - 1);
     const float sc = Q4 ? 1.0f : scales[rowC], bi = (MODE != FEW_SWIGLU && sg.bias) ? sg.bias[rowC] : 0.f;
     float gain = 1.0f, old[4] = {0.f, 0.f, 0.f, 0.f}, cs[4], sn[4];
-    if (MODE == FEW_RESID || MODE == FEW_STORE) {
-        if (MODE == FEW_RESID && p.nextGain) gain = p.nextGain[rowC];
-        if (MODE == FEW_RESID || p.accumulate)
+    if (MODE == FEW_RESID) {
+        if (p.nextGain) gain = p.nextGain[rowC];
 #pragma unroll
-            for (int e = 0; e < 4; e++) old[e] = sg.Y[(size_t)min(m0 + mq + e, T - 1) * N + rowC];
+        for (int e = 0; e < 4; e++) old[e] = sg.Y[(size_t)min(m0 + mq + e, T - 1) * N + rowC];
     }
     if (MODE == FEW_QKV) {
         const int half = p.headDim >> 1;
@@ -358,16 +356,7 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
         }
         v[e] = v[e] * sc * rs + bi;
     }
-    if (MODE == FEW_STORE) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int m = m0 + mq + e;
-            if (okN && m < T) {
-                float* y = sg.Y + (size_t)m * N + row;
-                *y = old[e] + v[e];
-            }
-        }
-    } else if (MODE == FEW_RESID) {
+    if (MODE == FEW_RESID) {
         float q2[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -460,7 +449,7 @@ static hipError_t launch_few_l(const FewParams& p, hipStream_t s) {
 
 template <int MODE, int MT, int NB, int Q4>
 static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
-    if constexpr (MODE != FEW_STORE && MT <= FEW_MT3)
+    if constexpr (MT <= FEW_MT3)
         if (p.Ax) return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0, 3>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1, 3>(p, s);
     if (p.Ax) return hipErrorInvalidValue;
     return p.K <= 64 * 2 * FR_WAVES ? launch_few_l<MODE, MT, NB, Q4, 0, 2>(p, s) : launch_few_l<MODE, MT, NB, Q4, 1, 2>(p, s);
@@ -516,12 +505,11 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
     if (p.T <= 0) return hipSuccess;
     if (p.K <= 0 || p.K % 32 || !p.Ahi || !p.Alo || p.seg[0].N <= 0) return hipErrorInvalidValue;
     const int terms = p.Ax ? 3 : 2;
-    if (terms == 3 && (mode == FEW_STORE || (p.nextHi && !p.nextX))) return hipErrorInvalidValue;
+    if (terms == 3 && p.nextHi && !p.nextX) return hipErrorInvalidValue;
     const int N = p.seg[0].N;
-    if (mode == FEW_STORE || mode == FEW_RESID) {
+    if (mode == FEW_RESID) {
         const FewTile t = few_tile(N, p.T, p.K, 1, 4, p.q4, terms);
         p.nTiles = (N + 16 * t.nb - 1) / (16 * t.nb);
-        if (mode == FEW_STORE) return t.nb == 1 ? launch_few_mt<FEW_STORE, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_STORE, 2>(t.mt, p, s) : launch_few_mt<FEW_STORE, 4>(t.mt, p, s);
         return t.nb == 1 ? launch_few_mt<FEW_RESID, 1>(t.mt, p, s) : t.nb == 2 ? launch_few_mt<FEW_RESID, 2>(t.mt, p, s) : launch_few_mt<FEW_RESID, 4>(t.mt, p, s);
     }
     if (mode == FEW_SWIGLU) {
@@ -567,39 +555,6 @@ hipError_t launch_embed_split(int kind, const void* table, const float* scales, 
                               hipStream_t s) {
     if (T <= 0) return hipSuccess;
     hipLaunchKernelGGL(embed_split_kernel, dim3((unsigned)T), dim3(WG), 0, s, kind, table, scales, tokens, x, gain, hi, lo, ext, sumSq, dim, vocab, q4);
-    return hipGetLastError();
-}
-
-// Rows of a caller's activations (per-op GEMM), one workgroup per 16 rows x 256 k: the planes are written whole lanes at a
-// time, rows past T as zeros.
-__global__ __launch_bounds__(WG) void few_split_kernel(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4) {
-    const int k = blockIdx.x * 256 + (threadIdx.x >> 4) * 8, r = threadIdx.x & 15;
-    const int t = blockIdx.y * 16 + r;
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const int kk = k + half * 128;
-        if (kk >= K) continue;
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f), c = a;
-        if (t < T) {
-            a = *reinterpret_cast<const float4*>(in + (size_t)t * K + kk);
-            c = *reinterpret_cast<const float4*>(in + (size_t)t * K + kk + 4);
-        }
-        const float v[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
-        unsigned h[4], l[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            h[i] = bf16_pair(v[2 * i], v[2 * i + 1]);
-            l[i] = bf16_pair(v[2 * i] - bf16_value((unsigned short)(h[i] & 0xffffu)), v[2 * i + 1] - bf16_value((unsigned short)(h[i] >> 16)));
-        }
-        const size_t o = few_index(t, kk, K, q4);
-        *reinterpret_cast<uint4*>(hi + o) = make_uint4(h[0], h[1], h[2], h[3]);
-        *reinterpret_cast<uint4*>(lo + o) = make_uint4(l[0], l[1], l[2], l[3]);
-    }
-}
-hipError_t launch_few_split(const float* in, unsigned short* hi, unsigned short* lo, int T, int K, int q4, hipStream_t s) {
-    if (T <= 0) return hipSuccess;
-    if (K % 32 || ((uintptr_t)in & 15)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(few_split_kernel, dim3((unsigned)((K + 255) / 256), (unsigned)((T + 15) / 16)), dim3(WG), 0, s, in, hi, lo, T, K, q4);
     return hipGetLastError();
 }
 

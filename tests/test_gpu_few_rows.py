@@ -100,6 +100,43 @@ def test_few_row_gemm_matches_float64(hip, rows, n, k, accumulate):
         t.Release()
 
 
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (15, 16, 64), (16, 17, 96), (17, 129, 544), (33, 40, 1056), (64, 128, 1024), (65, 600, 1088),
+                                      (5, 48, 8192), (9, 20, 8224), (3, 30, 16384)])
+def test_few_row_gemm_digits(hip, rows, n, k):
+    """Activations as 24-bit numbers with a scale a row and eighth of K, at edges of the runs and tiles, for rows of any
+    magnitude: a value is off by half a step, 2^-24 of its run's largest one; a result by sqrt(k) such errors times weights of
+    75 at random, six times that for the worst of a row, plus what fp32 sums and factors lose (1e-6 of the largest).  A row
+    with a NaN or an infinity is NaN."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((rows, k), dtype=np.float32)
+    for i, scale in enumerate((1e-37, 1e30, 1e-21, 0.0, 2.0 ** -64, 1.0)):
+        if i + 2 < rows:
+            a[i + 2] *= np.float32(scale)
+    if rows > 12:
+        a[9, rng.integers(k)] = 3e4
+        a[10, k // 2], a[11, k - 1] = np.inf, np.nan
+        a[12, 0] = -1e36
+    w = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    sc = (0.01 * (1 + rng.random(n))).astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        ref = a.astype(np.float64) @ (w.astype(np.float64) * sc[:, None].astype(np.float64)).T
+    ta, tw, ts, to = hip.FromHost(a, a.shape), hip.UploadRawBytes(w), hip.FromHost(sc, sc.shape), hip.Zeros([rows, n])
+    nbytes = 4 * ((rows + 127) // 128 * 128) * ((k + 63) // 64 * 64)
+    ws = hip.UploadRawBytes(np.full(nbytes, 0xff, np.uint8))
+    E.KQ8Gemm(ta, tw, ts, None, to, rows, n, k, 0, ws, nbytes)
+    E.KSync()
+    assert E.HIPCheck() == 0
+    got = hip.ToHost(to).reshape(rows, n)
+    for i in range(rows):
+        if not np.isfinite(a[i]).all():
+            assert np.isnan(got[i]).all()
+        else:
+            bar = 6 * 2.0 ** -24 * np.abs(a[i]).max() * np.sqrt(k) * 75 * 0.015 + 1e-6 * np.abs(ref[i]).max()
+            assert np.abs(got[i] - ref[i]).max() <= bar + 1e-45, i
+    for t in (ta, tw, ts, to, ws):
+        t.Release()
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 4), (2, 2048), (3, 2052), (1, 4100), (2, 8192), (1, 8196), (2, 30)])
 def test_rmsnorm_rows_kept_in_registers_and_others(hip, rows, dim):
     rng = np.random.default_rng(dim)
