@@ -528,8 +528,10 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
-// Embedding rows, their split times the first gain, their sums of squares: one workgroup a row.
+// Embedding rows, their split times the first gain, their sums of squares: one workgroup a row.  Rows of up to EV * 256
+// elements have all of their loads under way at once.
 // ---------------------------------------------------------------------------
+constexpr int EV = 8;
 __global__ __launch_bounds__(WG) void embed_split_kernel(int kind, const void* table, const float* scales, const int* tokens, float* x,
                                                          const float* gain, unsigned short* hi, unsigned short* lo, unsigned short* ext, float* sumSq,
                                                          int dim, int vocab, int q4) {
@@ -538,14 +540,24 @@ __global__ __launch_bounds__(WG) void embed_split_kernel(int kind, const void* t
     int tok = tokens[t];
     tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);
     float ss = 0.f;
-    for (int i = threadIdx.x; i < dim; i += WG) {
-        const float v = embed_value(kind, table, scales, tok, dim, vocab, i);
-        x[(size_t)t * dim + i] = v;
-        ss += v * v;
-        const float a = v * gain[i];
-        const size_t o = few_index(t, i, dim, q4);
-        if (ext) put_split<true>(hi, lo, ext, o, a);
-        else put_split<false>(hi, lo, ext, o, a);
+    for (int i0 = threadIdx.x; i0 < dim; i0 += EV * WG) {
+        float v[EV], g[EV];
+#pragma unroll
+        for (int j = 0; j < EV; j++) {
+            const int i = min(i0 + j * WG, dim - 1);
+            v[j] = embed_value(kind, table, scales, tok, dim, vocab, i);
+            g[j] = gain[i];
+        }
+#pragma unroll
+        for (int j = 0; j < EV; j++) {
+            const int i = i0 + j * WG;
+            if (i >= dim) continue;
+            x[(size_t)t * dim + i] = v[j];
+            ss += v[j] * v[j];
+            const size_t o = few_index(t, i, dim, q4);
+            if (ext) put_split<true>(hi, lo, ext, o, v[j] * g[j]);
+            else put_split<false>(hi, lo, ext, o, v[j] * g[j]);
+        }
     }
     ss = block_sum(ss, red);
     if (threadIdx.x == 0) sumSq[t] = ss;

@@ -134,9 +134,11 @@ public:
     float* hidden[2] = {nullptr, nullptr};
     int hiddenIdx = 0;
     int enqueueLayer(const LayerWeights& L, int layer, const StepState* st, int posImm);
-    int enqueueFinal(bool withArgmax);
+    // row / parts: the lm_head of that row (instead of the hidden buffer), its argmax partials left for the caller
+    int enqueueFinal(bool withArgmax, const float* row = nullptr, int* parts = nullptr);
     int publish(const float* src, int n, const int* ints, int nInts);      // results on their way to hOut
-    int collect(float* out, int n, int* ints, int nInts);                  // ... waited for and copied to the caller
+    PublishParams publishParams(const float* src, int n);
+    int collect(float* out, int n, int* ints, int nInts, bool prefill = false);      // ... waited for and copied to the caller
     float* logits = nullptr;
     float* finalNorm = nullptr;
     DevMat lmHead;

@@ -154,7 +154,7 @@ HIPFusedInference* HIPFusedInference::New(int dim, int kvDim, int headDim, int n
     f->hGate = static_cast<int*>(hp);
     *f->hGate = 1;
     // what calls hand over and take in: flags, error word, token ids, floats out; words in
-    f->hOutInts = 64 + 16 * PUBLISH_MAX_SLICES;
+    f->hOutInts = 64 + 16 * (PUBLISH_MAX_SLICES + 1);
     f->hOutFloats = (f->hOutInts + maxSeq + 1 + 63) / 64 * 64;
     const size_t outWords = (size_t)f->hOutFloats + std::max(vocabSize, dim), inWords = (size_t)std::max(maxSeq, dim);
     if (hipHostMalloc(&hp, outWords * 4, hipHostMallocDefault) != hipSuccess) return fail("pinned alloc");
@@ -1075,18 +1075,24 @@ int HIPFusedInference::setState(int pos, int token, int count, int nPrompt) {
 // Queues n floats of src, nInts ints and the persistent launch's error word behind everything queued so far; collect()
 // waits for them.  One small launch writes them to page-locked memory and the host watches for its flags: a synchronous
 // copy each of logits, token and error word, behind a stream synchronisation, cost 125 us a token of the 1.1B shape.
-int HIPFusedInference::publish(const float* src, int n, const int* ints, int nInts) {
+PublishParams HIPFusedInference::publishParams(const float* src, int n) {
     PublishParams p{};
     p.src = src; p.dst = reinterpret_cast<float*>(hOut + hOutFloats); p.n = n;
-    p.ints = ints; p.intDst = reinterpret_cast<int*>(hOut + hOutInts); p.nInts = nInts;
+    p.intDst = reinterpret_cast<int*>(hOut + hOutInts);
     p.err = dFlowErr; p.errDst = reinterpret_cast<int*>(hOut);
     p.flags = hOut + 64; p.seq = ++hOutSeq;
+    return p;
+}
+int HIPFusedInference::publish(const float* src, int n, const int* ints, int nInts) {
+    PublishParams p = publishParams(src, n);
+    p.ints = ints; p.nInts = nInts;
     HIPCHK(launch_publish(p, stream));
     return MG_OK;
 }
 
-int HIPFusedInference::collect(float* out, int n, int* ints, int nInts) {
-    const int per = publish_slice_floats(n), slices = publish_slices(n);
+// prefill: what launch_publish_prefill hands over.
+int HIPFusedInference::collect(float* out, int n, int* ints, int nInts, bool prefill) {
+    const int per = publish_slice_floats(n), slices = prefill ? (n > 0 ? publish_slices(n) : 0) + 1 : publish_slices(n);
     const auto t0 = std::chrono::steady_clock::now();
     bool waited = false;
     for (int b = 0; b < slices; b++) {
@@ -1172,7 +1178,7 @@ int HIPFusedInference::enqueueLayer(const LayerWeights& L, int layer, const Step
 
 // Final norm + lm_head (cuda_fused_infer.go:446-448) with the per-workgroup
 // argmax folded into the matvec epilogue.
-int HIPFusedInference::enqueueFinal(bool withArgmax) {
+int HIPFusedInference::enqueueFinal(bool withArgmax, const float* row, int* parts) {
     if (withArgmax) statePosHost = -1;              // (the argmax's last kernel advances the device state)
     if (!finalNorm || !lmHead.w) { set_error("final norm / lm_head not set"); return MG_E_STATE; }
     if (execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P) {
@@ -1190,7 +1196,7 @@ int HIPFusedInference::enqueueFinal(bool withArgmax) {
     }
     MvParams p{};
     p.seg[0] = MvSeg{lmHead.w, lmHead.scales, nullptr, logits, vocabSize};
-    p.nseg = 1; p.K = dim; p.act = hidden[hiddenIdx]; p.gain = finalNorm; p.eps = eps;
+    p.nseg = 1; p.K = dim; p.act = row ? row : hidden[hiddenIdx]; p.gain = finalNorm; p.eps = eps;
     p.amaxVal = amaxVal; p.amaxIdx = amaxIdx;
     if (fuseEmbed && flowEligible(0, nLayers)) {
         // inside the captured token: the lm_head launch also leaves the exchange area of the persistent
@@ -1204,6 +1210,7 @@ int HIPFusedInference::enqueueFinal(bool withArgmax) {
     if (mark(7)) return MG_E_HIP;
     if (withArgmax) {
         if (c.grid > amaxParts) { set_error("argmax partial buffer too small"); return MG_E_STATE; }
+        if (parts) { *parts = c.grid; return MG_OK; }
         HIPCHK(launch_argmax_finish(amaxVal, amaxIdx, c.grid, dState, nullptr, dHistory, maxSeq + 1, vocabSize, ropeRef(), embedRef(), stream));
     }
     return MG_OK;
@@ -1950,15 +1957,23 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
     }
     if (rc) return rc;
     // the last position continues on the decode path: final norm, lm_head, greedy token, state -> pos0 + T
-    HIPCHK(launch_prefill_tail(pfX + (size_t)(T - 1) * dim, hidden[hiddenIdx], dim, dState, pos0 + T - 1, tokens[T - 1], ropeRef(), stream));
-    rc = enqueueFinal(true);
-    if (rc) return rc;
-    statePosHost = pos0 + T;                        // where the argmax's last kernel leaves the state
-    if (elapsedMs) HIPCHK(hipEventRecord(ev1, stream));
+    const float* row = pfX + (size_t)(T - 1) * dim;
     const int n = logitsOut ? vocabSize : 0;
     int next = 0;
-    rc = publish(logits, n, dHistory, 1);
-    if (rc == 0) rc = collect(logitsOut, n, &next, 1);
+    const bool quantized = execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P;      // (a tail that wants the hidden buffer)
+    if (quantized) {
+        HIPCHK(launch_prefill_tail(row, hidden[hiddenIdx], dim, dState, pos0 + T - 1, tokens[T - 1], ropeRef(), stream));
+        rc = enqueueFinal(true);
+        if (rc == 0) rc = publish(logits, n, dHistory, 1);
+    } else {
+        PrefillEnd e{amaxVal, amaxIdx, 0, dState, pos0 + T, dHistory, vocabSize, ropeRef(), row, hidden[hiddenIdx], dim};
+        rc = enqueueFinal(true, row, &e.nparts);
+        if (rc == 0) HIPCHK(launch_publish_prefill(publishParams(logits, n), e, stream));
+    }
+    if (rc) return rc;
+    statePosHost = pos0 + T;                        // where the last kernel leaves the state
+    if (elapsedMs) HIPCHK(hipEventRecord(ev1, stream));
+    rc = collect(logitsOut, n, &next, 1, !quantized);
     if (rc) return rc;
     if (nextToken) *nextToken = next;
     if (elapsedMs) {

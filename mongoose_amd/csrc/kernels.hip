@@ -1865,6 +1865,46 @@ hipError_t launch_publish(const PublishParams& p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// With the argmax's last step, the state and the last row's copy as launches of their own, two dependent launches of 4 us each
+// stood between the lm_head and this one.
+__global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, PrefillEnd e, int per) {
+    const int b = blockIdx.x;
+    if (b + 1 < (int)gridDim.x) {
+        const int i0 = b * per, i1 = min(p.n, i0 + per), n4 = (i1 - i0) >> 2;
+        const float4* s4 = reinterpret_cast<const float4*>(p.src + i0);
+        float4* d4 = reinterpret_cast<float4*>(p.dst + i0);
+        for (int i = threadIdx.x; i < n4; i += WG) d4[i] = s4[i];
+        for (int i = i0 + n4 * 4 + threadIdx.x; i < i1; i += WG) p.dst[i] = p.src[i];
+    } else {
+        __shared__ float bv[WG / 64];
+        __shared__ int bi[WG / 64];
+        float v = -INFINITY;
+        int idx = INT_MAX;
+        for (int i = threadIdx.x; i < e.nparts; i += WG) argmax_pick(v, idx, e.pv[i], e.pi[i]);
+        copy_rope_row(e.rope, e.pos);
+        for (int i = threadIdx.x; i < e.dim; i += WG) e.hidden[i] = e.row[i];
+        wave_argmax(v, idx);
+        if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < WG / 64; w++) argmax_pick(v, idx, bv[w], bi[w]);
+            const int tok = idx < 0 || idx >= e.vocab ? 0 : idx;
+            e.history[0] = tok;
+            e.state->pos = e.pos; e.state->token = tok; e.state->count = 1; e.state->nPrompt = 0;
+            p.intDst[0] = tok;
+            *p.errDst = p.err ? *p.err : 0;
+        }
+    }
+    __threadfence_system();                          // every thread's own stores have reached the host's memory
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(p.flags + b * 16, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+hipError_t launch_publish_prefill(const PublishParams& p, const PrefillEnd& e, hipStream_t s) {
+    const int slices = p.n > 0 ? publish_slices(p.n) : 0;
+    hipLaunchKernelGGL(publish_prefill_kernel, dim3((unsigned)slices + 1), dim3(WG), 0, s, p, e, publish_slice_floats(p.n));
+    return hipGetLastError();
+}
+
 // Bound by the link: 16 workgroups of 512 threads, four 16-byte loads each in flight, read page-locked memory at 55 GB/s
 // (8.4 MB in 156 us; 64 workgroups 53 GB/s, 256 43; the copy engine 160 us).  hipMemcpyAsync writes anything up to 64 KB
 // from the host, at 0.26 GB/s and before it returns: the row scales of an 896 x 4864 matrix alone were 75 us.
