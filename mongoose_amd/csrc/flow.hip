@@ -598,7 +598,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     constexpr bool GL = CBD > 1;
     __shared__ float4 sqkv[2 + QHMAX][HD / 4];         // K and V row of the current position, q of the workgroup's heads
     __shared__ float4 accbuf[QHMAX][FWAVES][HD / 4];   // per query head of the workgroup: the waves' partial outputs, sums, maxima
-    __shared__ float lbuf[QHMAX][FWAVES], wred[QHMAX][FWAVES];
+    __shared__ __attribute__((aligned(16))) float lbuf[QHMAX][FWAVES], wred[QHMAX][FWAVES];
     __shared__ float outbuf[FLOW_MAX_ROUNDS][FWAVES];                // a phase's results of the workgroup, stored by one wave as whole 32-byte runs
     __shared__ int4 pfScrap[64];                       // where the prefetching loads land (never read)
     __shared__ float tailV[FWAVES];                    // the tail's argmax: the waves' best values and indices
@@ -1132,6 +1132,33 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                         }
                         // the waves' partials of all the workgroup's heads combined together: one barrier, a thread per head and piece
                         __syncthreads();
+                        if constexpr (!GQA && (FIX & 7) != 1) {
+                            // One head: one wave, whose four row groups take two waves' partials each -- a chain of two terms and
+                            // two exchanges instead of eight terms a thread.  (Microseconds a token, by waves' partials one after the
+                            // other / so: toy shape 50.3 / 49.8, hidden size 256 70.0 / 69.2, 1.1B 356 / 354, at 600 positions 429 /
+                            // 426.5; the variants with the 0.5B shape's sizes 266.0 / 268.4, Q4_0 the same: not there.)
+                            if (wave == 0) {
+                                constexpr int NP = HD / 64;
+                                const int i = lane & 15, k0 = lane >> 4;
+                                const float4 ma = *reinterpret_cast<const float4*>(&wred[0][0]), mb = *reinterpret_cast<const float4*>(&wred[0][4]);
+                                const float m0 = wred[0][k0], m1 = wred[0][k0 + 4], l0 = lbuf[0][k0], l1 = lbuf[0][k0 + 4];
+                                float4 x0[NP], x1[NP];
+#pragma unroll
+                                for (int j = 0; j < NP; j++) { x0[j] = accbuf[0][k0][i + 16 * j]; x1[j] = accbuf[0][k0 + 4][i + 16 * j]; }
+                                const float mg_ = fmaxf(fmaxf(fmaxf(ma.x, ma.y), fmaxf(ma.z, ma.w)), fmaxf(fmaxf(mb.x, mb.y), fmaxf(mb.z, mb.w)));
+                                const float w0 = exp_neg(m0 - mg_), w1 = exp_neg(m1 - mg_);
+                                float lg = tg_sum(fmaf(w1, l1, w0 * l0));
+                                const float il = nsplit == 1 ? __builtin_amdgcn_rcpf(lg) : 1.0f;      // (one split: see below)
+                                if (nsplit == 1) lg = 1.0f;
+#pragma unroll
+                                for (int j = 0; j < NP; j++) {
+                                    const f4 r = {tg_sum(fmaf(w1, x1[j].x, w0 * x0[j].x)) * il, tg_sum(fmaf(w1, x1[j].y, w0 * x0[j].y)) * il,
+                                                  tg_sum(fmaf(w1, x1[j].z, w0 * x0[j].z)) * il, tg_sum(fmaf(w1, x1[j].w, w0 * x0[j].w)) * il};
+                                    if (lane < 16) stx4(reinterpret_cast<f4*>(X + G.offPacc + (size_t)split * dim + h0 * HD) + i + 16 * j, r);
+                                }
+                                if (lane == 0) { stx(X + G.offPm + split * nHeadsV + h0, mg_); stx(X + G.offPl + split * nHeadsV + h0, lg); }
+                            }
+                        } else
                         if (tid < QH * (HD / 4)) {
                             const int hq = tid / (HD / 4), i = tid % (HD / 4), h = h0 + hq;
                             float mg_ = wred[hq][0];
