@@ -174,9 +174,9 @@ hipError_t launch_advance_prompt(StepState* state, const int* prompt, RopeCur ro
 hipError_t launch_signal_mailbox(unsigned* counter, unsigned value, hipStream_t s);
 
 // What a call hands to its caller -> page-locked host memory, behind everything queued before it on the stream: n floats of
-// src in publish_slices(n) slices, nInts ints, the error word.  A
+// src in publish_slices(n) slices, in their order, nInts ints, the error word.  A
 // slice's flag (64 bytes apart) takes the value seq once the slice is in host memory, so the host copies one slice on
-// while the next one crosses the link; the ints and the error word are there with the first.  Host addresses are what
+// while the next ones cross the link; the ints and the error word are there with the first.  Host addresses are what
 // hipHostMalloc returned.
 struct PublishParams {
     const float* src; float* dst; int n;

@@ -1844,37 +1844,48 @@ hipError_t launch_signal_mailbox(unsigned* counter, unsigned value, hipStream_t 
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(WG) void publish_kernel(PublishParams p, int per) {
-    const int b = blockIdx.x;
-    const int i0 = b * per, i1 = min(p.n, i0 + per);
-    const float4* s4 = reinterpret_cast<const float4*>(p.src + i0);
-    float4* d4 = reinterpret_cast<float4*>(p.dst + i0);
-    const int n4 = (i1 - i0) >> 2;
-    for (int i = threadIdx.x; i < n4; i += WG) d4[i] = s4[i];
-    for (int i = i0 + n4 * 4 + threadIdx.x; i < i1; i += WG) p.dst[i] = p.src[i];
-    if (b == 0) {
-        for (int i = threadIdx.x; i < p.nInts; i += WG) p.intDst[i] = p.ints[i];
-        if (threadIdx.x == 0) *p.errDst = p.err ? *p.err : 0;
+// Bound by the link (55 GB/s: 11 us for 152K floats) and by the host's copy out of the page-locked buffer (6 us), which can
+// run beside it only if the slices arrive one after the other.  A workgroup a slice brought all of them in together, at the
+// end: a token with its logits took 77.1 us where 8 workgroups that go through the slices in order take 69.9 (151,936 floats;
+// 70.9 -> 64.3 at 128,256, 44.1 -> 41.4 at 32,000; 4 workgroups do not fill the link, 16 leave 72.9).  The fence is one wave's:
+// one of every wave writes the L2 back four times a slice, 43.7 us at 32,000.
+constexpr int PUBLISH_WGS = 8;
+__device__ __forceinline__ void publish_flag(const PublishParams& p, int b) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this wave's stores have arrived ...
+    __syncthreads();                                 // ... and the other waves'
+    if (threadIdx.x == 0) {
+        __threadfence_system();
+        __hip_atomic_store(p.flags + b * 16, p.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    __threadfence_system();                          // every thread's own stores have reached the host's memory
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(p.flags + b * 16, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-hipError_t launch_publish(const PublishParams& p, hipStream_t s) {
-    hipLaunchKernelGGL(publish_kernel, dim3((unsigned)publish_slices(p.n)), dim3(WG), 0, s, p, publish_slice_floats(p.n));
-    return hipGetLastError();
-}
-
-// With the argmax's last step, the state and the last row's copy as launches of their own, two dependent launches of 4 us each
-// stood between the lm_head and this one.
-__global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, PrefillEnd e, int per) {
-    const int b = blockIdx.x;
-    if (b + 1 < (int)gridDim.x) {
+__device__ __forceinline__ void publish_floats(const PublishParams& p, int per, int slices) {
+    for (int b = blockIdx.x; b < slices; b += PUBLISH_WGS) {
         const int i0 = b * per, i1 = min(p.n, i0 + per), n4 = (i1 - i0) >> 2;
         const float4* s4 = reinterpret_cast<const float4*>(p.src + i0);
         float4* d4 = reinterpret_cast<float4*>(p.dst + i0);
         for (int i = threadIdx.x; i < n4; i += WG) d4[i] = s4[i];
         for (int i = i0 + n4 * 4 + threadIdx.x; i < i1; i += WG) p.dst[i] = p.src[i];
+        publish_flag(p, b);
+    }
+}
+__global__ __launch_bounds__(WG) void publish_kernel(PublishParams p, int per, int slices) {
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < p.nInts; i += WG) p.intDst[i] = p.ints[i];
+        if (threadIdx.x == 0) *p.errDst = p.err ? *p.err : 0;
+    }
+    publish_floats(p, per, slices);
+}
+hipError_t launch_publish(const PublishParams& p, hipStream_t s) {
+    const int slices = publish_slices(p.n), wgs = slices < PUBLISH_WGS ? slices : PUBLISH_WGS;
+    hipLaunchKernelGGL(publish_kernel, dim3((unsigned)wgs), dim3(WG), 0, s, p, publish_slice_floats(p.n), slices);
+    return hipGetLastError();
+}
+
+// With the argmax's last step, the state and the last row's copy as launches of their own, two dependent launches of 4 us each
+// stood between the lm_head and this one.
+__global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, PrefillEnd e, int per, int slices) {
+    if (blockIdx.x < PUBLISH_WGS) {
+        publish_floats(p, per, slices);
     } else {
         __shared__ float bv[WG / 64];
         __shared__ int bi[WG / 64];
@@ -1894,14 +1905,12 @@ __global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, Pr
             p.intDst[0] = tok;
             *p.errDst = p.err ? *p.err : 0;
         }
+        publish_flag(p, slices);
     }
-    __threadfence_system();                          // every thread's own stores have reached the host's memory
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(p.flags + b * 16, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 hipError_t launch_publish_prefill(const PublishParams& p, const PrefillEnd& e, hipStream_t s) {
     const int slices = p.n > 0 ? publish_slices(p.n) : 0;
-    hipLaunchKernelGGL(publish_prefill_kernel, dim3((unsigned)slices + 1), dim3(WG), 0, s, p, e, publish_slice_floats(p.n));
+    hipLaunchKernelGGL(publish_prefill_kernel, dim3(PUBLISH_WGS + 1), dim3(WG), 0, s, p, e, publish_slice_floats(p.n), slices);
     return hipGetLastError();
 }
 

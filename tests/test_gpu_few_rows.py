@@ -153,3 +153,20 @@ def test_rmsnorm_rows_kept_in_registers_and_others(hip, rows, dim):
     assert H.rel_err(hip.ToHost(tb).reshape(rows, dim), ref(a.astype(np.float64) + b)) < 1e-6
     for t in (ta, tb, tw, to):
         t.Release()
+
+
+@pytest.mark.parametrize("vocab", [3, 1023, 1024, 1025, 8190, 8193, 9219, 32767, 32770, 40001])
+def test_logits_arrive_whole(hip, vocab):
+    """The logits cross to the host in slices of at least 1,024 floats, of which eight workgroups take one each in turn: below,
+    at and above a slice, eight slices and the most there can be (32), against the oracle, for a single token and behind a
+    prompt.  The page-locked buffer holds the call before's values: a slice copied too early would show those."""
+    m = H.Model(SMALL._replace(vocab=vocab, nLayers=1), seed=vocab, maxSeq=16, eng=hip)
+    toks, got = m.prompt(8), np.empty(vocab, np.float32)
+    want = [m.orc.step(m.orc.embed(int(t)), pos, shadow=True)[1] for pos, t in enumerate(toks)]
+    for pos, t in enumerate(toks):
+        rc, _ = m.hip.DecodeToken(int(t), pos, got)
+        assert rc == 0 and H.rel_err(got, want[pos]) < 1e-4, E.last_error()
+    for n in (8, 5):
+        rc, nxt, logits, _ = m.hip.Prefill(toks[:n], 0, wantLogits=True)
+        assert rc == 0 and H.rel_err(logits, want[n - 1]) < 1e-3 and logits[nxt] == logits.max(), E.last_error()
+    m.close()
