@@ -572,13 +572,20 @@ hipError_t launch_embed_split(int kind, const void* table, const float* scales, 
 
 // ---------------------------------------------------------------------------
 // Causal attention over fp32 (or fp16) cache rows in fp32, on v_mfma_f32_16x16x4_f32: no split of the operands, no pass
-// over the cache rows beforehand.  A workgroup = one query head x 16 queries; its 8 waves take the 16-position tiles in
-// turn, each with a running maximum / sum / output of its own, combined through LDS at the end.
+// over the cache rows beforehand.  A workgroup = one query head x 16 queries x 1 / CS of the output's columns; its 8
+// waves take the 16-position tiles in turn, each with a running maximum / sum / output of its own, combined through LDS at the end.
 //   S^T[kpos][q] = K . Q^T   A = K rows (lane: row l%16), B = Q rows; the quarter l/16 of a lane holds the head elements
 //                            HD/4 * (l/16) + s, s = 0 .. HD/4 - 1, of both
 //   O^T[d][q]    = V^T . P^T a lane holds S^T rows 4 (l/16) + e of its query: as the B operand of step e it is position
-//                            4 (l/16) + e, which is the V row the lane loads; its elements HD/16 * (l%16) + b make up
-//                            row l%16 of output block b
+//                            4 (l/16) + e, which is the V row the lane loads; its elements HD/16/CS * (l%16) + b of the
+//                            workgroup's columns make up row l%16 of output block b
+// A prompt of a few rows has fewer (head, 16 queries) than the chip has CUs, and each is bound by its own matrix products and
+// V loads.  So CS = 2 or 4 workgroups share one as long as 256 are not exceeded: all of them form the scores (half of the
+// products), each a share of the columns, by the same sums.  Microseconds a layer with 1 / 2 / 4, all five launches:
+//   14 heads of 64 on 2: 37 rows behind 200 37.1 / 36.1 / 35.8, behind 1,000 46.2 / 43.8 / 42.9; 128 rows 47.2 / 46.7 / 47.2
+//   32 heads of 128 on 8: 16 rows behind 500 113.4 / 109.6 / 107.9; 64 behind 1,000 188.4 / 182.8 / 198.0
+// and past 256 workgroups the repeated scores cost more than they save: 14 heads, 256 rows behind 1,000 76.6 / 83.8 / 98.0.
+// (16 waves a workgroup: 0.3 to 1.3 us more at every size.)
 // ---------------------------------------------------------------------------
 template <bool KVH>
 __device__ __forceinline__ float4 ld_row4(const void* base, size_t i) {
@@ -588,17 +595,36 @@ __device__ __forceinline__ float4 ld_row4(const void* base, size_t i) {
                        half_bits_to_float((unsigned short)(u.y & 0xffffu)), half_bits_to_float((unsigned short)(u.y >> 16)));
 }
 
-template <int HD, bool KVH>
+// n consecutive cache values
+template <bool KVH, int N>
+__device__ __forceinline__ void ld_row(const void* base, size_t i, float (&r)[N]) {
+    if constexpr (N >= 4) {
+#pragma unroll
+        for (int j = 0; j < N; j += 4) {
+            const float4 t = ld_row4<KVH>(base, i + j);
+            r[j] = t.x; r[j + 1] = t.y; r[j + 2] = t.z; r[j + 3] = t.w;
+        }
+    } else if constexpr (!KVH) {
+#pragma unroll
+        for (int j = 0; j < N; j++) r[j] = static_cast<const float*>(base)[i + j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; j++) r[j] = half_bits_to_float(static_cast<const unsigned short*>(base)[i + j]);
+    }
+}
+
+template <int HD, bool KVH, int CS>
 __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, const void* Kc, const void* Vc, unsigned short* hi,
                                                              unsigned short* lo, unsigned short* ext, int T, int pos0, int dim, int kvDim, int nHeads,
                                                              int nKVHeads, int q4) {
-    constexpr int KF = HD / 16, VF = HD / 16;              // K: float4 a lane and row (HD/4 elements); V: elements a lane and row
+    constexpr int KF = HD / 16, VF = HD / 16 / CS;         // K: float4 a lane and row (HD/4 elements); V: elements a lane and row
     constexpr int OST = 17;
     extern __shared__ float ob[];                          // [wave][HD][OST]
     __shared__ float wm[FR_WAVES][16], wl[FR_WAVES][16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, fq = lane >> 4;
-    const int head = blockIdx.x % nHeads, q0 = ((int)gridDim.x / nHeads - 1 - (int)blockIdx.x / nHeads) * 16;    // the longest ranges first
+    const int item = blockIdx.x / CS, d0 = (int)blockIdx.x % CS * (HD / CS);
+    const int head = item % nHeads, q0 = ((int)gridDim.x / CS / nHeads - 1 - item / nHeads) * 16;    // the longest ranges first
     const int kvh = head / (nHeads / nKVHeads);
     const int myq = min(q0 + fr, T - 1), qpos = pos0 + myq;
     const int last = pos0 + min(q0 + 15, T - 1), nTiles = last / 16 + 1;
@@ -615,8 +641,9 @@ __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, co
 #pragma unroll
         for (int e = 0; e < 4; e++) o[b][e] = 0.f;
     float m = -INFINITY, l = 0.f;
-    float4 kf[2][KF], vf[2][4][VF / 4];
-    auto load = [&](int t, float4 (&k)[KF], float4 (&v)[4][VF / 4]) __attribute__((always_inline)) {
+    float4 kf[2][KF];
+    float vf[2][4][VF];
+    auto load = [&](int t, float4 (&k)[KF], float (&v)[4][VF]) __attribute__((always_inline)) {
         const int t0 = min(t, nTiles - 1) * 16;
         // K: whole rows at a time, HD/4 lanes a row (they change lanes through LDS when they are wanted)
 #pragma unroll
@@ -624,14 +651,13 @@ __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, co
             k[i] = ld_row4<KVH>(Kc, (size_t)min(t0 + i * (256 / HD) + lane / (HD / 4), last) * kvDim + (size_t)kvh * HD + 4 * (lane % (HD / 4)));
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const size_t vr = (size_t)min(t0 + 4 * fq + e, last) * kvDim + (size_t)kvh * HD + VF * fr;
-#pragma unroll
-            for (int i = 0; i < VF / 4; i++) v[e][i] = ld_row4<KVH>(Vc, vr + 4 * i);
+            const size_t vr = (size_t)min(t0 + 4 * fq + e, last) * kvDim + (size_t)kvh * HD + d0 + VF * fr;
+            ld_row<KVH>(Vc, vr, v[e]);
         }
     };
     float* kt = ob + wave * (HD * OST);                    // this wave's K tile: 16 rows of HD + HD/16 floats
     constexpr int KST = HD + HD / 16;
-    auto step = [&](int t, const float4 (&kl)[KF], const float4 (&v)[4][VF / 4]) __attribute__((always_inline)) {
+    auto step = [&](int t, const float4 (&kl)[KF], const float (&v)[4][VF]) __attribute__((always_inline)) {
         float4 k[KF];
 #pragma unroll
         for (int i = 0; i < KF; i++)
@@ -673,12 +699,7 @@ __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, co
 #pragma unroll
         for (int e = 0; e < 4; e++)
 #pragma unroll
-            for (int i = 0; i < VF / 4; i++) {
-                o[4 * i + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].x, sv[e], o[4 * i + 0], 0, 0, 0);
-                o[4 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].y, sv[e], o[4 * i + 1], 0, 0, 0);
-                o[4 * i + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].z, sv[e], o[4 * i + 2], 0, 0, 0);
-                o[4 * i + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i].w, sv[e], o[4 * i + 3], 0, 0, 0);
-            }
+            for (int i = 0; i < VF; i++) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][i], sv[e], o[i], 0, 0, 0);
     };
     load(wave, kf[0], vf[0]);
     for (int t = wave; t < nTiles; t += 2 * FR_WAVES) {
@@ -695,8 +716,8 @@ __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, co
         for (int e = 0; e < 4; e++) ob[(wave * HD + VF * (4 * fq + e) + b) * OST + fr] = o[b][e];
     if (fq == 0) { wm[wave][fr] = m; wl[wave][fr] = l; }
     __syncthreads();
-    for (int i = tid; i < 16 * HD; i += FR_WG) {
-        const int qq = i / HD, d = i % HD;
+    for (int i = tid; i < 16 * (HD / CS); i += FR_WG) {
+        const int qq = i / (HD / CS), d = i % (HD / CS);
         if (q0 + qq >= T) continue;
         float M = wm[0][qq];
 #pragma unroll
@@ -709,27 +730,32 @@ __global__ __launch_bounds__(FR_WG) void few_attention_kernel(const float* q, co
             den = fmaf(g, wl[w][qq], den);
         }
         const float a = num / den;
-        const size_t ix = few_index(q0 + qq, head * HD + d, dim, q4);
+        const size_t ix = few_index(q0 + qq, head * HD + d0 + d, dim, q4);
         if (ext) put_split<true>(hi, lo, ext, ix, a);
         else put_split<false>(hi, lo, ext, ix, a);
     }
 }
 
-template <int HD, bool KVH>
+template <int HD, bool KVH, int CS>
 static hipError_t launch_few_attn_t(unsigned grid, hipStream_t s, const float* q, const void* Kc, const void* Vc, unsigned short* hi,
                                     unsigned short* lo, unsigned short* ext, int T, int pos0, int dim, int kvDim, int nHeads, int nKVHeads, int q4) {
     constexpr int bytes = FR_WAVES * HD * 17 * 4;
     if (bytes > 48 * 1024) {
         static bool raised = false;
         if (!raised) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_attention_kernel<HD, KVH>),
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_attention_kernel<HD, KVH, CS>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
             if (e != hipSuccess) return e;
             raised = true;
         }
     }
-    hipLaunchKernelGGL((few_attention_kernel<HD, KVH>), dim3(grid), dim3(FR_WG), bytes, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    hipLaunchKernelGGL((few_attention_kernel<HD, KVH, CS>), dim3(grid * CS), dim3(FR_WG), bytes, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
     return hipGetLastError();
+}
+
+template <int HD, bool KVH, typename... A>
+static hipError_t launch_few_attn(int cs, A... a) {
+    return cs == 4 ? launch_few_attn_t<HD, KVH, 4>(a...) : (cs == 2 ? launch_few_attn_t<HD, KVH, 2>(a...) : launch_few_attn_t<HD, KVH, 1>(a...));
 }
 
 hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
@@ -738,10 +764,11 @@ hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, 
     if (nKVHeads <= 0 || nHeads % nKVHeads || pos0 < 0 || pos0 + T > rowLimit || dim != nHeads * headDim || kvDim != nKVHeads * headDim ||
         (headDim != 64 && headDim != 128) || !hi || !lo) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)nHeads * (unsigned)((T + 15) / 16);
-    if (headDim == 64) return kvHalf ? launch_few_attn_t<64, true>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
-                                     : launch_few_attn_t<64, false>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
-    return kvHalf ? launch_few_attn_t<128, true>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
-                  : launch_few_attn_t<128, false>(grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    const int cs = grid <= 64 ? 4 : (grid <= 128 ? 2 : 1);             // workgroups a head's 16 queries are shared by: see the kernel
+    if (headDim == 64) return kvHalf ? launch_few_attn<64, true>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
+                                     : launch_few_attn<64, false>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
+    return kvHalf ? launch_few_attn<128, true>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4)
+                  : launch_few_attn<128, false>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4);
 }
 
 }  // namespace mg

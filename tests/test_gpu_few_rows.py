@@ -170,3 +170,27 @@ def test_logits_arrive_whole(hip, vocab):
         rc, nxt, logits, _ = m.hip.Prefill(toks[:n], 0, wantLogits=True)
         assert rc == 0 and H.rel_err(logits, want[n - 1]) < 1e-3 and logits[nxt] == logits.max(), E.last_error()
     m.close()
+
+
+HEADS8 = configs.TOY._replace(name="heads8", nLayers=2, dim=1024, nHeads=8, nKVHeads=2, headDim=128, ffnDim=608, vocab=300)
+
+
+@pytest.mark.parametrize("shape,kv_f16,pos0,rows,shares", [
+    (SMALL, False, 7, 144, 4), (SMALL, False, 0, 145, 2), (SMALL, True, 3, 288, 2), (SMALL, False, 0, 289, 1), (SMALL, True, 30, 16, 4),
+    (HEADS8, False, 5, 128, 4), (HEADS8, True, 0, 129, 2), (HEADS8, False, 0, 256, 2), (HEADS8, False, 2, 257, 1), (HEADS8, True, 200, 1, 4)])
+def test_prompt_attention_by_columns(hip, shape, kv_f16, pos0, rows, shares):
+    """16 queries of a head are shared by four workgroups up to 64 of them, by two up to 128: both sides of each line, against
+    the same positions token by token.  Bar: that of test_few_rows_match_token_by_token (fp16 rows: 1e-3)."""
+    m = H.Model(shape, seed=rows, maxSeq=pos0 + rows + 2, eng=hip, oracle=False, kv_f16=kv_f16)
+    toks = m.prompt(pos0 + rows)
+    ref = np.empty(shape.vocab, np.float32)
+    for pos in range(pos0 + rows):
+        rc, nref = m.hip.DecodeToken(int(toks[pos]), pos, ref if pos == pos0 + rows - 1 else None)
+        assert rc == 0, E.last_error()
+    out = []
+    names = H.launched(lambda: out.append(m.hip.Prefill(toks[pos0:], pos0, wantLogits=True)))
+    rc, nxt, logits, _ = out[0]
+    assert rc == 0, E.last_error()
+    assert any(f"few_attention_kernel<{shape.headDim}, {str(kv_f16).lower()}, {shares}>" in n for n in names), names
+    assert H.rel_err(logits, ref) < (1e-3 if kv_f16 else 1e-4)
+    m.close()
