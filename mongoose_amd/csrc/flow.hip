@@ -72,6 +72,7 @@ struct Waiter {
     int* err;
     bool dead;
     const f4* idle;      // a line nothing writes during the launch (see poll_batch)
+    int pause;           // a constant of the variant: sleeps of 128 clocks between a staged vector's polls (see poll_batch)
     __device__ __forceinline__ void fail() {
         dead = true;
         __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -205,7 +206,7 @@ __device__ __forceinline__ void poll_batch(const f4* const (&ptr)[PB], f4 (&v)[P
             if (!unset4(v[0]) || w.dead) break;
             if (!timing) { timing = true; t0 = wall_clock64(); }
             else if (wall_clock64() - t0 > w.limit) { w.fail(); break; }
-            __builtin_amdgcn_s_sleep(2);
+            for (int z = 0; z < w.pause; z++) __builtin_amdgcn_s_sleep(2);
         }
         return;
     }
@@ -219,8 +220,9 @@ __device__ __forceinline__ void poll_batch(const f4* const (&ptr)[PB], f4 (&v)[P
         // the space is also the spread of the moments at which the workgroups notice the vector, and the phase ends with
         // the last of them.  128 clocks; us a token at the 0.5B shape, 24 layers, by clocks 0 / 128 / 256 / 512: 263.6 / 264.1 /
         // 265.9 / 274; sizes in registers 295.0 / 293.3 / 294.9 / 296.3 (1024: 300.7); the toy shape 51.4 / 51.2 / 51.3 / 51.6;
-        // 1.1B and 0.5B Q4_0 within 0.3 %.
-        if (PAUSE) __builtin_amdgcn_s_sleep(2);
+        // 1.1B and 0.5B Q4_0 within 0.3 %.  512 where sizes in registers meet long vectors, whose re-reading costs more: three
+        // layers of 3840 (Q4_0) 121.4 / 120.3 us by 128 / 512, five of 2560 the same, eight of 1536 121.7 / 120.9.
+        if (PAUSE) for (int z = 0; z < w.pause; z++) __builtin_amdgcn_s_sleep(2);
     }
 }
 
@@ -237,6 +239,26 @@ __device__ __forceinline__ void poll_ml(const float* const (&pm)[PB], const floa
                      : "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(l[0]), "=&v"(l[1]), "=&v"(l[2])
                      : "v"(pm[0]), "v"(pm[1]), "v"(pm[2]), "v"(pl[0]), "v"(pl[1]), "v"(pl[2]) : "memory");
         const unsigned missing = unset1(m[0]) | unset1(l[0]) | (n > 1 ? unset1(m[1]) | unset1(l[1]) : 0u) | (n > 2 ? unset1(m[2]) | unset1(l[2]) : 0u);
+        if (!missing || w.dead) break;
+        if (!timing) { timing = true; t0 = wall_clock64(); }
+        else if (wall_clock64() - t0 > w.limit) { w.fail(); break; }
+    }
+}
+// The same, and the accumulator pieces of the round after (nn > 0 of them), which have mostly landed with this round's: a round
+// after the first costs one round trip, not two.
+__device__ __forceinline__ void poll_ml_next(const float* const (&pm)[PB], const float* const (&pl)[PB], float (&m)[PB], float (&l)[PB],
+                                             const f4* const (&pa)[PB], f4 (&a)[PB], int nn, Waiter& w) {
+    long long t0 = 0;
+    bool timing = false;
+    for (;;) {
+        asm volatile("global_load_dword %0, %9, off sc1\n\tglobal_load_dword %1, %10, off sc1\n\tglobal_load_dword %2, %11, off sc1\n\t"
+                     "global_load_dword %3, %12, off sc1\n\tglobal_load_dword %4, %13, off sc1\n\tglobal_load_dword %5, %14, off sc1\n\t"
+                     "global_load_dwordx4 %6, %15, off sc1\n\tglobal_load_dwordx4 %7, %16, off sc1\n\tglobal_load_dwordx4 %8, %17, off sc1\n\t"
+                     "s_waitcnt vmcnt(0)"
+                     : "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(l[0]), "=&v"(l[1]), "=&v"(l[2]), "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2])
+                     : "v"(pm[0]), "v"(pm[1]), "v"(pm[2]), "v"(pl[0]), "v"(pl[1]), "v"(pl[2]), "v"(pa[0]), "v"(pa[1]), "v"(pa[2]) : "memory");
+        const unsigned missing = unset1(m[0]) | unset1(l[0]) | unset1(m[1]) | unset1(l[1]) | unset1(m[2]) | unset1(l[2]) |
+                                 unset4(a[0]) | (nn > 1 ? unset4(a[1]) : 0u) | (nn > 2 ? unset4(a[2]) : 0u);
         if (!missing || w.dead) break;
         if (!timing) { timing = true; t0 = wall_clock64(); }
         else if (wall_clock64() - t0 > w.limit) { w.fail(); break; }
@@ -599,6 +621,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     __shared__ float4 sqkv[2 + QHMAX][HD / 4];         // K and V row of the current position, q of the workgroup's heads
     __shared__ float4 accbuf[QHMAX][FWAVES][HD / 4];   // per query head of the workgroup: the waves' partial outputs, sums, maxima
     __shared__ __attribute__((aligned(16))) float lbuf[QHMAX][FWAVES], wred[QHMAX][FWAVES];
+    __shared__ float4 mnum[FWG];                       // the groups of threads that share out a vector's KV splits: numerator, maximum, sum
+    __shared__ float mM[FWG], mden[FWG];
     __shared__ float outbuf[FLOW_MAX_ROUNDS][FWAVES];                // a phase's results of the workgroup, stored by one wave as whole 32-byte runs
     __shared__ int4 pfScrap[64];                       // where the prefetching loads land (never read)
     __shared__ float tailV[FWAVES];                    // the tail's argmax: the waves' best values and indices
@@ -656,7 +680,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
         G.offAttn = GH.offAttn; G.offPacc = GH.offPacc;
     }
     // (the idle lines follow the error word's 256 bytes: 16 lines of 128 bytes, two workgroups of an XCD on each)
-    Waiter wt{p.limitTicks, p.err, false, reinterpret_cast<const f4*>(reinterpret_cast<const char*>(p.err) + 256 + ((blockIdx.x >> 3) & 15) * 128)};
+    Waiter wt{p.limitTicks, p.err, false, reinterpret_cast<const f4*>(reinterpret_cast<const char*>(p.err) + 256 + ((blockIdx.x >> 3) & 15) * 128),
+              CBD == 2 && FIX == 0 ? 4 : 1};
 
     // attention geometry (decode attention of kernels.hip with one query head per workgroup): a thread group of 16
     // lanes holds a K/V row, a thread VU rows of its workgroup's tile of FLOW_TILE positions.  (Measured on the 0.5B
@@ -1175,8 +1200,9 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                             }
                             // A single split is the whole softmax: its output leaves divided by its sum, and nobody has to wait
                             // for the maximum and the sum as well (a round trip after the accumulators': 282 -> 274 us a token
-                            // at the 0.5B shape, Q4_0 285 -> 280, 1.1B 364 -> 357).
-                            if (nsplit == 1) { const float il = __builtin_amdgcn_rcpf(lg); r.x *= il; r.y *= il; r.z *= il; r.w *= il; lg = 1.0f; }
+                            // at the 0.5B shape, Q4_0 285 -> 280, 1.1B 364 -> 357).  Not where long vectors meet grouped attention, a
+                            // variant for many splits (eight layers of the 1.1B shape at 1,200 positions 204.2 us without, 206.1 with).
+                            if (!(GQA && CBD == 2) && nsplit == 1) { const float il = __builtin_amdgcn_rcpf(lg); r.x *= il; r.y *= il; r.z *= il; r.w *= il; lg = 1.0f; }
                             stx4(reinterpret_cast<f4*>(X + G.offPacc + (size_t)split * dim + h * HD) + i, r);
                             if (i == 0) {
                                 stx(X + G.offPm + split * nHeadsV + h, mg_);
@@ -1192,8 +1218,6 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                     // one vector -- every consumer merging all partials itself re-reads tens of KB per workgroup and layer.
                     if ((int)blockIdx.x < nHeadsV) {
                         constexpr int P4 = HD / 4, SG = FWG / P4;          // pieces of a head, split groups (thread = piece x group)
-                        __shared__ float4 mnum[SG][P4];
-                        __shared__ float mM[SG][P4], mden[SG][P4];
                         const int h = blockIdx.x, i = tid % P4, sg = tid / P4;
                         const int ns = min(pos / TILE + 1, G.smax);
                         const unsigned Xo = xoff + (unsigned)l * G.stride;
@@ -1233,17 +1257,17 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                 }
                             }
                         }
-                        mnum[sg][i] = tof4(num); mM[sg][i] = M; mden[sg][i] = den;
+                        mnum[tid] = tof4(num); mM[tid] = M; mden[tid] = den;              // (tid = sg * P4 + i)
                         __syncthreads();
                         if (tid < P4) {
-                            float Mg = mM[0][tid];
-                            for (int g2 = 1; g2 < SG; g2++) Mg = fmaxf(Mg, mM[g2][tid]);
+                            float Mg = mM[tid];
+                            for (int g2 = 1; g2 < SG; g2++) Mg = fmaxf(Mg, mM[g2 * P4 + tid]);
                             float dn = 0.f;
                             f4 nm = {0.f, 0.f, 0.f, 0.f};
                             for (int g2 = 0; g2 < SG; g2++) {
-                                const float wgt = exp_neg(mM[g2][tid] - Mg);     // a group without splits has M = -inf: weight 0
-                                const float4 a = mnum[g2][tid];
-                                dn = fmaf(wgt, mden[g2][tid], dn);
+                                const float wgt = exp_neg(mM[g2 * P4 + tid] - Mg);     // a group without splits has M = -inf: weight 0
+                                const float4 a = mnum[g2 * P4 + tid];
+                                dn = fmaf(wgt, mden[g2 * P4 + tid], dn);
                                 nm.x = fmaf(wgt, a.x, nm.x); nm.y = fmaf(wgt, a.y, nm.y); nm.z = fmaf(wgt, a.z, nm.z); nm.w = fmaf(wgt, a.w, nm.w);
                             }
                             const float il = __builtin_amdgcn_rcpf(dn);
@@ -1280,11 +1304,21 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                         {
                             const int nsplit = pos / TILE + 1;
                             const int ns = nsplit < G.smax ? nsplit : G.smax;
-                            if (ns == 1) {                                 // uniform in the launch
+                            if (!(GQA && CBD == 2) && ns == 1) {                         // uniform in the launch
                                 for (int i = tid; i < (dim >> 2); i += FWG) a4[slot4<Q4>(i, nchD)] = tof4(poll4(reinterpret_cast<const f4*>(X + G.offPacc) + i, wt));
-                            } else
-                            for (int i = tid; i < (dim >> 2); i += FWG) {
-                                const int h = (i * 4) / HD;
+                            } else {
+                            // A vector of at most half as many pieces as there are threads: NG groups of threads share out the splits (a
+                            // group for every PB of them) and are combined through LDS, so that a long context costs fewer dependent
+                            // rounds.  With the rounds overlapped (poll_ml_next): us a token at the toy shape (4 groups) at 600 / 1,200 /
+                            // 2,000 positions 57.4 / 67.2 / 75.6 -> 56.4 / 59.1 / 62.6 (overlap alone 57.2 / 64.0 / 70.6), hidden size 256
+                            // at 2,000 102.2 -> 82.8.  The other variants do neither: it costs them registers at every position (sizes
+                            // compiled in, 0.5B shape at 4 positions 267 -> 275 us, 1.1B at 600 428 -> 432; long vectors, three layers of
+                            // 3840 at 20 and 600 positions 121.4 -> 124.1 and 136.4 -> 140.7), and grouped attention has few splits here.
+                            constexpr bool SHARED = !FX && !GQA && CBD == 1;
+                            const int nPieces = dim >> 2;
+                            const int NG = SHARED ? min(max(1, FWG / nPieces), (ns + PB - 1) / PB) : 1;
+                            for (int ii = tid; ii < nPieces * NG; ii += FWG) {
+                                const int g = NG == 1 ? 0 : ii / nPieces, i = ii - g * nPieces, h = (i * 4) / HD;
                                 float M = -INFINITY, den = 0.f;
                                 f4 num = {0.f, 0.f, 0.f, 0.f};
                                 auto mergeIn = [&](f4 a, float ms, float ls) {
@@ -1304,8 +1338,10 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                 // Two round trips after the last partial has landed, however many splits (one by one they
                                 // were one more per split: 4 % of the step at 1000 positions).
                                 const float* idle1 = reinterpret_cast<const float*>(wt.idle);
-                                for (int s0 = 0; s0 < ns; s0 += PB) {
-                                    const int nbt = min(PB, ns - s0);
+                                const int cnt = NG == 1 ? ns : (ns - g + NG - 1) / NG;          // this group's splits: g, g + NG, ...
+                                if constexpr (!SHARED) {
+                                for (int k0 = 0; k0 < cnt; k0 += PB) {
+                                    const int nbt = min(PB, cnt - k0);
                                     const f4* pa[PB];
                                     const float* pm[PB];
                                     const float* pl[PB];
@@ -1314,9 +1350,9 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 #pragma unroll
                                     for (int u = 0; u < PB; u++) {
                                         const bool on = u < nbt;
-                                        pa[u] = on ? reinterpret_cast<const f4*>(X + G.offPacc + (size_t)(s0 + u) * dim) + i : wt.idle;
-                                        pm[u] = on ? X + G.offPm + (s0 + u) * nHeadsV + h : idle1;
-                                        pl[u] = on ? X + G.offPl + (s0 + u) * nHeadsV + h : idle1;
+                                        pa[u] = on ? reinterpret_cast<const f4*>(X + G.offPacc + (size_t)(g + (k0 + u) * NG) * dim) + i : wt.idle;
+                                        pm[u] = on ? X + G.offPm + (g + (k0 + u) * NG) * nHeadsV + h : idle1;
+                                        pl[u] = on ? X + G.offPl + (g + (k0 + u) * NG) * nHeadsV + h : idle1;
                                         a[u] = f4{0.f, 0.f, 0.f, 0.f};
                                     }
                                     poll_batch<false, false>(pa, a, nbt, wt);
@@ -1324,8 +1360,61 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 #pragma unroll
                                     for (int u = 0; u < PB; u++) if (u < nbt) mergeIn(a[u], ms[u], ls[u]);
                                 }
+                                } else {
+                                    auto accAt = [&](int k) __attribute__((always_inline)) {
+                                        return k < cnt ? reinterpret_cast<const f4*>(X + G.offPacc + (size_t)(g + k * NG) * dim) + i : wt.idle;
+                                    };
+                                    f4 a[PB];
+                                    {
+                                        const f4* const pa[PB] = {accAt(0), accAt(1), accAt(2)};
+                                        poll_batch<false, false>(pa, a, min(PB, cnt), wt);
+                                    }
+                                    for (int k0 = 0; k0 < cnt; k0 += PB) {
+                                        const int nbt = min(PB, cnt - k0), nn = cnt - k0 - PB;
+                                        const float* pm[PB];
+                                        const float* pl[PB];
+                                        float ms[PB], ls[PB];
+#pragma unroll
+                                        for (int u = 0; u < PB; u++) {
+                                            const unsigned o = (unsigned)((g + (k0 + u) * NG) * nHeadsV + h);
+                                            pm[u] = u < nbt ? X + G.offPm + o : idle1;
+                                            pl[u] = u < nbt ? X + G.offPl + o : idle1;
+                                        }
+                                        if (nn > 0) {
+                                            const f4* const pa[PB] = {accAt(k0 + PB), accAt(k0 + PB + 1), accAt(k0 + PB + 2)};
+                                            f4 an[PB];
+                                            poll_ml_next(pm, pl, ms, ls, pa, an, nn, wt);
+#pragma unroll
+                                            for (int u = 0; u < PB; u++) { mergeIn(a[u], ms[u], ls[u]); a[u] = an[u]; }
+                                        } else {
+                                            poll_ml(pm, pl, ms, ls, nbt, wt);
+#pragma unroll
+                                            for (int u = 0; u < PB; u++) if (u < nbt) mergeIn(a[u], ms[u], ls[u]);
+                                        }
+                                    }
+                                }
+                                if (NG > 1) { mnum[ii] = tof4(num); mM[ii] = M; mden[ii] = den; break; }
                                 const float il = __builtin_amdgcn_rcpf(den);
                                 a4[slot4<Q4>(i, nchD)] = make_float4(num.x * il, num.y * il, num.z * il, num.w * il);
+                            }
+                            if (NG > 1) {                                  // uniform in the launch
+                                __syncthreads();
+                                if (tid < nPieces) {
+                                    float Mg = mM[tid];
+                                    for (int g = 1; g < NG; g++) Mg = fmaxf(Mg, mM[tid + g * nPieces]);
+                                    float dn = 0.f;
+                                    f4 nm = {0.f, 0.f, 0.f, 0.f};
+                                    for (int g = 0; g < NG; g++) {
+                                        const int o = tid + g * nPieces;
+                                        const float wgt = exp_neg(mM[o] - Mg);
+                                        const float4 a = mnum[o];
+                                        dn = fmaf(wgt, mden[o], dn);
+                                        nm.x = fmaf(wgt, a.x, nm.x); nm.y = fmaf(wgt, a.y, nm.y); nm.z = fmaf(wgt, a.z, nm.z); nm.w = fmaf(wgt, a.w, nm.w);
+                                    }
+                                    const float il = __builtin_amdgcn_rcpf(dn);
+                                    a4[slot4<Q4>(tid, nchD)] = make_float4(nm.x * il, nm.y * il, nm.z * il, nm.w * il);
+                                }
+                            }
                             }
                         }
                         __syncthreads();
@@ -1836,7 +1925,7 @@ bool flow_grid_fits(int ffn, int nHeads, const FlowGeometry& g, int nCompute) {
 
 bool flow_shape_supported(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim) {
     if (headDim != 64 && headDim != 128) return false;
-    // LDS: the staged vector (dynamic, up to 60 KB) beside the kernel's own arrays (4 to 7 KB; 33 to 52 KB in the
+    // LDS: the staged vector (dynamic, up to 60 KB) beside the kernel's own arrays (4 to 20 KB; 33 to 52 KB in the
     // variants with grouped attention, which keep every query head's partials) stays inside the CU's 160 KB
     if (dim % 16 || ffn % 16 || kvDim % 16 || dim > 15360 || ffn > 15360) return false;
     if (nKVHeads <= 0 || nHeads % nKVHeads || nHeads * headDim != dim || nKVHeads * headDim != kvDim) return false;
@@ -1930,7 +2019,7 @@ hipError_t launch_flow_reset_all(float* xchg, const FlowGeometry& g, int nLayers
     return hipGetLastError();
 }
 size_t flow_lds_bytes(int dim, int ffn, int headDim, int gqa, bool tokenMode) {
-    const size_t own = headDim == 64 ? (gqa ? (34u << 10) : (5u << 10)) : (gqa ? (53u << 10) : (8u << 10));
+    const size_t own = headDim == 64 ? (gqa ? (34u << 10) : (17u << 10)) : (gqa ? (53u << 10) : (20u << 10));
     return own + (size_t)((dim > ffn ? dim : ffn) + (tokenMode ? dim : 0)) * sizeof(float);
 }
 
