@@ -67,6 +67,7 @@ constexpr int FLOW_TRACE_SLOTS = 11;
 #define FLOW_TRACE_NAMES "layer-top", "qkv-input-staged", "qkv-done", "q-k-v-rows-in", "attention-done", "attention-merged", \
                          "wo-done", "gate-up-input-staged", "gate-up-done", "down-input-staged", "down-done"
 
+constexpr int FLOW_MANY_SPLITS = 6;      // see launch_flow_layers
 struct FlowParams {
     const FlowLayer* layers;     // indexed by layer
     int l0, l1;                  // layers [l0, l1)
@@ -95,6 +96,7 @@ struct FlowParams {
     int nTokens;                 // 0: layers [l0, l1) of one step, hidden in and out; n >= 1: token mode -- n whole tokens from the
                                  // device state on (all layers; xchg holds two halves and the argmax exchange; state != NULL)
     const FlowTail* tail;        // token mode
+    int manySplits;              // 1: a position of this launch has FLOW_MANY_SPLITS KV splits or more (the variant that shares their merge out)
     int gqaCode;                 // geo.gqa only: 1 = a position of this launch may need the grouped attention (the variant that can do
                                  // it is launched); 0 = none does (positions below nCompute / nHeads tiles): the plain variant, which
                                  // is faster there, runs on the same geometry and reports a position past its reach as error 3

@@ -652,7 +652,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
             }
         }
     };
-    constexpr bool FX = FIX != 0;
+    constexpr bool FX = (FIX & 31) != 0;
+    constexpr bool SHARED = (FIX & 32) != 0;           // launches that reach many KV splits, vectors of at most 1,024 elements: see the merge
     constexpr FlowFixedShape FS = flow_fixed_shape(FIX & 7);
     static_assert(!FX || FS.headDim == HD, "the fixed shape's head size is the variant's");
     int dim = FX ? FS.dim : p.dim, kvDim = FX ? FS.kvDim : p.kvDim, ffn = FX ? FS.ffn : p.ffn;
@@ -1311,12 +1312,13 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                             // group for every PB of them) and are combined through LDS, so that a long context costs fewer dependent
                             // rounds.  With the rounds overlapped (poll_ml_next): us a token at the toy shape (4 groups) at 600 / 1,200 /
                             // 2,000 positions 57.4 / 67.2 / 75.6 -> 56.4 / 59.1 / 62.6 (overlap alone 57.2 / 64.0 / 70.6), hidden size 256
-                            // at 2,000 102.2 -> 82.8.  The other variants do neither: it costs them registers at every position (sizes
-                            // compiled in, 0.5B shape at 4 positions 267 -> 275 us, 1.1B at 600 428 -> 432; long vectors, three layers of
-                            // 3840 at 20 and 600 positions 121.4 -> 124.1 and 136.4 -> 140.7), and grouped attention has few splits here.
-                            constexpr bool SHARED = !FX && !GQA && CBD == 1;
+                            // at 2,000 102.2 -> 82.8.  Only in a variant of its own, for launches that reach FLOW_MANY_SPLITS: the code alone
+                            // costs registers at every position (sizes compiled in, 0.5B shape at 4 positions 267 -> 275 us, 1.1B at 600 428 ->
+                            // 432; long vectors, three layers of 3840 at 20 and 600 positions 121.4 -> 124.1 and 136.4 -> 140.7; short ones, six
+                            // layers of 768, Q4_0, at 200 79.6 -> 83.7), and grouped attention has few splits here.  Fewer splits are merged as in
+                            // the other variants, one after the other, also in such a launch.
                             const int nPieces = dim >> 2;
-                            const int NG = SHARED ? min(max(1, FWG / nPieces), (ns + PB - 1) / PB) : 1;
+                            const int NG = SHARED && ns >= FLOW_MANY_SPLITS ? min(max(1, FWG / nPieces), (ns + PB - 1) / PB) : 1;
                             for (int ii = tid; ii < nPieces * NG; ii += FWG) {
                                 const int g = NG == 1 ? 0 : ii / nPieces, i = ii - g * nPieces, h = (i * 4) / HD;
                                 float M = -INFINITY, den = 0.f;
@@ -1974,6 +1976,13 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         else FLOW_LAUNCH_F(128, 2, true, false, false, 3);
     } else if (fix == 3 && !p.q4 && gqa) {              // fp16 K / V rows at a long context
         FLOW_LAUNCH_F(128, 2, true, true, false, 11);
+    } else if (p.manySplits && !gqa && !wide && !p.trace) {
+        // Six splits: hidden size 768, six layers, Q8, at 600 positions (five) 82.9 us a token with / 83.0 without, Q4_0 87.9 / 86.0,
+        // the toy shape 56.7 / 57.8; at 1,200 (ten) 88.5 / 95.3, 93.2 / 98.0 and 59.0 / 66.8.
+#define FLOW_LAUNCH_S(HDv, Q4v) hipLaunchKernelGGL((flow_layers_kernel<HDv, 1, false, false, Q4v, false, 32>), dim3(grid), dim3(FWG), lds, s, p)
+        if (p.headDim == 64) { if (p.q4) FLOW_LAUNCH_S(64, true); else FLOW_LAUNCH_S(64, false); }
+        else { if (p.q4) FLOW_LAUNCH_S(128, true); else FLOW_LAUNCH_S(128, false); }
+#undef FLOW_LAUNCH_S
     } else if (p.headDim == 64) {
         if (ring) FLOW_LAUNCH_G(64, 2, true);
         else if (wide) FLOW_LAUNCH_G(64, 2, false);

@@ -330,10 +330,11 @@ def test_heads_of_128_grouped_kv(hip):
     ("q8", 4, 4, 64, 383), ("q8", 4, 4, 64, 500), ("q8", 8, 8, 64, 640), ("q8", 7, 7, 64, 1400), ("q4_0", 3, 1, 128, 900),
     ("q8", 16, 16, 64, 896), ("q8", 17, 1, 64, 500), ("q8", 1, 1, 64, 2040), ("q4_0", 5, 5, 64, 770)])
 def test_kv_splits_shared_out_among_threads(hip, fmt, heads, kv, hd, pos):
-    """From four KV splits of 128 positions on, groups of threads merge every n-th split each where the vector is short
+    """From six KV splits of 128 positions on (640), groups of threads merge every n-th split each where the vector is short
     enough (up to 1,024 elements; three splits a group, or as many groups as there are threads for), with the rounds of a
-    group overlapped; longer vectors (17 heads) have one group.  At the last position of three splits and around the
-    first ones of 4, 5, 6, 7, 8, 11 and 16, against the separate launches, whose attention knows no splits of this kind."""
+    group overlapped; longer vectors (17 heads) and fewer splits go one after the other.  At the last position of three
+    splits, across the line inside one run, and at 7 to 16 splits, against the separate launches, whose attention knows no splits of
+    this kind."""
     s = configs.TOY._replace(name="splits", nLayers=2, dim=heads * hd, nHeads=heads, nKVHeads=kv, headDim=hd, ffnDim=608, vocab=300)
     m = H.Model(s, seed=pos, maxSeq=pos + 40, eng=hip, oracle=False, fmt=fmt)
     assert _in_use(m.hip)
