@@ -141,8 +141,12 @@ void mongoose_dequant_q4_0(const void* w_q4_0, float* out, int rows, int cols, v
  * cuda.go:230); here the int8 weights are read directly.  workspace: device
  * memory of at least 4 * roundup(T,128) * roundup(K,64) bytes for the split
  * activations (up to some hundred rows three planes of signed bytes and a scale
- * a row and eighth of K, beyond two bf16 planes).  K a multiple of 32; w and workspace
- * 16-byte aligned. */
+ * a row and eighth of K, beyond two bf16 planes).  An activation is held to 2^-17 of
+ * itself with two bf16 planes.  With signed bytes it is held to 2^-24 of the largest
+ * value of its row's eighth of K, and where more than an eighth of the values lie so far
+ * below that one that this would be the larger error, those are multiplied in two bf16
+ * terms besides (correct at any magnitude, slower the more rows and eighths it takes).
+ * K a multiple of 32; w and workspace 16-byte aligned. */
 void mongoose_q8_gemm(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
                       int K, int accumulate, void* workspace, size_t workspaceBytes, void* stream);
 /* No counterpart in the reference.  mongoose_q8_gemm for callers that cannot allocate and have no

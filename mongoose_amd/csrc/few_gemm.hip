@@ -4,16 +4,24 @@
 // Y[T,N] = A[T,K] . W[N,K]^T: an activation becomes a whole number of 24 bits times a scale, a = s (65536 d2 + 256 d1 + d0)
 // with signed digits of a byte, so that v_mfma_i32_16x16x64_i8 multiplies the int8 weights as they are -- three products at
 // twice the bf16 rate where two bf16 terms need two at the plain one, no conversion of a weight (which was a third of a
-// workgroup's time: no other workgroup's conversions serve it), three bytes an activation instead of four.  The sums of a
-// wave are whole numbers, exact; scale, row scale, bias and the sum of the waves are fp32.  Bound by the operands a workgroup
-// pulls through its CU's L1.  Microseconds a call, weights from memory, two bf16 terms / this: 77 x 5632 x 2048 19.0 / 13.9,
-// 16 x 5632 x 2048 10.2 / 9.2, 37 x 896 x 4864 11.4 / 10.3, 500 x 5632 x 2048 57 / 48, 48 x 9000 x 8192 50 / 39, 500 x 9000 x
-// 8192 241 / 209.
+// workgroup's time: no other workgroup's conversions serve it), three bytes an activation instead of four.  (Operands split
+// into small integers for an integer matrix unit: the Ozaki scheme, as in Ootomo, Ozaki and Yokota, "DGEMM on integer matrix
+// multiplication unit", 2024.)  The sums of a wave are whole numbers, exact; scale, row scale, bias and the sum of the waves are
+// fp32.  Bound by the operands a workgroup pulls through its CU's L1.  Microseconds a call, weights from memory, two bf16 terms
+// / this: 77 x 5632 x 2048 19.5 / 14.3, 16 x 5632 x 2048 10.4 / 9.9, 37 x 896 x 4864 11.4 / 10.6, 300 x 5632 x 2048 35.5 / 31.9,
+// 48 x 9000 x 8192 49.6 / 39.7, 500 x 9000 x 8192 240 / 207.
 //
 // Precision: the eight waves of a workgroup split K into eight runs, and every row has a scale for each run, the run's
-// largest value / 8355584.  A value is off by half a step at most, 2^-24 of the run's largest one, against 2^-18 of itself
-// with two bf16 terms.  Against 64 bits, K 32 to 8192: normal samples 2.5e-6 with two bf16 terms, 0.9e-7 to 1.5e-7 so; rows
-// whose one value outweighs all others (the error then grows with sqrt(K / 8) steps) 2.6e-6 to 3.7e-6 and 1.3e-7 to 1.1e-6.
+// largest value / 8355584.  A value is off by half a step at most, 2^-24 of the run's largest one: no more than two bf16
+// terms leave of it (2^-18 of itself) down to a 64th of that one.  The smaller ones of a run (3 to 5 % of normal samples, 28 %
+// of a SwiGLU's outputs) are weighed against each other in mean square, their share of the run times the digits' error
+// against the error of two bf16 terms of them; where the digits lose -- a few large values among small ones, a part of the run
+// on a scale of its own -- the run is a wide one, and what the digits leave of its small values is multiplied as well, as two
+// bf16 terms: they then keep 2^-17 of themselves however large their neighbours are.  Against 64 bits, K 32 to 8192: normal
+// samples 2.5e-6 with two bf16 terms, 0.9e-7 to 1.5e-7 so; one value 10,000 times the others, seen through weights that are
+// zero there, 2.4e-6 and 1.3e-7 (1.2e-4 without the wide runs); at every ratio from 30 to 1e20 the digits' error is the lower
+// one or equal.  A wide run costs its chunks a second time, with conversions, shared by the eight waves: 77 x 5632 x 2048 14.3 us
+// without any, 15.8 with one run of eight, 26 with all (two bf16 terms 19.5); 300 rows 32, 42 and 100 (35).
 #include "few_rows.h"
 #include "few_rules.h"
 #include "kernels.h"
@@ -24,9 +32,12 @@ namespace mg {
 
 typedef int int4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 constexpr int FG_WAVES = 8, FG_WG = 64 * FG_WAVES;
 constexpr int FG_TOP = 127 * 65536 + 127 * 256;             // three signed digits go to 127 more: a product may round up past it
+constexpr float FG_KEPT = 131072.f;                         // whole numbers from here on are off by 2^-18 of themselves at most
+constexpr float FG_EVEN = 6.58e9f;                          // 2^37.2 / 24: 1 / 12 of a step^2 against twice 2^-37.2 of a value^2
 
 // chunks of 64 k (a last half one counts), and of them a wave's
 __host__ __device__ inline int fg_chunks(int K) { return (K + 63) >> 6; }
@@ -36,7 +47,8 @@ __host__ __device__ inline int fg_per_wave(int K) { return (fg_chunks(K) + FG_WA
 // Digits and scales, a wave per row and run of K (a workgroup four rows): a lane holds pieces of four k.  A 16-row block of a
 // chunk is 3 KB, a KB a digit, in each the operand of a lane (lane = 16 q + row: k 16 q .. + 15 of the chunk) at lane * 16.
 // Rows past T and k past K are zeros.  A run with a NaN or an infinity gets the scale NaN (so did the two bf16 terms of an
-// infinity); one whose values are below 2^-64 is brought up by 2^64 first, which a negative scale says.
+// infinity); one whose values are below 2^-64 is brought up by 2^64 first, which a negative scale says.  wide: 1 for a row's
+// wide run (see above).
 // ---------------------------------------------------------------------------
 constexpr int FG_PIECES = 4;                                // a lane's pieces: runs of up to 1024 k
 __device__ __forceinline__ unsigned max_bits(unsigned m, float4 v) {
@@ -44,7 +56,7 @@ __device__ __forceinline__ unsigned max_bits(unsigned m, float4 v) {
     return max(max(m, max(bits(v.x), bits(v.y))), max(bits(v.z), bits(v.w)));
 }
 
-__global__ __launch_bounds__(WG) void few_digits_kernel(const float* in, signed char* out, float* scales, int T, int K) {
+__global__ __launch_bounds__(WG) void few_digits_kernel(const float* in, signed char* out, float* scales, unsigned char* wide, int T, int K) {
     const int run = blockIdx.y, t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int chunks = fg_chunks(K), per = fg_per_wave(K);
     const int c0 = run * per, pieces = max(0, min(per, chunks - c0)) * 16;      // (a last run may be empty)
@@ -69,27 +81,38 @@ __global__ __launch_bounds__(WG) void few_digits_kernel(const float* in, signed 
     const size_t tb = (size_t)(t >> 4);
     const int r = t & 15;
     if (lane == 0) scales[(tb * FG_WAVES + run) * 16 + r] = tiny ? -s : s;
-    auto put = [&](int p, float4 a) {
-        if (p >= pieces) return;
+    int some = 0, small = 0;                                // of the wave: values that are not zero, small ones among them,
+    float squares = 0.f;                                    // and of the lane: their squares
+    auto put = [&](int p, float4 a) {                       // (called by whole waves; pieces past the run are zeros)
         const float x[4] = {a.x, a.y, a.z, a.w};
         unsigned d[3] = {0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            float y = rintf(x[e] * up * inv);
+            const float z = x[e] * up * inv;
+            float y = rintf(z);
             if (bad) y = 0.f;
+            const bool low = x[e] != 0.f && fabsf(z) < FG_KEPT;
+            some += __popcll(__ballot(x[e] != 0.f));
+            small += __popcll(__ballot(low));
+            squares = fmaf(low ? z : 0.f, z, squares);
             const unsigned n = ((unsigned)(int)y + 0x808080u) ^ 0x808080u;          // bytes = signed digits, carries taken along
             d[0] |= (n & 0xffu) << (8 * e);
             d[1] |= ((n >> 8) & 0xffu) << (8 * e);
             d[2] |= ((n >> 16) & 0xffu) << (8 * e);
         }
+        if (p >= pieces) return;
         const int i = p & 15;
         signed char* o = out + ((tb * chunks + c0 + (p >> 4)) * 3) * 1024 + ((i >> 2) * 16 + r) * 16 + (i & 3) * 4;
 #pragma unroll
         for (int g = 0; g < 3; g++) *reinterpret_cast<unsigned*>(o + g * 1024) = d[g];
     };
 #pragma unroll
-    for (int j = 0; j < FG_PIECES; j++) put(lane + 64 * j, v[j]);
-    for (int p = lane + 64 * FG_PIECES; p < pieces; p += 64) put(p, get(p));
+    for (int j = 0; j < FG_PIECES; j++)
+        if (64 * j < pieces) put(lane + 64 * j, v[j]);
+    for (int p = 64 * FG_PIECES; p < pieces; p += 64) put(p + lane, get(p + lane));
+    squares = wave_sum(squares);
+    const float f = (float)small;
+    if (lane == 0) wide[(tb * FG_WAVES + run) * 16 + r] = !bad && small * 8 > some && (float)some * squares < FG_EVEN * f * f ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -139,6 +162,10 @@ __global__ __launch_bounds__(FG_WG) void few_gemm_kernel(FewGemmParams p) {
     float4_t aS[MT];
 #pragma unroll
     for (int i = 0; i < MT; i++) aS[i] = *reinterpret_cast<const float4_t*>(sP[i]);
+    int wides[MT];                                                    // lane = 8 run + pair of rows: whether one of the two has a wide run
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+        wides[i] = *reinterpret_cast<const unsigned short*>(p.wide + (size_t)min((m0 >> 4) + i, (T - 1) >> 4) * FG_WAVES * 16 + lane * 2);
 
     int4_t acc[MT][NB][3];
 #pragma unroll
@@ -200,19 +227,82 @@ __global__ __launch_bounds__(FG_WG) void few_gemm_kernel(FewGemmParams p) {
     }
 
     // C layout: lane holds column fr, rows 4 fq .. 4 fq + 3 of a block
+    float4_t sum[MT][NB];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            float4_t v;
+        for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float x = fmaf((float)acc[i][b][2][e], 65536.f, fmaf((float)acc[i][b][1][e], 256.f, (float)acc[i][b][0][e]));
-                v[e] = x * (aS[i][e] < 0.f ? aS[i][e] * -1.0f : aS[i][e]);
-                if (aS[i][e] < 0.f) v[e] *= 0x1p-64f;
+                sum[i][b][e] = x * fabsf(aS[i][e]);
+                if (aS[i][e] < 0.f) sum[i][b][e] *= 0x1p-64f;
             }
-            *reinterpret_cast<float4_t*>(&part[(wave * NCOL + b * 16 + fr) * LST + i * 16 + 4 * fq]) = v;
+    // Wide runs: what is left of their small values, as two bf16 terms; all waves share a run's chunks (the same lane of both
+    // operands holds the same 16 k, so they go in as two halves of 8 k of every lane).
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const unsigned long long runs = __ballot(wides[i] != 0);      // a byte a run
+        if (runs == 0) continue;
+        const int tb = min((m0 >> 4) + i, (T - 1) >> 4);
+        const float* aRow = p.act + (size_t)min(tb * 16 + fr, T - 1) * K;
+        float4_t left[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) left[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int run = 0; run < FG_WAVES; run++) {
+            if (((runs >> (8 * run)) & 0xff) == 0) continue;
+            const size_t at = ((size_t)tb * FG_WAVES + run) * 16 + fr;
+            const bool mineWide = p.wide[at] != 0;
+            const float s0 = p.aScales[at], s = fabsf(s0), up = s0 < 0.f ? 0x1p64f : 1.0f, down = s0 < 0.f ? 0x1p-64f : 1.0f;
+            for (int c = run * per + ((wave - run * per) & (FG_WAVES - 1)); c < min(run * per + per, chunks); c += FG_WAVES) {
+                const int k = c * 64 + fq * 16;
+                const bool on = mineWide && k < K;
+                int4_t w[NB], d[3];
+                float4_t a[4];
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    w[b] = *reinterpret_cast<const int4_t*>(c < whole ? wP[b] + (size_t)c * few_chunk_bytes(0)
+                        : p.W + (size_t)min(r0 + b * 16 + ldRow, N - 1) * K + (size_t)whole * 64 + (ldPiece & 1) * 16);
+#pragma unroll
+                for (int e = 0; e < 4; e++) a[e] = *reinterpret_cast<const float4_t*>(aRow + (on ? k + 4 * e : 0));
+#pragma unroll
+                for (int g = 0; g < 3; g++) d[g] = *reinterpret_cast<const int4_t*>(aP[i] + (size_t)c * 3072 + g * 1024);
+                asm volatile("" ::: "memory");
+                bf16x8_t hi[2], lo[2];
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int sh = 24 - 8 * (e & 3);
+                    const int n = (d[2][e >> 2] << sh >> 24) * 65536 + (d[1][e >> 2] << sh >> 24) * 256 + (d[0][e >> 2] << sh >> 24);
+                    const float y = (float)n, r = on && fabsf(y) < FG_KEPT ? fmaf(-s, y, a[e >> 2][e & 3] * up) * down : 0.f;
+                    const __bf16 h = (__bf16)r;
+                    hi[e >> 3][e & 7] = h;
+                    lo[e >> 3][e & 7] = (__bf16)(r - (float)h);
+                }
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    bf16x8_t x[2];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int q = __builtin_amdgcn_ds_bpermute(from, w[b][e]);
+#pragma unroll
+                        for (int y = 0; y < 4; y++) x[e >> 1][(e & 1) * 4 + y] = (__bf16)(float)(q << (24 - 8 * y) >> 24);
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        left[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[h], x[h], left[b], 0, 0, 0);
+                        left[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[h], x[h], left[b], 0, 0, 0);
+                    }
+                }
+            }
         }
+#pragma unroll
+        for (int b = 0; b < NB; b++) sum[i][b] += left[b];
+    }
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+            *reinterpret_cast<float4_t*>(&part[(wave * NCOL + b * 16 + fr) * LST + i * 16 + 4 * fq]) = sum[i][b];
     __syncthreads();
     if (!mine) return;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -253,7 +343,7 @@ static hipError_t launch_fg_loop(FewGemmParams& p, hipStream_t s) {
 
 size_t few_gemm_bytes(int T, int K) {
     const size_t tb = (size_t)((T > 0 ? T : 0) + 15) / 16;
-    return tb * fg_chunks(K) * 3072 + tb * FG_WAVES * 16 * sizeof(float);
+    return tb * fg_chunks(K) * 3072 + tb * FG_WAVES * 16 * (sizeof(float) + 1);
 }
 
 hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, hipStream_t s) {
@@ -262,8 +352,9 @@ hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, hipStre
     const unsigned tb = (unsigned)((p.T + 15) / 16);
     signed char* digits = static_cast<signed char*>(ws);
     float* scales = reinterpret_cast<float*>(digits + (size_t)tb * fg_chunks(p.K) * 3072);
-    hipLaunchKernelGGL(few_digits_kernel, dim3(tb * 4, FG_WAVES), dim3(WG), 0, s, act, digits, scales, p.T, p.K);
-    p.A = digits; p.aScales = scales;
+    unsigned char* wide = reinterpret_cast<unsigned char*>(scales + (size_t)tb * FG_WAVES * 16);
+    hipLaunchKernelGGL(few_digits_kernel, dim3(tb * 4, FG_WAVES), dim3(WG), 0, s, act, digits, scales, wide, p.T, p.K);
+    p.act = act; p.A = digits; p.aScales = scales; p.wide = wide;
     // The tile (few_rows.hip's model without conversions): a workgroup's bytes at 80 a nanosecond and the sums it exchanges,
     // times the workgroups of the busiest CU, a quarter of which overlap evenly over the chip.  Against every tile in turn, 8
     // to 500 rows, twelve shapes: the best or within 6 % of it (77 x 5632 x 2048: 13.9 us, the best 13.1, the others 16 to 24).

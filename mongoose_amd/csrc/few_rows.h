@@ -55,7 +55,7 @@ struct FewGemmParams {
     const signed char* W; const float* scales; const float* bias; float* Y;
     int T, N, K, accumulate;
     // filled by the launcher
-    const signed char* A; const float* aScales;
+    const float* act; const signed char* A; const float* aScales; const unsigned char* wide;
     int nTiles;
 };
 size_t few_gemm_bytes(int T, int K);

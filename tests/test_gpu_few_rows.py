@@ -137,6 +137,49 @@ def test_few_row_gemm_digits(hip, rows, n, k):
         t.Release()
 
 
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (17, 33, 96), (33, 40, 544), (16, 130, 1056), (64, 1000, 1024), (65, 600, 2048), (77, 5632, 2048),
+                                      (40, 64, 8224)])
+@pytest.mark.parametrize("spread", [100.0, 1e3, 1e5, 1e7, 1e20, "lognormal", "half"])
+def test_few_row_gemm_keeps_small_values(hip, rows, n, k, spread):
+    """Values far below the largest of their row, seen through weights that are zero at the large ones: each is held to 2^-17 of
+    itself at worst (two bf16 terms), so a result is off by 2^-18 of sqrt(sum of squared products) at random, six times that for
+    the worst of a call, plus fp32 sums: 2^-24 of a partial sum for each of a wave's k / 16 steps and the eight waves.
+    "lognormal": magnitudes over eight decades, weights where |a| is below the median; "half": one half a thousandth of the other."""
+    rng = np.random.default_rng(k + rows)
+    a = rng.standard_normal((rows, k), dtype=np.float32)
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    if spread == "lognormal":
+        a *= np.exp(4 * rng.standard_normal(k)).astype(np.float32)
+        w[:, np.abs(a).mean(axis=0) > np.median(np.abs(a))] = 0
+    elif spread == "half":
+        small = rng.permutation(k)[:k // 2]
+        a[:, small] *= np.float32(1e-3)
+        w[:, np.setdiff1d(np.arange(k), small)] = 0
+    else:
+        at = rng.integers(k)
+        a[:, at] = np.float32(spread) * np.where(rng.random(rows) < 0.5, -1, 1)
+        w[:, at] = 0
+        if rows > 2:
+            a[1] *= np.float32(1e-25)                        # a row of tiny values, and one whose large value is alone
+            a[2, np.arange(k) != at] = 0
+    sc = (0.01 * (1 + rng.random(n))).astype(np.float32)
+    wd = w.astype(np.float64) * sc[:, None].astype(np.float64)
+    ref = a.astype(np.float64) @ wd.T
+    size = np.sqrt((a.astype(np.float64) ** 2) @ (wd ** 2).T)
+    ta, tw, ts, to = hip.FromHost(a, a.shape), hip.UploadRawBytes(w), hip.FromHost(sc, sc.shape), hip.Zeros([rows, n])
+    nbytes = 4 * ((rows + 127) // 128 * 128) * ((k + 63) // 64 * 64)
+    ws = hip.UploadRawBytes(np.full(nbytes, 0xff, np.uint8))
+    E.KQ8Gemm(ta, tw, ts, None, to, rows, n, k, 0, ws, nbytes)
+    E.KSync()
+    assert E.HIPCheck() == 0
+    got = hip.ToHost(to).reshape(rows, n)
+    bar = 6 * 2.0 ** -18 * size + 2.0 ** -24 * np.sqrt(k / 16 + 16) * size
+    worst = (np.abs(got - ref) / (bar + 1e-300)).max()
+    assert worst <= 1, worst
+    for t in (ta, tw, ts, to, ws):
+        t.Release()
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 4), (2, 2048), (3, 2052), (1, 4100), (2, 8192), (1, 8196), (2, 30)])
 def test_rmsnorm_rows_kept_in_registers_and_others(hip, rows, dim):
     rng = np.random.default_rng(dim)
