@@ -234,7 +234,7 @@ static hipError_t q8_gemm_launches(const float* act, const void* w, const float*
                                    int K, int accumulate, void* ws, size_t plane, hipStream_t s) {
     void* hi = ws;
     void* lo = static_cast<char*>(ws) + plane;
-    if (T > 0 && N > 0 && (T <= 512 || (long long)T * N <= 1500000) && aligned16(act)) {
+    if (T > 0 && N > 0 && (T <= 512 || (long long)T * N <= 1500000) && aligned16(act) && mg::few_gemm_sums_fit(K)) {
         mg::FewGemmParams f{};
         f.W = static_cast<const signed char*>(w); f.scales = scales; f.bias = bias; f.Y = out;
         f.T = T; f.N = N; f.K = K; f.accumulate = accumulate;

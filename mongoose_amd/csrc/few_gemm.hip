@@ -348,7 +348,7 @@ size_t few_gemm_bytes(int T, int K) {
 
 hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, hipStream_t s) {
     if (p.T <= 0 || p.N <= 0) return hipSuccess;
-    if (p.K <= 0 || p.K % 32 || ((uintptr_t)act & 15) || ((uintptr_t)p.W & 15) || ((uintptr_t)ws & 15)) return hipErrorInvalidValue;
+    if (p.K <= 0 || p.K % 32 || !few_gemm_sums_fit(p.K) || ((uintptr_t)act & 15) || ((uintptr_t)p.W & 15) || ((uintptr_t)ws & 15)) return hipErrorInvalidValue;
     const unsigned tb = (unsigned)((p.T + 15) / 16);
     signed char* digits = static_cast<signed char*>(ws);
     float* scales = reinterpret_cast<float*>(digits + (size_t)tb * fg_chunks(p.K) * 3072);

@@ -1,4 +1,4 @@
-// few_rules.h -- where the few-row kernels (few_rows.hip) read a weight matrix and which prefills take them, in plain C++:
+// few_rules.h -- where the few-row kernels (few_rows.hip, few_gemm.hip) read a weight matrix and which calls take them, in plain C++:
 // the kernels and the dispatch use these functions, and so do the host tests that walk them over whole matrices and over
 // what was measured.
 #pragma once
@@ -23,6 +23,11 @@ constexpr int few_last_chunk(int K) { return K < 64 ? 0 : (K >> 6) - 1; }
 // which the last row does not have.  few_own_scale: where the row's first scale then lies.
 constexpr int few_own_scale(int K) { return K < 64 ? 1 : 0; }
 constexpr long long few_scales_at(int row, int K) { return (long long)row * (K >> 5) - few_own_scale(K); }
+
+// ---- which products take the integer form (few_gemm.hip) ----
+// Eight waves sum a run of K each, whole chunks of 64, of products of two signed bytes in 32 bits.  Past this K a run of them
+// could exceed those (K = 1,048,064 is the last that cannot); the tiled kernel's fp32 sums take any.
+constexpr bool few_gemm_sums_fit(int K) { return (long long)(((K >> 6) + ((K & 63) ? 1 : 0) + 7) / 8) * 64 * (128 * 128) < (1LL << 31); }
 
 // ---- which prefills take the few-row kernels, and which the tiled GEMMs (prefill.hip) ----
 // Rows up to which some prefill takes them.  The tiled GEMMs want work for every CU, so the line falls with the weights of a

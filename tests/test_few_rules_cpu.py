@@ -47,6 +47,22 @@ int main() {
     assert out == "ok\n", out
 
 
+def test_integer_sums_fit_32_bits(tmp_path):
+    """A wave's run of the few-row GEMM: whole chunks of 64 k, an eighth of them, of products up to (-128) (-128)."""
+    out = _run(tmp_path, r"""
+#include "few_rules.h"
+#include <cstdio>
+int main() {
+    for (int K = 32; K > 0 && K < 2147483647 - 64; K += K < 1500000 ? 32 : 1048576) {
+        const long long chunks = ((long long)K + 63) / 64, run = (chunks + 7) / 8 * 64;
+        if (mg::few_gemm_sums_fit(K) != (run * 16384 <= 2147483647ll)) { std::printf("K %d\n", K); return 0; }
+    }
+    std::printf("%d %d\n", mg::few_gemm_sums_fit(1048064), mg::few_gemm_sums_fit(1048096));
+}
+""")
+    assert out == "1 0\n", out
+
+
 QWEN, TINY, LLAMA, TOY = (896, 128, 4864, 14), (2048, 256, 5632, 32), (4096, 1024, 14336, 32), (512, 128, 1376, 8)
 
 

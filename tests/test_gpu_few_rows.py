@@ -180,6 +180,32 @@ def test_few_row_gemm_keeps_small_values(hip, rows, n, k, spread):
         t.Release()
 
 
+@pytest.mark.parametrize("k,kernel", [(1048064, "few_gemm_kernel"), (1049088, "gemm_q8")])
+def test_gemm_at_the_longest_rows(hip, k, kernel):
+    """One step below and one above the K up to which 32-bit sums hold: every middle digit is -128 and so is every weight (the
+    values are 4161536 = 64 * 65536 - 128 * 256 steps of the row's scale, but for one a run at the top), which takes a run's
+    sum to the limit.  Bar: fp32 sums of equal terms, every one of k / 16 steps rounded the same way by up to 2^-24 of a sum
+    that is half the last one on average; a sum past 32 bits is off by twice the result."""
+    a = np.full((1, k), np.float32(4161536 / 8355584), np.float32)
+    a[0, ::((k // 64 + 7) // 8 * 64)] = 1.0
+    w = np.full((3, k), -128, np.int8)
+    w[1, :k // 2] = 127
+    sc = np.array([0.01, 0.02, 0.03], np.float32)
+    ref = a.astype(np.float64) @ (w.astype(np.float64) * sc[:, None].astype(np.float64)).T
+    ta, tw, ts, to = hip.FromHost(a, a.shape), hip.UploadRawBytes(w), hip.FromHost(sc, sc.shape), hip.Zeros([1, 3])
+    nbytes = 4 * 128 * ((k + 63) // 64 * 64)
+    ws = hip.Zeros([nbytes // 4])
+    names = H.launched(lambda: E.KQ8Gemm(ta, tw, ts, None, to, 1, 3, k, 0, ws, nbytes))
+    E.KSync()
+    assert E.HIPCheck() == 0
+    assert any(kernel in n for n in names) and ("few_gemm" in kernel) == any("few_gemm" in n for n in names), names
+    got = hip.ToHost(to).reshape(1, 3)
+    size = np.abs(a.astype(np.float64)) @ (np.abs(w.astype(np.float64)) * sc[:, None]).T
+    assert (np.abs(got - ref) <= k / 16 * 2.0 ** -25 * size).all(), (got, ref)
+    for t in (ta, tw, ts, to, ws):
+        t.Release()
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 4), (2, 2048), (3, 2052), (1, 4100), (2, 8192), (1, 8196), (2, 30)])
 def test_rmsnorm_rows_kept_in_registers_and_others(hip, rows, dim):
     rng = np.random.default_rng(dim)
