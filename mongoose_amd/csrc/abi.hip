@@ -5,6 +5,7 @@
 #include "kernels.h"
 #include "prefill.h"
 #include "few_rows.h"
+#include "few_rules.h"
 #include "fused_infer.h"
 
 #include <atomic>
@@ -238,7 +239,7 @@ static hipError_t q8_gemm_launches(const float* act, const void* w, const float*
         mg::FewGemmParams f{};
         f.W = static_cast<const signed char*>(w); f.scales = scales; f.bias = bias; f.Y = out;
         f.T = T; f.N = N; f.K = K; f.accumulate = accumulate;
-        return mg::launch_few_gemm(act, f, ws, s);
+        return mg::launch_few_gemm(act, f, ws, 2 * plane, s);
     }
     hipError_t e = mg::launch_split_rows(act, nullptr, 0.f, T, K, hi, lo, s);
     if (e != hipSuccess || T == 0 || N == 0) return e;

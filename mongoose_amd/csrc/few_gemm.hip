@@ -341,14 +341,9 @@ static hipError_t launch_fg_loop(FewGemmParams& p, hipStream_t s) {
     return fg_per_wave(p.K) <= 2 ? launch_fg<MT, NB, 0>(p, s) : launch_fg<MT, NB, 1>(p, s);
 }
 
-size_t few_gemm_bytes(int T, int K) {
-    const size_t tb = (size_t)((T > 0 ? T : 0) + 15) / 16;
-    return tb * fg_chunks(K) * 3072 + tb * FG_WAVES * 16 * (sizeof(float) + 1);
-}
-
-hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, hipStream_t s) {
+hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, size_t wsBytes, hipStream_t s) {
     if (p.T <= 0 || p.N <= 0) return hipSuccess;
-    if (p.K <= 0 || p.K % 32 || !few_gemm_sums_fit(p.K) || ((uintptr_t)act & 15) || ((uintptr_t)p.W & 15) || ((uintptr_t)ws & 15)) return hipErrorInvalidValue;
+    if (p.K <= 0 || p.K % 32 || !few_gemm_sums_fit(p.K) || few_gemm_bytes(p.T, p.K) > wsBytes || ((uintptr_t)act & 15) || ((uintptr_t)p.W & 15) || ((uintptr_t)ws & 15)) return hipErrorInvalidValue;
     const unsigned tb = (unsigned)((p.T + 15) / 16);
     signed char* digits = static_cast<signed char*>(ws);
     float* scales = reinterpret_cast<float*>(digits + (size_t)tb * fg_chunks(p.K) * 3072);

@@ -50,7 +50,7 @@ hipError_t launch_embed_split(int kind, const void* table, const float* scales, 
                               unsigned short* hi, unsigned short* lo, unsigned short* ext, float* sumSq, int T, int dim, int vocab, int q4,
                               hipStream_t s);
 // Several rows through one Q8 matrix on the integer matrix instruction (few_gemm.hip): Y[T,N] (+)= act[T,K] . W[N,K]^T *
-// scales[n] (+ bias[n]).  act, W and ws 16-byte aligned, K a multiple of 32; ws: few_gemm_bytes(T, K).
+// scales[n] (+ bias[n]).  act, W and ws 16-byte aligned, K a multiple of 32; ws: few_gemm_bytes(T, K) (few_rules.h).
 struct FewGemmParams {
     const signed char* W; const float* scales; const float* bias; float* Y;
     int T, N, K, accumulate;
@@ -58,8 +58,7 @@ struct FewGemmParams {
     const float* act; const signed char* A; const float* aScales; const unsigned char* wide;
     int nTiles;
 };
-size_t few_gemm_bytes(int T, int K);
-hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, hipStream_t s);
+hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, size_t wsBytes, hipStream_t s);
 
 // Causal attention of T query rows (rotated) at positions pos0 .. over the cache rows [0, pos0 + T), all products and sums
 // in fp32; the result goes out as the split the output projection reads.

@@ -29,6 +29,12 @@ constexpr long long few_scales_at(int row, int K) { return (long long)row * (K >
 // could exceed those (K = 1,048,064 is the last that cannot); the tiled kernel's fp32 sums take any.
 constexpr bool few_gemm_sums_fit(int K) { return (long long)(((K >> 6) + ((K & 63) ? 1 : 0) + 7) / 8) * 64 * (128 * 128) < (1LL << 31); }
 
+// What it keeps of T rows, 16 at a time: three digit planes, and for each of the eight runs a scale and a mark a row.
+constexpr size_t few_gemm_bytes(int T, int K) {
+    const size_t blocks = ((size_t)(T > 0 ? T : 0) + 15) / 16, chunks = ((size_t)K + 63) / 64;
+    return blocks * (chunks * 3 * 1024 + 8 * 16 * (sizeof(float) + 1));
+}
+
 // ---- which prefills take the few-row kernels, and which the tiled GEMMs (prefill.hip) ----
 // Rows up to which some prefill takes them.  The tiled GEMMs want work for every CU, so the line falls with the weights of a
 // layer.  Microseconds a layer, few-row / tiled, Q8 and Q4_0, nothing cached: 0.5B shape (15 million weights) 36 / 69 and

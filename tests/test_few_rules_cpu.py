@@ -63,6 +63,22 @@ int main() {
     assert out == "1 0\n", out
 
 
+def test_digits_fit_the_callers_planes(tmp_path):
+    """What the few-row GEMM keeps of the activations against the workspace that mongoose_q8_gemm asks a caller for (two bf16
+    planes of T rounded up to 128 rows and K to 64), over rows and K, K = 64 and whole blocks of 128 rows the tightest."""
+    out = _run(tmp_path, r"""
+#include "few_rules.h"
+#include <cstdio>
+int main() {
+    for (int T = 0; T <= 1100; T++)
+        for (int K = 32; K < 1048096; K += K < 2048 ? 32 : 8160)
+            if (mg::few_gemm_bytes(T, K) > 2 * (size_t)((T + 127) / 128 * 128) * ((K + 63) / 64 * 64) * 2) { std::printf("T %d K %d\n", T, K); return 0; }
+    std::printf("%zu\n", mg::few_gemm_bytes(128, 64));
+}
+""")
+    assert out == "%d\n" % (8 * (3072 + 640)), out
+
+
 QWEN, TINY, LLAMA, TOY = (896, 128, 4864, 14), (2048, 256, 5632, 32), (4096, 1024, 14336, 32), (512, 128, 1376, 8)
 
 
