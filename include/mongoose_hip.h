@@ -143,9 +143,9 @@ void mongoose_dequant_q4_0(const void* w_q4_0, float* out, int rows, int cols, v
  * activations (up to some hundred rows three planes of signed bytes and a scale
  * a row and eighth of K, beyond two bf16 planes).  An activation is held to 2^-17 of
  * itself with two bf16 planes.  With signed bytes it is held to 2^-24 of the largest
- * value of its row's eighth of K, and where more than an eighth of the values lie so far
- * below that one that this would be the larger error, those are multiplied in two bf16
- * terms besides (correct at any magnitude, slower the more rows and eighths it takes).
+ * value of its row's eighth of K; where more than an eighth of the values lie so far
+ * below that one that this would be the larger error, those are multiplied as two bf16
+ * terms (2^-17 of themselves at any magnitude; slower the more rows and eighths it takes).
  * K a multiple of 32; w and workspace 16-byte aligned. */
 void mongoose_q8_gemm(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
                       int K, int accumulate, void* workspace, size_t workspaceBytes, void* stream);

@@ -12,16 +12,19 @@
 // 48 x 9000 x 8192 49.6 / 39.7, 500 x 9000 x 8192 240 / 207.
 //
 // Precision: the eight waves of a workgroup split K into eight runs, and every row has a scale for each run, the run's
-// largest value / 8355584.  A value is off by half a step at most, 2^-24 of the run's largest one: no more than two bf16
-// terms leave of it (2^-18 of itself) down to a 64th of that one.  The smaller ones of a run (3 to 5 % of normal samples, 28 %
-// of a SwiGLU's outputs) are weighed against each other in mean square, their share of the run times the digits' error
-// against the error of two bf16 terms of them; where the digits lose -- a few large values among small ones, a part of the run
-// on a scale of its own -- the run is a wide one, and what the digits leave of its small values is multiplied as well, as two
-// bf16 terms: they then keep 2^-17 of themselves however large their neighbours are.  Against 64 bits, K 32 to 8192: normal
-// samples 2.5e-6 with two bf16 terms, 0.9e-7 to 1.5e-7 so; one value 10,000 times the others, seen through weights that are
-// zero there, 2.4e-6 and 1.3e-7 (1.2e-4 without the wide runs); at every ratio from 30 to 1e20 the digits' error is the lower
-// one or equal.  A wide run costs its chunks a second time, with conversions, shared by the eight waves: 77 x 5632 x 2048 14.3 us
-// without any, 15.8 with one run of eight, 26 with all (two bf16 terms 19.5); 300 rows 32, 42 and 100 (35).
+// largest value / 8355584.  A value is off by half a step, 2^-24 of the run's largest one (by up to 1.4 steps next to that one,
+// where the roundings of factor, product and scale weigh as much): no more than two bf16 terms leave of it (up to 2^-17 of
+// itself) down to a 64th of the largest.  The smaller ones of a run (3 to 5 % of normal samples, 28 % of a SwiGLU's outputs) are
+// weighed against each other in mean square, their share of the run times the digits' error against the error of two bf16 terms
+// of them; where the digits lose -- a few large values among small ones, a part of the run on a scale of its own -- the run is a
+// wide one, its small values go in as two bf16 terms instead, and so keep 2^-17 of themselves however large their neighbours
+// are.  Against 64 bits, two bf16 terms / digits alone / as it is: normal samples, K 64 to 8192 2.5e-6 / 1.5e-7 / 1.5e-7; one
+// value R times the others, seen through weights that are zero there, K = 2048 (eight runs, one of them wide) R = 30 2.5e-6 /
+// 3.9e-7 / 3.9e-7, 100 2.5e-6 / 1.2e-6 / 7.7e-7, 1,000 2.5e-6 / 1.2e-5 / 8.8e-7, 10^5 2.5e-6 / 1.2e-3 / 8.7e-7, 10^20 2.5e-6 /
+// 0.35 / 8.7e-7; K = 64 (one run) 100 2.4e-6 / 3.4e-6 / 2.1e-6, from 1,000 on two bf16 terms' own.
+// A wide run costs its chunks a second time, with conversions, shared by the eight waves.  Microseconds a call with no wide
+// run, one of eight, about half of them, all (two bf16 terms): 77 x 5632 x 2048 14.3, 15.8, 19.2, 23.2 (19.7), 48 x 9000 x 8192
+// 40, 45, 54, 74 (50), 300 x 5632 x 2048 32, 38, 55, 86 (36), 500 x 9000 x 8192 209, 257, 386, 555 (241).
 #include "few_rows.h"
 #include "few_rules.h"
 #include "kernels.h"
@@ -32,11 +35,13 @@ namespace mg {
 
 typedef int int4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 constexpr int FG_WAVES = 8, FG_WG = 64 * FG_WAVES;
 constexpr int FG_TOP = 127 * 65536 + 127 * 256;             // three signed digits go to 127 more: a product may round up past it
-constexpr float FG_KEPT = 131072.f;                         // whole numbers from here on are off by 2^-18 of themselves at most
+constexpr float FG_KEPT = 131072.f;                         // whole numbers from here on keep 2^-17 of themselves, as two bf16 terms do
 constexpr float FG_EVEN = 6.58e9f;                          // 2^37.2 / 24: 1 / 12 of a step^2 against twice 2^-37.2 of a value^2
 
 // chunks of 64 k (a last half one counts), and of them a wave's
@@ -48,7 +53,7 @@ __host__ __device__ inline int fg_per_wave(int K) { return (fg_chunks(K) + FG_WA
 // chunk is 3 KB, a KB a digit, in each the operand of a lane (lane = 16 q + row: k 16 q .. + 15 of the chunk) at lane * 16.
 // Rows past T and k past K are zeros.  A run with a NaN or an infinity gets the scale NaN (so did the two bf16 terms of an
 // infinity); one whose values are below 2^-64 is brought up by 2^64 first, which a negative scale says.  wide: 1 for a row's
-// wide run (see above).
+// wide run (see above), whose small values are zeros here.
 // ---------------------------------------------------------------------------
 constexpr int FG_PIECES = 4;                                // a lane's pieces: runs of up to 1024 k
 __device__ __forceinline__ unsigned max_bits(unsigned m, float4 v) {
@@ -81,38 +86,51 @@ __global__ __launch_bounds__(WG) void few_digits_kernel(const float* in, signed 
     const size_t tb = (size_t)(t >> 4);
     const int r = t & 15;
     if (lane == 0) scales[(tb * FG_WAVES + run) * 16 + r] = tiny ? -s : s;
-    int some = 0, small = 0;                                // of the wave: values that are not zero, small ones among them,
-    float squares = 0.f;                                    // and of the lane: their squares
-    auto put = [&](int p, float4 a) {                       // (called by whole waves; pieces past the run are zeros)
+    // values below this are small; of the wave: values that are not zero, small ones among them, and of the lane their squares
+    const float lim = tiny ? s * FG_KEPT * 0x1p-64f : s * FG_KEPT;
+    int some = 0, small = 0;
+    float squares = 0.f;
+    auto weigh = [&](float4 a) {                            // (called by whole waves; pieces past the run are zeros)
+        const float x[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const bool low = x[e] != 0.f && fabsf(x[e]) < lim;
+            some += __popcll(__ballot(x[e] != 0.f));
+            small += __popcll(__ballot(low));
+            const float z = low ? x[e] * up * inv : 0.f;
+            squares = fmaf(z, z, squares);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < FG_PIECES; j++)
+        if (64 * j < pieces) weigh(v[j]);
+    for (int p = 64 * FG_PIECES; p < pieces; p += 64) weigh(get(p + lane));
+    squares = wave_sum(squares);
+    const float f = (float)small;
+    const bool isWide = !bad && small * 8 > some && (float)some * squares < FG_EVEN * f * f;
+    if (lane == 0) wide[(tb * FG_WAVES + run) * 16 + r] = isWide ? 1 : 0;
+    const float least = isWide ? lim : 0.f;
+    auto put = [&](int p, float4 a) {
+        if (p >= pieces) return;
         const float x[4] = {a.x, a.y, a.z, a.w};
         unsigned d[3] = {0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const float z = x[e] * up * inv;
-            float y = rintf(z);
-            if (bad) y = 0.f;
-            const bool low = x[e] != 0.f && fabsf(z) < FG_KEPT;
-            some += __popcll(__ballot(x[e] != 0.f));
-            small += __popcll(__ballot(low));
-            squares = fmaf(low ? z : 0.f, z, squares);
+            float y = rintf(x[e] * up * inv);
+            if (bad || fabsf(x[e]) < least) y = 0.f;
             const unsigned n = ((unsigned)(int)y + 0x808080u) ^ 0x808080u;          // bytes = signed digits, carries taken along
             d[0] |= (n & 0xffu) << (8 * e);
             d[1] |= ((n >> 8) & 0xffu) << (8 * e);
             d[2] |= ((n >> 16) & 0xffu) << (8 * e);
         }
-        if (p >= pieces) return;
         const int i = p & 15;
         signed char* o = out + ((tb * chunks + c0 + (p >> 4)) * 3) * 1024 + ((i >> 2) * 16 + r) * 16 + (i & 3) * 4;
 #pragma unroll
         for (int g = 0; g < 3; g++) *reinterpret_cast<unsigned*>(o + g * 1024) = d[g];
     };
 #pragma unroll
-    for (int j = 0; j < FG_PIECES; j++)
-        if (64 * j < pieces) put(lane + 64 * j, v[j]);
-    for (int p = 64 * FG_PIECES; p < pieces; p += 64) put(p + lane, get(p + lane));
-    squares = wave_sum(squares);
-    const float f = (float)small;
-    if (lane == 0) wide[(tb * FG_WAVES + run) * 16 + r] = !bad && small * 8 > some && (float)some * squares < FG_EVEN * f * f ? 1 : 0;
+    for (int j = 0; j < FG_PIECES; j++) put(lane + 64 * j, v[j]);
+    for (int p = lane + 64 * FG_PIECES; p < pieces; p += 64) put(p, get(p));
 }
 
 // ---------------------------------------------------------------------------
@@ -238,65 +256,90 @@ __global__ __launch_bounds__(FG_WG) void few_gemm_kernel(FewGemmParams p) {
                 sum[i][b][e] = x * fabsf(aS[i][e]);
                 if (aS[i][e] < 0.f) sum[i][b][e] *= 0x1p-64f;
             }
-    // Wide runs: what is left of their small values, as two bf16 terms; all waves share a run's chunks (the same lane of both
-    // operands holds the same 16 k, so they go in as two halves of 8 k of every lane).
+    // Wide runs: their small values, as two bf16 terms; all waves share a run's chunks, a chunk's weights are converted once for
+    // all rows of the tile (the same lane of both operands holds the same 16 k, so they go in as two halves of 8 k of every lane).
+    unsigned long long runs[MT], any = 0;                             // a byte a run
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-        const unsigned long long runs = __ballot(wides[i] != 0);      // a byte a run
-        if (runs == 0) continue;
-        const int tb = min((m0 >> 4) + i, (T - 1) >> 4);
-        const float* aRow = p.act + (size_t)min(tb * 16 + fr, T - 1) * K;
-        float4_t left[NB];
+    for (int i = 0; i < MT; i++) { runs[i] = __ballot(wides[i] != 0); any |= runs[i]; }
+    if (any) {
+        float4_t left[MT][NB];
+        const float* aRow[MT];
 #pragma unroll
-        for (int b = 0; b < NB; b++) left[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < MT; i++) {
+            aRow[i] = p.act + (size_t)min(min((m0 >> 4) + i, (T - 1) >> 4) * 16 + fr, T - 1) * K;
+#pragma unroll
+            for (int b = 0; b < NB; b++) left[i][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+        }
         for (int run = 0; run < FG_WAVES; run++) {
-            if (((runs >> (8 * run)) & 0xff) == 0) continue;
-            const size_t at = ((size_t)tb * FG_WAVES + run) * 16 + fr;
-            const bool mineWide = p.wide[at] != 0;
-            const float s0 = p.aScales[at], s = fabsf(s0), up = s0 < 0.f ? 0x1p64f : 1.0f, down = s0 < 0.f ? 0x1p-64f : 1.0f;
+            if (((any >> (8 * run)) & 0xff) == 0) continue;
+            float lim[MT];                                            // of a row whose run is not wide no value is small
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                const size_t at = ((size_t)min((m0 >> 4) + i, (T - 1) >> 4) * FG_WAVES + run) * 16 + fr;
+                const float s = p.aScales[at];
+                lim[i] = !p.wide[at] ? 0.f : s < 0.f ? s * -FG_KEPT * 0x1p-64f : s * FG_KEPT;
+            }
             for (int c = run * per + ((wave - run * per) & (FG_WAVES - 1)); c < min(run * per + per, chunks); c += FG_WAVES) {
-                const int k = c * 64 + fq * 16;
-                const bool on = mineWide && k < K;
-                int4_t w[NB], d[3];
-                float4_t a[4];
+                const int k = c * 64 + fq * 16, kA = k < K ? k : 0;
+                int4_t w[NB];
+                float4_t a[2][4];                                     // a block's values, and those of the next
+                auto loadA = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) a[i & 1][e] = *reinterpret_cast<const float4_t*>(aRow[i] + kA + 4 * e);
+                };
 #pragma unroll
                 for (int b = 0; b < NB; b++)
                     w[b] = *reinterpret_cast<const int4_t*>(c < whole ? wP[b] + (size_t)c * few_chunk_bytes(0)
                         : p.W + (size_t)min(r0 + b * 16 + ldRow, N - 1) * K + (size_t)whole * 64 + (ldPiece & 1) * 16);
-#pragma unroll
-                for (int e = 0; e < 4; e++) a[e] = *reinterpret_cast<const float4_t*>(aRow + (on ? k + 4 * e : 0));
-#pragma unroll
-                for (int g = 0; g < 3; g++) d[g] = *reinterpret_cast<const int4_t*>(aP[i] + (size_t)c * 3072 + g * 1024);
+                loadA(0);
                 asm volatile("" ::: "memory");
-                bf16x8_t hi[2], lo[2];
+                bf16x8_t x[NB][2];
 #pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int sh = 24 - 8 * (e & 3);
-                    const int n = (d[2][e >> 2] << sh >> 24) * 65536 + (d[1][e >> 2] << sh >> 24) * 256 + (d[0][e >> 2] << sh >> 24);
-                    const float y = (float)n, r = on && fabsf(y) < FG_KEPT ? fmaf(-s, y, a[e >> 2][e & 3] * up) * down : 0.f;
-                    const __bf16 h = (__bf16)r;
-                    hi[e >> 3][e & 7] = h;
-                    lo[e >> 3][e & 7] = (__bf16)(r - (float)h);
-                }
-#pragma unroll
-                for (int b = 0; b < NB; b++) {
-                    bf16x8_t x[2];
+                for (int b = 0; b < NB; b++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const int q = __builtin_amdgcn_ds_bpermute(from, w[b][e]);
 #pragma unroll
-                        for (int y = 0; y < 4; y++) x[e >> 1][(e & 1) * 4 + y] = (__bf16)(float)(q << (24 - 8 * y) >> 24);
+                        for (int y = 0; y < 4; y++) x[b][e >> 1][(e & 1) * 4 + y] = (__bf16)(float)(q << (24 - 8 * y) >> 24);
                     }
 #pragma unroll
+                for (int i = 0; i < MT; i++) {
+                    if (i + 1 < MT) loadA(i + 1);
+                    asm volatile("" ::: "memory");
+                    if (((runs[i] >> (8 * run)) & 0xff) == 0) continue;
+                    const float below = k < K ? lim[i] : 0.f;
+#pragma unroll
                     for (int h = 0; h < 2; h++) {
-                        left[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[h], x[h], left[b], 0, 0, 0);
-                        left[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[h], x[h], left[b], 0, 0, 0);
+                        bf16x8_t hi, lo;
+#pragma unroll
+                        for (int e = 0; e < 8; e += 2) {                      // (pairs: one conversion for two values)
+                            float2_t v;
+#pragma unroll
+                            for (int y = 0; y < 2; y++) {
+                                const float u = a[i & 1][2 * h + (e >> 2)][(e & 3) + y];
+                                v[y] = fabsf(u) < below ? u : 0.f;
+                            }
+                            const bf16x2_t t = __builtin_convertvector(v, bf16x2_t);
+                            const unsigned bits = __builtin_bit_cast(unsigned, t);
+                            v[0] -= __builtin_bit_cast(float, bits << 16);
+                            v[1] -= __builtin_bit_cast(float, bits & 0xffff0000u);
+                            const bf16x2_t r = __builtin_convertvector(v, bf16x2_t);
+                            hi[e] = t[0]; hi[e + 1] = t[1];
+                            lo[e] = r[0]; lo[e + 1] = r[1];
+                        }
+#pragma unroll
+                        for (int b = 0; b < NB; b++) {
+                            left[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, x[b][h], left[i][b], 0, 0, 0);
+                            left[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, x[b][h], left[i][b], 0, 0, 0);
+                        }
                     }
                 }
             }
         }
 #pragma unroll
-        for (int b = 0; b < NB; b++) sum[i][b] += left[b];
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) sum[i][b] += left[i][b];
     }
 #pragma unroll
     for (int i = 0; i < MT; i++)
