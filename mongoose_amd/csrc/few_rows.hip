@@ -87,7 +87,7 @@ __device__ __forceinline__ void put_split(unsigned short* hi, unsigned short* lo
 // each of the two Q4_0 blocks -- any order serves as long as both operands have the same.
 // ---------------------------------------------------------------------------
 //   LOOP = 0: K of at most 16 chunks, two a wave: both are requested at once, no ring.
-//   TERMS: bf16 terms of an activation, one plane each: 2 (2^-16 of the value left over), or 3 -- all 24 bits of an fp32 value,
+//   TERMS: bf16 terms of an activation, one plane each: 2 (2^-17 of the value left over), or 3 -- all 24 bits of an fp32 value,
 //   so that the products are those of the decode step and only the order of the fp32 sums differs.
 template <int MODE, int MT, int NB, int Q4, int LOOP, int TERMS>
 __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {

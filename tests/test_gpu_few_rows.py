@@ -55,7 +55,7 @@ def test_prompts_of_generate_match_token_by_token(hip, shape, fmt, kv_f16, n):
     the logits of the step after, which reads every cache row, against the same tokens one by one.  Bar: the products are the
     same (three bf16 terms are an fp32 value), so what differs are the roundings of fp32 sums: 2^-24 of a partial sum each,
     some 20 that matter in each of 7 products and 4 norms of 2 layers, at random: 2^-24 sqrt(20 * 11 * 2) = 1.3e-6, and
-    4e-6 for the largest of the logits.  Two terms would be off by 2^-18 a value: 1e-5 and more."""
+    4e-6 for the largest of the logits.  Two terms would be off by 2^-17 a value at worst, 2^-18 at random: 1e-5 and more."""
     m = H.Model(shape, seed=n, maxSeq=n + 3, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
     toks = m.prompt(n)
     for pos in range(n):
@@ -103,10 +103,13 @@ def test_few_row_gemm_matches_float64(hip, rows, n, k, accumulate):
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (15, 16, 64), (16, 17, 96), (17, 129, 544), (33, 40, 1056), (64, 128, 1024), (65, 600, 1088),
                                       (5, 48, 8192), (9, 20, 8224), (3, 30, 16384)])
 def test_few_row_gemm_digits(hip, rows, n, k):
-    """Activations as 24-bit numbers with a scale a row and eighth of K, at edges of the runs and tiles, for rows of any
-    magnitude: a value is off by half a step, 2^-24 of its run's largest one; a result by sqrt(k) such errors times weights of
-    75 at random, six times that for the worst of a row, plus what fp32 sums and factors lose (1e-6 of the largest).  A row
-    with a NaN or an infinity is NaN."""
+    """Activations as whole numbers of 24 bits times a scale a row and eighth of K, at edges of the runs and tiles, for rows of
+    any magnitude.  A value is off by half a step of its run (2^-23 of the largest value), and by three fp32 roundings of itself,
+    so a result by sqrt(sum of (step^2 / 12 + (2^-24 a)^2) weight^2) at random: five times that for the worst of up to 20,000,
+    and what fp32 loses in a dozen sums and factors, 2^-21 of its terms' root sum of squares in all.  The rows with one large
+    value may hold their values as two bf16 terms instead, off by 2^-18 of themselves at random.  A bit fewer would be ten
+    deviations, a step of another run (one is 10,000 times the others, with weights of zero for half of the columns)
+    thousands.  A row with a NaN or an infinity is NaN."""
     rng = np.random.default_rng(k)
     a = rng.standard_normal((rows, k), dtype=np.float32)
     for i, scale in enumerate((1e-37, 1e30, 1e-21, 0.0, 2.0 ** -64, 1.0)):
@@ -117,9 +120,14 @@ def test_few_row_gemm_digits(hip, rows, n, k):
         a[10, k // 2], a[11, k - 1] = np.inf, np.nan
         a[12, 0] = -1e36
     w = rng.integers(-128, 128, (n, k), dtype=np.int8)
+    per = ((k + 63) // 64 + 7) // 8 * 64                                # k of a run
+    if rows > 1 and k > per:
+        a[1, per:2 * per] *= np.float32(1e4)
+        w[:(n + 1) // 2, per:2 * per] = 0
     sc = (0.01 * (1 + rng.random(n))).astype(np.float32)
+    wd = w.astype(np.float64) * sc[:, None].astype(np.float64)
     with np.errstate(invalid="ignore"):
-        ref = a.astype(np.float64) @ (w.astype(np.float64) * sc[:, None].astype(np.float64)).T
+        ref = a.astype(np.float64) @ wd.T
     ta, tw, ts, to = hip.FromHost(a, a.shape), hip.UploadRawBytes(w), hip.FromHost(sc, sc.shape), hip.Zeros([rows, n])
     nbytes = 4 * ((rows + 127) // 128 * 128) * ((k + 63) // 64 * 64)
     ws = hip.UploadRawBytes(np.full(nbytes, 0xff, np.uint8))
@@ -131,8 +139,13 @@ def test_few_row_gemm_digits(hip, rows, n, k):
         if not np.isfinite(a[i]).all():
             assert np.isnan(got[i]).all()
         else:
-            bar = 6 * 2.0 ** -24 * np.abs(a[i]).max() * np.sqrt(k) * 75 * 0.015 + 1e-6 * np.abs(ref[i]).max()
-            assert np.abs(got[i] - ref[i]).max() <= bar + 1e-45, i
+            x = a[i].astype(np.float64)
+            top = np.concatenate([np.full(len(x[r:r + per]), np.abs(x[r:r + per]).max()) for r in range(0, k, per)])
+            each = (top / 8355584) ** 2 / 12 + (2.0 ** -24 * x) ** 2
+            if i in (9, 12):
+                each = np.maximum(each, (2.0 ** -18 * x) ** 2)
+            bar = 5 * np.sqrt((wd ** 2) @ each) + 2.0 ** -21 * np.sqrt((wd ** 2) @ (x ** 2))
+            assert (np.abs(got[i] - ref[i]) <= bar + 1e-45).all(), (i, (np.abs(got[i] - ref[i]) / (bar + 1e-45)).max())
     for t in (ta, tw, ts, to, ws):
         t.Release()
 
@@ -183,11 +196,11 @@ def test_few_row_gemm_keeps_small_values(hip, rows, n, k, spread):
 @pytest.mark.parametrize("k,kernel", [(1048064, "few_gemm_kernel"), (1049088, "gemm_q8")])
 def test_gemm_at_the_longest_rows(hip, k, kernel):
     """One step below and one above the K up to which 32-bit sums hold: every middle digit is -128 and so is every weight (the
-    values are 4161536 = 64 * 65536 - 128 * 256 steps of the row's scale, but for one a run at the top), which takes a run's
+    values are 4161536 = 64 * 65536 - 128 * 256 steps of the run, whose largest value is 8355584 of them), which takes a run's
     sum to the limit.  Bar: fp32 sums of equal terms, every one of k / 16 steps rounded the same way by up to 2^-24 of a sum
     that is half the last one on average; a sum past 32 bits is off by twice the result."""
-    a = np.full((1, k), np.float32(4161536 / 8355584), np.float32)
-    a[0, ::((k // 64 + 7) // 8 * 64)] = 1.0
+    a = np.full((1, k), 4161536 * 2.0 ** -23, np.float32)
+    a[0, ::((k // 64 + 7) // 8 * 64)] = 8355584 * 2.0 ** -23
     w = np.full((3, k), -128, np.int8)
     w[1, :k // 2] = 127
     sc = np.array([0.01, 0.02, 0.03], np.float32)
