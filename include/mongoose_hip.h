@@ -299,7 +299,9 @@ int mg_decode_token(mg_ctx* ctx, int token, int pos, int* nextToken, float* logi
  * captured hipGraph per token (CaptureGraph / Launch, cuda_graph.go:315-669);
  * the position and the token stay in device memory between steps.  Where runs of
  * tokens go inside the persistent launch, the prompt's positions before the last
- * go through the layers together, at the precision of a decode step. */
+ * go through the layers together, at the precision of a decode step (not bit for bit
+ * the cache rows that mg_decode_token leaves: fp32 sums in another order); where there
+ * is no device memory for their rows, they go one by one. */
 int mg_generate(mg_ctx* ctx, const int* prompt, int nPrompt, int nDecode, int* outTokens, int useGraph);
 
 /* Whole-token graphs (embedding gather .. argmax), the form the decode loop replays: capture once;

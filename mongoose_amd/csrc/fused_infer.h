@@ -177,7 +177,7 @@ private:
     FewScratch promptScratch{};
     int promptCap = 0;              // rows promptSlab holds
     int ensurePrompt(int rows);
-    int enqueuePrompt(const int* tokens, int n);    // the cache rows of positions 0 .. n - 1 (tokens: page-locked)
+    int enqueuePrompt(const int* tokens, int n);    // the cache rows of positions 0 .. n - 1 (tokens: page-locked), ensurePrompt before
     int enqueuePrefillTiles(int T, int pos0);
     std::vector<Slab> layerSlabs, kvSlabs;
     size_t slotOff[12] = {0};

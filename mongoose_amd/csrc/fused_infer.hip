@@ -1633,7 +1633,10 @@ int HIPFusedInference::Generate(const int* prompt, int nPrompt, int nDecode, int
     if (runsInLaunch(useGraph)) {
         rc = ensureFlow();
         int first = 0;                              // where the tokens of the launches begin
-        if (rc == MG_OK && nDecode > 0 && nPrompt - 1 >= PROMPT_ROWS_FROM) {
+        // (no room for a prompt's rows: its positions are tokens of the launches, as a short prompt's are)
+        bool rows = rc == MG_OK && nDecode > 0 && nPrompt - 1 >= PROMPT_ROWS_FROM;
+        if (rows && ensurePrompt(std::min(nPrompt - 1, PROMPT_ROWS)) != MG_OK) { rows = false; set_error(""); }
+        if (rows) {
             first = nPrompt - 1;
             rc = enqueuePrompt(reinterpret_cast<const int*>(hIn), first);
         } else if (rc == MG_OK) {
@@ -1923,7 +1926,7 @@ int HIPFusedInference::ensurePrompt(int rows) {
 //   128      892 / 18134    1014 / 17750    1317 / 25213    235 / 6500     394 / 11786       (Q4_0 within 10 % of these)
 // Against the 64-bit oracle the logits after the prompt are off by 2.4e-7 to 8e-7 either way.
 int HIPFusedInference::enqueuePrompt(const int* tokens, int n) {
-    int rc = ensurePrompt(std::min(n, PROMPT_ROWS));
+    int rc = MG_OK;
     for (int at = 0; at < n && rc == MG_OK; at += PROMPT_ROWS)
         rc = enqueuePrefillFew(tokens + at, std::min(PROMPT_ROWS, n - at), at, promptScratch, true);
     return rc;

@@ -1,10 +1,14 @@
 """The few-row prefill kernels (few_rows.hip) against the token-by-token path, at the edges of their tiles."""
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 from mongoose_amd import configs
 from mongoose_amd import engine as E
 from tests import helpers as H
+from tests.conftest import ROOT
 
 pytestmark = pytest.mark.gpu
 
@@ -77,6 +81,54 @@ def test_prompts_of_generate_match_token_by_token(hip, shape, fmt, kv_f16, n):
     rc, t = m.hip.Generate(toks, 1)
     assert rc == 0 and int(t[0]) == want
     m.close()
+
+
+def test_prompt_without_room_for_its_rows(tmp_path):
+    """Generate where the buffer for a prompt's rows cannot be had: the positions go one by one, as where a prompt is short, and
+    once there is room they go together.  A hipMalloc that fails when told to stands before the runtime's own, in a process
+    of its own (the buffer is the only allocation of such a call: the context has generated two tokens before)."""
+    src = tmp_path / "refuse.c"
+    src.write_text("""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+int refuse, refused;
+int hipMalloc(void** p, size_t n) {
+    static int (*real)(void**, size_t);
+    if (!real) real = (int (*)(void**, size_t))dlsym(RTLD_NEXT, "hipMalloc");
+    if (refuse) { refused++; return real(p, (size_t)1 << 50); }      /* the runtime's own refusal */
+    return real(p, n);
+}
+""")
+    shim = tmp_path / "refuse.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(shim), "-L/opt/rocm/lib", "-Wl,--no-as-needed", "-lamdhip64", "-ldl",
+                    "-Wl,-rpath,/opt/rocm/lib"], check=True)
+    out = subprocess.run([sys.executable, "-c", """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+from mongoose_amd import engine as E
+from tests import helpers as H
+from tests.test_gpu_few_rows import SMALL
+refuse, refused = (ctypes.c_int.in_dll(shim, n) for n in ("refuse", "refused"))
+m = H.Model(SMALL, seed=5, maxSeq=64, eng=E.NewHIP(), oracle=False)
+toks = m.prompt(40)
+assert m.hip.Generate(toks[:1], 2)[0] == 0
+got = []
+for r in (1, 0):
+    refuse.value = r
+    rc, t = m.hip.Generate(toks, 6)
+    assert rc == 0, E.last_error()
+    got.append(t.tolist())
+    after = np.empty(SMALL.vocab, np.float32)
+    assert m.hip.DecodeToken(int(t[-1]), 45, after)[0] == 0
+    got.append(after)
+assert refused.value == 1, refused.value
+assert got[0] == got[2], got
+assert H.rel_err(got[1], got[3]) < 4e-6
+print("same", flush=True)
+""", str(shim)], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and "same" in out.stdout, out.stdout + out.stderr
 
 
 @pytest.mark.parametrize("rows,n,k,accumulate", [(1, 16, 32, 0), (17, 33, 96, 1), (64, 300, 1056, 0), (77, 129, 2080, 1), (130, 1000, 4864, 0),
