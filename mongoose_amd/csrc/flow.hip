@@ -1976,13 +1976,11 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         else FLOW_LAUNCH_F(128, 2, true, false, false, 3);
     } else if (fix == 3 && !p.q4 && gqa) {              // fp16 K / V rows at a long context
         FLOW_LAUNCH_F(128, 2, true, true, false, 11);
-    } else if (p.manySplits && !gqa && !wide && !p.trace) {
+    } else if (p.manySplits && !gqa && !wide) {
         // Six splits: hidden size 768, six layers, Q8, at 600 positions (five) 82.9 us a token with / 83.0 without, Q4_0 87.9 / 86.0,
         // the toy shape 56.7 / 57.8; at 1,200 (ten) 88.5 / 95.3, 93.2 / 98.0 and 59.0 / 66.8.
-#define FLOW_LAUNCH_S(HDv, Q4v) hipLaunchKernelGGL((flow_layers_kernel<HDv, 1, false, false, Q4v, false, 32>), dim3(grid), dim3(FWG), lds, s, p)
-        if (p.headDim == 64) { if (p.q4) FLOW_LAUNCH_S(64, true); else FLOW_LAUNCH_S(64, false); }
-        else { if (p.q4) FLOW_LAUNCH_S(128, true); else FLOW_LAUNCH_S(128, false); }
-#undef FLOW_LAUNCH_S
+        if (p.headDim == 64) { if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 32); else FLOW_LAUNCH_F(64, 1, false, false, false, 32); }
+        else { if (p.q4) FLOW_LAUNCH_F(128, 1, false, false, true, 32); else FLOW_LAUNCH_F(128, 1, false, false, false, 32); }
     } else if (p.headDim == 64) {
         if (ring) FLOW_LAUNCH_G(64, 2, true);
         else if (wide) FLOW_LAUNCH_G(64, 2, false);

@@ -342,6 +342,26 @@ def test_kv_splits_shared_out_among_threads(hip, fmt, heads, kv, hd, pos):
     m.close()
 
 
+@pytest.mark.parametrize("fmt,heads,kv,hd,kv_f16", [
+    ("q8", 4, 4, 64, False), ("q4_0", 3, 1, 64, False), ("q8", 4, 2, 128, False), ("q4_0", 3, 1, 128, False), ("q8", 6, 2, 64, True),
+    ("q4_0", 4, 2, 128, True)])
+def test_variant_with_the_shared_merge(hip, fmt, heads, kv, hd, kv_f16):
+    """The variant whose threads share out a vector's KV splits, and only from six splits on (position 640), with the timing
+    diagnostic on as with it off; its results at 900 positions against the separate launches where the test above has no such
+    shape (fp16 rows, Q8 heads of 128; their bar as there)."""
+    s = configs.TOY._replace(name="splits", nLayers=2, dim=heads * hd, nHeads=heads, nKVHeads=kv, headDim=hd, ffnDim=608, vocab=300)
+    m = H.Model(s, seed=heads, maxSeq=940, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
+    _modes_agree(m, m.prompt(888), 24, f"{heads} heads of {hd}, {fmt}, fp16 rows: {kv_f16}")
+    for trace in (False, True):
+        assert m.hip.FlowTrace(trace)[0] == 0
+        for pos, shared in ((639, False), (640, True)):
+            names = [n for n in H.launched(lambda: m.hip.DecodeToken(1, pos)) if "flow_layers_kernel<" in n]
+            assert len(names) == 1, names
+            args = names[0].split("<")[1].split(">")[0].replace(" ", "").split(",")
+            assert args[5] == str(trace).lower() and (args[6] == "32") == shared, names
+    m.close()
+
+
 def test_fp16_kv_rows_in_the_launch(hip):
     """fp16 K/V rows (SetKVFormat(1)) through the persistent launch: rounded where the q|k|v phase writes them (the
     cache and the copy it hands to the attention workgroups), widened where the attention phase reads them.  Tokens
