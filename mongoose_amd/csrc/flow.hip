@@ -220,8 +220,9 @@ __device__ __forceinline__ void poll_batch(const f4* const (&ptr)[PB], f4 (&v)[P
         // the space is also the spread of the moments at which the workgroups notice the vector, and the phase ends with
         // the last of them.  128 clocks; us a token at the 0.5B shape, 24 layers, by clocks 0 / 128 / 256 / 512: 263.6 / 264.1 /
         // 265.9 / 274; sizes in registers 295.0 / 293.3 / 294.9 / 296.3 (1024: 300.7); the toy shape 51.4 / 51.2 / 51.3 / 51.6;
-        // 1.1B and 0.5B Q4_0 within 0.3 %.  512 where sizes in registers meet long vectors, whose re-reading costs more: three
-        // layers of 3840 (Q4_0) 121.4 / 120.3 us by 128 / 512, five of 2560 the same, eight of 1536 121.7 / 120.9.
+        // 0.5B Q4_0 within 0.3 %.  512 for vectors of more than 1,024 elements, whose re-reading costs more: three
+        // layers of 3840 (Q4_0) 121.4 / 120.3 us by 128 / 512, five of 2560 the same, eight of 1536 121.7 / 120.9, 1.1B 22 layers
+        // 396.4 / 395.8, at 600 positions 435.2 / 434.4, 8B six layers at 3,900 435.0 / 433.9.
         if (PAUSE) for (int z = 0; z < w.pause; z++) __builtin_amdgcn_s_sleep(2);
     }
 }
@@ -663,11 +664,10 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     // Measured per variant, ms a token with / without: 0.5B Q8 0.3141 / 0.3230, 8B 1.558 / 1.561 (fp16 rows at 4,000
     // positions 1.841 / 1.847), 0.5B Q4_0 0.3235 / 0.3230, 1.1B 0.378 / 0.372 -- the last two keep them in registers.
     constexpr bool FXF = FX && (((FIX & 7) == 1 && !Q4) || (FIX & 7) == 3);
-    // (0.5B Q4_0 0.3267 -> 0.3204 ms a token, Q8 0.3141 -> 0.3138; 1.1B 0.366 -> 0.364, at 600 positions 0.433 -> 0.430; 8B gains nothing)
-    constexpr bool FXD = FX && ((FIX & 7) == 1 || (FIX & 7) == 2);
     // whether workgroups past the computing ones prefetch (then none prefetches while idle during the attention): of the
-    // two roles a known shape has one, the other's code is not in its variant
-    const bool hasPrefetchers = FXD ? FS.dedicated != 0 : nC != (int)gridDim.x;
+    // two roles a known shape has one, the other's code is not in its variant (0.5B Q4_0 0.3267 -> 0.3204 ms a token, Q8 0.3141 ->
+    // 0.3138; 1.1B 0.366 -> 0.364, at 600 positions 0.433 -> 0.430; 8B, six layers at 900 and 3,900, 0.4237 -> 0.4224 and 0.4339 -> 0.4333)
+    const bool hasPrefetchers = FX ? FS.dedicated != 0 : nC != (int)gridDim.x;
     // (1.1B: the row sharing alone as a constant 0.3734 -> 0.3695 ms a token, the row format alone 0.3818)
     const bool downSplitV = (FXF || (FIX & 7) == 2) ? FS.downSplit != 0 : p.downSplit != 0;
     const bool kvHalfV = FXF ? (FIX & 8) != 0 : p.kvHalf != 0;
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     }
     // (the idle lines follow the error word's 256 bytes: 16 lines of 128 bytes, two workgroups of an XCD on each)
     Waiter wt{p.limitTicks, p.err, false, reinterpret_cast<const f4*>(reinterpret_cast<const char*>(p.err) + 256 + ((blockIdx.x >> 3) & 15) * 128),
-              CBD == 2 && FIX == 0 ? 4 : 1};
+              CBD == 2 ? 4 : 1};
 
     // attention geometry (decode attention of kernels.hip with one query head per workgroup): a thread group of 16
     // lanes holds a K/V row, a thread VU rows of its workgroup's tile of FLOW_TILE positions.  (Measured on the 0.5B
@@ -1158,11 +1158,12 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                         }
                         // the waves' partials of all the workgroup's heads combined together: one barrier, a thread per head and piece
                         __syncthreads();
-                        if constexpr (!GQA && (FIX & 7) != 1) {
+                        if constexpr (!GQA) {
                             // One head: one wave, whose four row groups take two waves' partials each -- a chain of two terms and
                             // two exchanges instead of eight terms a thread.  (Microseconds a token, by waves' partials one after the
                             // other / so: toy shape 50.3 / 49.8, hidden size 256 70.0 / 69.2, 1.1B 356 / 354, at 600 positions 429 /
-                            // 426.5; the variants with the 0.5B shape's sizes 266.0 / 268.4, Q4_0 the same: not there.)
+                            // 426.5; 0.5B Q4_0 at 100 / 320 / 1,000 positions 307.1 / 304.4, 320.7 / 316.7, 373.2 / 373.6, Q8 at 20 / 600
+                            // / 1,900 291.4 / 292.4, 338.1 / 339.4, 435.3 / 437.8.)
                             if (wave == 0) {
                                 constexpr int NP = HD / 64;
                                 const int i = lane & 15, k0 = lane >> 4;
@@ -1959,7 +1960,7 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         for (int k = 1; k <= 3 && !fix; k++) {
             const FlowFixedShape fs = flow_fixed_shape(k);
             if (p.dim == fs.dim && p.kvDim == fs.kvDim && p.ffn == fs.ffn && p.nHeads == fs.nHeads && p.nKVHeads == fs.nKVHeads &&
-                p.headDim == fs.headDim && (p.downSplit != 0) == (fs.downSplit != 0) && (k == 3 || (nC != grid) == (fs.dedicated != 0))) fix = k;
+                p.headDim == fs.headDim && (p.downSplit != 0) == (fs.downSplit != 0) && (nC != grid) == (fs.dedicated != 0)) fix = k;
         }
 #define FLOW_LAUNCH_F(HDv, CBv, RGv, GQv, Q4v, FXv) do { \
         if (p.trace) hipLaunchKernelGGL((flow_layers_kernel<HDv, CBv, RGv, GQv, Q4v, true, FXv>), dim3(grid), dim3(FWG), lds, s, p); \
