@@ -49,6 +49,7 @@ inline void note(hipError_t e) {
 }
 inline hipStream_t S(void* s) { return static_cast<hipStream_t>(s); }
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+inline bool overlap(const float* a, long long na, const float* b, long long nb) { return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na); }
 }  // namespace
 
 extern "C" {
@@ -196,8 +197,12 @@ void mongoose_decode_attention(const float* Q, const float* K, const float* V, f
     if (cacheLen <= 0 || nHeads <= 0) return;
     // No room for partial results here, so the context is not split.  Four workgroups a query head share out its columns while
     // that is at most a workgroup for every CU (kernels.hip); with more heads the K rows they read again cost more than the
-    // idle CUs do, and a workgroup takes a head.
-    if (nHeads <= 64) { note(mg::launch_attention_columns(Q, K, V, out, cacheLen, kvDim, nHeads, nKVHeads, dim / nHeads, S(stream))); return; }
+    // idle CUs do, and a workgroup takes a head.  So it does where the output goes over the query: of four workgroups one could
+    // read what another has written.
+    if (nHeads <= 64 && !overlap(Q, dim, out, dim)) {
+        note(mg::launch_attention_columns(Q, K, V, out, cacheLen, kvDim, nHeads, nKVHeads, dim / nHeads, S(stream)));
+        return;
+    }
     mg::AttnParams p{};
     p.q = Q; p.Kc = K; p.Vc = V;
     p.posImm = cacheLen - 1;

@@ -214,6 +214,19 @@ def test_decode_attention_by_columns(hip, nH, nKV, hd, T):
     assert H.rel_err(hip.ToHost(do), ref) < 1e-5
 
 
+@pytest.mark.parametrize("nH,nKV,hd,T", [(14, 2, 64, 1025), (64, 8, 128, 300)])
+def test_decode_attention_over_its_query(hip, nH, nKV, hd, T):
+    """out may be Q: then a head's output comes from one workgroup, which has read the query before it writes.  Bar as above."""
+    dim, kvDim = nH * hd, nKV * hd
+    Q = rng.standard_normal(dim).astype(np.float32)
+    Kc, Vc = rng.standard_normal((2, T, kvDim)).astype(np.float32)
+    dq, dk, dv = _up(hip, Q), _up(hip, Kc), _up(hip, Vc)
+    names = H.launched(lambda: E.KDecodeAttention(dq, dk, dv, dq, T, dim, kvDim, nH, nKV))
+    _check()
+    assert not any("attn_columns" in n for n in names), names
+    assert H.rel_err(hip.ToHost(dq), ob.decode_attention(Q, Kc, Vc, T, kvDim, nH, nKV, hd, shadow=True)) < 1e-5
+
+
 def test_elementwise_ops(hip):
     n = 4864
     g = (rng.standard_normal(n) * 3).astype(np.float32)
