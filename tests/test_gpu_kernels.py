@@ -220,7 +220,7 @@ def test_decode_attention_over_its_query(hip, nH, nKV, hd, T):
     dim, kvDim = nH * hd, nKV * hd
     Q = rng.standard_normal(dim).astype(np.float32)
     Kc, Vc = rng.standard_normal((2, T, kvDim)).astype(np.float32)
-    dq, dk, dv = _up(hip, Q), _up(hip, Kc), _up(hip, Vc)
+    dq, dk, dv = hip.FromHost(Q, Q.shape), _up(hip, Kc), _up(hip, Vc)
     names = H.launched(lambda: E.KDecodeAttention(dq, dk, dv, dq, T, dim, kvDim, nH, nKV))
     _check()
     assert not any("attn_columns" in n for n in names), names
