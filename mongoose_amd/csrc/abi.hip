@@ -236,11 +236,13 @@ void mongoose_dequant_q4_0(const void* w, float* out, int rows, int cols, void* 
 // kernel has no room for K splits here and leaves most CUs idle until N / 128 x T / 64 tiles fill them.  Microseconds a call,
 // few rows / tiled: 5632 x 2048 54 / 58 at 513 rows, 74 / 68 at 800; 9000 x 8192 230 / 239 at 513, 400 / 317 at 800; 900 x
 // 2048 28 / 31 at 1000, 38 / 42 at 1500, 48 / 45 at 2000; 28672 x 4096 400 / 373 at 513.
+// Its wide runs are read from act a second time, so it is not for results that go over act.
 static hipError_t q8_gemm_launches(const float* act, const void* w, const float* scales, const float* bias, float* out, int T, int N,
                                    int K, int accumulate, void* ws, size_t plane, hipStream_t s) {
     void* hi = ws;
     void* lo = static_cast<char*>(ws) + plane;
-    if (T > 0 && N > 0 && (T <= 512 || (long long)T * N <= 1500000) && aligned16(act) && mg::few_gemm_sums_fit(K)) {
+    if (T > 0 && N > 0 && (T <= 512 || (long long)T * N <= 1500000) && aligned16(act) && mg::few_gemm_sums_fit(K) &&
+        !overlap(act, (long long)T * K, out, (long long)T * N)) {
         mg::FewGemmParams f{};
         f.W = static_cast<const signed char*>(w); f.scales = scales; f.bias = bias; f.Y = out;
         f.T = T; f.N = N; f.K = K; f.accumulate = accumulate;

@@ -245,6 +245,27 @@ def test_few_row_gemm_keeps_small_values(hip, rows, n, k, spread):
         t.Release()
 
 
+@pytest.mark.parametrize("rows,n,accumulate", [(300, 2048, 0), (16, 2048, 1), (40, 1024, 0)])
+def test_gemm_over_its_activations(hip, rows, n, accumulate):
+    """out may lie over act: the kernel that reads act again, for its small values beside a large one, does not serve such a call.
+    Bar: two bf16 terms."""
+    k, rng = 2048, np.random.default_rng(rows)
+    a = rng.standard_normal((rows, k), dtype=np.float32)
+    a[:, 5] *= 1e4
+    w = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    sc = (0.01 * (1 + rng.random(n))).astype(np.float32)
+    ref = a.astype(np.float64) @ (w.astype(np.float64) * sc[:, None]).T + (a if accumulate else 0)
+    ta, tw, ts = hip.FromHost(a, a.shape), hip.UploadRawBytes(w), hip.FromHost(sc, sc.shape)
+    nbytes = 4 * ((rows + 127) // 128 * 128) * k
+    ws = hip.Zeros([nbytes // 4])
+    names = H.launched(lambda: E.KQ8Gemm(ta, tw, ts, None, ta, rows, n, k, accumulate, ws, nbytes))
+    assert E.HIPCheck() == 0
+    assert not any("few_gemm" in x for x in names) and len(names) > 1, names
+    assert H.rel_err(hip.ToHost(ta).reshape(-1)[:rows * n].reshape(rows, n), ref) < 3e-5
+    for t in (ta, tw, ts, ws):
+        t.Release()
+
+
 @pytest.mark.parametrize("k,kernel", [(1048064, "few_gemm_kernel"), (1049088, "gemm_q8")])
 def test_gemm_at_the_longest_rows(hip, k, kernel):
     """One step below and one above the K up to which 32-bit sums hold: every middle digit is -128 and so is every weight (the
