@@ -8,8 +8,8 @@
 // into small integers for an integer matrix unit: the Ozaki scheme, as in Ootomo, Ozaki and Yokota, "DGEMM on integer matrix
 // multiplication unit", 2024.)  The sums of a wave are whole numbers, exact; scale, row scale, bias and the sum of the waves are
 // fp32.  Bound by the operands a workgroup pulls through its CU's L1.  Microseconds a call, weights from memory, two bf16 terms
-// / this: 77 x 5632 x 2048 19.5 / 14.3, 16 x 5632 x 2048 10.4 / 9.9, 37 x 896 x 4864 11.4 / 10.6, 300 x 5632 x 2048 35.5 / 31.9,
-// 48 x 9000 x 8192 49.6 / 39.7, 500 x 9000 x 8192 240 / 207.
+// / this: 77 x 5632 x 2048 19.7 / 14.1, 16 x 5632 x 2048 10.4 / 9.9, 37 x 896 x 4864 11.8 / 11.1, 300 x 5632 x 2048 36.5 / 31.9,
+// 48 x 9000 x 8192 49.7 / 39.8, 500 x 9000 x 8192 240 / 207.
 //
 // Precision: the eight waves of a workgroup split K into eight runs, and every row has a scale for each run, the run's
 // largest value / 8355584.  A value is off by half a step, 2^-24 of the run's largest one (by up to 1.4 steps next to that one,
@@ -23,7 +23,7 @@
 // 3.9e-7 / 3.9e-7, 100 2.5e-6 / 1.2e-6 / 7.7e-7, 1,000 2.5e-6 / 1.2e-5 / 8.8e-7, 10^5 2.5e-6 / 1.2e-3 / 8.7e-7, 10^20 2.5e-6 /
 // 0.35 / 8.7e-7; K = 64 (one run) 100 2.4e-6 / 3.4e-6 / 2.1e-6, from 1,000 on two bf16 terms' own.
 // A wide run costs its chunks a second time, with conversions, shared by the eight waves.  Microseconds a call with no wide
-// run, one of eight, about half of them, all (two bf16 terms): 77 x 5632 x 2048 14.3, 15.8, 19.2, 23.2 (19.7), 48 x 9000 x 8192
+// run, one of eight, about half of them, all (two bf16 terms): 77 x 5632 x 2048 14.1, 15.7, 19.2, 23.2 (19.7), 48 x 9000 x 8192
 // 40, 45, 54, 74 (50), 300 x 5632 x 2048 32, 38, 55, 86 (36), 500 x 9000 x 8192 209, 257, 386, 555 (241).
 #include "few_rows.h"
 #include "few_rules.h"
@@ -101,16 +101,7 @@ __global__ __launch_bounds__(WG) void few_digits_kernel(const float* in, signed 
             squares = fmaf(z, z, squares);
         }
     };
-#pragma unroll
-    for (int j = 0; j < FG_PIECES; j++)
-        if (64 * j < pieces) weigh(v[j]);
-    for (int p = 64 * FG_PIECES; p < pieces; p += 64) weigh(get(p + lane));
-    squares = wave_sum(squares);
-    const float f = (float)small;
-    const bool isWide = !bad && small * 8 > some && (float)some * squares < FG_EVEN * f * f;
-    if (lane == 0) wide[(tb * FG_WAVES + run) * 16 + r] = isWide ? 1 : 0;
-    const float least = isWide ? lim : 0.f;
-    auto put = [&](int p, float4 a) {
+    auto put = [&](int p, float4 a, float least) {
         if (p >= pieces) return;
         const float x[4] = {a.x, a.y, a.z, a.w};
         unsigned d[3] = {0, 0, 0};
@@ -128,9 +119,19 @@ __global__ __launch_bounds__(WG) void few_digits_kernel(const float* in, signed 
 #pragma unroll
         for (int g = 0; g < 3; g++) *reinterpret_cast<unsigned*>(o + g * 1024) = d[g];
     };
+    // (digits of all values first, which hides the weighing; those of a wide run again)
 #pragma unroll
-    for (int j = 0; j < FG_PIECES; j++) put(lane + 64 * j, v[j]);
-    for (int p = lane + 64 * FG_PIECES; p < pieces; p += 64) put(p, get(p));
+    for (int j = 0; j < FG_PIECES; j++)
+        if (64 * j < pieces) { weigh(v[j]); put(lane + 64 * j, v[j], 0.f); }
+    for (int p = 64 * FG_PIECES; p < pieces; p += 64) { const float4 a = get(p + lane); weigh(a); put(p + lane, a, 0.f); }
+    squares = wave_sum(squares);
+    const float f = (float)small;
+    const bool isWide = !bad && small * 8 > some && (float)some * squares < FG_EVEN * f * f;
+    if (lane == 0) wide[(tb * FG_WAVES + run) * 16 + r] = isWide ? 1 : 0;
+    if (!isWide) return;
+#pragma unroll
+    for (int j = 0; j < FG_PIECES; j++) put(lane + 64 * j, v[j], lim);
+    for (int p = lane + 64 * FG_PIECES; p < pieces; p += 64) put(p, get(p), lim);
 }
 
 // ---------------------------------------------------------------------------
