@@ -135,7 +135,7 @@ public:
     int hiddenIdx = 0;
     int enqueueLayer(const LayerWeights& L, int layer, const StepState* st, int posImm);
     // row / parts: the lm_head of that row (instead of the hidden buffer), its argmax partials left for the caller
-    int enqueueFinal(bool withArgmax, const float* row = nullptr, int* parts = nullptr);
+    int enqueueFinal(bool withArgmax, int* parts = nullptr);
     int publish(const float* src, int n, const int* ints, int nInts);      // results on their way to hOut
     PublishParams publishParams(const float* src, int n);
     int collect(float* out, int n, int* ints, int nInts, bool prefill = false);      // ... waited for and copied to the caller
@@ -170,7 +170,7 @@ private:
     float* pfSumSq = nullptr;               // few-row path: partial sums of squares of the rows
     // Buffers of the few-row path; the third planes: NULL, or the third terms of the activations (few_rows.h).
     struct FewScratch { float *x, *q, *sumSq; unsigned short *a[3], *b[3]; };
-    int enqueuePrefillFew(const int* tokens, int T, int pos0, const FewScratch& S, bool cachesOnly);
+    int enqueuePrefillFew(const int* tokens, int T, int pos0, const FewScratch& S, bool wholeLast);
     static constexpr int PROMPT_ROWS = 128;      // prompt positions that go through the layers together
     static constexpr int PROMPT_ROWS_FROM = 3;   // ... from as many on (below, Generate has them as tokens of its launches)
     Slab promptSlab;
@@ -178,12 +178,13 @@ private:
     int promptCap = 0;              // rows promptSlab holds
     int ensurePrompt(int rows);
     int enqueuePrompt(const int* tokens, int n);    // the cache rows of positions 0 .. n - 1 (tokens: page-locked), ensurePrompt before
-    int enqueuePrefillTiles(int T, int pos0);
+    int enqueuePrefillTiles(int T, int pos0, bool wholeLast);
     std::vector<Slab> layerSlabs, kvSlabs;
     size_t slotOff[12] = {0};
     size_t layerSlabBytes = 0;
     DevMat* matSlot(int idx, int* rows, int* cols);
     int enqueueLayerFused(const LayerWeights& L, int layer, const StepState* st, int posImm);
+    int enqueueLayerRest(const LayerWeights& L, int layer, const StepState* st, int posImm, const float* q, const float* resid);
     MvParams qkvParams(const LayerWeights& L, int layer, const StepState* st, int posImm) const;
     MvParams woParams(const LayerWeights& L) const;
     MvParams gateUpParams(const LayerWeights& L) const;

@@ -668,11 +668,17 @@ int HIPFusedInference::enqueueLayerFused(const LayerWeights& L, int layer, const
         MvParams p = qkvParams(L, layer, st, posImm);
         HIPCHK(launch_matvec(L.wq.kind, EPI_QKV, PRO_RMS, p, nullptr, stream));
     }
+    return enqueueLayerRest(L, layer, st, posImm, Q, hidden[hiddenIdx]);
+}
+
+// The layer behind its q|k|v: attention of the (rotated) q over the cache, Wo added to resid, gate | up, down.  The row ends up in
+// the hidden buffer.
+int HIPFusedInference::enqueueLayerRest(const LayerWeights& L, int layer, const StepState* st, int posImm, const float* q, const float* resid) {
     if (mark(2)) return MG_E_HIP;
     {
         AttnParams a{};
         a.kvHalf = kvHalf;
-        a.q = Q; a.Kc = kCache[layer]; a.Vc = vCache[layer];
+        a.q = q; a.Kc = kCache[layer]; a.Vc = vCache[layer];
         a.state = st; a.posImm = posImm; a.rowLimit = maxSeq;
         a.kvDim = kvDim; a.nHeads = nHeads; a.nKVHeads = nKVHeads; a.headDim = headDim;
         a.smax = smax; a.splitLen = splitLen; a.headsPerWG = attnHeadsPerWG;
@@ -686,6 +692,7 @@ int HIPFusedInference::enqueueLayerFused(const LayerWeights& L, int layer, const
     if (mark(3)) return MG_E_HIP;
     {
         MvParams p = woParams(L);
+        p.resid = resid;
         HIPCHK(launch_matvec(L.wo.kind, EPI_RESID, PRO_PLAIN, p, nullptr, stream));
     }
     if (mark(4)) return MG_E_HIP;
@@ -1179,7 +1186,7 @@ int HIPFusedInference::enqueueLayer(const LayerWeights& L, int layer, const Step
 
 // Final norm + lm_head (cuda_fused_infer.go:446-448) with the per-workgroup
 // argmax folded into the matvec epilogue.
-int HIPFusedInference::enqueueFinal(bool withArgmax, const float* row, int* parts) {
+int HIPFusedInference::enqueueFinal(bool withArgmax, int* parts) {
     if (withArgmax) statePosHost = -1;              // (the argmax's last kernel advances the device state)
     if (!finalNorm || !lmHead.w) { set_error("final norm / lm_head not set"); return MG_E_STATE; }
     if (execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P) {
@@ -1197,7 +1204,7 @@ int HIPFusedInference::enqueueFinal(bool withArgmax, const float* row, int* part
     }
     MvParams p{};
     p.seg[0] = MvSeg{lmHead.w, lmHead.scales, nullptr, logits, vocabSize};
-    p.nseg = 1; p.K = dim; p.act = row ? row : hidden[hiddenIdx]; p.gain = finalNorm; p.eps = eps;
+    p.nseg = 1; p.K = dim; p.act = hidden[hiddenIdx]; p.gain = finalNorm; p.eps = eps;
     p.amaxVal = amaxVal; p.amaxIdx = amaxIdx;
     if (fuseEmbed && flowEligible(0, nLayers)) {
         // inside the captured token: the lm_head launch also leaves the exchange area of the persistent
@@ -1786,8 +1793,9 @@ int HIPFusedInference::ensurePrefill(int rows, int kvRows) {
     return MG_OK;
 }
 
-// The layers over T rows through the tiled GEMMs of prefill.hip; the rows end up in pfX.
-int HIPFusedInference::enqueuePrefillTiles(int T, int pos0) {
+// The layers over T rows through the tiled GEMMs of prefill.hip, the last one up to its cache rows -- its input rows are then in pfX,
+// its q rows in pfQ -- or, with wholeLast, to its end (rows in pfX).
+int HIPFusedInference::enqueuePrefillTiles(int T, int pos0, bool wholeLast) {
     if (embedKind == 1 || embedKind == 2) {
         HIPCHK(launch_embed_rows(embedKind, embedTable, nullptr, pfTokens, pfX, T, dim, vocabSize, stream));
     } else {
@@ -1812,6 +1820,7 @@ int HIPFusedInference::enqueuePrefillTiles(int T, int pos0) {
         HIPCHK(launch_gemm_q8(g, 0, stream));
         if (!g.wroteRope)
             HIPCHK(launch_rope_store_rows(pfQ, pfK, pfV, kCache[l], vCache[l], kvHalf, cosTab, sinTab, pos0, T, dim, kvDim, headDim, stream));
+        if (l + 1 == nLayers && !wholeLast) break;
         g.ropeKc = nullptr; g.ropeVc = nullptr;
         // the attention writes its rows as the hi/lo split the output projection reads
         HIPCHK(launch_prefill_attention(pfQ, kCache[l], vCache[l], kvHalf, pfKVSplit, nullptr, pfHi, pfLo, T, pos0, maxSeq, dim, kvDim, nHeads,
@@ -1843,9 +1852,8 @@ int HIPFusedInference::enqueuePrefillTiles(int T, int pos0) {
     return MG_OK;
 }
 
-// The same through the few-row kernels (few_rows.hip): five launches a layer; the rows end up in S.x.  cachesOnly: what
-// is wanted are the K / V rows, so the last layer ends with them.
-int HIPFusedInference::enqueuePrefillFew(const int* tokens, int T, int pos0, const FewScratch& S, bool cachesOnly) {
+// The same through the few-row kernels (few_rows.hip): five launches a layer; rows in S.x, q rows in S.q.
+int HIPFusedInference::enqueuePrefillFew(const int* tokens, int T, int pos0, const FewScratch& S, bool wholeLast) {
     // S.a: normed rows, S.b: attention output, SwiGLU rows
     const bool table = embedKind == 1 || embedKind == 2;
     const int terms = S.a[2] ? 3 : 2;
@@ -1866,7 +1874,7 @@ int HIPFusedInference::enqueuePrefillFew(const int* tokens, int T, int pos0, con
         f.seg[0] = seg(L.wq, L.bq, S.q); f.seg[1] = seg(L.wk, L.bk, nullptr); f.seg[2] = seg(L.wv, L.bv, nullptr);
         f.Kc = kCache[l]; f.Vc = vCache[l]; f.cosTab = cosTab; f.sinTab = sinTab; f.pos0 = pos0; f.headDim = headDim; f.kvHalf = kvHalf;
         HIPCHK(launch_few_rows(FEW_QKV, f, stream));
-        if (cachesOnly && l + 1 == nLayers) break;
+        if (l + 1 == nLayers && !wholeLast) break;
         HIPCHK(launch_few_attention(S.q, kCache[l], vCache[l], kvHalf, S.b[0], S.b[1], S.b[2], T, pos0, maxSeq, dim, kvDim, nHeads, nKVHeads,
                                     headDim, L.wo.kind == WF_Q4P, stream));
         FewParams r{};
@@ -1928,7 +1936,7 @@ int HIPFusedInference::ensurePrompt(int rows) {
 int HIPFusedInference::enqueuePrompt(const int* tokens, int n) {
     int rc = MG_OK;
     for (int at = 0; at < n && rc == MG_OK; at += PROMPT_ROWS)
-        rc = enqueuePrefillFew(tokens + at, std::min(PROMPT_ROWS, n - at), at, promptScratch, true);
+        rc = enqueuePrefillFew(tokens + at, std::min(PROMPT_ROWS, n - at), at, promptScratch, false);
     return rc;
 }
 
@@ -1951,27 +1959,34 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
     const bool few = few_rows_pay(T, pos0, dim, kvDim, ffnDim, nHeads, layers[0].gate.kind == WF_Q4P);
     std::memcpy(hIn, tokens, sizeof(int) * (size_t)T);              // (the embedding rows' launch reads them there)
     pfTokens = reinterpret_cast<const int*>(hIn);
+    // Of the last layer only the last position is wanted behind the cache rows; the rest of it then runs as a decode step's layer
+    // does.  8B shape: 512 rows through eight layers 3,919 -> 3,605 us, 37 through four 601 -> 536; 1.1B, eight layers, 37 rows 487 ->
+    // 463; 0.5B, 24 layers, 855 -> 851.  (A model of one layer goes through whole: the batched kernels are checked on such models.)
+    const bool single = nLayers == 1;
     if (elapsedMs) HIPCHK(hipEventRecord(ev0, stream));
     if (few) {
         auto plane = [](void* p) { return static_cast<unsigned short*>(p); };
         const FewScratch S{pfX, pfQ, pfSumSq, {plane(pfHi), plane(pfLo), nullptr}, {plane(pfHi2), plane(pfLo2), nullptr}};
-        rc = enqueuePrefillFew(pfTokens, T, pos0, S, false);
+        rc = enqueuePrefillFew(pfTokens, T, pos0, S, single);
     } else {
-        rc = enqueuePrefillTiles(T, pos0);
+        rc = enqueuePrefillTiles(T, pos0, single);
     }
     if (rc) return rc;
-    // the last position continues on the decode path: final norm, lm_head, greedy token, state -> pos0 + T
+    // the last position continues on the decode path: the rest of its last layer, final norm, lm_head, greedy token, state -> pos0 + T
     const float* row = pfX + (size_t)(T - 1) * dim;
+    if (single) HIPCHK(hipMemcpyAsync(hidden[hiddenIdx], row, (size_t)dim * 4, hipMemcpyDeviceToDevice, stream));
+    else rc = enqueueLayerRest(layers[nLayers - 1], nLayers - 1, nullptr, pos0 + T - 1, pfQ + (size_t)(T - 1) * dim, row);
+    if (rc) return rc;
     const int n = logitsOut ? vocabSize : 0;
     int next = 0;
-    const bool quantized = execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P;      // (a tail that wants the hidden buffer)
+    const bool quantized = execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P;      // (a tail of its own)
     if (quantized) {
-        HIPCHK(launch_prefill_tail(row, hidden[hiddenIdx], dim, dState, pos0 + T - 1, tokens[T - 1], ropeRef(), stream));
+        HIPCHK(launch_set_state(dState, pos0 + T - 1, tokens[T - 1], 0, 0, ropeRef(), stream));
         rc = enqueueFinal(true);
         if (rc == 0) rc = publish(logits, n, dHistory, 1);
     } else {
-        PrefillEnd e{amaxVal, amaxIdx, 0, dState, pos0 + T, dHistory, vocabSize, ropeRef(), row, hidden[hiddenIdx], dim};
-        rc = enqueueFinal(true, row, &e.nparts);
+        PrefillEnd e{amaxVal, amaxIdx, 0, dState, pos0 + T, dHistory, vocabSize, ropeRef()};
+        rc = enqueueFinal(true, &e.nparts);
         if (rc == 0) HIPCHK(launch_publish_prefill(publishParams(logits, n), e, stream));
     }
     if (rc) return rc;

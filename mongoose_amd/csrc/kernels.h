@@ -189,13 +189,12 @@ inline int publish_slice_floats(int n) { const int per = (n + PUBLISH_MAX_SLICES
 inline int publish_slices(int n) { return n > 0 ? (n + publish_slice_floats(n) - 1) / publish_slice_floats(n) : 1; }
 hipError_t launch_publish(const PublishParams& p, hipStream_t s);
 // The same at the end of a prefill, whose lm_head has left its argmax partials: one more workgroup (and flag, behind the
-// slices') picks the greedy token, hands it over as the only int, and leaves the step state, the history's first entry, the
-// RoPE row and the hidden buffer as the step after needs them.  Its flag is the first where there are no slices (n = 0).
+// slices') picks the greedy token, hands it over as the only int, and leaves the step state, the history's first entry and the
+// RoPE row as the step after needs them.  Its flag is the first where there are no slices (n = 0).
 struct PrefillEnd {
     const float* pv; const int* pi; int nparts;
     StepState* state; int pos; int* history; int vocab;      // pos: of the next token
     RopeCur rope;
-    const float* row; float* hidden; int dim;                // the last position's row
 };
 hipError_t launch_publish_prefill(const PublishParams& p, const PrefillEnd& e, hipStream_t s);
 // Page-locked host memory -> device memory, up to three pieces in one launch (16-byte aligned on both sides; a length need
@@ -204,8 +203,6 @@ struct HostPieces { const void* src[3]; void* dst[3]; size_t bytes[3]; int n; };
 hipError_t launch_host_pieces(const HostPieces& p, hipStream_t s);
 // n words of page-locked host memory -> device memory.
 hipError_t launch_take_words(const unsigned* src, unsigned* dst, int n, hipStream_t s);
-// The last row of a prefill -> the hidden buffer, and the step state for its lm_head (where that needs both).
-hipError_t launch_prefill_tail(const float* row, float* hidden, int dim, StepState* state, int pos, int token, RopeCur rope, hipStream_t s);
 
 // Stream gate for timing runs: waits for *flag != 0 (host-pinned) or limitTicks of the 100 MHz wall clock.
 hipError_t launch_gate(const int* flag, long long limitTicks, hipStream_t s);

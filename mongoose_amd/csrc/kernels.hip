@@ -1881,7 +1881,7 @@ hipError_t launch_publish(const PublishParams& p, hipStream_t s) {
     return hipGetLastError();
 }
 
-// With the argmax's last step, the state and the last row's copy as launches of their own, two dependent launches of 4 us each
+// With the argmax's last step and the state as launches of their own, two dependent launches of 4 us each
 // stood between the lm_head and this one.
 __global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, PrefillEnd e, int per, int slices) {
     if (blockIdx.x < PUBLISH_WGS) {
@@ -1893,7 +1893,6 @@ __global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, Pr
         int idx = INT_MAX;
         for (int i = threadIdx.x; i < e.nparts; i += WG) argmax_pick(v, idx, e.pv[i], e.pi[i]);
         copy_rope_row(e.rope, e.pos);
-        for (int i = threadIdx.x; i < e.dim; i += WG) e.hidden[i] = e.row[i];
         wave_argmax(v, idx);
         if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
         __syncthreads();
@@ -1952,19 +1951,6 @@ __global__ void take_words_kernel(const unsigned* src, unsigned* dst, int n) {
 hipError_t launch_take_words(const unsigned* src, unsigned* dst, int n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(take_words_kernel, dim3((unsigned)((n + WG - 1) / WG)), dim3(WG), 0, s, src, dst, n);
-    return hipGetLastError();
-}
-
-__global__ void prefill_tail_kernel(const float* row, float* hidden, int dim, StepState* state, int pos, int token, RopeCur rope) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < dim) hidden[i] = row[i];
-    if (blockIdx.x == 0) {
-        copy_rope_row(rope, pos);
-        if (threadIdx.x == 0) { state->pos = pos; state->token = token; state->count = 0; state->nPrompt = 0; }
-    }
-}
-hipError_t launch_prefill_tail(const float* row, float* hidden, int dim, StepState* state, int pos, int token, RopeCur rope, hipStream_t s) {
-    hipLaunchKernelGGL(prefill_tail_kernel, dim3((unsigned)((dim + WG - 1) / WG)), dim3(WG), 0, s, row, hidden, dim, state, pos, token, rope);
     return hipGetLastError();
 }
 

@@ -290,3 +290,36 @@ def test_tiled_prefill(hip, s, fmt, kv_f16, pos0, rows, kernels):
     rc, _ = m.hip.DecodeToken(int(toks[-1]), pos0 + rows, after)
     assert rc == 0 and H.rel_err(after, want[1]) < bar
     m.close()
+
+
+@pytest.mark.parametrize("s,fmt,kv_f16,pos0,rows,attention", [
+    (H.with_layers(configs.TOY, 3), "q8", False, 0, 1, "few_attention_kernel"), (H.with_layers(configs.QWEN, 2), "q8", False, 300, 33, "few_attention_kernel"),
+    (H.with_layers(configs.QWEN_Q4, 2), "q4_0", True, 20, 16, "few_attention_kernel"), (MINI, "q8", True, 127, 2, "few_attention_kernel"),
+    (ODD, "q8", False, 0, 1505, "prefill_attn_kernel"), (ODD, "q4_0", True, 3, 1505, "prefill_attn_kernel"),
+    (H.with_layers(configs.TOY, 1), "q8", False, 0, 18, "few_attention_kernel")], ids=lambda v: getattr(v, "name", None))
+def test_last_layer_for_the_last_position(hip, s, fmt, kv_f16, pos0, rows, attention):
+    """Behind its cache rows the last of several layers runs for the last position alone, by the decode step's launches: logits, the
+    hidden buffer (whose bar is that of the logits: an element is off by what two bf16 terms leave, 2^-16, over the layers) and the
+    token behind it, against the same tokens one by one."""
+    m = H.Model(s, seed=rows, maxSeq=pos0 + rows + 2, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
+    toks = m.prompt(pos0 + rows + 1)
+    ref, after, got = (np.empty(s.vocab, np.float32) for _ in range(3))
+    m.hip.SetExecMode(1)                                       # (a token's last row stays in the hidden buffer)
+    for pos in range(pos0 + rows):
+        rc, nref = m.hip.DecodeToken(int(toks[pos]), pos, ref if pos == pos0 + rows - 1 else None)
+        assert rc == 0, E.last_error()
+    href = m.hip.ExportHidden().copy()
+    assert m.hip.DecodeToken(int(toks[-1]), pos0 + rows, after)[0] == 0
+    assert m.hip.ResetKV() == 0
+    for pos in range(pos0):
+        assert m.hip.DecodeToken(int(toks[pos]), pos)[0] == 0
+    out = []
+    names = H.launched(lambda: out.append(m.hip.Prefill(toks[pos0:pos0 + rows], pos0, wantLogits=True)))
+    rc, nxt, logits, _ = out[0]
+    assert rc == 0, E.last_error()
+    assert sum(attention in n for n in names) == max(1, s.nLayers - 1) and any("attn_decode" in n for n in names) == (s.nLayers > 1), names
+    bar = 1e-3 if kv_f16 else 1e-4
+    assert H.rel_err(logits, ref) < bar and nxt == nref
+    assert H.rel_err(m.hip.ExportHidden(), href) < bar
+    assert m.hip.DecodeToken(int(toks[-1]), pos0 + rows, got)[0] == 0 and H.rel_err(got, after) < bar
+    m.close()
