@@ -60,10 +60,13 @@ struct FewGemmParams {
 };
 hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, size_t wsBytes, hipStream_t s);
 
+// What the launches behind an attention launch multiply T rows by, in their order (launch_few_rows: W1 and W2 where the mode has them,
+// N1 their rows): its idle CUs read it into the L2s.
+struct FewNext { FewMode mode; const void* W0; const void* W1; const void* W2; int N, N1, K, q4; };
 // Causal attention of T query rows (rotated) at positions pos0 .. over the cache rows [0, pos0 + T), all products and sums
 // in fp32; the result goes out as the split the output projection reads.
 hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
                                 unsigned short* ext, int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4,
-                                hipStream_t s);
+                                const FewNext* next, int nNext, int terms, hipStream_t s);
 
 }  // namespace mg

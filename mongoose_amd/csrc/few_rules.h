@@ -24,6 +24,24 @@ constexpr int few_last_chunk(int K) { return K < 64 ? 0 : (K >> 6) - 1; }
 constexpr int few_own_scale(int K) { return K < 64 ? 1 : 0; }
 constexpr long long few_scales_at(int row, int K) { return (long long)row * (K >> 5) - few_own_scale(K); }
 
+// ---- weights read ahead of the launches that multiply them (few_rows.hip) ----
+// A region is a plane of a matrix (rows of int8 weights or of nibbles, or fp16 scales; `bytes` in all): its tiles below `tiles`, `run`
+// bytes each, of which tile t is wanted on XCD (t + tile0) mod 8.  per: 0, or the 16-row blocks of half a head, of which tile t is
+// block t % per in head t / per (base: the first or the second halves').  run, bytes: multiples of 16.
+struct FewRegion { const char* base; unsigned run, bytes; int tiles, tile0, per; };
+// What an XCD's workgroups read of it, in pieces of a KB, and where a lane's 16 bytes of piece p are.  (The last piece of a tile
+// reads the tile's end again, a tile past the matrix's end the matrix's.)
+constexpr unsigned few_ahead_per(const FewRegion& r) { return (r.run + 1023) >> 10; }
+constexpr unsigned few_ahead_pieces(const FewRegion& r, int xcd) {
+    const int t0 = (xcd - r.tile0) & 7;
+    return t0 < r.tiles ? ((unsigned)(r.tiles - t0 + 7) >> 3) * few_ahead_per(r) : 0;
+}
+constexpr unsigned few_ahead_at(const FewRegion& r, int xcd, unsigned p, int lane) {
+    const unsigned i = p / few_ahead_per(r), t = (unsigned)((xcd - r.tile0) & 7) + 8 * i, in = ((p - i * few_ahead_per(r)) << 10) + (unsigned)lane * 16;
+    const unsigned at = (r.per ? t / r.per * 2 * r.per + t % r.per : t) * r.run + (in < r.run - 16 ? in : r.run - 16);
+    return at < r.bytes - 16 ? at : r.bytes - 16;
+}
+
 // ---- which products take the integer form (few_gemm.hip) ----
 // Eight waves sum a run of K each, whole chunks of 64, of products of two signed bytes in 32 bits.  Past this K a run of them
 // could exceed those (K = 1,048,064 is the last that cannot); the tiled kernel's fp32 sums take any.

@@ -95,3 +95,52 @@ def test_the_faster_path_is_taken(tmp_path, shape, q4, rows, pos0, few, tiled):
     out = _run(tmp_path, '#include "few_rules.h"\n#include <cstdio>\nint main() { std::puts(mg::few_rows_pay(%d, %d, %d, %d, %d, %d, %d != 0) ? "few" : "tiled"); }'
                % (rows, pos0, *shape, q4))
     assert out.strip() == ("few" if few < tiled else "tiled")
+
+
+def test_reading_ahead_covers_the_tiles_and_stays_inside(tmp_path):
+    """Regions as an attention launch forms them (whole and partial matrices, last tiles cut off by the matrix's end, halves of heads
+    of 64 and 128, both formats' planes, rows of 32 weights up): every 16 bytes of a tile are read on the XCD that the tile's
+    workgroup will run on, and nothing outside the plane is."""
+    out = _run(tmp_path, r"""
+#include "few_rules.h"
+#include <cstdio>
+#include <vector>
+using namespace mg;
+int walk(unsigned row, int N, int rows, int tiles, int tile0, int per, int half) {
+    const unsigned run = rows * row, skip = half ? per * run : 0;
+    FewRegion r{nullptr, run, N * row - skip, tiles, tile0, per};
+    std::vector<int> by((N * row + 15) / 16, -1);
+    for (int x = 0; x < 8; x++)
+        for (unsigned p = 0; p < few_ahead_pieces(r, x); p++)
+            for (int lane = 0; lane < 64; lane++) {
+                const unsigned at = skip + few_ahead_at(r, x, p, lane);
+                if (at % 16 || at + 16 > N * row) return 1;
+                if (by[at / 16] < 0) by[at / 16] = x;
+            }
+    for (int t = 0; t < tiles; t++) {
+        const unsigned first = (per ? t / per * 2 * per + t % per + (half ? per : 0) : t) * rows;
+        for (unsigned b = first * row; b < (first + rows) * row && b < N * row; b += 16)
+            if (by[b / 16] != ((t + tile0) & 7)) return 2;
+    }
+    return 0;
+}
+int main() {
+    for (int K : {32, 96, 448, 896, 4864})
+        for (int div : {1, 2, 16})                         // bytes of a row: int8, nibbles, scales
+            for (int N : {64, 128, 200, 896, 1000}) {
+                const unsigned row = K / div;
+                for (int rows : {16, 32, 64}) {
+                    const int tiles = (N + rows - 1) / rows;
+                    for (int n : {tiles, tiles / 8 * 8})
+                        if (int e = n ? walk(row, N, rows, n, 0, 0, 0) : 0) { std::printf("K %d / %d N %d rows %d tiles %d: %d\n", K, div, N, rows, n, e); return 0; }
+                }
+                for (int hd : {64, 128})
+                    if (N % hd == 0)
+                        for (int tile0 : {0, 28, 3})
+                            for (int half : {0, 1})
+                                if (int e = walk(row, N, 16, N / 32, tile0, hd / 32, half)) { std::printf("K %d / %d N %d heads of %d: %d\n", K, div, N, hd, e); return 0; }
+            }
+    std::puts("ok");
+}
+""")
+    assert out == "ok\n", out
