@@ -53,6 +53,7 @@ constexpr int FLOW_TILE = 128;         // positions of an attention tile: one wo
 struct FlowGeometry {
     int stride;
     int offQ, offKc, offVc, offPacc, offPm, offPl, offX1, offM, offX2, offAttn;
+    int offMl;       // (maximum, sum) of a split's head beside every 16-byte piece of its accumulator, for the variants that merge by them
     int smax;
     int gqa;         // 1: an attention workgroup per (KV head, split) taking all its query heads; 0: per (query head, split)
 };
@@ -67,7 +68,7 @@ constexpr int FLOW_TRACE_SLOTS = 11;
 #define FLOW_TRACE_NAMES "layer-top", "qkv-input-staged", "qkv-done", "q-k-v-rows-in", "attention-done", "attention-merged", \
                          "wo-done", "gate-up-input-staged", "gate-up-done", "down-input-staged", "down-done"
 
-constexpr int FLOW_MANY_SPLITS = 6;      // see launch_flow_layers
+constexpr int FLOW_MANY_SPLITS = 6, FLOW_MANY_SPLITS_Q4 = 4;      // see launch_flow_layers
 struct FlowParams {
     const FlowLayer* layers;     // indexed by layer
     int l0, l1;                  // layers [l0, l1)
@@ -96,7 +97,7 @@ struct FlowParams {
     int nTokens;                 // 0: layers [l0, l1) of one step, hidden in and out; n >= 1: token mode -- n whole tokens from the
                                  // device state on (all layers; xchg holds two halves and the argmax exchange; state != NULL)
     const FlowTail* tail;        // token mode
-    int manySplits;              // 1: a position of this launch has FLOW_MANY_SPLITS KV splits or more (the variant that shares their merge out)
+    int mostSplits;              // KV splits at the launch's last position (0: not known); from some on a variant that shares their merge out
     int gqaCode;                 // geo.gqa only: 1 = a position of this launch may need the grouped attention (the variant that can do
                                  // it is launched); 0 = none does (positions below nCompute / nHeads tiles): the plain variant, which
                                  // is faster there, runs on the same geometry and reports a position past its reach as error 3

@@ -13,6 +13,7 @@
 // own in the same fixed order, so with all workgroups resident every wait ends; every wait is bounded by
 // a time limit all the same, after which the workgroup stops waiting (results are then garbage and
 // *err is set, which the host checks).
+#include <algorithm>
 #include <cstddef>
 #include "flow.h"
 #include "device_util.h"
@@ -240,6 +241,25 @@ __device__ __forceinline__ void poll_ml(const float* const (&pm)[PB], const floa
                      : "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(l[0]), "=&v"(l[1]), "=&v"(l[2])
                      : "v"(pm[0]), "v"(pm[1]), "v"(pm[2]), "v"(pl[0]), "v"(pl[1]), "v"(pl[2]) : "memory");
         const unsigned missing = unset1(m[0]) | unset1(l[0]) | (n > 1 ? unset1(m[1]) | unset1(l[1]) : 0u) | (n > 2 ? unset1(m[2]) | unset1(l[2]) : 0u);
+        if (!missing || w.dead) break;
+        if (!timing) { timing = true; t0 = wall_clock64(); }
+        else if (wall_clock64() - t0 > w.limit) { w.fail(); break; }
+    }
+}
+// Accumulator pieces of up to PB KV splits, each with its head's maximum and sum, all in one round trip.
+typedef float f2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void poll_pairs(const f4* const (&pa)[PB], const f2* const (&pq)[PB], f4 (&a)[PB], f2 (&q)[PB], int n, Waiter& w) {
+    static_assert(PB == 3, "three splits a round");
+    long long t0 = 0;
+    bool timing = false;
+    for (;;) {
+        asm volatile("global_load_dwordx4 %0, %6, off sc1\n\tglobal_load_dwordx4 %1, %7, off sc1\n\tglobal_load_dwordx4 %2, %8, off sc1\n\t"
+                     "global_load_dwordx2 %3, %9, off sc1\n\tglobal_load_dwordx2 %4, %10, off sc1\n\tglobal_load_dwordx2 %5, %11, off sc1\n\t"
+                     "s_waitcnt vmcnt(0)"
+                     : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2])
+                     : "v"(pa[0]), "v"(pa[1]), "v"(pa[2]), "v"(pq[0]), "v"(pq[1]), "v"(pq[2]) : "memory");
+        const unsigned missing = unset4(a[0]) | unset1(q[0].x) | unset1(q[0].y) | (n > 1 ? unset4(a[1]) | unset1(q[1].x) | unset1(q[1].y) : 0u) |
+                                 (n > 2 ? unset4(a[2]) | unset1(q[2].x) | unset1(q[2].y) : 0u);
         if (!missing || w.dead) break;
         if (!timing) { timing = true; t0 = wall_clock64(); }
         else if (wall_clock64() - t0 > w.limit) { w.fail(); break; }
@@ -587,12 +607,12 @@ constexpr int NID = 8 / FWAVES;    // down rows a wave holds in flight
 //      addresses, trip counts and divisions fold (0.5B shape: 0.3294 -> 0.3231 ms a token).  Bit 8: the caches hold fp16 rows;
 //      bit 16: the launch runs whole tokens (FlowParams::nTokens > 0).  Same formulas over the same rows; results agree with
 //      the other variants' to rounding (the compiler contracts and schedules differently).  launch_flow_layers picks them.
-struct FlowFixedShape { int dim, kvDim, ffn, nHeads, nKVHeads, headDim, downSplit, dedicated; };
+struct FlowFixedShape { int dim, kvDim, ffn, nHeads, nKVHeads, headDim, downSplit, dedicated, pairs; };
 __host__ __device__ constexpr FlowFixedShape flow_fixed_shape(int fix) {
-    return fix == 1 ? FlowFixedShape{896, 128, 4864, 14, 2, 64, 1, 1}      // Qwen2.5-0.5B
-         : fix == 2 ? FlowFixedShape{2048, 256, 5632, 32, 4, 64, 0, 0}     // TinyLlama-1.1B
-         : fix == 3 ? FlowFixedShape{4096, 1024, 14336, 32, 8, 128, 0, 0}  // Llama-3-8B
-                    : FlowFixedShape{0, 0, 0, 0, 0, 0, 0, 0};
+    return fix == 1 ? FlowFixedShape{896, 128, 4864, 14, 2, 64, 1, 1, 1}     // Qwen2.5-0.5B
+         : fix == 2 ? FlowFixedShape{2048, 256, 5632, 32, 4, 64, 0, 0, 0}    // TinyLlama-1.1B
+         : fix == 3 ? FlowFixedShape{4096, 1024, 14336, 32, 8, 128, 0, 0, 0} // Llama-3-8B
+                    : FlowFixedShape{0, 0, 0, 0, 0, 0, 0, 0, 0};
 }
 // The part of a layer's exchange area whose layout follows from the sizes alone: q, current K row, current V row, hidden
 // after attention, SwiGLU vector, layer output, merged attention output, and where the KV splits' partial slots begin.
@@ -656,6 +676,10 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     constexpr bool FX = (FIX & 31) != 0;
     constexpr bool SHARED = (FIX & 32) != 0;           // launches that reach many KV splits, vectors of at most 1,024 elements: see the merge
     constexpr FlowFixedShape FS = flow_fixed_shape(FIX & 7);
+    // A split's maximum and sum beside every piece of its accumulator, a line a head written once: a round of the merge is one round
+    // trip, not two.  Twice the lines to poll, which longer vectors lose by (1.1B at 300 positions 397 -> 401.5 us a token), and the
+    // variants with their sizes in registers do not gain (the toy shape 54.3 -> 54.4 at 200, 60.1 -> 60.6 at 1,200).
+    constexpr bool PAIRS = SHARED && FS.pairs != 0;
     static_assert(!FX || FS.headDim == HD, "the fixed shape's head size is the variant's");
     int dim = FX ? FS.dim : p.dim, kvDim = FX ? FS.kvDim : p.kvDim, ffn = FX ? FS.ffn : p.ffn;
     const int nHeadsV = FX ? FS.nHeads : p.nHeads, nKVHeadsV = FX ? FS.nKVHeads : p.nKVHeads;
@@ -1182,6 +1206,11 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                     const f4 r = {tg_sum(fmaf(w1, x1[j].x, w0 * x0[j].x)) * il, tg_sum(fmaf(w1, x1[j].y, w0 * x0[j].y)) * il,
                                                   tg_sum(fmaf(w1, x1[j].z, w0 * x0[j].z)) * il, tg_sum(fmaf(w1, x1[j].w, w0 * x0[j].w)) * il};
                                     if (lane < 16) stx4(reinterpret_cast<f4*>(X + G.offPacc + (size_t)split * dim + h0 * HD) + i + 16 * j, r);
+                                    if (PAIRS && nsplit > 1 && lane < 16) {
+                                        const f2 ml = {canon(mg_), canon(lg)};
+                                        asm volatile("global_store_dwordx2 %0, %1, off sc1" : :
+                                                     "v"(reinterpret_cast<f2*>(X + G.offMl + (size_t)split * (dim >> 1) + h0 * (HD / 2)) + i + 16 * j), "v"(ml) : "memory");
+                                    }
                                 }
                                 if (lane == 0) { stx(X + G.offPm + split * nHeadsV + h0, mg_); stx(X + G.offPl + split * nHeadsV + h0, lg); }
                             }
@@ -1305,7 +1334,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                         __syncthreads();
                         {
                             const int nsplit = pos / TILE + 1;
-                            const int ns = nsplit < G.smax ? nsplit : G.smax;
+                            const int ns = min(nsplit, PAIRS ? min(G.smax, (nC + nHeadsV - 1) / nHeadsV) : G.smax);      // (a position past the variant's reach stays inside the area)
                             if (!(GQA && CBD == 2) && ns == 1) {                         // uniform in the launch
                                 for (int i = tid; i < (dim >> 2); i += FWG) a4[slot4<Q4>(i, nchD)] = tof4(poll4(reinterpret_cast<const f4*>(X + G.offPacc) + i, wt));
                             } else {
@@ -1319,7 +1348,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                             // layers of 768, Q4_0, at 200 79.6 -> 83.7), and grouped attention has few splits here.  Fewer splits are merged as in
                             // the other variants, one after the other, also in such a launch.
                             const int nPieces = dim >> 2;
-                            const int NG = SHARED && ns >= FLOW_MANY_SPLITS ? min(max(1, FWG / nPieces), (ns + PB - 1) / PB) : 1;
+                            const int NG = SHARED && ns >= (PAIRS ? PB + 1 : FLOW_MANY_SPLITS) ? min(max(1, FWG / nPieces), (ns + PB - 1) / PB) : 1;
                             for (int ii = tid; ii < nPieces * NG; ii += FWG) {
                                 const int g = NG == 1 ? 0 : ii / nPieces, i = ii - g * nPieces, h = (i * 4) / HD;
                                 float M = -INFINITY, den = 0.f;
@@ -1342,7 +1371,26 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                 // were one more per split: 4 % of the step at 1000 positions).
                                 const float* idle1 = reinterpret_cast<const float*>(wt.idle);
                                 const int cnt = NG == 1 ? ns : (ns - g + NG - 1) / NG;          // this group's splits: g, g + NG, ...
-                                if constexpr (!SHARED) {
+                                if constexpr (PAIRS) {
+                                    const f2* idle2p = reinterpret_cast<const f2*>(wt.idle);
+                                    for (int k0 = 0; k0 < cnt; k0 += PB) {
+                                        const int nbt = min(PB, cnt - k0);
+                                        const f4* pa[PB];
+                                        const f2* pq[PB];
+                                        f4 a[PB];
+                                        f2 q[PB];
+#pragma unroll
+                                        for (int u = 0; u < PB; u++) {
+                                            const bool on = u < nbt;
+                                            const int sp = g + (k0 + u) * NG;
+                                            pa[u] = on ? reinterpret_cast<const f4*>(X + G.offPacc + (size_t)sp * dim) + i : wt.idle;
+                                            pq[u] = on ? reinterpret_cast<const f2*>(X + G.offMl + (size_t)sp * (dim >> 1)) + i : idle2p;
+                                        }
+                                        poll_pairs(pa, pq, a, q, nbt, wt);
+#pragma unroll
+                                        for (int u = 0; u < PB; u++) if (u < nbt) mergeIn(a[u], q[u].x, q[u].y);
+                                    }
+                                } else if constexpr (!SHARED) {
                                 for (int k0 = 0; k0 < cnt; k0 += PB) {
                                     const int nbt = min(PB, cnt - k0);
                                     const f4* pa[PB];
@@ -1897,6 +1945,13 @@ FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads
     int o = g.offPacc + up64(g.smax * dim);
     g.offPm = o; o += up64(g.smax * nHeads);
     g.offPl = o; o += up64(g.smax * nHeads);
+    // (the plain variant alone merges by the pairs: of a grouped geometry the splits that one reaches)
+    g.offMl = o;
+    for (int k = 1; k <= 3; k++) {
+        const FlowFixedShape f = flow_fixed_shape(k);
+        if (f.pairs && f.dim == dim && f.kvDim == kvDim && f.ffn == ffn && f.nHeads == nHeads && f.nKVHeads == nKVHeads && f.headDim == headDim)
+            o += up64((g.gqa ? std::min(g.smax, (grid + nHeads - 1) / nHeads) : g.smax) * (dim / 2));
+    }
     g.stride = o;
     return g;
 }
@@ -1966,7 +2021,13 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         if (p.trace) hipLaunchKernelGGL((flow_layers_kernel<HDv, CBv, RGv, GQv, Q4v, true, FXv>), dim3(grid), dim3(FWG), lds, s, p); \
         else hipLaunchKernelGGL((flow_layers_kernel<HDv, CBv, RGv, GQv, Q4v, false, FXv>), dim3(grid), dim3(FWG), lds, s, p); } while (0)
     if (fix == 1 && !gqa && !p.kvHalf) {
-        if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 1);
+        // Many splits, shared out among groups of threads and merged by pairs (see PAIRS); us a token without / with, Q8 at 600 (five
+        // splits) 340.1 / 340.0, 900 371.7 / 360.1, 1,300 400.0 / 373.6, 1,900 439.9 / 395.1, but at 20 291.8 / 300.3 and 320 316.3 / 327.9 for
+        // the registers the code costs; Q4_0 at 320 (three) 317.0 / 320.4, 450 332.8 / 327.4, 900 369.6 / 356.1, 1,900 440.8 / 390.1.
+        if (p.mostSplits >= (p.q4 ? FLOW_MANY_SPLITS_Q4 : FLOW_MANY_SPLITS)) {
+            if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 33);
+            else FLOW_LAUNCH_F(64, 1, false, false, false, 33);
+        } else if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 1);
         else if (p.nTokens > 0 && !p.trace)             // (whole tokens as a constant: 0.3140 -> 0.3130 ms a token; slower in the other variants)
             hipLaunchKernelGGL((flow_layers_kernel<64, 1, false, false, false, false, 17>), dim3(grid), dim3(FWG), lds, s, p);
         else FLOW_LAUNCH_F(64, 1, false, false, false, 1);
@@ -1977,7 +2038,7 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         else FLOW_LAUNCH_F(128, 2, true, false, false, 3);
     } else if (fix == 3 && !p.q4 && gqa) {              // fp16 K / V rows at a long context
         FLOW_LAUNCH_F(128, 2, true, true, false, 11);
-    } else if (p.manySplits && !gqa && !wide) {
+    } else if (p.mostSplits >= FLOW_MANY_SPLITS && !gqa && !wide) {
         // Six splits: hidden size 768, six layers, Q8, at 600 positions (five) 82.9 us a token with / 83.0 without, Q4_0 87.9 / 86.0,
         // the toy shape 56.7 / 57.8; at 1,200 (ten) 88.5 / 95.3, 93.2 / 98.0 and 59.0 / 66.8.
         if (p.headDim == 64) { if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 32); else FLOW_LAUNCH_F(64, 1, false, false, false, 32); }

@@ -1015,7 +1015,7 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
         if (!st) posMax = posImm;
         else if (statePosHost >= 0) posMax = (long long)statePosHost + (nTokens > 0 ? nTokens - 1 : 0);
         p.gqaCode = (posMax < 0 || (long long)nHeads * (posMax / FLOW_TILE + 1) > flowCompute) ? 1 : 0;
-        p.manySplits = posMax / FLOW_TILE + 1 >= FLOW_MANY_SPLITS ? 1 : 0;
+        p.mostSplits = posMax < 0 ? 0 : (int)(posMax / FLOW_TILE) + 1;
         p.generic = flowGeneric ? 1 : 0;
         // the half of the exchange area a run of whole tokens starts in has to be as a reset leaves it: the launch before
         // left the half of its last position's successor so (DecodeToken at consecutive positions resets nothing)

@@ -303,6 +303,37 @@ def test_variants_with_a_shape_compiled_in_change_nothing(hip, name, positions, 
     m.close()
 
 
+@pytest.mark.parametrize("fmt,maxSeq,positions,first", [
+    ("q8", 2048, (639, 640, 767, 768, 1151, 2047), 615), ("q8", 4000, (640, 1024, 2047, 2048), 2021), ("q4_0", 2048, (511, 512, 640, 1536, 2047), 485)])
+def test_many_splits_of_a_known_shape(hip, fmt, maxSeq, positions, first):
+    """0.5B shape: from six KV splits on (position 640; Q4_0 four, 512) a variant of its own shares their merge out and reads a
+    split's maximum and sum beside its accumulator.  At the edges of rounds and splits and at the last position of the plain
+    attention (sixteen splits, with a geometry laid out for the grouped one as well), against the variants whose sizes come with
+    the launch: the same sums in another order of a few dozen terms, 1e-6 of the largest logit, ten times that is asked for.  A
+    run of tokens across the line gives the same tokens."""
+    s = H.with_layers(configs.QWEN if fmt == "q8" else configs.QWEN_Q4, 2)._replace(vocab=2048)
+    m = H.Model(s, seed=43, maxSeq=maxSeq, eng=hip, oracle=False, fmt=fmt)
+    toks = m.prompt(max(positions) + 1)
+    outs = {}
+    for generic in (0, 1):
+        assert m.hip.SetFlowGeneric(generic) == 0 and m.hip.ResetKV() == 0
+        for p in range(0, max(positions), 500):
+            assert m.hip.Prefill(toks[p:min(max(positions), p + 500)], p)[0] == 0, E.last_error()
+        outs[generic] = []
+        for pos in positions:
+            logits = np.empty(s.vocab, np.float32)
+            rc, nxt = m.hip.DecodeToken(int(toks[pos]), pos, logits)
+            assert rc == 0 and m.hip.FlowInUse(), E.last_error()
+            outs[generic].append((nxt, logits))
+        rc, run = m.hip.GeneratePrefill(toks[:first], 50)
+        assert rc == 0, E.last_error()
+        outs[generic].append(run.tolist())
+    assert outs[0][-1] == outs[1][-1]
+    for (n0, l0), (n1, l1) in zip(outs[0][:-1], outs[1][:-1]):
+        assert n0 == n1 and H.rel_err(l0, l1) < 1e-5
+    m.close()
+
+
 def test_heads_of_128_grouped_kv(hip):
     """Llama-3-8B attention geometry (32 query heads of 128 on 8 KV heads, dim 4096: rows of two chunks a lane), 2
     layers, FFN and vocabulary cut: 8 partial slots, tile 128."""
