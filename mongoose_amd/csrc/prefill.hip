@@ -613,8 +613,8 @@ __global__ __launch_bounds__(NT) void gemm_q8_bf16x2_kernel(GemmParams p) {
         for (int r = 0; r < BR; r++)
             if (bActive) *reinterpret_cast<int4*>(&sB[(bRow + (NT / WSEG) * r) * WSTRIDE + bSeg * 16]) = gB[r];
         if (Q4 && tid < BN) {
-            sD[tid * 2] = (float)__builtin_bit_cast(_Float16, gD[0]);
-            sD[tid * 2 + 1] = (float)__builtin_bit_cast(_Float16, gD[1]);
+            sD[tid * 2] = (float)__builtin_bit_cast(_Float16, gD[0]) * 0.0625f;
+            sD[tid * 2 + 1] = (float)__builtin_bit_cast(_Float16, gD[1]) * 0.0625f;
         }
         __syncthreads();
         if (step + 1 < stepEnd) MG_GEMM_GLOAD((step + 1) * BK);       // next tile in flight while this one is multiplied
@@ -634,13 +634,16 @@ __global__ __launch_bounds__(NT) void gemm_q8_bf16x2_kernel(GemmParams p) {
                     for (int h2 = 0; h2 < 2; h2++) {
                         const int e0 = 16 * h2 + 8 * (lane >> 5);
                         const int2 w = *reinterpret_cast<const int2*>(&sB[nrow * WSTRIDE + bl * 16 + (e0 & 8)]);
-                        const unsigned sh = h2 ? 4u : 0u;   // elements 16..31 are the high nibbles
-                        const unsigned n0v = ((unsigned)w.x >> sh) & 0x0f0f0f0fu, n1v = ((unsigned)w.y >> sh) & 0x0f0f0f0fu;
+                        // (elements 16..31 are the high nibbles.)  A nibble in the upper half of a byte, its highest bit
+                        // flipped, is (nibble - 8) * 16 as a signed byte, which converts in one instruction; sD is a
+                        // sixteenth of the scale.  (0.5B shape, 700 rows 4,294 -> 4,136 us)
+                        const unsigned sh = h2 ? 0u : 4u;
+                        const int n0v = (int)((((unsigned)w.x << sh) & 0xf0f0f0f0u) ^ 0x80808080u), n1v = (int)((((unsigned)w.y << sh) & 0xf0f0f0f0u) ^ 0x80808080u);
                         uint4 u;
-                        u.x = pack_bf16_exact((float)(n0v & 0xff) - 8.0f, (float)((n0v >> 8) & 0xff) - 8.0f);
-                        u.y = pack_bf16_exact((float)((n0v >> 16) & 0xff) - 8.0f, (float)(n0v >> 24) - 8.0f);
-                        u.z = pack_bf16_exact((float)(n1v & 0xff) - 8.0f, (float)((n1v >> 8) & 0xff) - 8.0f);
-                        u.w = pack_bf16_exact((float)((n1v >> 16) & 0xff) - 8.0f, (float)(n1v >> 24) - 8.0f);
+                        u.x = pack_bf16_exact((float)(signed char)(n0v), (float)(signed char)(n0v >> 8));
+                        u.y = pack_bf16_exact((float)(signed char)(n0v >> 16), (float)(n0v >> 24));
+                        u.z = pack_bf16_exact((float)(signed char)(n1v), (float)(signed char)(n1v >> 8));
+                        u.w = pack_bf16_exact((float)(signed char)(n1v >> 16), (float)(n1v >> 24));
                         b[h2] = __builtin_bit_cast(bf16x8_t, u);
                     }
 #pragma unroll
