@@ -456,12 +456,14 @@ static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
 
 // The tile of a launch (16 MT activation rows x 16 NB weight rows a workgroup): the one with the shortest time by a model of
 // a workgroup's nanoseconds -- the bytes it pulls (a CU gets some 80 a nanosecond, whether they come from its L2 or from
-// beyond it), the weights it converts (no other workgroup's conversions serve it: a Q4_0 weight costs three int8 ones), the
-// sums it exchanges -- times the workgroups of the busiest CU, a quarter of which overlap evenly over the chip.  Short rows
-// go through two workgroups a CU at once; tiles of more than four blocks take too many registers for that (1.5).  The
-// constants are a fit to every tile of gate | up and of Wo + down at 64 to 512 rows of the three benchmark shapes, both
-// formats: what it picks is within 3 % of a layer of the best one at all of them, and at 16 and 37 rows.  (Bytes alone and 2.5 us a round of 256
-// workgroups: 301 rows of the 0.5B shape 88 -> 78 us a layer, Q4_0 111 -> 86; 1.1B Q4_0 238 -> 180.)
+// beyond it), the weights it converts (no other workgroup's conversions serve it: a Q4_0 weight costs four int8 ones), its
+// matrix instructions, the sums it exchanges -- times the workgroups of the busiest CU, a fifth of which overlap evenly over the
+// chip.  A launch is made up to a multiple of eight weight tiles, and those count: they end at once, but until then another CU has
+// two workgroups (Q4_0 0.5B shape, down at 400 rows: 252 workgroups of 3 x 2, 288 launched, 11 us longer than 196 of 4 x 2).  Short rows
+// go through two workgroups a CU at once; tiles of more than four blocks take too many registers for that (1.5), which matters where
+// there are two, and 128 weight rows at any number.  The constants are a fit to every tile of gate | up, Wo and down at 16 to 512
+// rows of the benchmark shapes, both formats: what it picks is within 2 % of a prefill of the best one at all of them (without matrix
+// instructions, made-up tiles and the line at one workgroup a CU 10 %: 0.5B shape, 301 rows 1,808 -> 1,718 us, Q4_0 400 rows 2,642 -> 2,310).
 struct FewTile { int mt, nb; };
 // With three terms an activation row is half as many bytes again, and a tile has at most FEW_MT3 row blocks.
 static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4, int terms) {
@@ -470,11 +472,12 @@ static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4
     double least = 1e30;
     for (int nb = nbFirst; nb <= nbLast; nb *= 2)
         for (int mt = 1; mt <= (terms == 3 ? FEW_MT3 : 4) && mt <= b16 && mt * nb <= 8; mt++) {
-            const double wgs = (double)((rowsN + 16 * nb - 1) / (16 * nb)) * ((b16 + mt - 1) / mt);
+            const int nTiles = (rowsN + 16 * nb - 1) / (16 * nb), mTiles = (b16 + mt - 1) / mt;
+            const double wgs = (double)nTiles * mTiles, launched = (double)((nTiles + 7) / 8 * 8) * mTiles;
             const double bytes = (32.0 * terms * mt + (q4 ? 9.0 : 16.0) * nb) * K;
-            double each = bytes / 80.0 + (q4 ? 0.74 : 0.225) * nb * K + 25.0 * mt * nb;
-            if (K <= 64 * 2 * FR_WAVES && mt * nb > 4) each *= 1.5;
-            const double cost = (0.75 * ceil(wgs / 256.0) + 0.25 * wgs / 256.0) * each;
+            double each = bytes / 80.0 + (q4 ? 0.9 : 0.225) * nb * K + 0.03 * terms * mt * nb * K + 160.0 * mt * nb;
+            if (K <= 64 * 2 * FR_WAVES && mt * nb > 4 && (nb > 4 || launched > 256)) each *= 1.5;
+            const double cost = (0.8 * ceil(launched / 256.0) + 0.2 * wgs / 256.0) * each;
             if (cost < least) { least = cost; best = FewTile{mt, nb}; }
         }
     return best;
