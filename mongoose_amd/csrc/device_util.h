@@ -162,14 +162,22 @@ __device__ __forceinline__ float dot_q4_half(int2 w, float d, const float4 (&av)
     q = (unsigned)w.y; s = dot4_nib(q & 0x0f0f0f0fu, av[1], s); s = dot4_nib((q >> 4) & 0x0f0f0f0fu, av[3], s);
     return fmaf(s, d, acc);
 }
-// The sum of a chunk's 16 activations, in the order every Q4_0 path uses.
-__device__ __forceinline__ float chunk_act_sum(const float4 (&av)[4]) {
-    float4 t;
-    t.x = (av[0].x + av[1].x) + (av[2].x + av[3].x);
-    t.y = (av[0].y + av[1].y) + (av[2].y + av[3].y);
-    t.z = (av[0].z + av[1].z) + (av[2].z + av[3].z);
-    t.w = (av[0].w + av[1].w) + (av[2].w + av[3].w);
-    return (t.x + t.y) + (t.z + t.w);
+// The same without the activations' sum, which takes as many additions as half of the products: a nibble in the upper half of a
+// byte, its highest bit flipped, is (nib - 8) * 16 as a signed byte, which converts in one instruction.  For the persistent
+// launch (flow.hip), whose phases are bound by their instructions (8B shape in Q4_0, six layers 340.5 -> 330.5 us a token, at 900 positions
+// 391 -> 383; 1.1B, eight layers 151.2 -> 150.2, at 600 169.9 -> 168.0); the separate launches wait for their loads instead and
+// are no faster by it (5632 x 2048 5.3 -> 5.7 us, 32000 x 2048 14.5 -> 14.9, 4096 x 14336 15.5 -> 14.9).  Its error against
+// a shadow of the same roundings is half that of dot_q4_half (two layers of three shapes: 7e-7 -> 3.5e-7), whose sum has to cancel.
+__device__ __forceinline__ int nib_bytes(unsigned q) {
+    int b = (int)((q & 0xf0f0f0f0u) ^ 0x80808080u);
+    asm("" : "+v"(b));                       // (the compiler otherwise takes every nibble out of q by itself)
+    return b;
+}
+__device__ __forceinline__ float dot_q4_half_signed(int2 w, float d, const float4 (&av)[4], float acc) {
+    float s = 0.f;
+    s = dot4_i8(nib_bytes((unsigned)w.x << 4), av[0], s); s = dot4_i8(nib_bytes((unsigned)w.x), av[2], s);
+    s = dot4_i8(nib_bytes((unsigned)w.y << 4), av[1], s); s = dot4_i8(nib_bytes((unsigned)w.y), av[3], s);
+    return fmaf(s, d * 0.0625f, acc);
 }
 
 // Element i of token tok's embedding row.  kind 0: int8 rows [vocab, dim] times the row's scale (a tied Q8 lm_head),

@@ -68,7 +68,7 @@ constexpr int FLOW_TRACE_SLOTS = 11;
 #define FLOW_TRACE_NAMES "layer-top", "qkv-input-staged", "qkv-done", "q-k-v-rows-in", "attention-done", "attention-merged", \
                          "wo-done", "gate-up-input-staged", "gate-up-done", "down-input-staged", "down-done"
 
-constexpr int FLOW_MANY_SPLITS = 6, FLOW_MANY_SPLITS_Q4 = 4;      // see launch_flow_layers
+constexpr int FLOW_MANY_SPLITS = 6;      // see launch_flow_layers
 struct FlowParams {
     const FlowLayer* layers;     // indexed by layer
     int l0, l1;                  // layers [l0, l1)

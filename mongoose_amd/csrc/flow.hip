@@ -488,10 +488,9 @@ __device__ __forceinline__ void dot_rows(const int4 (&wr)[NR][CB], const float4*
         if (c < nch) {
             const float4 av[4] = {a4[c], a4[nch + c], a4[2 * nch + c], a4[3 * nch + c]};
             if (Q4) {
-                const float asum = chunk_act_sum(av);
 #pragma unroll
                 for (int r = 0; r < NR; r++)
-                    acc[r] = dot_q4_half(make_int2(wr[r][i].x, wr[r][i].y), half_bits_to_float((unsigned short)wr[r][i].z), av, asum, acc[r]);
+                    acc[r] = dot_q4_half_signed(make_int2(wr[r][i].x, wr[r][i].y), half_bits_to_float((unsigned short)wr[r][i].z), av, acc[r]);
             } else {
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
@@ -526,7 +525,7 @@ __device__ __forceinline__ float dot_row_rng(const int4 (&wr)[CB], const float4*
         if (c < cHi) {
             const float4 av[4] = {a4[c], a4[nch + c], a4[2 * nch + c], a4[3 * nch + c]};
             if (Q4) {
-                acc = dot_q4_half(make_int2(wr[i].x, wr[i].y), half_bits_to_float((unsigned short)wr[i].z), av, chunk_act_sum(av), acc);
+                acc = dot_q4_half_signed(make_int2(wr[i].x, wr[i].y), half_bits_to_float((unsigned short)wr[i].z), av, acc);
             } else {
                 acc = dot4_i8(wr[i].x, av[0], acc); acc = dot4_i8(wr[i].y, av[1], acc);
                 acc = dot4_i8(wr[i].z, av[2], acc); acc = dot4_i8(wr[i].w, av[3], acc);
@@ -2023,8 +2022,8 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
     if (fix == 1 && !gqa && !p.kvHalf) {
         // Many splits, shared out among groups of threads and merged by pairs (see PAIRS); us a token without / with, Q8 at 600 (five
         // splits) 340.1 / 340.0, 900 371.7 / 360.1, 1,300 400.0 / 373.6, 1,900 439.9 / 395.1, but at 20 291.8 / 300.3 and 320 316.3 / 327.9 for
-        // the registers the code costs; Q4_0 at 320 (three) 317.0 / 320.4, 450 332.8 / 327.4, 900 369.6 / 356.1, 1,900 440.8 / 390.1.
-        if (p.mostSplits >= (p.q4 ? FLOW_MANY_SPLITS_Q4 : FLOW_MANY_SPLITS)) {
+        // the registers the code costs; Q4_0 at 320 (three) 317.0 / 320.4, 600 340.5 / 342.1, 900 369.9 / 356.2, 1,900 440.8 / 391.5.
+        if (p.mostSplits >= FLOW_MANY_SPLITS) {
             if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 33);
             else FLOW_LAUNCH_F(64, 1, false, false, false, 33);
         } else if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 1);
