@@ -1234,7 +1234,10 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                             // variant for many splits (eight layers of the 1.1B shape at 1,200 positions 204.2 us without, 206.1 with).
                             if (!(GQA && CBD == 2) && nsplit == 1) { const float il = __builtin_amdgcn_rcpf(lg); r.x *= il; r.y *= il; r.z *= il; r.w *= il; lg = 1.0f; }
                             stx4(reinterpret_cast<f4*>(X + G.offPacc + (size_t)split * dim + h * HD) + i, r);
-                            if (i == 0) {
+                            if (i == 0 && grouped) {
+                                const f2 ml = {canon(mg_), canon(lg)};
+                                asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(X + G.offPm + 2 * (h * G.smax + split)), "v"(ml) : "memory");
+                            } else if (i == 0) {
                                 stx(X + G.offPm + split * nHeadsV + h, mg_);
                                 stx(X + G.offPl + split * nHeadsV + h, lg);
                             }
@@ -1243,33 +1246,36 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                 }
 
                 if (grouped) {
-                    // Long contexts, tens of KV splits: merged once per head, by workgroup h for head h (every thread a 16-byte piece
-                    // and every eighth split, eight splits' loads in flight together, then combined through LDS), and handed on as
-                    // one vector -- every consumer merging all partials itself re-reads tens of KB per workgroup and layer.
+                    // Long contexts, tens of KV splits: merged once per head, by workgroup h for head h, and handed on as one vector -- every
+                    // consumer merging all partials itself re-reads tens of KB per workgroup and layer.  A thread takes a 16-byte piece of
+                    // every SG-th split, MBG of them at a time; the splits a wave holds meet in registers, the eight waves in LDS.  A head's
+                    // maxima and sums lie together, split after split (offPm, pairs), and only this workgroup polls them.  Bound by the round
+                    // trip after the last partial has landed and the chain of combines.  (With the heads' maxima of a split in one line that
+                    // every merging workgroup polled, threads without a second split asking for the last one again, and a chain of 32
+                    // groups in LDS a merge took 6 us, now 2.6: us a token at 1,300 / 3,900 positions, 1.1B 594 / 624 -> 524 / 568, 0.5B at
+                    // 2,600 480 -> 413, eight layers of 8B at 1,030 / 3,900 459 / 481 -> 445 / 471.)
                     if ((int)blockIdx.x < nHeadsV) {
-                        constexpr int P4 = HD / 4, SG = FWG / P4;          // pieces of a head, split groups (thread = piece x group)
+                        constexpr int P4 = HD / 4, SG = FWG / P4, MBG = 2;          // pieces of a head, split groups (thread = piece x group)
                         const int h = blockIdx.x, i = tid % P4, sg = tid / P4;
                         const int ns = min(pos / TILE + 1, G.smax);
                         const unsigned Xo = xoff + (unsigned)l * G.stride;
                         float M = -INFINITY, den = 0.f;
                         f4 num = {0.f, 0.f, 0.f, 0.f};
-                        constexpr int MBG = 4;
                         for (int s1 = sg; s1 < ns; s1 += SG * MBG) {
                             f4 a[MBG];
-                            float ms[MBG], ls[MBG];
+                            f2 ml[MBG];
                             long long t0w = 0;
                             bool timing = false;
                             for (;;) {
                                 unsigned missing = 0;
 #pragma unroll
                                 for (int j = 0; j < MBG; j++) {
-                                    const int sj = min(s1 + j * SG, ns - 1);
+                                    const int sj = s1 + j * SG < ns ? s1 + j * SG : s1;      // (past the end: the thread's own again, not a line others wait for)
                                     a[j] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (Xo + G.offPacc + (unsigned)sj * dim + h * HD + i * 4) * 4u, 0, 16));
-                                    ms[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrsrc, (Xo + G.offPm + sj * nHeadsV + h) * 4u, 0, 16));
-                                    ls[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrsrc, (Xo + G.offPl + sj * nHeadsV + h) * 4u, 0, 16));
+                                    ml[j] = __builtin_bit_cast(f2, __builtin_amdgcn_raw_buffer_load_b64(xrsrc, (Xo + G.offPm + 2 * (h * G.smax + sj)) * 4u, 0, 16));
                                 }
 #pragma unroll
-                                for (int j = 0; j < MBG; j++) missing |= unset4(a[j]) | unset1(ms[j]) | unset1(ls[j]);
+                                for (int j = 0; j < MBG; j++) missing |= unset4(a[j]) | unset1(ml[j].x) | unset1(ml[j].y);
                                 if (!missing || wt.dead) break;
                                 if (!timing) { timing = true; t0w = wall_clock64(); }
                                 else if (wall_clock64() - t0w > wt.limit) { wt.fail(); break; }
@@ -1278,27 +1284,35 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 #pragma unroll
                             for (int j = 0; j < MBG; j++) {
                                 if (s1 + j * SG < ns) {
-                                    const float Mn = fmaxf(M, ms[j]);
-                                    const float c = exp_neg(M - Mn), wgt = exp_neg(ms[j] - Mn);
-                                    den = den * c + wgt * ls[j];
+                                    const float Mn = fmaxf(M, ml[j].x);
+                                    const float c = exp_neg(M - Mn), wgt = exp_neg(ml[j].x - Mn);
+                                    den = den * c + wgt * ml[j].y;
                                     num.x = num.x * c + wgt * a[j].x; num.y = num.y * c + wgt * a[j].y;
                                     num.z = num.z * c + wgt * a[j].z; num.w = num.w * c + wgt * a[j].w;
                                     M = Mn;
                                 }
                             }
                         }
-                        mnum[tid] = tof4(num); mM[tid] = M; mden[tid] = den;              // (tid = sg * P4 + i)
+                        // over the wave's split groups: lanes P4 apart (a group without splits has M = -inf: weight 0)
+                        auto over = [&](float v) { if constexpr (HD == 64) return rows_sum(v); float u = v; row_swap32(v, u); return v + u; };
+                        const float Mw = rows_max(M), wgt = M == -INFINITY ? 0.f : exp_neg(M - Mw);
+                        num.x = over(num.x * wgt); num.y = over(num.y * wgt); num.z = over(num.z * wgt); num.w = over(num.w * wgt);
+                        den = over(den * wgt);
+                        if (lane < P4) mnum[wave * P4 + i] = tof4(num);
+                        if (lane == 0) { mM[wave] = Mw; mden[wave] = den; }
                         __syncthreads();
                         if (tid < P4) {
-                            float Mg = mM[tid];
-                            for (int g2 = 1; g2 < SG; g2++) Mg = fmaxf(Mg, mM[g2 * P4 + tid]);
+                            float Mg = mM[0];
+#pragma unroll
+                            for (int k = 1; k < FWAVES; k++) Mg = fmaxf(Mg, mM[k]);
                             float dn = 0.f;
                             f4 nm = {0.f, 0.f, 0.f, 0.f};
-                            for (int g2 = 0; g2 < SG; g2++) {
-                                const float wgt = exp_neg(mM[g2 * P4 + tid] - Mg);     // a group without splits has M = -inf: weight 0
-                                const float4 a = mnum[g2 * P4 + tid];
-                                dn = fmaf(wgt, mden[g2 * P4 + tid], dn);
-                                nm.x = fmaf(wgt, a.x, nm.x); nm.y = fmaf(wgt, a.y, nm.y); nm.z = fmaf(wgt, a.z, nm.z); nm.w = fmaf(wgt, a.w, nm.w);
+#pragma unroll
+                            for (int k = 0; k < FWAVES; k++) {
+                                const float wk = exp_neg(mM[k] - Mg);
+                                const float4 a = mnum[k * P4 + tid];
+                                dn = fmaf(wk, mden[k], dn);
+                                nm.x = fmaf(wk, a.x, nm.x); nm.y = fmaf(wk, a.y, nm.y); nm.z = fmaf(wk, a.z, nm.z); nm.w = fmaf(wk, a.w, nm.w);
                             }
                             const float il = __builtin_amdgcn_rcpf(dn);
                             stx4(reinterpret_cast<f4*>(X + G.offAttn + h * HD) + tid, f4{nm.x * il, nm.y * il, nm.z * il, nm.w * il});
