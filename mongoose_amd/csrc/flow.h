@@ -57,7 +57,10 @@ struct FlowGeometry {
     int smax;
     int gqa;         // 1: an attention workgroup per (KV head, split) taking all its query heads; 0: per (query head, split)
 };
-FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim, int maxSeq, int grid);
+// grid: computing workgroups, of cus the launch has.
+FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim, int maxSeq, int grid, int cus);
+// Attention workgroups, one a query head and KV split, up to which a launch that can group query heads does not.
+int flow_plain_most(int nC, int cus, int nHeads, int dim);
 bool flow_context_fits(int maxSeq, const FlowGeometry& g);
 
 constexpr size_t FLOW_ERR_BYTES = 4096;
@@ -98,8 +101,8 @@ struct FlowParams {
                                  // device state on (all layers; xchg holds two halves and the argmax exchange; state != NULL)
     const FlowTail* tail;        // token mode
     int mostSplits;              // KV splits at the launch's last position (0: not known); from some on a variant that shares their merge out
-    int gqaCode;                 // geo.gqa only: 1 = a position of this launch may need the grouped attention (the variant that can do
-                                 // it is launched); 0 = none does (positions below nCompute / nHeads tiles): the plain variant, which
+    int gqaCode;                 // geo.gqa only: not 0 = a position of this launch may take the grouped attention (the variant that has it is
+                                 // launched), which does so past this many attention workgroups; 0 = none does: the plain variant, which
                                  // is faster there, runs on the same geometry and reports a position past its reach as error 3
     int generic;                 // 1: never a variant with a known shape's sizes compiled in (comparisons, tests)
 };

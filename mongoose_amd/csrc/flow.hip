@@ -1013,8 +1013,8 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 
                 FLOW_TRACE(2);
                 // ------------------------------------------------------------------ attention: one (head, KV split) per workgroup
-                // grouped only while a workgroup per query head and split would not fit the launch (positions far into a long context)
-                const bool grouped = GQA && nHeadsV * (pos / TILE + 1) > nC;
+                // grouped only past what a workgroup per query head and split serves best (flow_plain_most; it comes with the launch)
+                const bool grouped = GQA && nHeadsV * (pos / TILE + 1) > p.gqaCode;
                 {
                     const int nsplit = pos / TILE + 1;
                     // Grouped: the query heads of a KV head are shared out over as many workgroups as the launch has left for
@@ -1042,13 +1042,14 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                     // 0.470), else half of the first round of rows, which is what a phase waits for before it streams (8B shape
                     // with both: 1.845 -> 1.790; the whole first round 1.804, a quarter 1.800).
                     // Only while at least a third of the launch is idle (1.1B shape at 600 positions, 96 of 256 idle: 477 -> 457 us a token; a
-                    // half before, an eighth gives no more), and only without dedicated prefetchers.
+                    // half before, an eighth gives no more; grouped attention a quarter: 1.1B at 1,300 positions, 80 idle, 524 -> 499), and
+                    // only without dedicated prefetchers.
                     if (!hasPrefetchers && (p.idleWoRows > 0 || p.idleGateUpRows > 0)) {
                         const int live = nsplit < G.smax ? nsplit : G.smax;
                         int nBusy = unit * live;
                         if (grouped && nBusy < nHeadsV) nBusy = nHeadsV;
                         nBusy = (nBusy + 7) & ~7;
-                        if ((int)blockIdx.x >= nBusy && 3 * ((int)gridDim.x - nBusy) >= (int)gridDim.x) {
+                        if ((int)blockIdx.x >= nBusy && (GQA ? 4 : 3) * ((int)gridDim.x - nBusy) >= (int)gridDim.x) {
                             Prefetcher pf{(int)blockIdx.x & 7, ((int)blockIdx.x - nBusy) >> 3, ((int)gridDim.x - nBusy) >> 3, tid, pfScrap};
                             const size_t rbD = Q4 ? dim >> 1 : dim, rdD = dim >> 4;
                             // (a workgroup without q | k | v rows gets here at the top of the layer; holding it back until q | k | v is
@@ -1938,13 +1939,27 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     }
 }
 
-FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim, int maxSeq, int grid) {
+// Grouped attention costs a hand-over more, but shares a K / V tile among query heads, leaves workgroups idle that read ahead, and its
+// consumers stage one vector instead of merging every split's.  So it starts before the launch is full.  Vectors past 2,048 elements,
+// several pieces a thread: when the splits no longer fit a round of the merge (PB; us a token without / with it, eight layers
+// of 8B at three splits Q8 425 / 430, Q4_0 406 / 419, fp16 rows 435 / 424, at four 445 / 436, 420 / 421, 452 / 428, at five 444 / 437, 424 / 421,
+// 452 / 428, at eight 463 / 446, 451 / 423, 479 / 434).  Shorter ones: past three quarters of the launch (1.1B, six splits 466 / 478, Q4_0
+// 473 / 480, seven 484 / 479 and 491 / 481, eight 490 / 484 and 496 / 482; eight layers of 1,536, 24 heads, Q8 at eight 189 / 186, Q4_0 184 /
+// 185).  With dedicated prefetchers, when it is full (0.5B, twelve splits 370 / 397, sixteen 394 / 414).
+int flow_plain_most(int nC, int cus, int nHeads, int dim) {
+    if (nC != cus) return nC;
+    return dim > 2048 ? std::min(nC, PB * nHeads) : nC * 3 / 4;
+}
+
+FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim, int maxSeq, int grid, int cus) {
     FlowGeometry g{};
     // partial slots: one per FLOW_TILE positions, at most as many as the workgroups of the launch can serve.  One
-    // workgroup a query head where that covers the context (the shorter phase), else one a KV head, taking all its
-    // query heads in turn on one load of the K / V rows.
+    // workgroup a query head where that covers the context and is the better choice (flow_plain_most), else one a KV head, taking its
+    // query heads in turn on one load of the K / V rows -- which takes more LDS: only a context that cannot do without insists on it.
     const int want = (maxSeq + FLOW_TILE - 1) / FLOW_TILE;
-    g.gqa = (nHeads > 0 && want > grid / nHeads && nKVHeads > 0 && nHeads / nKVHeads > 1 && nHeads / nKVHeads <= FLOW_GQA_MAX) ? 1 : 0;
+    if (nHeads > 0 && nKVHeads > 0 && nHeads / nKVHeads > 1 && nHeads / nKVHeads <= FLOW_GQA_MAX)
+        g.gqa = want > grid / nHeads || ((long long)want * nHeads > flow_plain_most(grid, cus, nHeads, dim) && nHeads <= grid &&
+                                         flow_lds_bytes(dim, ffn, headDim, 1, true) <= ((size_t)160 << 10)) ? 1 : 0;
     const int unit = g.gqa ? nKVHeads : nHeads;
     g.smax = want;
     if (unit > 0 && g.smax > grid / unit) g.smax = grid / unit;

@@ -818,7 +818,7 @@ int HIPFusedInference::flowComputeWgs(int cus) const {
     const int pf = execMode == 4 ? 0 : flow_prefetch_workgroups(cus, layerBytes, dim, kvDim, ffnDim);
     const int tries[2] = {cus - pf, cus};
     for (int nC : tries) {
-        const FlowGeometry g = flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, nC);
+        const FlowGeometry g = flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, nC, cus);
         // (the same limits as launch_flow_layers checks: a shape it would refuse runs the fused launches instead)
         if (flow_min_grid(nHeads, nKVHeads, g) <= nC && flow_context_fits(maxSeq, g) && flow_grid_fits(ffnDim, nHeads, g, nC) &&
             (size_t)nLayers * g.stride * 4 < (1ull << 31)) return nC;
@@ -864,7 +864,7 @@ int HIPFusedInference::ensureFlow() {
         }
         flowGrid = prop.multiProcessorCount;
         flowCompute = flowComputeWgs(flowGrid);
-        flowGeo = flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, flowCompute);
+        flowGeo = flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, flowCompute, flowGrid);
         void* v = nullptr;
         HIPCHK(hipMalloc(&v, sizeof(FlowLayer) * (size_t)nLayers));
         dFlowLayers = static_cast<FlowLayer*>(v);
@@ -1009,12 +1009,15 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
     p.err = dFlowErr;
     p.limitTicks = flowLimitTicks;
     {
-        // the last position this launch can reach, where the host knows it: the plain attention variant serves while a
-        // workgroup per query head and KV split fits the launch, also in a context laid out for grouped attention
+        // the last position this launch can reach, where the host knows it: the plain attention variant serves while it is the faster
+        // one, also in a context laid out for grouped attention; where the position is not known, in contexts that it covers
         long long posMax = -1;
         if (!st) posMax = posImm;
         else if (statePosHost >= 0) posMax = (long long)statePosHost + (nTokens > 0 ? nTokens - 1 : 0);
-        p.gqaCode = (posMax < 0 || (long long)nHeads * (posMax / FLOW_TILE + 1) > flowCompute) ? 1 : 0;
+        const int plainMost = flow_plain_most(flowCompute, flowGrid, nHeads, dim);
+        const bool grouped = posMax < 0 ? (long long)nHeads * ((maxSeq + FLOW_TILE - 1) / FLOW_TILE) > flowCompute
+                                        : (long long)nHeads * (posMax / FLOW_TILE + 1) > plainMost;
+        p.gqaCode = grouped ? plainMost : 0;
         p.mostSplits = posMax < 0 ? 0 : (int)(posMax / FLOW_TILE) + 1;
         p.generic = flowGeneric ? 1 : 0;
         // the half of the exchange area a run of whole tokens starts in has to be as a reset leaves it: the launch before
@@ -1053,7 +1056,7 @@ bool HIPFusedInference::flowTailEligible() const {
     if (!flowTail || !flowEligible(0, nLayers)) return false;
     if (!finalNorm || !lmHead.w || lmHead.kind != layers[0].wq.kind || lmHead.cols != dim || lmHead.rows != vocabSize) return false;
     if (lmHead.kind == WF_Q4P && dim % 32) return false;
-    const FlowGeometry g = flowGrid ? flowGeo : flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, 8);
+    const FlowGeometry g = flowGrid ? flowGeo : flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, 8, 8);
     const int gqa = flowGrid ? flowGeo.gqa : 1;        // before the launch is set up: the larger bound
     (void)g;
     return flow_lds_bytes(dim, ffnDim, headDim, gqa, true) <= ((size_t)160 << 10);

@@ -111,6 +111,19 @@ def test_context_past_16384_head64_two_tiles_per_split(hip):
     m.close()
 
 
+@pytest.mark.parametrize("shape,maxSeq,check", [
+    # vectors of more than 2,048 elements: from four splits on
+    (configs.Shape("g3-hd128-ring", 1, 2304, 18, 6, 128, 512, 512, 1e-5, 5e5, False, True, "q8"), 660, {0, 383, 384, 511, 512, 639, 640, 659}),
+    # shorter ones: past three quarters of the launch, seven splits of 32 heads
+    (configs.Shape("g8-hd64", 1, 2048, 32, 4, 64, 512, 512, 1e-5, 1e4, True, True, "q8"), 1000, {0, 767, 768, 895, 896, 999}),
+], ids=lambda v: getattr(v, "name", None))
+def test_grouped_attention_before_the_launch_is_full(hip, shape, maxSeq, check):
+    """Contexts that a workgroup per query head and split would cover, at positions where query heads are grouped all the same."""
+    m = H.load_fast(shape, seed=56, maxSeq=maxSeq, eng=hip, threads=16)
+    _walk(m, maxSeq, check, modes=(1, 3))
+    m.close()
+
+
 @pytest.mark.parametrize("name,shape,maxSeq", [
     ("hd64", configs.Shape("g7-hd64-modes", 1, 896, 14, 2, 64, 256, 512, 1e-6, 1e6, True, True, "q8"), 8300),
     ("hd128", configs.Shape("g4-hd128-modes", 1, 1024, 8, 2, 128, 256, 512, 1e-5, 5e5, False, True, "q8"), 8300),
