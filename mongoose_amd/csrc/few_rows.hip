@@ -466,9 +466,9 @@ static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
 // instructions, made-up tiles and the line at one workgroup a CU 10 %: 0.5B shape, 301 rows 1,808 -> 1,718 us, Q4_0 400 rows 2,642 -> 2,310).
 struct FewTile { int mt, nb; };
 // With three terms an activation row is half as many bytes again, and a tile has at most FEW_MT3 row blocks.
-static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4, int terms) {
+static double few_tile_cost(int rowsN, int T, int K, int nbFirst, int nbLast, int q4, int terms, FewTile& best) {
     const int b16 = (T + 15) / 16;
-    FewTile best{1, nbFirst};
+    best = FewTile{1, nbFirst};
     double least = 1e30;
     for (int nb = nbFirst; nb <= nbLast; nb *= 2)
         for (int mt = 1; mt <= (terms == 3 ? FEW_MT3 : 4) && mt <= b16 && mt * nb <= 8; mt++) {
@@ -480,11 +480,219 @@ static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4
             const double cost = (0.8 * ceil(launched / 256.0) + 0.2 * wgs / 256.0) * each;
             if (cost < least) { least = cost; best = FewTile{mt, nb}; }
         }
-    return best;
+    return least;
+}
+static FewTile few_tile(int rowsN, int T, int K, int nbFirst, int nbLast, int q4, int terms) {
+    FewTile t;
+    few_tile_cost(rowsN, T, K, nbFirst, nbLast, q4, terms, t);
+    return t;
 }
 int few_rows_sum_parts(int N, int T, int K, int q4, int terms) {
     const int b = few_tile(N, T, K, 1, 4, q4, terms).nb;
     return (N + 16 * b - 1) / (16 * b);
+}
+
+// ---------------------------------------------------------------------------
+// gate | up + SwiGLU of more rows.  few_rows_kernel reads an operand once a workgroup of at most 64 x 32 rows, all from L2: from some
+// hundred rows on that is what a CU pulls (0.5B shape, 301 rows, 31 us of a layer's 72), with the matrix pipe mostly idle.  Here a
+// workgroup takes 64 MT / 2 activation rows x (64 gate + 64 up rows), eight waves as two halves of the rows x four quarters of the
+// columns, and a chunk of 64 k of both operands comes through LDS, straight from memory (a ring of three, two chunks under way): 12 to
+// 20 bytes a product row instead of 30 and more.  Activations lie in LDS as the instruction holds them, weights as they are (a row's
+// 16-byte pieces permuted so that 16 rows fall on different banks), converted by the wave that multiplies them.  A wave has the same 16
+// columns of gate and of up, so SwiGLU stays in registers, and a tile's columns are one chunk of the down projection's input: its split
+// is put together in LDS and leaves in whole lines.  Sums over K in one wave, in the order of k.
+//   K a multiple of 64, two terms.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ unsigned few_lds_offset(const void* p) {
+    return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)(p);
+}
+constexpr int FS_RING = 3;
+template <int Q4, int BM>
+__global__ __launch_bounds__(FR_WG) void few_swiglu_kernel(FewParams p) {
+    constexpr int MT = BM / 32, BLK = BM / 16, AB = BLK * 4096, WB = Q4 ? 4608 : 8192, STAGE = AB + WB, LA = BLK / 2, G = FR_WG / BM;
+    extern __shared__ __attribute__((aligned(16))) float part[];
+    __shared__ float sq[G][BM], rs[BM];
+    unsigned char* const ring = reinterpret_cast<unsigned char*>(part);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fq = lane >> 4, wm = wave >> 2, wn = wave & 3;
+    const int T = p.T, K = p.K, N = p.seg[0].N, numM = (T + BM - 1) / BM;
+    const int L = blockIdx.x, grp = L / (8 * numM), rem = L % (8 * numM);
+    const int nTile = grp * 8 + (rem & 7), mTile = rem >> 3;          // the row tiles of a weight tile on one XCD
+    if (nTile >= p.nTiles) return;
+    const int m0 = mTile * BM, n0 = nTile * 64, chunks = K >> 6;
+
+    // what this wave brings of a chunk: LA KB of activations, a KB of weights (Q4_0: waves 0 .. 3 nibbles, 4 .. 7 block scales, twice)
+    const size_t aBlk = (size_t)chunks * 1024;
+    // (uniform bases, a byte offset a lane that stays)
+    const int aBlock = BM == 128 ? wave : wave & 3;
+    const unsigned aOff = ((unsigned)min((m0 >> 4) + aBlock, (T - 1) >> 4) * (unsigned)aBlk + lane * 8) * 2;      // (blocks past the last row repeat the last one)
+    const unsigned short* const a0 = BM == 128 || wave < 4 ? p.Ahi : p.Alo;
+    const unsigned aDst = aBlock * 4096 + (BM == 128 ? 0 : (wave >> 2) * 2048);
+    const signed char* wBase;
+    unsigned wOff, wDst;
+    if (!Q4) {
+        wBase = wave < 4 ? p.seg[0].W : p.seg[1].W;
+        wOff = (unsigned)min(n0 + (wave & 3) * 16 + (lane >> 2), N - 1) * (unsigned)K + ((lane & 3) ^ fq) * 16;
+        wDst = AB + wave * 1024;
+    } else if (wave < 4) {
+        wBase = wave < 2 ? p.seg[0].W : p.seg[1].W;
+        wOff = (unsigned)min(n0 + (wave & 1) * 32 + (lane >> 1), N - 1) * (unsigned)(K >> 1) + ((lane & 1) ^ (fq & 1)) * 16;
+        wDst = AB + wave * 1024;
+    } else {
+        wBase = (wave & 1 ? p.seg[1].W : p.seg[0].W) + (size_t)N * (K >> 1);
+        wOff = (unsigned)min(n0 + lane, N - 1) * (unsigned)(K >> 4);
+        wDst = AB + 4096 + (wave & 1) * 256;
+    }
+    // (written out, M0 the LDS address of the wave's first slot: the compiler's own form has every LDS read behind it wait for all loads)
+    auto issue = [&](int c, int stage) __attribute__((always_inline)) {
+        const int cc = min(c, chunks - 1);                            // past the end: a reload that keeps the count of loads
+        const unsigned base = few_lds_offset(ring) + stage * STAGE;
+#pragma unroll
+        for (int t = 0; t < LA / 2; t++) {
+            const unsigned short* const src = (t ? p.Alo : a0) + (size_t)cc * 1024;
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(base + aDst + t * 2048), "v"(aOff), "s"(src) : "memory");
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(base + aDst + t * 2048 + 1024), "v"(aOff), "s"(src + 512) : "memory");
+        }
+        if (Q4 && wave >= 4) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" : : "s"(base + wDst), "v"(wOff), "s"(wBase + (size_t)cc * 4) : "memory");
+        else asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(base + wDst), "v"(wOff), "s"(wBase + (size_t)cc * (Q4 ? 32 : 64)) : "memory");
+    };
+#pragma unroll
+    for (int c = 0; c < FS_RING - 1; c++) issue(c, c);
+
+    // the rows' RMS factors
+    {
+        const int row = tid % BM, g = tid / BM, t = min(m0 + row, T - 1);
+        float v = 0.f;
+        if (p.sumSq)
+#pragma unroll 4
+            for (int i = g; i < p.sumParts; i += G) v += p.sumSq[(size_t)i * p.sumStride + t];
+        sq[g][row] = v;
+        __syncthreads();
+        if (tid < BM) {
+            float x = 0.f;
+#pragma unroll
+            for (int j = 0; j < G; j++) x += sq[j][tid];
+            rs[tid] = p.sumSq ? 1.0f / sqrtf(x / (float)K + p.eps) : 1.0f;
+        }
+    }
+    const int col = n0 + wn * 16 + fr, colC = min(col, N - 1);
+    const float scG = Q4 ? 0.0625f : p.seg[0].scales[colC], scU = Q4 ? 0.0625f : p.seg[1].scales[colC];
+
+    float4_t acc[MT][2];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) acc[i][b] = float4_t{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int stage) __attribute__((always_inline)) {
+        const unsigned char* const A = ring + stage * STAGE + wm * (MT * 4096) + lane * 16;
+        const unsigned char* const W = ring + stage * STAGE + AB;
+        bf16x8_t f[2][2];
+        unsigned d[2] = {0, 0};
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            if (!Q4) {
+                const int4 x = *reinterpret_cast<const int4*>(W + (b * 4 + wn) * 1024 + fr * 64 + (fq ^ (fr >> 2)) * 16);
+                f[b][0] = frag_i8(x.x, x.y);
+                f[b][1] = frag_i8(x.z, x.w);
+            } else {
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+                    f[b][s] = frag_nib16(*reinterpret_cast<const int2*>(W + (b * 4 + wn) * 512 + fr * 32 + (s ^ (fr >> 3)) * 16 + (fq & 1) * 8), fq >= 2 ? 0u : 4u);
+                d[b] = *reinterpret_cast<const unsigned*>(W + 4096 + b * 256 + (wn * 16 + fr) * 4);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                const bf16x8_t hi = *reinterpret_cast<const bf16x8_t*>(A + i * 4096 + s * 1024);
+                const bf16x8_t lo = *reinterpret_cast<const bf16x8_t*>(A + i * 4096 + 2048 + s * 1024);
+#pragma unroll
+                for (int b = 0; b < 2; b++) {
+                    if (Q4) {
+                        // a Q4_0 block's sum, then its fp16 scale
+                        float4_t t = {0.f, 0.f, 0.f, 0.f};
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, f[b][s], t, 0, 0, 0);
+                        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, f[b][s], t, 0, 0, 0);
+                        const float dd = half_bits_to_float((unsigned short)(s ? d[b] >> 16 : d[b] & 0xffffu));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[i][b][e] = fmaf(dd, t[e], acc[i][b][e]);
+                    } else {
+                        acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, f[b][s], acc[i][b], 0, 0, 0);
+                        acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, f[b][s], acc[i][b], 0, 0, 0);
+                    }
+                }
+            }
+    };
+    int stage = 0;
+    for (int c = 0; c < chunks; c++) {
+        // chunk c has landed (of what is under way only chunk c + 1's loads are younger), and nobody reads chunk c - 1 any more
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((FS_RING - 2) * (LA + 1)) : "memory");
+        const int s2 = stage == 0 ? FS_RING - 1 : stage - 1;
+        issue(c + FS_RING - 1, s2);
+        multiply(stage);
+        stage = stage + 1 == FS_RING ? 0 : stage + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the ring is nobody's any more
+
+    // C layout: lane holds column fr, rows 4 fq .. 4 fq + 3 of a block
+    unsigned short* const out = reinterpret_cast<unsigned short*>(part);      // [plane][block][1024], as few_index has a block's chunk
+    const int kk = wn * 16 + fr, slot = (p.nextQ4 ? (kk >> 5) * 512 + ((kk >> 3) & 3) * 128 : ((kk >> 3) & 1) * 512 + (kk >> 4) * 128) + (kk & 7);
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int blk = wm * MT + i, t = 4 * fq + e;
+            const float r = rs[blk * 16 + t];
+            const float g = acc[i][0][e] * scG * r, u = acc[i][1][e] * scU * r;
+            const float a = g * (1.0f / (1.0f + expf(-g))) * u;      // mongoose.cu:949-956
+            put_split<false>(out, out + BLK * 1024, nullptr, (size_t)(blk * 1024 + slot + t * 8), a);
+        }
+    __syncthreads();
+    const size_t o0 = (size_t)(m0 >> 4) * ((N + 63) >> 6) * 1024 + (size_t)nTile * 1024;
+#pragma unroll
+    for (int j = 0; j < 2 * BLK * 128 / FR_WG; j++) {
+        const int x = tid + j * FR_WG, plane = x / (BLK * 128), blk = x / 128 % BLK, piece = x & 127;
+        const int s = piece >> 6, q = (piece >> 4) & 3, k0 = n0 + (p.nextQ4 ? 32 * s + 8 * q : 16 * q + 8 * s);
+        if (k0 >= N || m0 + blk * 16 + (piece & 15) >= T) continue;
+        const uint4 v = *reinterpret_cast<const uint4*>(out + (size_t)x * 8);
+        *reinterpret_cast<uint4*>((plane ? p.nextLo : p.nextHi) + o0 + (size_t)blk * ((N + 63) >> 6) * 1024 + piece * 8) = v;
+    }
+}
+
+template <int Q4, int BM>
+static hipError_t launch_few_swiglu(FewParams& p, hipStream_t s) {
+    constexpr int bytes = FS_RING * (BM / 16 * 4096 + (Q4 ? 4608 : 8192));
+    static bool raised = false;                                        // (more than the default cap on dynamic LDS)
+    if (!raised) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_swiglu_kernel<Q4, BM>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e != hipSuccess) return e;
+        raised = true;
+    }
+    p.nTiles = (p.seg[0].N + 63) / 64;
+    const unsigned grid = (unsigned)((p.nTiles + 7) / 8 * 8) * (unsigned)((p.T + BM - 1) / BM);
+    hipLaunchKernelGGL((few_swiglu_kernel<Q4, BM>), dim3(grid), dim3(FR_WG), bytes, s, p);
+    return hipGetLastError();
+}
+// 0: gate | up of T rows is few_rows_kernel's; else the activation rows of a workgroup's tile in few_swiglu_kernel.  The least of three
+// models in microseconds: few_tile's, and for tiles of 64 and 128 rows a start and end and so much a chunk of 64 k, times the
+// workgroups of the busiest CU (of 64 rows two run on it together and hide each other's waits).  Fitted to the launches of five
+// shapes at 16 to 1,000 rows; what it picks is within 6 % of the best at all but three of 123 points (15 %), and none of it is slower than few_rows_kernel.  Microseconds a launch, old / 64 /
+// 128 rows, Q8 and Q4_0: 0.5B shape 77 rows 12.6 / 14.8 / 20.3 and 15.0 / 17.0 / 24.0, 301 31.6 / 20.7 / 21.5 and 36.0 / 24.6 / 24.8, 512 47.0 /
+// 29.1 / 37.3 and 51.8 / 33.7 / 43.3; 1.1B 64 rows 19.1 / 23.0 / 34.2 and 27.7 / 27.6 / 42.8, 200 41.1 / 34.9 / 35.0 and 58.2 / 43.4 / 42.6; 8B
+// 16 rows 32.4 / 46.1 / 71.0, 37 62.8 / 42.6 / 63.0, 128 109.5 / 69.8 / 67.6, Q4_0 144.1 / 87.0 / 83.0.
+static int few_swiglu_rows(int N, int T, int K, int q4, int terms) {
+    if (terms != 2 || K % 64) return 0;
+    FewTile t;
+    const double cost = 1e-3 * few_tile_cost(2 * N, T, K, 2, 8, q4, terms, t), chunks = K / 64;
+    const double old = q4 && K <= 64 * 2 * FR_WAVES ? 6.0 + 0.7 * cost : 4.0 + 0.9 * cost;
+    const int launched = ((N + 63) / 64 + 7) / 8 * 8;
+    auto busiest = [&](int bm) { return (launched * ((T + bm - 1) / bm) + 255) / 256; };
+    const int c64 = busiest(64), c128 = busiest(128);
+    const double t64 = c64 == 1 ? (q4 ? 6.5 + 0.75 * chunks : 5.5 + 0.62 * chunks) : 7.0 + (q4 ? 0.61 : 0.50) * chunks * c64;
+    const double t128 = 7.0 + (q4 ? 1.18 : 0.93) * chunks * c128;
+    if (old <= t64 && old <= t128) return 0;
+    return t64 <= t128 ? 64 : 128;
 }
 
 template <int MODE, int MT, int NB>
@@ -516,6 +724,9 @@ hipError_t launch_few_rows(int mode, FewParams& p, hipStream_t s) {
     }
     if (mode == FEW_SWIGLU) {
         if (p.seg[1].N != N || !p.nextHi || !p.nextLo) return hipErrorInvalidValue;
+        const int bm = few_swiglu_rows(N, p.T, p.K, p.q4, terms);
+        if (bm == 64) return p.q4 ? launch_few_swiglu<1, 64>(p, s) : launch_few_swiglu<0, 64>(p, s);
+        if (bm == 128) return p.q4 ? launch_few_swiglu<1, 128>(p, s) : launch_few_swiglu<0, 128>(p, s);
         const FewTile t = few_tile(2 * N, p.T, p.K, 2, 8, p.q4, terms);
         p.nTiles = (N + 8 * t.nb - 1) / (8 * t.nb);
         return t.nb == 2 ? launch_few_mt<FEW_SWIGLU, 2>(t.mt, p, s) : t.nb == 4 ? launch_few_mt<FEW_SWIGLU, 4>(t.mt, p, s) : launch_few_mt<FEW_SWIGLU, 8>(t.mt, p, s);
@@ -825,7 +1036,7 @@ static FewAhead few_plan(unsigned grid, const FewNext* next, int nNext, int T, i
             take(m.W2, nullptr, m.N1, m.K, m.q4, 32, tk, tq + tk, 0);
         } else {
             const bool two = m.mode == FEW_SWIGLU;
-            const int rows = two ? 8 * few_tile(2 * m.N, T, m.K, 2, 8, m.q4, terms).nb : 16 * few_tile(m.N, T, m.K, 1, 4, m.q4, terms).nb;
+            const int rows = two ? (few_swiglu_rows(m.N, T, m.K, m.q4, terms) ? 64 : 8 * few_tile(2 * m.N, T, m.K, 2, 8, m.q4, terms).nb) : 16 * few_tile(m.N, T, m.K, 1, 4, m.q4, terms).nb;
             take(m.W0, m.W1, m.N, m.K, m.q4, rows, (m.N + rows - 1) / rows, 0, 0);
         }
     }

@@ -26,6 +26,22 @@ NARROW = SMALL._replace(name="narrow", ffnDim=32)          # the down projection
     (SMALL, "q4_0", False, 5, 33), (SMALL, "q4_0", True, 0, 48), (ODD, "q8", False, 100, 15), (ODD, "q8", True, 17, 63),
     (ODD, "q4_0", False, 250, 31), (NARROW, "q8", False, 0, 17), (NARROW, "q4_0", False, 2, 33)])
 def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
+    _prefill_against_tokens(hip, shape, fmt, kv_f16, pos0, rows)
+
+
+# gate | up through LDS: one chunk of 64 k, two (less than the ring holds) and seven, a last tile of 32 columns, rows one past and one
+# short of the tiles of 64 and 128 rows
+@pytest.mark.parametrize("heads,ffn,fmt,kv_f16,pos0,rows,bm", [
+    (1, 9760, "q8", False, 0, 129, 64), (1, 9760, "q4_0", False, 3, 257, 128), (2, 14304, "q8", False, 0, 193, 128), (2, 14304, "q4_0", True, 0, 129, 64),
+    (7, 9760, "q8", False, 5, 65, 128), (7, 9760, "q8", True, 0, 255, 64), (7, 9760, "q4_0", False, 0, 127, 128), (7, 9760, "q4_0", False, 9, 191, 64)])
+def test_gate_up_tiles_match_token_by_token(hip, heads, ffn, fmt, kv_f16, pos0, rows, bm):
+    shape = configs.TOY._replace(name="swiglu", nLayers=2, dim=64 * heads, nHeads=heads, nKVHeads=1, ffnDim=ffn, vocab=300)
+    names = _prefill_against_tokens(hip, shape, fmt, kv_f16, pos0, rows)
+    assert any("few_swiglu_kernel<%d, %d>" % (fmt == "q4_0", bm) in n for n in names), sorted(set(names))
+
+
+def _prefill_against_tokens(hip, shape, fmt, kv_f16, pos0, rows):
+    """A prompt in one call against the same tokens one by one; the names of the kernels the call launched."""
     m = H.Model(shape, seed=rows, maxSeq=pos0 + rows + 3, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
     toks = m.prompt(pos0 + rows + 1)
     ref = np.empty(shape.vocab, np.float32)
@@ -40,7 +56,9 @@ def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
     for pos in range(pos0):
         rc, _ = m.hip.DecodeToken(int(toks[pos]), pos)
         assert rc == 0
-    rc, nxt, logits, _ = m.hip.Prefill(toks[pos0:pos0 + rows], pos0, wantLogits=True)
+    out = []
+    names = H.launched(lambda: out.append(m.hip.Prefill(toks[pos0:pos0 + rows], pos0, wantLogits=True)))
+    rc, nxt, logits, _ = out[0]
     assert rc == 0, E.last_error()
     bar = 1e-3 if kv_f16 else 1e-4
     assert H.rel_err(logits, ref) < bar and nxt == nref
@@ -48,6 +66,7 @@ def test_few_rows_match_token_by_token(hip, shape, fmt, kv_f16, pos0, rows):
     rc, _ = m.hip.DecodeToken(int(toks[-1]), pos0 + rows, got)
     assert rc == 0 and H.rel_err(got, after) < bar
     m.close()
+    return names
 
 
 @pytest.mark.parametrize("shape,fmt,kv_f16,n", [
