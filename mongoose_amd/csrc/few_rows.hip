@@ -495,13 +495,16 @@ int few_rows_sum_parts(int N, int T, int K, int q4, int terms) {
 // ---------------------------------------------------------------------------
 // gate | up + SwiGLU of more rows.  few_rows_kernel reads an operand once a workgroup of at most 64 x 32 rows, all from L2: from some
 // hundred rows on that is what a CU pulls (0.5B shape, 301 rows, 31 us of a layer's 72), with the matrix pipe mostly idle.  Here a
-// workgroup takes 64 MT / 2 activation rows x (64 gate + 64 up rows), eight waves as two halves of the rows x four quarters of the
-// columns, and a chunk of 64 k of both operands comes through LDS, straight from memory (a ring of three, two chunks under way): 12 to
-// 20 bytes a product row instead of 30 and more.  Activations lie in LDS as the instruction holds them, weights as they are (a row's
+// workgroup takes BM = 64 or 128 activation rows x (64 gate + 64 up rows), eight waves as two halves of the rows x four quarters of the
+// columns, and a chunk of 64 k of both operands comes through LDS, straight from memory (a ring of three, two chunks under way): 0.04 to
+// 0.05 bytes a product instead of 0.14 and more.  Activations lie in LDS as the instruction holds them, weights as they are (a row's
 // 16-byte pieces permuted so that 16 rows fall on different banks), converted by the wave that multiplies them.  A wave has the same 16
 // columns of gate and of up, so SwiGLU stays in registers, and a tile's columns are one chunk of the down projection's input: its split
-// is put together in LDS and leaves in whole lines.  Sums over K in one wave, in the order of k.
-//   K a multiple of 64, two terms.
+// is put together in LDS and leaves in whole lines.  Sums over K in one wave, in the order of k.  Bound by a wave's own chain in a chunk --
+// LDS reads, conversions, products -- with two waves a SIMD: 64 rows 0.62 us a chunk with one workgroup on a CU, 0.50 with two (products
+// 0.21, conversions 0.17), 128 rows 0.93; a ring of six changes nothing with one and keeps two from fitting (0.70), products ordered so that
+// none waits for the one before 1 to 3 % slower.  Microseconds a launch: few_swiglu_rows.
+//   K a multiple of 64, N K below 2^31, two terms.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ unsigned few_lds_offset(const void* p) {
     return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)(p);
@@ -682,7 +685,7 @@ static hipError_t launch_few_swiglu(FewParams& p, hipStream_t s) {
 // 29.1 / 37.3 and 51.8 / 33.7 / 43.3; 1.1B 64 rows 19.1 / 23.0 / 34.2 and 27.7 / 27.6 / 42.8, 200 41.1 / 34.9 / 35.0 and 58.2 / 43.4 / 42.6; 8B
 // 16 rows 32.4 / 46.1 / 71.0, 37 62.8 / 42.6 / 63.0, 128 109.5 / 69.8 / 67.6, Q4_0 144.1 / 87.0 / 83.0.
 static int few_swiglu_rows(int N, int T, int K, int q4, int terms) {
-    if (terms != 2 || K % 64) return 0;
+    if (terms != 2 || K % 64 || (long long)N * K >= 1LL << 31) return 0;      // (offsets in 32 bits)
     FewTile t;
     const double cost = 1e-3 * few_tile_cost(2 * N, T, K, 2, 8, q4, terms, t), chunks = K / 64;
     const double old = q4 && K <= 64 * 2 * FR_WAVES ? 6.0 + 0.7 * cost : 4.0 + 0.9 * cost;

@@ -57,7 +57,9 @@ constexpr size_t few_gemm_bytes(int T, int K) {
 // Rows up to which some prefill takes them.  The tiled GEMMs want work for every CU, so the line falls with the weights of a
 // layer.  Microseconds a layer, few-row / tiled, Q8 and Q4_0, nothing cached: 0.5B shape (15 million weights) 36 / 69 and
 // 39 / 77 at 37 rows, 103 / 119 and 118 / 141 at 506, 138 / 136 and 156 / 154 at 625; 1.1B (44) 147 / 164 and 182 / 203 at
-// 294, 161 / 173 and 203 / 211 at 346, 183 / 191 and 239 / 219 at 415; 8B (218) 236 / 243 and 286 / 297 at 124.
+// 294, 161 / 173 and 203 / 211 at 346, 183 / 191 and 239 / 219 at 415; 8B (218) 236 / 243 and 286 / 297 at 124.  (Drawn before gate | up of
+// many rows went through LDS (few_swiglu_kernel); with that the few-row kernels lead up to it everywhere and some way past it: 0.5B 78 / 110
+// at 512 rows, 118 / 132 at 700, 157 / 157 at 1,024, Q4_0 131 / 166 at 700; 1.1B 122 / 152 at 301, 150 / 173 at 400, 237 / 231 at 600.)
 inline int few_rows_most(int dim, int kvDim, int ffn) {
     const double millions = ((double)dim * (2.0 * dim + 2.0 * kvDim) + 3.0 * dim * ffn) * 1e-6;
     const int n = (int)(2300.0 / std::sqrt(millions));

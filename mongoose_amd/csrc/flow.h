@@ -46,7 +46,8 @@ struct FlowTail {
 
 // Exchange area: per layer one block of `stride` floats holding, at the offsets below, the rotated query,
 // the K and V rows of the current position, the attention partials of up to smax KV splits (accumulator,
-// maximum, sum), the hidden state after the attention block, the SwiGLU vector and the layer's output.
+// maximum, sum), the hidden state after the attention block, the SwiGLU vector and the layer's output.  Maxima and sums: split by
+// split, all heads of one together, at offPm and offPl; where query heads are grouped pairs of them from offPm on, head by head.
 // Every float is the pattern 0xFFFFFFFF until its producer has written it.
 constexpr int FLOW_GQA_MAX = 8;        // query heads a KV head may have for the grouped attention
 constexpr int FLOW_TILE = 128;         // positions of an attention tile: one workgroup per (query head, tile)
