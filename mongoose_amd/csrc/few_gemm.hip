@@ -165,9 +165,11 @@ __global__ __launch_bounds__(FG_WG) void few_gemm_kernel(FewGemmParams p) {
     const signed char* aP[MT];
     const float* sP[MT];
 #pragma unroll
-    for (int i = 0; i < MT; i++) {                                    // (blocks past the last row repeat the last one)
+    for (int i = 0; i < MT; i++) {
+        // Blocks past the last row repeat the last one, and so do rows: half a block's lines where it has eight rows or fewer (1 to 8 rows
+        // 896 x 4864 9.8 -> 8.9 us a call, 9000 x 8192 30.8 -> 28.0; 20 rows 35.0 -> 32.7, 72 49.3 -> 47.3).
         const size_t tb = (size_t)min((m0 >> 4) + i, (T - 1) >> 4);
-        aP[i] = p.A + tb * chunks * 3072 + lane * 16;
+        aP[i] = p.A + tb * chunks * 3072 + (fq * 16 + min(fr, T - 1 - (int)tb * 16)) * 16;
         sP[i] = p.aScales + (tb * FG_WAVES + wave) * 16 + 4 * fq;
     }
     // what the epilogue needs, requested before the operands: this thread's column n, rows mq .. mq + 3

@@ -146,8 +146,11 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
     const size_t aBlk = (size_t)planeChunks * 1024;                   // elements from one 16-row block to the next
     const unsigned short* aP[TERMS][MT];
 #pragma unroll
-    for (int i = 0; i < MT; i++) {                                    // (blocks past the last row repeat the last one)
-        const size_t o = (size_t)min((m0 >> 4) + i, (T - 1) >> 4) * aBlk + lane * 8;
+    for (int i = 0; i < MT; i++) {
+        // Blocks past the last row repeat the last one, and so do rows: half a block's lines where it has eight rows or fewer (us a call,
+        // eight 1.1B layers at 3 / 20 rows 370 / 387 -> 338 / 367, four of 8B 361 / 441 -> 332 / 422, Q4_0 385 / 495 -> 356 / 475).
+        const int block = min((m0 >> 4) + i, (T - 1) >> 4);
+        const size_t o = (size_t)block * aBlk + (fq * 16 + min(fr, T - 1 - block * 16)) * 8;
         aP[0][i] = p.Ahi + o;
         aP[1][i] = p.Alo + o;
         if constexpr (TERMS == 3) aP[2][i] = p.Ax + o;
@@ -308,7 +311,7 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
                 dd[b] = 1.0f;
             }
         }
-        const int at = chunks * 1024 + (Q4 ? 0 : (fq & 1) * 512 + ((fq >> 1) * 16 + fr) * 8 - lane * 8);      // k = 8 q .. 8 q + 7
+        const int at = chunks * 1024 + (Q4 ? 0 : (fq & 1) * 512 + ((fq >> 1) - fq) * 128);      // k = 8 q .. 8 q + 7
 #pragma unroll
         for (int i = 0; i < MT; i++) {
             uint4 a[TERMS];
