@@ -9,6 +9,11 @@ namespace mg {
 
 constexpr int WG = 256;
 
+// Opens an asm string that loads into LDS (operand 0: the LDS address of the wave's first slot).  A load that reads M0 may not be the
+// instruction behind a scalar write of it; the compiler keeps them apart by itself, but not inside a string.  (M0 is a reserved
+// register that no clobber list takes: the compiler writes it anew before each use of its own.)
+#define MG_SET_M0 "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+
 // ---------------------------------------------------------------------------
 // wave64 / workgroup reductions
 // ---------------------------------------------------------------------------

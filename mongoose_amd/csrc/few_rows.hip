@@ -556,11 +556,11 @@ __global__ __launch_bounds__(FR_WG) void few_swiglu_kernel(FewParams p) {
 #pragma unroll
         for (int t = 0; t < LA / 2; t++) {
             const unsigned short* const src = (t ? p.Alo : a0) + (size_t)cc * 1024;
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(base + aDst + t * 2048), "v"(aOff), "s"(src) : "memory");
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(base + aDst + t * 2048 + 1024), "v"(aOff), "s"(src + 512) : "memory");
+            asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(base + aDst + t * 2048), "v"(aOff), "s"(src) : "memory");
+            asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(base + aDst + t * 2048 + 1024), "v"(aOff), "s"(src + 512) : "memory");
         }
-        if (Q4 && wave >= 4) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" : : "s"(base + wDst), "v"(wOff), "s"(wBase + (size_t)cc * 4) : "memory");
-        else asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(base + wDst), "v"(wOff), "s"(wBase + (size_t)cc * (Q4 ? 32 : 64)) : "memory");
+        if (Q4 && wave >= 4) asm volatile(MG_SET_M0 "global_load_lds_dword %1, %2" : : "s"(base + wDst), "v"(wOff), "s"(wBase + (size_t)cc * 4) : "memory");
+        else asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(base + wDst), "v"(wOff), "s"(wBase + (size_t)cc * (Q4 ? 32 : 64)) : "memory");
     };
 #pragma unroll
     for (int c = 0; c < FS_RING - 1; c++) issue(c, c);

@@ -11,6 +11,7 @@
 // (causal attention as kernels/mongoose.cu:251-353 does for training).
 #include "kernels.h"
 #include "prefill.h"
+#include "device_util.h"
 
 namespace mg {
 
@@ -852,10 +853,10 @@ __global__ __launch_bounds__(512) void gemm_q8_ring_kernel(GemmParams p) {
             const unsigned short* ah = p.Ahi + ko;
             const unsigned short* al = p.Alo + ko;
             const unsigned l0 = lds_offset(base);
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(l0), "v"(aOff[0] * 2u), "s"(ah));
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(l0 + 1024u), "v"(aOff[1] * 2u), "s"(ah));
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(l0 + (unsigned)RING_PLANE), "v"(aOff[0] * 2u), "s"(al));
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(l0 + (unsigned)RING_PLANE + 1024u), "v"(aOff[1] * 2u), "s"(al));
+            asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(l0), "v"(aOff[0] * 2u), "s"(ah));
+            asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(l0 + 1024u), "v"(aOff[1] * 2u), "s"(ah));
+            asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(l0 + (unsigned)RING_PLANE), "v"(aOff[0] * 2u), "s"(al));
+            asm volatile(MG_SET_M0 "global_load_lds_dwordx4 %1, %2" : : "s"(l0 + (unsigned)RING_PLANE + 1024u), "v"(aOff[1] * 2u), "s"(al));
         } else {
             // (K split or short launches: the compiler's form of the same loads schedules better there -- measured)
             __builtin_amdgcn_global_load_lds(p.Ahi + aOff[0] + ko, reinterpret_cast<int4*>(base), 16, 0, 0);
