@@ -135,7 +135,7 @@ public:
     int hiddenIdx = 0;
     int enqueueLayer(const LayerWeights& L, int layer, const StepState* st, int posImm);
     // row / parts: the lm_head of that row (instead of the hidden buffer), its argmax partials left for the caller
-    int enqueueFinal(bool withArgmax, int* parts = nullptr);
+    int enqueueFinal(bool withArgmax, int* parts = nullptr, const float* row = nullptr);
     int publish(const float* src, int n, const int* ints, int nInts);      // results on their way to hOut
     PublishParams publishParams(const float* src, int n);
     int collect(float* out, int n, int* ints, int nInts, bool prefill = false);      // ... waited for and copied to the caller

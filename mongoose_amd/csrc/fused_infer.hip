@@ -1189,7 +1189,7 @@ int HIPFusedInference::enqueueLayer(const LayerWeights& L, int layer, const Step
 
 // Final norm + lm_head (cuda_fused_infer.go:446-448) with the per-workgroup
 // argmax folded into the matvec epilogue.
-int HIPFusedInference::enqueueFinal(bool withArgmax, int* parts) {
+int HIPFusedInference::enqueueFinal(bool withArgmax, int* parts, const float* row) {
     if (withArgmax) statePosHost = -1;              // (the argmax's last kernel advances the device state)
     if (!finalNorm || !lmHead.w) { set_error("final norm / lm_head not set"); return MG_E_STATE; }
     if (execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P) {
@@ -1207,7 +1207,7 @@ int HIPFusedInference::enqueueFinal(bool withArgmax, int* parts) {
     }
     MvParams p{};
     p.seg[0] = MvSeg{lmHead.w, lmHead.scales, nullptr, logits, vocabSize};
-    p.nseg = 1; p.K = dim; p.act = hidden[hiddenIdx]; p.gain = finalNorm; p.eps = eps;
+    p.nseg = 1; p.K = dim; p.act = row ? row : hidden[hiddenIdx]; p.gain = finalNorm; p.eps = eps;
     p.amaxVal = amaxVal; p.amaxIdx = amaxIdx;
     if (fuseEmbed && flowEligible(0, nLayers)) {
         // inside the captured token: the lm_head launch also leaves the exchange area of the persistent
@@ -1973,8 +1973,10 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
     pfTokens = reinterpret_cast<const int*>(hIn);
     // Of the last layer only the last position is wanted behind the cache rows; the rest of it then runs as a decode step's layer
     // does.  8B shape: 512 rows through eight layers 3,919 -> 3,605 us, 37 through four 601 -> 536; 1.1B, eight layers, 37 rows 487 ->
-    // 463; 0.5B, 24 layers, 855 -> 851.  (A model of one layer goes through whole: the batched kernels are checked on such models.)
-    const bool single = nLayers == 1;
+    // 463; 0.5B, 24 layers, 855 -> 851.  (A model of one layer goes through whole, which is what the batched
+    // kernels are checked on, but for a lm_head on quantized activations, which wants the row in the hidden buffer.)
+    const bool quantized = execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P;
+    const bool single = nLayers == 1 && !quantized;
     if (elapsedMs) HIPCHK(hipEventRecord(ev0, stream));
     if (few) {
         auto plane = [](void* p) { return static_cast<unsigned short*>(p); };
@@ -1986,19 +1988,18 @@ int HIPFusedInference::Prefill(const int* tokens, int nTokens, int pos0, int* ne
     if (rc) return rc;
     // the last position continues on the decode path: the rest of its last layer, final norm, lm_head, greedy token, state -> pos0 + T
     const float* row = pfX + (size_t)(T - 1) * dim;
-    if (single) HIPCHK(hipMemcpyAsync(hidden[hiddenIdx], row, (size_t)dim * 4, hipMemcpyDeviceToDevice, stream));
-    else rc = enqueueLayerRest(layers[nLayers - 1], nLayers - 1, nullptr, pos0 + T - 1, pfQ + (size_t)(T - 1) * dim, row);
+    if (!single) rc = enqueueLayerRest(layers[nLayers - 1], nLayers - 1, nullptr, pos0 + T - 1, pfQ + (size_t)(T - 1) * dim, row);
     if (rc) return rc;
     const int n = logitsOut ? vocabSize : 0;
     int next = 0;
-    const bool quantized = execMode == 0 && q4ActQuant && lmHead.kind == WF_Q4P;      // (a tail of its own)
     if (quantized) {
         HIPCHK(launch_set_state(dState, pos0 + T - 1, tokens[T - 1], 0, 0, ropeRef(), stream));
         rc = enqueueFinal(true);
         if (rc == 0) rc = publish(logits, n, dHistory, 1);
     } else {
-        PrefillEnd e{amaxVal, amaxIdx, 0, dState, pos0 + T, dHistory, vocabSize, ropeRef()};
-        rc = enqueueFinal(true, &e.nparts);
+        // (one layer: the row goes into the hidden buffer beside the token's way out, not by a copy of its own, 1.3 to 2 us of a call)
+        PrefillEnd e{amaxVal, amaxIdx, 0, dState, pos0 + T, dHistory, vocabSize, ropeRef(), single ? row : nullptr, hidden[hiddenIdx], dim};
+        rc = enqueueFinal(true, &e.nparts, e.row);
         if (rc == 0) HIPCHK(launch_publish_prefill(publishParams(logits, n), e, stream));
     }
     if (rc) return rc;

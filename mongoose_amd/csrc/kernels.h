@@ -189,12 +189,13 @@ inline int publish_slice_floats(int n) { const int per = (n + PUBLISH_MAX_SLICES
 inline int publish_slices(int n) { return n > 0 ? (n + publish_slice_floats(n) - 1) / publish_slice_floats(n) : 1; }
 hipError_t launch_publish(const PublishParams& p, hipStream_t s);
 // The same at the end of a prefill, whose lm_head has left its argmax partials: one more workgroup (and flag, behind the
-// slices') picks the greedy token, hands it over as the only int, and leaves the step state, the history's first entry and the
-// RoPE row as the step after needs them.  Its flag is the first where there are no slices (n = 0).
+// slices') picks the greedy token, hands it over as the only int, and leaves the step state, the history's first entry, the
+// RoPE row and, where row is set, the hidden buffer as the step after needs them.  Its flag is the first where there are no slices (n = 0).
 struct PrefillEnd {
     const float* pv; const int* pi; int nparts;
     StepState* state; int pos; int* history; int vocab;      // pos: of the next token
     RopeCur rope;
+    const float* row; float* hidden; int dim;                // the last position's row, where it is not in the hidden buffer (else NULL)
 };
 hipError_t launch_publish_prefill(const PublishParams& p, const PrefillEnd& e, hipStream_t s);
 // Page-locked host memory -> device memory, up to three pieces in one launch (16-byte aligned on both sides; a length need

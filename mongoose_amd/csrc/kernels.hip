@@ -1881,7 +1881,7 @@ hipError_t launch_publish(const PublishParams& p, hipStream_t s) {
     return hipGetLastError();
 }
 
-// With the argmax's last step and the state as launches of their own, two dependent launches of 4 us each
+// With the argmax's last step, the state and the row's copy as launches of their own, two dependent launches of 4 us each
 // stood between the lm_head and this one.
 __global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, PrefillEnd e, int per, int slices) {
     if (blockIdx.x < PUBLISH_WGS) {
@@ -1893,6 +1893,7 @@ __global__ __launch_bounds__(WG) void publish_prefill_kernel(PublishParams p, Pr
         int idx = INT_MAX;
         for (int i = threadIdx.x; i < e.nparts; i += WG) argmax_pick(v, idx, e.pv[i], e.pi[i]);
         copy_rope_row(e.rope, e.pos);
+        if (e.row) for (int i = threadIdx.x; i < e.dim; i += WG) e.hidden[i] = e.row[i];
         wave_argmax(v, idx);
         if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = v; bi[threadIdx.x >> 6] = idx; }
         __syncthreads();

@@ -323,3 +323,15 @@ def test_last_layer_for_the_last_position(hip, s, fmt, kv_f16, pos0, rows, atten
     assert H.rel_err(m.hip.ExportHidden(), href) < bar
     assert m.hip.DecodeToken(int(toks[-1]), pos0 + rows, got)[0] == 0 and H.rel_err(got, after) < bar
     m.close()
+
+
+@pytest.mark.parametrize("s,rows", [(H.with_layers(configs.TOY, 1), 2), (H.with_layers(configs.TOY, 1), 1100), (MINI, 7)], ids=lambda v: getattr(v, "name", None))
+def test_the_last_row_takes_no_copy_of_its_own(hip, s, rows):
+    """A call's launches are its kernels, at any number of layers: the row that the lm_head reads reaches the hidden buffer in one of
+    them."""
+    m = H.Model(s, seed=rows, maxSeq=rows + 2, eng=hip, oracle=False)
+    toks = m.prompt(rows)
+    assert m.hip.Prefill(toks, 0)[0] == 0                      # (tables and buffers are there afterwards)
+    names = H.launched(lambda: m.hip.Prefill(toks, 0))
+    assert names and not any("memcpy" in n.lower() or "copybuffer" in n.lower() for n in names), names
+    m.close()
