@@ -1,16 +1,10 @@
 // few_rows.h -- launchers of the few-row prefill kernels (few_rows.hip): a handful of positions through the layers.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "few_rules.h"
 
 namespace mg {
 
-// One launch, tiles of 16 to 128 weight rows x 16 to 64 activation rows a workgroup (few_tile chooses); what follows the
-// product is the epilogue of the mode.
-enum FewMode {
-    FEW_RESID,       // Y += v * scale + bias; optionally the next projection's split of Y * nextGain and the rows' sums of squares
-    FEW_SWIGLU,    // seg0 = gate, seg1 = up: silu(g) * u as the split of the down projection's input
-    FEW_QKV,         // seg0 = q, seg1 = k, seg2 = v: bias, RoPE, q rows to seg0.Y, K / V rows into the caches at pos0 + row
-};
 struct FewSeg { const signed char* W; const float* scales; const float* bias; float* Y; int N; };
 struct FewParams {
     FewSeg seg[3];
@@ -60,9 +54,6 @@ struct FewGemmParams {
 };
 hipError_t launch_few_gemm(const float* act, FewGemmParams& p, void* ws, size_t wsBytes, hipStream_t s);
 
-// What the launches behind an attention launch multiply T rows by, in their order (launch_few_rows: W1 and W2 where the mode has them,
-// N1 their rows): its idle CUs read it into the L2s.
-struct FewNext { FewMode mode; const void* W0; const void* W1; const void* W2; int N, N1, K, q4; };
 // Causal attention of T query rows (rotated) at positions pos0 .. over the cache rows [0, pos0 + T), all products and sums
 // in fp32; the result goes out as the split the output projection reads.
 hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,

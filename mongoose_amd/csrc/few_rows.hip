@@ -14,8 +14,6 @@
 #include "few_rows.h"
 #include "few_rules.h"
 #include "device_util.h"
-#include <algorithm>
-#include <climits>
 
 namespace mg {
 
@@ -833,13 +831,11 @@ __device__ __forceinline__ void ld_row(const void* base, size_t i, float (&r)[N]
 }
 
 // Reading ahead.  The attention moves few bytes and leaves most CUs idle, and the projections behind it start cold, so workgroups
-// behind its own read what those multiply -- Wo, gate | up, down, the next layer's q|k|v -- into the L2s.  These are one an XCD: tile t
+// behind its own read what those multiply -- Wo, gate | up, down, in Q8 the next layer's q|k|v -- into the L2s.  These are one an XCD: tile t
 // of a launch runs on XCD t mod 8 (few_rows_kernel's mapping) and is read by workgroups there, a KB a wave and instruction, into
 // LDS that nothing reads.  Microseconds a call, without / with: 0.5B, 24 layers, 16 rows 811 / 722, 37 behind 200 902 / 826, 128
 // 1,180 / 1,100, 301 1,908 / 1,814, 512 2,641 / 2,440; Q4_0 16 rows 807 / 780, 301 1,906 / 1,902; 1.1B, eight layers, 77 rows 559 / 542, 200
 // 859 / 824; 8B, four layers, within 1 %: a layer is far more than the L2s hold.
-constexpr int FEW_REGIONS = 10;
-struct FewAhead { FewRegion r[FEW_REGIONS]; int n, first, readers; };      // first: the launch's first workgroup that reads ahead
 __device__ __forceinline__ void few_read_ahead(const FewAhead& a, float* scrap) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), xcd = (int)blockIdx.x & 7;
     const unsigned nW = (unsigned)(a.readers >> 3) * FR_WAVES, me = (((int)blockIdx.x - a.first) >> 3) * FR_WAVES + wave;
@@ -1003,56 +999,6 @@ static hipError_t launch_few_attn(int cs, A... a) {
     return cs == 4 ? launch_few_attn_t<HD, KVH, 4>(a...) : (cs == 2 ? launch_few_attn_t<HD, KVH, 2>(a...) : launch_few_attn_t<HD, KVH, 1>(a...));
 }
 
-// What an attention launch of `grid` workgroups reads ahead.  Up to 200 KB a reading workgroup (100: 0.5B, 200 rows 1,448 us a call
-// against 1,388) and 20 MB (12: 16 rows 777 against 714; past it the 1.1B shape, 44 MB a layer, loses, 16 rows 360 at 12, 371 at 20, 370 at
-// 24); a matrix that does not fit is taken in part, its first tiles.  Readers are the workgroups up to 256, but 96 at least -- they
-// then share CUs with the attention's, which wait more than they load (0.5B, 301 rows, 266 workgroups of attention, with 0 / 32 / 64
-// / 96 / 128 readers 1,908 / 1,896 / 1,849 / 1,814 / 1,799, 200 rows 1,388 / 1,388 / 1,386 / 1,410 / 1,402) -- and no more than
-// have 64 KB each.
-constexpr long long FEW_AHEAD_EACH = 200 << 10, FEW_AHEAD_MOST = 20 << 20, FEW_AHEAD_LEAST = 64 << 10;
-static FewAhead few_plan(unsigned grid, const FewNext* next, int nNext, int T, int terms, int headDim) {
-    FewAhead a{};
-    a.first = INT_MAX;
-    const unsigned own = (grid + 7) / 8 * 8, room = own + 96 > 256 ? 96 : 256 - own;
-    const long long most = std::min(room * FEW_AHEAD_EACH, FEW_AHEAD_MOST);
-    long long left = most, bytes = 0;
-    // one matrix, or two read tile by tile (W1; per: the halves of W0's heads)
-    auto take = [&](const void* W0, const void* W1, int N, int K, int q4, int rows, int tiles, int tile0, int per) {
-        const unsigned row = q4 ? K / 2 : K, run = rows * row;
-        const int two = per || W1 ? 2 : 1;
-        const long long one = (long long)run * two * (q4 ? 9 : 8) / 8;
-        int n = (int)std::min<long long>(tiles, left / one);
-        if (n < tiles) n = n / 8 * 8;
-        if (n <= 0 || a.n + two * (q4 ? 2 : 1) > FEW_REGIONS || (long long)N * row >= 1LL << 32) { left = 0; return; }
-        for (int h = 0; h < two; h++) {
-            const char* W = static_cast<const char*>(h && W1 ? W1 : W0);
-            const unsigned skip = h && per ? per * run : 0;
-            a.r[a.n++] = FewRegion{W + skip, run, N * row - skip, n, tile0, per};
-            if (q4) a.r[a.n++] = FewRegion{W + (size_t)N * row + skip / 8, run / 8, (N * row - skip) / 8, n, tile0, per};
-        }
-        left = n < tiles ? 0 : left - n * one;
-        bytes += n * one;
-    };
-    for (int i = 0; i < nNext; i++) {
-        const FewNext& m = next[i];
-        if (m.mode == FEW_QKV) {
-            const int per = headDim / 32, tq = m.N / 32, tk = m.N1 / 32;
-            take(m.W0, nullptr, m.N, m.K, m.q4, 16, tq, 0, per);
-            take(m.W1, nullptr, m.N1, m.K, m.q4, 16, tk, tq, per);
-            take(m.W2, nullptr, m.N1, m.K, m.q4, 32, tk, tq + tk, 0);
-        } else {
-            const bool two = m.mode == FEW_SWIGLU;
-            const int rows = two ? (few_swiglu_rows(m.N, T, m.K, m.q4, terms) ? 64 : 8 * few_tile(2 * m.N, T, m.K, 2, 8, m.q4, terms).nb) : 16 * few_tile(m.N, T, m.K, 1, 4, m.q4, terms).nb;
-            take(m.W0, m.W1, m.N, m.K, m.q4, rows, (m.N + rows - 1) / rows, 0, 0);
-        }
-    }
-    if (a.n) {
-        a.first = (int)own;
-        a.readers = (int)std::min<long long>(room, (bytes / FEW_AHEAD_LEAST + 8) / 8 * 8);
-    }
-    return a;
-}
-
 hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, int kvHalf, unsigned short* hi, unsigned short* lo,
                                 unsigned short* ext, int T, int pos0, int rowLimit, int dim, int kvDim, int nHeads, int nKVHeads, int headDim, int q4, const FewNext* next,
                                 int nNext, int terms, hipStream_t s) {
@@ -1061,7 +1007,10 @@ hipError_t launch_few_attention(const float* q, const void* Kc, const void* Vc, 
         (headDim != 64 && headDim != 128) || !hi || !lo) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)nHeads * (unsigned)((T + 15) / 16);
     const int cs = grid <= 64 ? 4 : (grid <= 128 ? 2 : 1);              // workgroups a head's 16 queries are shared by: see the kernel
-    const FewAhead ahead = few_plan(grid * cs, next, nNext, T, terms, headDim);
+    const FewAhead ahead = few_plan(grid * cs, next, nNext, headDim, [&](const FewNext& m) {
+        if (m.mode != FEW_SWIGLU) return 16 * few_tile(m.N, T, m.K, 1, 4, m.q4, terms).nb;
+        return few_swiglu_rows(m.N, T, m.K, m.q4, terms) ? 64 : 8 * few_tile(2 * m.N, T, m.K, 2, 8, m.q4, terms).nb;
+    });
     if (headDim == 64) return kvHalf ? launch_few_attn<64, true>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4, ahead)
                                      : launch_few_attn<64, false>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4, ahead);
     return kvHalf ? launch_few_attn<128, true>(cs, grid, s, q, Kc, Vc, hi, lo, ext, T, pos0, dim, kvDim, nHeads, nKVHeads, q4, ahead)

@@ -2,10 +2,20 @@
 // the kernels and the dispatch use these functions, and so do the host tests that walk them over whole matrices and over
 // what was measured.
 #pragma once
+#include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstddef>
 
 namespace mg {
+
+// One launch, tiles of 16 to 128 weight rows x 16 to 64 activation rows a workgroup (few_tile chooses); what follows the
+// product is the epilogue of the mode.
+enum FewMode {
+    FEW_RESID,       // Y += v * scale + bias; optionally the next projection's split of Y * nextGain and the rows' sums of squares
+    FEW_SWIGLU,    // seg0 = gate, seg1 = up: silu(g) * u as the split of the down projection's input
+    FEW_QKV,         // seg0 = q, seg1 = k, seg2 = v: bias, RoPE, q rows to seg0.Y, K / V rows into the caches at pos0 + row
+};
 
 // A lane (quarter fq = lane / 16, index fr = lane % 16 in it) loads a piece of 16 bytes (Q4_0: 8 bytes of nibbles) of a
 // 16-row block of weights: piece few_piece of row few_load_row, so that a quarter wave reads whole 64-k rows.  A row of
@@ -40,6 +50,65 @@ constexpr unsigned few_ahead_at(const FewRegion& r, int xcd, unsigned p, int lan
     const unsigned i = p / few_ahead_per(r), t = (unsigned)((xcd - r.tile0) & 7) + 8 * i, in = ((p - i * few_ahead_per(r)) << 10) + (unsigned)lane * 16;
     const unsigned at = (r.per ? t / r.per * 2 * r.per + t % r.per : t) * r.run + (in < r.run - 16 ? in : r.run - 16);
     return at < r.bytes - 16 ? at : r.bytes - 16;
+}
+
+// What the launches behind an attention launch multiply T rows by, in their order (launch_few_rows: W1 and W2 where the mode has them,
+// N1 their rows): its idle CUs read it into the L2s.
+struct FewNext { FewMode mode; const void* W0; const void* W1; const void* W2; int N, N1, K, q4; };
+// What an attention launch of `grid` workgroups reads ahead.  Up to 200 KB a reading workgroup (100: 0.5B, 200 rows 1,448 us a call
+// against 1,388) and 20 MB (12: 16 rows 777 against 714; past it the 1.1B shape, 44 MB a layer, loses, 16 rows 360 at 12, 371 at 20, 370 at
+// 24); a matrix that does not fit is taken in part, its first tiles.  Readers are the workgroups up to 256, but 96 at least -- they
+// then share CUs with the attention's, which wait more than they load (0.5B, 301 rows, 266 workgroups of attention, with 0 / 32 / 64
+// / 96 / 128 readers 1,908 / 1,896 / 1,849 / 1,814 / 1,799, 200 rows 1,388 / 1,388 / 1,386 / 1,410 / 1,402) -- and no more than
+// have 64 KB each.
+constexpr long long FEW_AHEAD_EACH = 200 << 10, FEW_AHEAD_MOST = 20 << 20, FEW_AHEAD_LEAST = 64 << 10;
+// Planes of Wo, gate | up and down, one a matrix or, in Q4_0, two, and of Q8 q|k|v: one of v, of q and k the halves of their heads.
+constexpr int FEW_REGIONS = 13;
+struct FewAhead { FewRegion r[FEW_REGIONS]; int n, first, readers; };      // first: the launch's first workgroup that reads ahead
+// tileRows(next): the weight rows of a tile of that launch.
+template <class TileRows>
+inline FewAhead few_plan(unsigned grid, const FewNext* next, int nNext, int headDim, TileRows tileRows) {
+    FewAhead a{};
+    a.first = INT_MAX;
+    const unsigned own = (grid + 7) / 8 * 8, room = own + 96 > 256 ? 96 : 256 - own;
+    long long left = std::min(room * FEW_AHEAD_EACH, FEW_AHEAD_MOST), bytes = 0;
+    // one matrix, or two read tile by tile (W1; per: the halves of W0's heads)
+    auto take = [&](const void* W0, const void* W1, int N, int K, int q4, int rows, int tiles, int tile0, int per) {
+        const unsigned row = q4 ? K / 2 : K, run = rows * row;
+        const int two = per || W1 ? 2 : 1;
+        const long long one = (long long)run * two * (q4 ? 9 : 8) / 8;
+        int n = (int)std::min<long long>(tiles, left / one);
+        if (n < tiles) n = n / 8 * 8;
+        if (n <= 0 || a.n + two * (q4 ? 2 : 1) > FEW_REGIONS || (long long)N * row >= 1LL << 32) { left = 0; return; }
+        for (int h = 0; h < two; h++) {
+            const char* W = static_cast<const char*>(h && W1 ? W1 : W0);
+            const unsigned skip = h && per ? per * run : 0;
+            a.r[a.n++] = FewRegion{W + skip, run, N * row - skip, n, tile0, per};
+            if (q4) a.r[a.n++] = FewRegion{W + (size_t)N * row + skip / 8, run / 8, (N * row - skip) / 8, n, tile0, per};
+        }
+        left = n < tiles ? 0 : left - n * one;
+        bytes += n * one;
+    };
+    for (int i = 0; i < nNext; i++) {
+        const FewNext& m = next[i];
+        if (m.mode == FEW_QKV) {
+            // (not in Q4_0, whose ten planes hold a fifteenth of a layer's bytes and take more turns than the other eight: 0.5B, without / with / nothing
+            // read at all, 2 rows 760 / 798 / 757 us a call, 16 795 / 825 / 830, 37 behind 200 887 / 898 / 914, 301 1,637 / 1,656 / 1,633)
+            if (m.q4) break;
+            const int per = headDim / 32, tq = m.N / 32, tk = m.N1 / 32;
+            take(m.W0, nullptr, m.N, m.K, m.q4, 16, tq, 0, per);
+            take(m.W1, nullptr, m.N1, m.K, m.q4, 16, tk, tq, per);
+            take(m.W2, nullptr, m.N1, m.K, m.q4, 32, tk, tq + tk, 0);
+        } else {
+            const int rows = tileRows(m);
+            take(m.W0, m.W1, m.N, m.K, m.q4, rows, (m.N + rows - 1) / rows, 0, 0);
+        }
+    }
+    if (a.n) {
+        a.first = (int)own;
+        a.readers = (int)std::min<long long>(room, (bytes / FEW_AHEAD_LEAST + 8) / 8 * 8);
+    }
+    return a;
 }
 
 // ---- which products take the integer form (few_gemm.hip) ----

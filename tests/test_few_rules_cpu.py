@@ -144,3 +144,69 @@ int main() {
 }
 """)
     assert out == "ok\n", out
+
+
+@pytest.mark.parametrize("q4", [0, 1])
+@pytest.mark.parametrize("dim,kvDim,ffn,head_dim,grid", [(896, 128, 4864, 64, 56), (2048, 256, 5632, 64, 64), (1024, 256, 2816, 128, 250), (256, 256, 96, 64, 16)])
+def test_what_an_attention_launch_reads_ahead(tmp_path, q4, dim, kvDim, ffn, head_dim, grid):
+    """few_plan over a layer's four launches: a layer below the limits is read whole -- every 16 bytes of Wo, gate, up and down and, in Q8,
+    the next layer's q, k and v, weights and scales, on the XCD of their tile -- and of a larger one the matrices in their
+    order, the last one in part, up to the limits; nothing outside a plane."""
+    out = _run(tmp_path, r"""
+#include "few_rules.h"
+#include <cstdint>
+#include <cstdio>
+#include <cstring>
+#include <vector>
+using namespace mg;
+struct Mat { int N, K, rows, tile0, per; std::vector<char> w; std::vector<int> by; };
+int main() {
+    const int q4 = %d, dim = %d, kvDim = %d, ffn = %d, hd = %d, grid = %d, per = hd / 32, tq = dim / 32, tk = kvDim / 32;
+    Mat m[7] = {{dim, dim, 16, 0, 0}, {ffn, dim, 64, 0, 0}, {ffn, dim, 64, 0, 0}, {dim, ffn, 32, 0, 0}, {dim, dim, 16, 0, per}, {kvDim, dim, 16, tq, per}, {kvDim, dim, 32, tq + tk, 0}};
+    long long total = 0;
+    for (auto& x : m) {
+        x.w.resize(q4 ? (size_t)x.N * x.K / 16 * 9 : (size_t)x.N * x.K);
+        x.by.assign(x.w.size() / 16, -1);
+        if (!q4 || &x < m + 4) total += x.w.size();
+    }
+    const FewNext next[4] = {{FEW_RESID, m[0].w.data(), nullptr, nullptr, dim, 0, dim, q4}, {FEW_SWIGLU, m[1].w.data(), m[2].w.data(), nullptr, ffn, 0, dim, q4},
+                             {FEW_RESID, m[3].w.data(), nullptr, nullptr, dim, 0, ffn, q4}, {FEW_QKV, m[4].w.data(), m[5].w.data(), m[6].w.data(), dim, kvDim, dim, q4}};
+    const FewAhead a = few_plan(grid, next, 4, hd, [&](const FewNext& n) { return n.mode == FEW_SWIGLU ? 64 : n.K == dim ? 16 : 32; });
+    if (a.first %% 8 || a.first < grid || a.readers %% 8 || a.readers < 8) return std::puts("workgroups"), 0;
+    for (int x = 0; x < 8; x++)
+        for (int r = 0; r < a.n; r++)
+            for (unsigned p = 0; p < few_ahead_pieces(a.r[r], x); p++)
+                for (int lane = 0; lane < 64; lane++) {
+                    const char* at = a.r[r].base + few_ahead_at(a.r[r], x, p, lane);
+                    int in = -1;
+                    for (int i = 0; i < 7; i++) if (at >= m[i].w.data() && at + 16 <= m[i].w.data() + m[i].w.size()) in = i;
+                    if (in < 0 || (at - m[in].w.data()) %% 16) return std::puts("outside"), 0;
+                    int& by = m[in].by[(at - m[in].w.data()) / 16];
+                    if (by < 0) by = x;
+                }
+    const long long most = std::min((grid + 7) / 8 * 8 + 96 > 256 ? 96 : 256 - (grid + 7) / 8 * 8, 1 << 20) * FEW_AHEAD_EACH;
+    const bool whole = total <= std::min(most, FEW_AHEAD_MOST);
+    long long read = 0;
+    bool cut = false;
+    for (int i = 0; i < 7; i++) {
+        Mat& x = m[i];
+        const size_t row = q4 ? x.K / 2 : x.K;
+        size_t got = 0;
+        for (size_t b = 0; b < x.w.size(); b += 16) {
+            if (x.by[b / 16] < 0) continue;
+            got += 16;
+            const size_t nr = b < x.N * row ? b / row : (b - x.N * row) / (x.K / 16);
+            if (q4 && b >= x.N * row && x.K %% 256) continue;          // (16 bytes of scales of more than a row)
+            const size_t tile = x.per ? nr / 16 / (2 * x.per) * x.per + nr / 16 %% x.per : nr / x.rows;
+            if (x.by[b / 16] != (int)((tile + x.tile0) %% 8)) return std::printf("matrix %%d row %%zu: XCD %%d\n", i, nr, x.by[b / 16]), 0;
+        }
+        read += got;
+        if (got && cut && i != 2) return std::puts("order"), 0;        // (up goes with gate)
+        if (q4 && i >= 4) { if (got) return std::puts("q|k|v"), 0; continue; }
+        if (got < x.w.size()) { cut = true; if (whole) return std::printf("matrix %%d: %%zu of %%zu bytes\n", i, got, x.w.size()), 0; }
+    }
+    if (read > std::min(most, FEW_AHEAD_MOST) || (!whole && 10 * read < 9 * std::min(most, FEW_AHEAD_MOST))) return std::printf("%%lld of %%lld bytes\n", read, total), 0;
+    std::puts("ok");
+}
+""" % (q4, dim, kvDim, ffn, head_dim, grid))
+    assert out == "ok\n", out
