@@ -720,7 +720,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
         p.trace[((size_t)(l - p.l0) * FLOW_TRACE_SLOTS + (b)) * nC + blockIdx.x] = wall_clock64(); } } while (0)
     // the exchange area as a buffer resource: agent-scope loads that the compiler keeps track of (used where many are
     // wanted in flight together)
-    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(p.xchg, 0, (int)((size_t)p.nLayersTotal * G.stride * 4 * (p.nTokens > 0 ? 2 : 1)), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(p.xchg, 0, (int)((size_t)p.nLayersTotal * (G.stride + G.pairs) * 4 * (p.nTokens > 0 ? 2 : 1)), 0x00020000);
     unsigned lw = layer_words(p.layers, p.l0, lane);
 
     // Token mode (p.nTokens > 0): the launch runs whole tokens -- the embedding of the token in the device state, all
@@ -739,7 +739,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     const int nPrompt = imm ? p.nPromptImm : (tokens ? p.state->nPrompt : 0);
     // the token chosen at position np - 1 is entry hist0 + np of the history (np >= nPrompt)
     const int hist0 = (tokens && !imm ? p.state->count : 0) - max(pos + 1, nPrompt);
-    const size_t halfFloats = (size_t)p.nLayersTotal * G.stride;
+    const size_t blockFloats = (size_t)p.nLayersTotal * G.stride, halfFloats = (size_t)p.nLayersTotal * (G.stride + G.pairs);
     float* const xemb = reinterpret_cast<float*>(a4) + (dim > ffn ? dim : ffn);      // the token's embedding (token mode)
     for (int tk = 0; tk < nTok; tk++) {
         // Nothing that depends on the thread or on the shape is to be computed once for all tokens and kept in registers
@@ -1209,7 +1209,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                     if (PAIRS && nsplit > 1 && lane < 16) {
                                         const f2 ml = {canon(mg_), canon(lg)};
                                         asm volatile("global_store_dwordx2 %0, %1, off sc1" : :
-                                                     "v"(reinterpret_cast<f2*>(X + G.offMl + (size_t)split * (dim >> 1) + h0 * (HD / 2)) + i + 16 * j), "v"(ml) : "memory");
+                                                     "v"(reinterpret_cast<f2*>(xb + blockFloats + (size_t)l * G.pairs + (size_t)split * (dim >> 1) + h0 * (HD / 2)) + i + 16 * j), "v"(ml) : "memory");
                                     }
                                 }
                                 if (lane == 0) { stx(X + G.offPm + split * nHeadsV + h0, mg_); stx(X + G.offPl + split * nHeadsV + h0, lg); }
@@ -1398,7 +1398,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                             const bool on = u < nbt;
                                             const int sp = g + (k0 + u) * NG;
                                             pa[u] = on ? reinterpret_cast<const f4*>(X + G.offPacc + (size_t)sp * dim) + i : wt.idle;
-                                            pq[u] = on ? reinterpret_cast<const f2*>(X + G.offMl + (size_t)sp * (dim >> 1)) + i : idle2p;
+                                            pq[u] = on ? reinterpret_cast<const f2*>(xb + blockFloats + (size_t)l * G.pairs + (size_t)sp * (dim >> 1)) + i : idle2p;
                                         }
                                         poll_pairs(pa, pq, a, q, nbt, wt);
 #pragma unroll
@@ -1766,10 +1766,12 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                 for (int i = 0; i < NRT; i++) acc[i] = 0.f;
             };
             auto resetOther = [&]() {
-                // the other half of the exchange area, and this workgroup's argmax slot there, for the token after this one
+                // the other half of the exchange area -- the pairs only where they are written: they are half as much again as the
+                // blocks (0.5B shape, fp16 rows, at 20 / 900 positions 293.6 / 361.6 -> 292.0 / 359.4 us a token, Q8 at 20 271.4 -> 270.7) --
+                // and this workgroup's argmax slot there, for the token after this one
                 const f4 sent = {__builtin_bit_cast(float, XSENT), __builtin_bit_cast(float, XSENT), __builtin_bit_cast(float, XSENT), __builtin_bit_cast(float, XSENT)};
                 f4* o4 = reinterpret_cast<f4*>(p.xchg + (size_t)(np & 1) * halfFloats);
-                for (size_t i = (size_t)blockIdx.x * FWG + tid; i < halfFloats / 4; i += (size_t)gridDim.x * FWG)
+                for (size_t i = (size_t)blockIdx.x * FWG + tid; i < (PAIRS ? halfFloats : blockFloats) / 4; i += (size_t)gridDim.x * FWG)
                     asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(o4 + i), "v"(sent) : "memory");
                 if (tid == 0) {
                     st_agent(amax + ((size_t)(np & 1) * gridDim.x + blockIdx.x) * FLOW_AMAX_STRIDE, sent.x);
@@ -1973,14 +1975,13 @@ FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads
     int o = g.offPacc + up64(g.smax * dim);
     g.offPm = o; o += up64(g.smax * nHeads);
     g.offPl = o; o += up64(g.smax * nHeads);
+    g.stride = o;
     // (the plain variant alone merges by the pairs: of a grouped geometry the splits that one reaches)
-    g.offMl = o;
-    for (int k = 1; k <= 3; k++) {
+    for (int k = 1; k <= 3 && want >= FLOW_MANY_SPLITS; k++) {
         const FlowFixedShape f = flow_fixed_shape(k);
         if (f.pairs && f.dim == dim && f.kvDim == kvDim && f.ffn == ffn && f.nHeads == nHeads && f.nKVHeads == nKVHeads && f.headDim == headDim)
-            o += up64((g.gqa ? std::min(g.smax, (grid + nHeads - 1) / nHeads) : g.smax) * (dim / 2));
+            g.pairs = up64((g.gqa ? std::min(g.smax, (grid + nHeads - 1) / nHeads) : g.smax) * (dim / 2));
     }
-    g.stride = o;
     return g;
 }
 
@@ -2018,13 +2019,27 @@ bool flow_shape_supported(int dim, int kvDim, int ffn, int nHeads, int nKVHeads,
     return true;
 }
 
+// The variant with a known shape's sizes compiled in (launches of exactly that shape, unless switched off), or 0.
+static int flow_fixed(const FlowParams& p, int grid) {
+    if (p.generic) return 0;
+    for (int k = 1; k <= 3; k++) {
+        const FlowFixedShape fs = flow_fixed_shape(k);
+        if (p.dim == fs.dim && p.kvDim == fs.kvDim && p.ffn == fs.ffn && p.nHeads == fs.nHeads && p.nKVHeads == fs.nKVHeads &&
+            p.headDim == fs.headDim && (p.downSplit != 0) == (fs.downSplit != 0) && (p.nCompute != grid) == (fs.dedicated != 0)) return k;
+    }
+    return 0;
+}
+bool flow_merges_pairs(const FlowParams& p, int grid) {
+    return flow_fixed_shape(flow_fixed(p, grid)).pairs && !p.kvHalf && !(p.geo.gqa && p.gqaCode) && p.mostSplits >= FLOW_MANY_SPLITS;
+}
+
 hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
     if (!flow_shape_supported(p.dim, p.kvDim, p.ffn, p.nHeads, p.nKVHeads, p.headDim)) return hipErrorInvalidValue;
     const int nC = p.nCompute;
     if (nC <= 0 || nC > grid || ((grid - nC) && (nC % 8 || (grid - nC) % 8))) return hipErrorInvalidValue;
     if (p.l0 < 0 || p.l1 <= p.l0 || p.l1 > p.nLayersTotal || nC < flow_min_grid(p.nHeads, p.nKVHeads, p.geo) ||
         !flow_context_fits(p.maxSeq, p.geo) || !p.layers || !p.xchg || !p.err || !p.hidden ||
-        !flow_grid_fits(p.ffn, p.nHeads, p.geo, nC) || (size_t)p.nLayersTotal * p.geo.stride * 4 >= (1ull << 31))
+        !flow_grid_fits(p.ffn, p.nHeads, p.geo, nC) || flow_half_floats(p.geo, p.nLayersTotal) * 4 >= (1ull << 31))
         return hipErrorInvalidValue;
     if (p.nTokens > 0 && (!p.tail || !p.state || p.l0 != 0 || p.l1 != p.nLayersTotal || p.nTokens > p.maxSeq ||
                           flow_lds_bytes(p.dim, p.ffn, p.headDim, p.geo.gqa, true) > ((size_t)160 << 10)))
@@ -2037,14 +2052,7 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
 #define FLOW_LAUNCH_G(HDv, CBv, RGv) do { \
         if (p.q4) { if (gqa) FLOW_LAUNCH(HDv, CBv, RGv, true, true); else FLOW_LAUNCH(HDv, CBv, RGv, false, true); } \
         else { if (gqa) FLOW_LAUNCH(HDv, CBv, RGv, true, false); else FLOW_LAUNCH(HDv, CBv, RGv, false, false); } } while (0)
-    // the variants with a known shape's sizes compiled in (launches of exactly that shape, unless switched off)
-    int fix = 0;
-    if (!p.generic)
-        for (int k = 1; k <= 3 && !fix; k++) {
-            const FlowFixedShape fs = flow_fixed_shape(k);
-            if (p.dim == fs.dim && p.kvDim == fs.kvDim && p.ffn == fs.ffn && p.nHeads == fs.nHeads && p.nKVHeads == fs.nKVHeads &&
-                p.headDim == fs.headDim && (p.downSplit != 0) == (fs.downSplit != 0) && (nC != grid) == (fs.dedicated != 0)) fix = k;
-        }
+    const int fix = flow_fixed(p, grid);
 #define FLOW_LAUNCH_F(HDv, CBv, RGv, GQv, Q4v, FXv) do { \
         if (p.trace) hipLaunchKernelGGL((flow_layers_kernel<HDv, CBv, RGv, GQv, Q4v, true, FXv>), dim3(grid), dim3(FWG), lds, s, p); \
         else hipLaunchKernelGGL((flow_layers_kernel<HDv, CBv, RGv, GQv, Q4v, false, FXv>), dim3(grid), dim3(FWG), lds, s, p); } while (0)
@@ -2052,7 +2060,7 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
         // Many splits, shared out among groups of threads and merged by pairs (see PAIRS); us a token without / with, Q8 at 600 (five
         // splits) 340.1 / 340.0, 900 371.7 / 360.1, 1,300 400.0 / 373.6, 1,900 439.9 / 395.1, but at 20 291.8 / 300.3 and 320 316.3 / 327.9 for
         // the registers the code costs; Q4_0 at 320 (three) 317.0 / 320.4, 600 340.5 / 342.1, 900 369.9 / 356.2, 1,900 440.8 / 391.5.
-        if (p.mostSplits >= FLOW_MANY_SPLITS) {
+        if (flow_merges_pairs(p, grid)) {
             if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 33);
             else FLOW_LAUNCH_F(64, 1, false, false, false, 33);
         } else if (p.q4) FLOW_LAUNCH_F(64, 1, false, false, true, 1);
@@ -2086,33 +2094,34 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
     return hipGetLastError();
 }
 
-__global__ void flow_reset_kernel(uint4* x, size_t n4, const float* hiddenIn, float* hidden, int dim) {
+__global__ void flow_reset_kernel(uint4* x, size_t n4, uint4* x2, size_t m4, const float* hiddenIn, float* hidden, int dim) {
     // (hiddenIn is page-locked host memory, a microsecond and a half away: one load a thread)
     if (hiddenIn)
         for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < dim / 4; i += gridDim.x * blockDim.x)
             reinterpret_cast<float4*>(hidden)[i] = reinterpret_cast<const float4*>(hiddenIn)[i];
     const uint4 sent = make_uint4(XSENT, XSENT, XSENT, XSENT);
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) x[i] = sent;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m4; i += (size_t)gridDim.x * blockDim.x) x2[i] = sent;
 }
-hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, const float* hiddenIn, float* hidden, int dim, hipStream_t s) {
+hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int nLayers, int l0, int l1, bool pairs, const float* hiddenIn, float* hidden, int dim, hipStream_t s) {
     if (l1 <= l0) return hipSuccess;
-    const size_t n4 = (size_t)(l1 - l0) * g.stride / 4;
+    const size_t n4 = (size_t)(l1 - l0) * g.stride / 4, m4 = pairs ? (size_t)(l1 - l0) * g.pairs / 4 : 0;
     size_t blocks = (n4 + WG - 1) / WG;
     if (blocks > 1024) blocks = 1024;
-    hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s,
-                       reinterpret_cast<uint4*>(xchg + (size_t)l0 * g.stride), n4, hiddenIn, hidden, dim);
+    hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s, reinterpret_cast<uint4*>(xchg + (size_t)l0 * g.stride), n4,
+                       reinterpret_cast<uint4*>(xchg + flow_block_floats(g, nLayers) + (size_t)l0 * g.pairs), m4, hiddenIn, hidden, dim);
     return hipGetLastError();
 }
 
 size_t flow_xchg_floats(const FlowGeometry& g, int nLayers, int grid) {
-    return (size_t)2 * nLayers * g.stride + (size_t)2 * grid * FLOW_AMAX_STRIDE;
+    return 2 * flow_half_floats(g, nLayers) + (size_t)2 * grid * FLOW_AMAX_STRIDE;
 }
 hipError_t launch_flow_reset_all(float* xchg, const FlowGeometry& g, int nLayers, int grid, hipStream_t s) {
     const size_t n4 = flow_xchg_floats(g, nLayers, grid) / 4;
     size_t blocks = (n4 + WG - 1) / WG;
     if (blocks > 1024) blocks = 1024;
     hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s, reinterpret_cast<uint4*>(xchg), n4,
-                       static_cast<const float*>(nullptr), static_cast<float*>(nullptr), 0);
+                       static_cast<uint4*>(nullptr), (size_t)0, static_cast<const float*>(nullptr), static_cast<float*>(nullptr), 0);
     return hipGetLastError();
 }
 size_t flow_lds_bytes(int dim, int ffn, int headDim, int gqa, bool tokenMode) {

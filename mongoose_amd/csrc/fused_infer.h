@@ -243,7 +243,7 @@ private:
     bool flowTailEligible() const;
     FlowTail* dFlowTail = nullptr;
     int enqueueTokensFlow(int nTokens, int pos = 0, int token = -1, int nPrompt = 0);
-    int flowClean = 0;              // halves of the exchange area known to be as a reset leaves them (bits 0 and 1)
+    int flowClean = 0;              // halves of the exchange area known to be as a reset leaves them: bits 0 and 1 the blocks, 2 and 3 the pairs
     unsigned* hOut = nullptr;       // pinned: error word, flags of the slices from word 64, ints and floats at the offsets below
     int hOutInts = 0, hOutFloats = 0;
     unsigned hOutSeq = 0;

@@ -821,7 +821,7 @@ int HIPFusedInference::flowComputeWgs(int cus) const {
         const FlowGeometry g = flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, nC, cus);
         // (the same limits as launch_flow_layers checks: a shape it would refuse runs the fused launches instead)
         if (flow_min_grid(nHeads, nKVHeads, g) <= nC && flow_context_fits(maxSeq, g) && flow_grid_fits(ffnDim, nHeads, g, nC) &&
-            (size_t)nLayers * g.stride * 4 < (1ull << 31)) return nC;
+            flow_half_floats(g, nLayers) * 4 < (1ull << 31)) return nC;
     }
     return 0;
 }
@@ -871,7 +871,7 @@ int HIPFusedInference::ensureFlow() {
         HIPCHK(hipMalloc(&v, sizeof(float) * flow_xchg_floats(flowGeo, nLayers, flowGrid)));
         flowXchg = static_cast<float*>(v);
         HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
-        flowClean = 3;
+        flowClean = 15;
         HIPCHK(hipMalloc(&v, sizeof(FlowTail)));
         dFlowTail = static_cast<FlowTail*>(v);
         HIPCHK(hipMalloc(&v, FLOW_ERR_BYTES));
@@ -1008,6 +1008,7 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
     p.xchg = flowXchg; p.geo = flowGeo;
     p.err = dFlowErr;
     p.limitTicks = flowLimitTicks;
+    bool pairs = false;
     {
         // the last position this launch can reach, where the host knows it: the plain attention variant serves while it is the faster
         // one, also in a context laid out for grouped attention; where the position is not known, in contexts that it covers
@@ -1020,21 +1021,23 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
         p.gqaCode = grouped ? plainMost : 0;
         p.mostSplits = posMax < 0 ? 0 : (int)(posMax / FLOW_TILE) + 1;
         p.generic = flowGeneric ? 1 : 0;
+        pairs = flow_merges_pairs(p, flowGrid);
+        const int written = pairs ? 5 : 1;
         // the half of the exchange area a run of whole tokens starts in has to be as a reset leaves it: the launch before
         // left the half of its last position's successor so (DecodeToken at consecutive positions resets nothing)
         if (nTokens > 0 && !capturing) {
-            const int need = statePosHost >= 0 ? 1 << (statePosHost & 1) : 3;
-            if ((flowClean & need) != need) HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
-            flowClean = statePosHost >= 0 ? 1 << ((statePosHost + nTokens) & 1) : 0;
+            const int need = (statePosHost >= 0 ? 1 << (statePosHost & 1) : 3) * written;
+            if ((flowClean & need) != need) { HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream)); flowClean = 15; }
+            flowClean = (flowClean & ~(3 * written)) | (statePosHost >= 0 ? (1 << ((statePosHost + nTokens) & 1)) * written : 0);
         } else {
-            flowClean &= ~1;                                                          // (layers only: the first half)
+            flowClean &= ~written;                                                    // (layers only: the first half)
         }
         if (st && nTokens > 0 && statePosHost >= 0) statePosHost += nTokens;          // whole tokens advance the device state
         else if (st) statePosHost = -1;                                               // (what follows this launch advances it)
     }
     p.trace = flowTrace;
     if (nTokens > 0) { p.nTokens = nTokens; p.tail = dFlowTail; }
-    if (resetFirst) HIPCHK(launch_flow_reset(flowXchg, flowGeo, l0, l1, hiddenIn, hidden[hiddenIdx], dim, stream));
+    if (resetFirst) HIPCHK(launch_flow_reset(flowXchg, flowGeo, nLayers, l0, l1, pairs, hiddenIn, hidden[hiddenIdx], dim, stream));
     if (mark(1)) return MG_E_HIP;
     if (capturing) { HIPCHK(launch_flow_layers(p, flowGrid, stream)); return MG_OK; }      // (the replay takes the turn)
     std::lock_guard<std::mutex> lk(flowTurnMutex());
@@ -1077,7 +1080,7 @@ int HIPFusedInference::setState(int pos, int token, int count, int nPrompt) {
     statePosHost = pos;
     if (flowXchg && (execMode == 3 || execMode == 4)) {
         HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
-        flowClean = 3;
+        flowClean = 15;
     }
     return MG_OK;
 }
@@ -1213,7 +1216,7 @@ int HIPFusedInference::enqueueFinal(bool withArgmax, int* parts, const float* ro
         // inside the captured token: the lm_head launch also leaves the exchange area of the persistent
         // layer launch in its "nothing written yet" state for the next token (one launch saved)
         p.xreset = reinterpret_cast<unsigned*>(flowXchg);
-        p.xresetWords = (unsigned)((size_t)nLayers * flowGeo.stride);
+        p.xresetWords = (unsigned)flow_block_floats(flowGeo, nLayers);
     }
     MvConfig c{0, 0, 0};
     if (mark(6)) return MG_E_HIP;
@@ -1384,9 +1387,9 @@ int HIPFusedInference::primeGraph() {
     // A captured token resets nothing before it reads: it finds its half of the exchange area as the token before it left
     // it.  The first one of a run finds it so from here, whatever ran before (setState has done it already where that was
     // called; a prefill does not touch the area, and eager launches leave a half of it written).
-    if (graphsUseFlow && flowClean != 3) {
+    if (graphsUseFlow && (flowClean & 3) != 3) {
         HIPCHK(launch_flow_reset_all(flowXchg, flowGeo, nLayers, flowGrid, stream));
-        flowClean = 3;
+        flowClean = 15;
     }
     return enqueueEmbed();
 }
@@ -1417,7 +1420,7 @@ int HIPFusedInference::enqueueToken(bool withHead) {
     // no lm_head launch to leave the exchange area reset for the next launch: a captured prompt step does it itself,
     // and so does any prompt step where whole tokens run in the launch (they expect to find it so)
     if (flow && (fuseEmbed || flowTailEligible())) {
-        HIPCHK(launch_flow_reset(flowXchg, flowGeo, 0, nLayers, nullptr, nullptr, 0, stream));
+        HIPCHK(launch_flow_reset(flowXchg, flowGeo, nLayers, 0, nLayers, !capturing, nullptr, nullptr, 0, stream));
         if (!capturing) flowClean = clean;          // (the layers' launch wrote the first half only)
     }
     return MG_OK;

@@ -334,6 +334,51 @@ def test_many_splits_of_a_known_shape(hip, fmt, maxSeq, positions, first):
     m.close()
 
 
+def test_pairs_are_reset_by_the_launches_that_write_them(hip):
+    """0.5B shape: the (maximum, sum) pairs that launches of many KV splits merge by lie behind the layers' blocks, so that other launches
+    have none to reset (a block ends with the splits' sums), and come out as first written whatever ran in between: shorter
+    positions, the same again, layer ranges, runs of tokens across the line -- against the variants without pairs, in the same order
+    (bar as above)."""
+    s = H.with_layers(configs.QWEN, 2)._replace(vocab=2048)
+    m = H.Model(s, seed=47, maxSeq=2048, eng=hip, oracle=False)
+    toks = m.prompt(1100)
+    outs = {}
+    for generic in (0, 1):
+        assert m.hip.SetFlowGeneric(generic) == 0 and m.hip.ResetKV() == 0
+        for p in range(0, 1100, 500):
+            assert m.hip.Prefill(toks[p:min(1100, p + 500)], p)[0] == 0, E.last_error()
+        outs[generic] = []
+
+        def token(pos):
+            logits = np.empty(s.vocab, np.float32)
+            rc, nxt = m.hip.DecodeToken(int(toks[pos]), pos, logits)
+            assert rc == 0 and m.hip.FlowInUse(), E.last_error()
+            outs[generic].append(logits)
+
+        for pos in (1000, 1001, 1002, 30, 1000, 31, 32, 1001, 700, 702, 701, 639, 640, 641):
+            token(pos)
+        for pos in (1003, 40, 1003):
+            x = 0.02 * np.arange(s.dim, dtype=np.float32) / s.dim
+            for first, last in ((0, 2), (0, 1), (1, 2)):
+                out = np.empty(s.vocab if last == 2 else s.dim, np.float32)
+                hidden, logits = (None, out) if last == 2 else (out, None)
+                assert m.hip.PartialStep(x, pos, first, last, hidden, logits) == 0, E.last_error()
+                outs[generic].append(out)
+            token(pos + 1)
+            token(pos + 2)
+        rc, run = m.hip.GeneratePrefill(toks[:615], 50)
+        assert rc == 0, E.last_error()
+        outs[generic].append(run.astype(np.float32))
+        token(1050)
+    for i, (a, b) in enumerate(zip(outs[0], outs[1])):
+        assert H.rel_err(a, b) < 1e-5, i
+    geo = np.zeros(11, np.int32)
+    assert E.lib.mg_flow_exchange(m.hip._h, 0, None, 0, E._ip(geo)) == 0
+    stride, opl, smax = int(geo[0]), int(geo[6]), int(geo[10])
+    assert stride - opl == (smax * s.nHeads + 63) // 64 * 64
+    m.close()
+
+
 def test_heads_of_128_grouped_kv(hip):
     """Llama-3-8B attention geometry (32 query heads of 128 on 8 KV heads, dim 4096: rows of two chunks a lane), 2
     layers, FFN and vocabulary cut: 8 partial slots, tile 128."""
