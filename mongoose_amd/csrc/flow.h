@@ -55,7 +55,7 @@ struct FlowGeometry {
     int stride;
     int offQ, offKc, offVc, offPacc, offPm, offPl, offX1, offM, offX2, offAttn;
     int pairs;       // (maximum, sum) of a split's head for every 16-byte piece of its accumulator, for the variant that merges by them: floats
-                     // a layer, behind all layers' blocks (0: no launch of this shape does); what it alone writes it alone resets
+                     // a layer (0: no launch of this shape does), in an area of their own that it alone resets
     int smax;
     int gqa;         // 1: an attention workgroup per (KV head, split) taking all its query heads; 0: per (query head, split)
 };
@@ -64,9 +64,6 @@ FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads
 // Attention workgroups, one a query head and KV split, up to which a launch that can group query heads does not.
 int flow_plain_most(int nC, int cus, int nHeads, int dim);
 bool flow_context_fits(int maxSeq, const FlowGeometry& g);
-// Floats of all layers' blocks, and with the pairs behind them (half of the exchange area).
-inline size_t flow_block_floats(const FlowGeometry& g, int nLayers) { return (size_t)nLayers * g.stride; }
-inline size_t flow_half_floats(const FlowGeometry& g, int nLayers) { return (size_t)nLayers * (g.stride + g.pairs); }
 
 constexpr size_t FLOW_ERR_BYTES = 4096;
 constexpr int FLOW_AMAX_STRIDE = 32;   // floats between two workgroups' argmax slots: a 128-byte line each
@@ -127,13 +124,15 @@ bool flow_grid_fits(int ffn, int nHeads, const FlowGeometry& g, int nCompute);
 hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s);
 // That launch merges KV splits by pairs: it expects them reset as well, and in token mode resets the other half's for its successor.
 bool flow_merges_pairs(const FlowParams& p, int grid);
-// Fills the blocks of layers [l0, l1) (of the first half), with pairs set also their pairs, with the "not written yet" pattern.
+// Fills the blocks of layers [l0, l1) (of the first half), and their pairs if given that area, with the "not written yet" pattern.
 // hiddenIn != NULL: also dim floats of (page-locked host) memory into hidden.
-hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int nLayers, int l0, int l1, bool pairs, const float* hiddenIn, float* hidden, int dim, hipStream_t s);
-// Floats of the whole exchange allocation: two halves of nLayers blocks and their pairs (token mode alternates between them; launches
-// over a range of layers use the first) and the argmax exchange [2][grid] pairs behind them.
+hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, float* pairs, const float* hiddenIn, float* hidden, int dim, hipStream_t s);
+// Floats of the whole exchange allocation: two halves of nLayers blocks (token mode alternates between them; launches
+// over a range of layers use the first) and behind them the argmax exchange, [2][grid]
+// slots, and the pairs, two halves as well.
 size_t flow_xchg_floats(const FlowGeometry& g, int nLayers, int grid);
-inline float* flow_amax_area(float* xchg, const FlowGeometry& g, int nLayers) { return xchg + 2 * flow_half_floats(g, nLayers); }
+inline float* flow_amax_area(float* xchg, const FlowGeometry& g, int nLayers) { return xchg + (size_t)2 * nLayers * g.stride; }
+inline float* flow_pairs_area(float* xchg, const FlowGeometry& g, int nLayers, int grid) { return flow_amax_area(xchg, g, nLayers) + (size_t)2 * grid * FLOW_AMAX_STRIDE; }
 // ... all of it (before a token-mode launch that does not find its half as another left it).
 hipError_t launch_flow_reset_all(float* xchg, const FlowGeometry& g, int nLayers, int grid, hipStream_t s);
 // LDS a workgroup of the launch takes (an upper bound: dynamic part plus the variant's own arrays); token mode keeps

@@ -720,7 +720,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
         p.trace[((size_t)(l - p.l0) * FLOW_TRACE_SLOTS + (b)) * nC + blockIdx.x] = wall_clock64(); } } while (0)
     // the exchange area as a buffer resource: agent-scope loads that the compiler keeps track of (used where many are
     // wanted in flight together)
-    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(p.xchg, 0, (int)((size_t)p.nLayersTotal * (G.stride + G.pairs) * 4 * (p.nTokens > 0 ? 2 : 1)), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(p.xchg, 0, (int)((size_t)p.nLayersTotal * G.stride * 4 * (p.nTokens > 0 ? 2 : 1)), 0x00020000);
     unsigned lw = layer_words(p.layers, p.l0, lane);
 
     // Token mode (p.nTokens > 0): the launch runs whole tokens -- the embedding of the token in the device state, all
@@ -739,7 +739,9 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
     const int nPrompt = imm ? p.nPromptImm : (tokens ? p.state->nPrompt : 0);
     // the token chosen at position np - 1 is entry hist0 + np of the history (np >= nPrompt)
     const int hist0 = (tokens && !imm ? p.state->count : 0) - max(pos + 1, nPrompt);
-    const size_t blockFloats = (size_t)p.nLayersTotal * G.stride, halfFloats = (size_t)p.nLayersTotal * (G.stride + G.pairs);
+    const size_t halfFloats = (size_t)p.nLayersTotal * G.stride;
+    // (of the variant with PAIRS alone: a value computed here, even one that is not used, changes the registers of the others)
+    auto pairsOf = [&](int parity, int layer) { return p.xchg + 2 * halfFloats + (size_t)2 * gridDim.x * FLOW_AMAX_STRIDE + ((size_t)parity * p.nLayersTotal + layer) * G.pairs; };
     float* const xemb = reinterpret_cast<float*>(a4) + (dim > ffn ? dim : ffn);      // the token's embedding (token mode)
     for (int tk = 0; tk < nTok; tk++) {
         // Nothing that depends on the thread or on the shape is to be computed once for all tokens and kept in registers
@@ -1209,7 +1211,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                     if (PAIRS && nsplit > 1 && lane < 16) {
                                         const f2 ml = {canon(mg_), canon(lg)};
                                         asm volatile("global_store_dwordx2 %0, %1, off sc1" : :
-                                                     "v"(reinterpret_cast<f2*>(xb + blockFloats + (size_t)l * G.pairs + (size_t)split * (dim >> 1) + h0 * (HD / 2)) + i + 16 * j), "v"(ml) : "memory");
+                                                     "v"(reinterpret_cast<f2*>(pairsOf(tokens ? pos & 1 : 0, l) + (size_t)split * (dim >> 1) + h0 * (HD / 2)) + i + 16 * j), "v"(ml) : "memory");
                                     }
                                 }
                                 if (lane == 0) { stx(X + G.offPm + split * nHeadsV + h0, mg_); stx(X + G.offPl + split * nHeadsV + h0, lg); }
@@ -1387,6 +1389,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                 const int cnt = NG == 1 ? ns : (ns - g + NG - 1) / NG;          // this group's splits: g, g + NG, ...
                                 if constexpr (PAIRS) {
                                     const f2* idle2p = reinterpret_cast<const f2*>(wt.idle);
+                                    const float* const xp = pairsOf(tokens ? pos & 1 : 0, l);
                                     for (int k0 = 0; k0 < cnt; k0 += PB) {
                                         const int nbt = min(PB, cnt - k0);
                                         const f4* pa[PB];
@@ -1398,7 +1401,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                                             const bool on = u < nbt;
                                             const int sp = g + (k0 + u) * NG;
                                             pa[u] = on ? reinterpret_cast<const f4*>(X + G.offPacc + (size_t)sp * dim) + i : wt.idle;
-                                            pq[u] = on ? reinterpret_cast<const f2*>(xb + blockFloats + (size_t)l * G.pairs + (size_t)sp * (dim >> 1)) + i : idle2p;
+                                            pq[u] = on ? reinterpret_cast<const f2*>(xp + (size_t)sp * (dim >> 1)) + i : idle2p;
                                         }
                                         poll_pairs(pa, pq, a, q, nbt, wt);
 #pragma unroll
@@ -1766,13 +1769,19 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
                 for (int i = 0; i < NRT; i++) acc[i] = 0.f;
             };
             auto resetOther = [&]() {
-                // the other half of the exchange area -- the pairs only where they are written: they are half as much again as the
-                // blocks (0.5B shape, fp16 rows, at 20 / 900 positions 293.6 / 361.6 -> 292.0 / 359.4 us a token, Q8 at 20 271.4 -> 270.7) --
-                // and this workgroup's argmax slot there, for the token after this one
+                // the other half of the exchange area -- the pairs only where they are written: they are half as much again as the blocks
+                // (0.5B shape at 20 positions, fp16 rows 293.6 -> 292.2 us a token, Q8 271.4 -> 270.7) -- and this workgroup's
+                // argmax slot there, for the token after this one
                 const f4 sent = {__builtin_bit_cast(float, XSENT), __builtin_bit_cast(float, XSENT), __builtin_bit_cast(float, XSENT), __builtin_bit_cast(float, XSENT)};
                 f4* o4 = reinterpret_cast<f4*>(p.xchg + (size_t)(np & 1) * halfFloats);
-                for (size_t i = (size_t)blockIdx.x * FWG + tid; i < (PAIRS ? halfFloats : blockFloats) / 4; i += (size_t)gridDim.x * FWG)
+                for (size_t i = (size_t)blockIdx.x * FWG + tid; i < halfFloats / 4; i += (size_t)gridDim.x * FWG)
                     asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(o4 + i), "v"(sent) : "memory");
+                if constexpr (PAIRS) {
+                    f4* q4 = reinterpret_cast<f4*>(pairsOf(np & 1, 0));
+                    const size_t n4 = (size_t)p.nLayersTotal * G.pairs / 4;
+                    for (size_t i = (size_t)blockIdx.x * FWG + tid; i < n4; i += (size_t)gridDim.x * FWG)
+                        asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(q4 + i), "v"(sent) : "memory");
+                }
                 if (tid == 0) {
                     st_agent(amax + ((size_t)(np & 1) * gridDim.x + blockIdx.x) * FLOW_AMAX_STRIDE, sent.x);
                     st_agent(amax + ((size_t)(np & 1) * gridDim.x + blockIdx.x) * FLOW_AMAX_STRIDE + 1, sent.x);
@@ -2039,7 +2048,7 @@ hipError_t launch_flow_layers(const FlowParams& p, int grid, hipStream_t s) {
     if (nC <= 0 || nC > grid || ((grid - nC) && (nC % 8 || (grid - nC) % 8))) return hipErrorInvalidValue;
     if (p.l0 < 0 || p.l1 <= p.l0 || p.l1 > p.nLayersTotal || nC < flow_min_grid(p.nHeads, p.nKVHeads, p.geo) ||
         !flow_context_fits(p.maxSeq, p.geo) || !p.layers || !p.xchg || !p.err || !p.hidden ||
-        !flow_grid_fits(p.ffn, p.nHeads, p.geo, nC) || flow_half_floats(p.geo, p.nLayersTotal) * 4 >= (1ull << 31))
+        !flow_grid_fits(p.ffn, p.nHeads, p.geo, nC) || (size_t)p.nLayersTotal * p.geo.stride * 4 >= (1ull << 31))
         return hipErrorInvalidValue;
     if (p.nTokens > 0 && (!p.tail || !p.state || p.l0 != 0 || p.l1 != p.nLayersTotal || p.nTokens > p.maxSeq ||
                           flow_lds_bytes(p.dim, p.ffn, p.headDim, p.geo.gqa, true) > ((size_t)160 << 10)))
@@ -2103,18 +2112,18 @@ __global__ void flow_reset_kernel(uint4* x, size_t n4, uint4* x2, size_t m4, con
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) x[i] = sent;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m4; i += (size_t)gridDim.x * blockDim.x) x2[i] = sent;
 }
-hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int nLayers, int l0, int l1, bool pairs, const float* hiddenIn, float* hidden, int dim, hipStream_t s) {
+hipError_t launch_flow_reset(float* xchg, const FlowGeometry& g, int l0, int l1, float* pairs, const float* hiddenIn, float* hidden, int dim, hipStream_t s) {
     if (l1 <= l0) return hipSuccess;
     const size_t n4 = (size_t)(l1 - l0) * g.stride / 4, m4 = pairs ? (size_t)(l1 - l0) * g.pairs / 4 : 0;
     size_t blocks = (n4 + WG - 1) / WG;
     if (blocks > 1024) blocks = 1024;
     hipLaunchKernelGGL(flow_reset_kernel, dim3((unsigned)blocks), dim3(WG), 0, s, reinterpret_cast<uint4*>(xchg + (size_t)l0 * g.stride), n4,
-                       reinterpret_cast<uint4*>(xchg + flow_block_floats(g, nLayers) + (size_t)l0 * g.pairs), m4, hiddenIn, hidden, dim);
+                       reinterpret_cast<uint4*>(m4 ? pairs + (size_t)l0 * g.pairs : nullptr), m4, hiddenIn, hidden, dim);
     return hipGetLastError();
 }
 
 size_t flow_xchg_floats(const FlowGeometry& g, int nLayers, int grid) {
-    return 2 * flow_half_floats(g, nLayers) + (size_t)2 * grid * FLOW_AMAX_STRIDE;
+    return (size_t)2 * nLayers * (g.stride + g.pairs) + (size_t)2 * grid * FLOW_AMAX_STRIDE;
 }
 hipError_t launch_flow_reset_all(float* xchg, const FlowGeometry& g, int nLayers, int grid, hipStream_t s) {
     const size_t n4 = flow_xchg_floats(g, nLayers, grid) / 4;

@@ -821,7 +821,7 @@ int HIPFusedInference::flowComputeWgs(int cus) const {
         const FlowGeometry g = flow_geometry(dim, kvDim, ffnDim, nHeads, nKVHeads, headDim, maxSeq, nC, cus);
         // (the same limits as launch_flow_layers checks: a shape it would refuse runs the fused launches instead)
         if (flow_min_grid(nHeads, nKVHeads, g) <= nC && flow_context_fits(maxSeq, g) && flow_grid_fits(ffnDim, nHeads, g, nC) &&
-            flow_half_floats(g, nLayers) * 4 < (1ull << 31)) return nC;
+            (size_t)nLayers * g.stride * 4 < (1ull << 31)) return nC;
     }
     return 0;
 }
@@ -1037,7 +1037,7 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
     }
     p.trace = flowTrace;
     if (nTokens > 0) { p.nTokens = nTokens; p.tail = dFlowTail; }
-    if (resetFirst) HIPCHK(launch_flow_reset(flowXchg, flowGeo, nLayers, l0, l1, pairs, hiddenIn, hidden[hiddenIdx], dim, stream));
+    if (resetFirst) HIPCHK(launch_flow_reset(flowXchg, flowGeo, l0, l1, pairs ? flow_pairs_area(flowXchg, flowGeo, nLayers, flowGrid) : nullptr, hiddenIn, hidden[hiddenIdx], dim, stream));
     if (mark(1)) return MG_E_HIP;
     if (capturing) { HIPCHK(launch_flow_layers(p, flowGrid, stream)); return MG_OK; }      // (the replay takes the turn)
     std::lock_guard<std::mutex> lk(flowTurnMutex());
@@ -1216,7 +1216,7 @@ int HIPFusedInference::enqueueFinal(bool withArgmax, int* parts, const float* ro
         // inside the captured token: the lm_head launch also leaves the exchange area of the persistent
         // layer launch in its "nothing written yet" state for the next token (one launch saved)
         p.xreset = reinterpret_cast<unsigned*>(flowXchg);
-        p.xresetWords = (unsigned)flow_block_floats(flowGeo, nLayers);
+        p.xresetWords = (unsigned)((size_t)nLayers * flowGeo.stride);
     }
     MvConfig c{0, 0, 0};
     if (mark(6)) return MG_E_HIP;
@@ -1420,7 +1420,7 @@ int HIPFusedInference::enqueueToken(bool withHead) {
     // no lm_head launch to leave the exchange area reset for the next launch: a captured prompt step does it itself,
     // and so does any prompt step where whole tokens run in the launch (they expect to find it so)
     if (flow && (fuseEmbed || flowTailEligible())) {
-        HIPCHK(launch_flow_reset(flowXchg, flowGeo, nLayers, 0, nLayers, !capturing, nullptr, nullptr, 0, stream));
+        HIPCHK(launch_flow_reset(flowXchg, flowGeo, 0, nLayers, capturing ? nullptr : flow_pairs_area(flowXchg, flowGeo, nLayers, flowGrid), nullptr, nullptr, 0, stream));
         if (!capturing) flowClean = clean;          // (the layers' launch wrote the first half only)
     }
     return MG_OK;

@@ -335,7 +335,7 @@ def test_many_splits_of_a_known_shape(hip, fmt, maxSeq, positions, first):
 
 
 def test_pairs_are_reset_by_the_launches_that_write_them(hip):
-    """0.5B shape: the (maximum, sum) pairs that launches of many KV splits merge by lie behind the layers' blocks, so that other launches
+    """0.5B shape: the (maximum, sum) pairs that launches of many KV splits merge by lie outside the layers' blocks, so that other launches
     have none to reset (a block ends with the splits' sums), and come out as first written whatever ran in between: shorter
     positions, the same again, layer ranges, runs of tokens across the line -- against the variants without pairs, in the same order
     (bar as above)."""
