@@ -62,7 +62,7 @@ struct FlowGeometry {
 // grid: computing workgroups, of cus the launch has.
 FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim, int maxSeq, int grid, int cus);
 // Attention workgroups, one a query head and KV split, up to which a launch that can group query heads does not.
-int flow_plain_most(int nC, int cus, int nHeads, int dim);
+int flow_plain_most(int nC, int cus, int nHeads, int nKVHeads, int dim);
 bool flow_context_fits(int maxSeq, const FlowGeometry& g);
 
 constexpr size_t FLOW_ERR_BYTES = 4096;

@@ -1951,15 +1951,24 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 }
 
 // Grouped attention costs a hand-over more, but shares a K / V tile among query heads, leaves workgroups idle that read ahead, and its
-// consumers stage one vector instead of merging every split's.  So it starts before the launch is full.  Vectors past 2,048 elements,
-// several pieces a thread: when the splits no longer fit a round of the merge (PB; us a token without / with it, eight layers
-// of 8B at three splits Q8 425 / 430, Q4_0 406 / 419, fp16 rows 435 / 424, at four 445 / 436, 420 / 421, 452 / 428, at five 444 / 437, 424 / 421,
-// 452 / 428, at eight 463 / 446, 451 / 423, 479 / 434).  Shorter ones: past three quarters of the launch (1.1B, six splits 466 / 478, Q4_0
-// 473 / 480, seven 484 / 479 and 491 / 481, eight 490 / 484 and 496 / 482; eight layers of 1,536, 24 heads, Q8 at eight 189 / 186, Q4_0 184 /
-// 185).  With dedicated prefetchers, when it is full (0.5B, twelve splits 370 / 397, sixteen 394 / 414).
-int flow_plain_most(int nC, int cus, int nHeads, int dim) {
+// consumers stage one vector instead of merging every split's.  So it starts before the launch is full.
+// Vectors past 2,048 elements, several pieces a thread: when the splits no longer fit a round of the merge (PB; us a token without / with
+// it, eight layers of 8B at three splits Q8 425 / 430, Q4_0 406 / 419, fp16 rows 435 / 424, at four 445 / 436, 420 / 421, 452 / 428, at
+// five 444 / 437, 424 / 421, 452 / 428, at eight 463 / 446, 451 / 423, 479 / 434; 24 heads on 8 at four 155.3 / 154.8, 150.5 / 151.2, 151.9 / 152.3).
+// Query heads in pairs share least: there when the splits do not fit a second round of five, or it would merge more than 15K elements, or
+// the launch is five eighths full.  Four layers, 20 heads of 128 on 10, Q8, Q4_0 and fp16 rows at four splits 143.1 / 147.2, 152.4 / 152.4,
+// 141.2 / 144.8, five 144.9 / 147.7, 154.4 / 152.9, 142.7 / 144.9, six 146.1 / 148.4, 156.0 / 153.7, 143.3 / 145.0, seven 152.1 / 148.9, 162.2 /
+// 153.7, 149.1 / 145.5; 24 on 12 at five 159.9 / 159.1, 154.7 / 157.2, 154.7 / 155.3, six 162.7 / 159.8, 157.5 / 157.6, 156.3 / 155.7; 32 on 16 at four
+// 225.9 / 225.3, 208.9 / 207.0, 219.1 / 221.1, five 231.0 / 226.9, 208.5 / 206.9, 226.1 / 221.4; 40 of 64 on 20, 160 workgroups 142.8 / 145.8, 147.7 /
+// 149.4, 142.7 / 144.7, 200 149.2 / 145.2, 149.1 / 149.9, 149.7 / 143.6; 44 on 22, 176 152.7 / 148.3, 150.9 / 149.7, 152.7 / 148.2.
+// Shorter ones: past three quarters of the launch (1.1B, six splits 466 / 478, Q4_0 473 / 480, seven 484 / 479 and 491 / 481, eight 490 / 484 and
+// 496 / 482; eight layers of 1,536, 24 heads, Q8 at eight 189 / 186, Q4_0 184 / 185).  With dedicated prefetchers, when it is full (0.5B,
+// twelve splits 370 / 397, sixteen 394 / 414).
+int flow_plain_most(int nC, int cus, int nHeads, int nKVHeads, int dim) {
     if (nC != cus) return nC;
-    return dim > 2048 ? std::min(nC, PB * nHeads) : nC * 3 / 4;
+    if (dim <= 2048) return nC * 3 / 4;
+    const int splits = nHeads == 2 * nKVHeads ? std::min((15 << 10) / dim, 5) : 0;
+    return std::min(nC, std::max(PB * nHeads, std::min(splits * nHeads, nC * 5 / 8)));
 }
 
 FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads, int headDim, int maxSeq, int grid, int cus) {
@@ -1969,7 +1978,7 @@ FlowGeometry flow_geometry(int dim, int kvDim, int ffn, int nHeads, int nKVHeads
     // query heads in turn on one load of the K / V rows -- which takes more LDS: only a context that cannot do without insists on it.
     const int want = (maxSeq + FLOW_TILE - 1) / FLOW_TILE;
     if (nHeads > 0 && nKVHeads > 0 && nHeads / nKVHeads > 1 && nHeads / nKVHeads <= FLOW_GQA_MAX)
-        g.gqa = want > grid / nHeads || ((long long)want * nHeads > flow_plain_most(grid, cus, nHeads, dim) && nHeads <= grid &&
+        g.gqa = want > grid / nHeads || ((long long)want * nHeads > flow_plain_most(grid, cus, nHeads, nKVHeads, dim) && nHeads <= grid &&
                                          flow_lds_bytes(dim, ffn, headDim, 1, true) <= ((size_t)160 << 10)) ? 1 : 0;
     const int unit = g.gqa ? nKVHeads : nHeads;
     g.smax = want;

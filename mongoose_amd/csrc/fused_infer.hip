@@ -1015,7 +1015,7 @@ int HIPFusedInference::enqueueLayersFlow(int l0, int l1, const StepState* st, in
         long long posMax = -1;
         if (!st) posMax = posImm;
         else if (statePosHost >= 0) posMax = (long long)statePosHost + (nTokens > 0 ? nTokens - 1 : 0);
-        const int plainMost = flow_plain_most(flowCompute, flowGrid, nHeads, dim);
+        const int plainMost = flow_plain_most(flowCompute, flowGrid, nHeads, nKVHeads, dim);
         const bool grouped = posMax < 0 ? (long long)nHeads * ((maxSeq + FLOW_TILE - 1) / FLOW_TILE) > flowCompute
                                         : (long long)nHeads * (posMax / FLOW_TILE + 1) > plainMost;
         p.gqaCode = grouped ? plainMost : 0;

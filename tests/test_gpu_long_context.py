@@ -124,6 +124,35 @@ def test_grouped_attention_before_the_launch_is_full(hip, shape, maxSeq, check):
     m.close()
 
 
+@pytest.mark.parametrize("heads,kv,hd,fmt,kv_f16,first", [
+    (32, 8, 128, "q8", False, 384), (18, 6, 128, "q4_0", True, 384), (20, 10, 128, "q8", False, 640), (24, 12, 128, "q4_0", False, 640),
+    (28, 14, 128, "q8", True, 512), (32, 16, 128, "q4_0", False, 384), (40, 20, 64, "q8", False, 512), (44, 22, 64, "q4_0", True, 384),
+    (32, 4, 64, "q8", False, 768)])
+def test_where_grouped_attention_starts(hip, heads, kv, hd, fmt, kv_f16, first):
+    """The variant with grouped attention runs from the first position past the rule's line and not before (256 CUs, launches without
+    dedicated prefetchers); tokens around the line against the separate launches (bar: the logit bar of every mode here)."""
+    dim = heads * hd
+    s = configs.TOY._replace(name="line", nLayers=1, dim=dim, nHeads=heads, nKVHeads=kv, headDim=hd, ffnDim=-(-(32 << 20) // (3 * dim) // 64) * 64, vocab=300)
+    m = H.Model(s, seed=heads, maxSeq=first + 3, eng=hip, oracle=False, fmt=fmt, kv_f16=kv_f16)
+    toks = m.prompt(first + 2)
+    got = {}
+    for mode in (1, 3):
+        assert m.hip.SetExecMode(mode) == 0 and m.hip.ResetKV() == 0
+        assert m.hip.Prefill(toks[:first - 2], 0)[0] == 0, E.last_error()
+        got[mode] = np.empty((4, s.vocab), np.float32)
+        for i, pos in enumerate(range(first - 2, first + 2)):
+            names = H.launched(lambda: m.hip.DecodeToken(int(toks[pos]), pos, got[mode][i]))
+            names = [n for n in names if "flow_layers_kernel<" in n]
+            if mode == 1:
+                assert not names
+                continue
+            assert len(names) == 1, names
+            args = names[0].split("<")[1].split(">")[0].replace(" ", "").split(",")
+            assert (args[3] == "true") == (pos >= first), (pos, names)
+    assert H.rel_err(got[3], got[1]) < LOGIT_TOL
+    m.close()
+
+
 @pytest.mark.parametrize("name,shape,maxSeq", [
     ("hd64", configs.Shape("g7-hd64-modes", 1, 896, 14, 2, 64, 256, 512, 1e-6, 1e6, True, True, "q8"), 8300),
     ("hd128", configs.Shape("g4-hd128-modes", 1, 1024, 8, 2, 128, 256, 512, 1e-5, 5e5, False, True, "q8"), 8300),
