@@ -60,8 +60,16 @@ struct FewNext { FewMode mode; const void* W0; const void* W1; const void* W2; i
 // 24); a matrix that does not fit is taken in part, its first tiles.  Readers are the workgroups up to 256, but 96 at least -- they
 // then share CUs with the attention's, which wait more than they load (0.5B, 301 rows, 266 workgroups of attention, with 0 / 32 / 64
 // / 96 / 128 readers 1,908 / 1,896 / 1,849 / 1,814 / 1,799, 200 rows 1,388 / 1,388 / 1,386 / 1,410 / 1,402) -- and no more than
-// have 64 KB each.
-constexpr long long FEW_AHEAD_EACH = 200 << 10, FEW_AHEAD_MOST = 20 << 20, FEW_AHEAD_LEAST = 64 << 10;
+// have 64 KB each.  There a layer that does not fit whole is read up to 4 MB past its first matrix: the attention waits for its CUs, and what many
+// rows are multiplied by is wanted too slowly for a cold start to matter past the first tiles.  Nothing read / 8 / 12 / 19.2 MB, us a
+// call, Q8: eight 1.1B layers (44 MB), 100 rows 549 / 545 / 549 / 562, 128 573 / 566 / 571 / 583, 256 788 / 786 / 796 / 806; six of 2048 x 8192, heads of 64, 100 rows
+// 465 / 460 / 463 / 475; eight of 1536 x 6144 (38) 521 / 514 / 521 / 532; four of 3072 x 8192, heads of 128 (101; Wo alone 9.4) 441 / 443 / 437 / 438; 1.1B Q4_0 (22) 975 /
+// 974 / 982 / 987.  Layers that fit: 0.5B, 100 behind 300, 1,137 / 1,128 / 1,129 / 1,092, 1536 x 6144 Q4_0 (17) 256 rows 1,513 / 1,486 / 1,485 / 1,463.
+constexpr long long FEW_AHEAD_EACH = 200 << 10, FEW_AHEAD_MOST = 20 << 20, FEW_AHEAD_LEAST = 64 << 10, FEW_AHEAD_SHARED = 4 << 20;
+constexpr long long few_ahead_bytes(const FewNext& m) {
+    const long long rows = m.mode == FEW_QKV ? m.N + 2LL * m.N1 : (m.mode == FEW_SWIGLU ? 2LL : 1LL) * m.N;
+    return m.q4 ? rows * m.K / 16 * 9 : rows * m.K;
+}
 // Planes of Wo, gate | up and down, one a matrix or, in Q4_0, two, and of Q8 q|k|v: one of v, of q and k the halves of their heads.
 constexpr int FEW_REGIONS = 13;
 struct FewAhead { FewRegion r[FEW_REGIONS]; int n, first, readers; };      // first: the launch's first workgroup that reads ahead
@@ -71,7 +79,9 @@ inline FewAhead few_plan(unsigned grid, const FewNext* next, int nNext, int head
     FewAhead a{};
     a.first = INT_MAX;
     const unsigned own = (grid + 7) / 8 * 8, room = own + 96 > 256 ? 96 : 256 - own;
-    long long left = std::min(room * FEW_AHEAD_EACH, FEW_AHEAD_MOST), bytes = 0;
+    long long left = std::min(room * FEW_AHEAD_EACH, FEW_AHEAD_MOST), bytes = 0, all = 0;
+    for (int i = 0; i < nNext; i++) all += next[i].mode == FEW_QKV && next[i].q4 ? 0 : few_ahead_bytes(next[i]);
+    if (own + 96 > 256 && all > left) left = std::min(left, few_ahead_bytes(next[0]) + FEW_AHEAD_SHARED);
     // one matrix, or two read tile by tile (W1; per: the halves of W0's heads)
     auto take = [&](const void* W0, const void* W1, int N, int K, int q4, int rows, int tiles, int tile0, int per) {
         const unsigned row = q4 ? K / 2 : K, run = rows * row;

@@ -210,3 +210,36 @@ int main() {
 }
 """ % (q4, dim, kvDim, ffn, head_dim, grid))
     assert out == "ok\n", out
+
+
+@pytest.mark.parametrize("q4", [0, 1])
+@pytest.mark.parametrize("dim,kvDim,ffn,head_dim", [(2048, 256, 5632, 64), (3072, 1024, 8192, 128), (4096, 1024, 14336, 128), (1280, 320, 3584, 64)])
+def test_what_is_read_ahead_beside_an_attention(tmp_path, q4, dim, kvDim, ffn, head_dim):
+    """Where the reading workgroups share CUs with the attention's (more than 160 of those), a layer that does not fit whole is read up to 4 MB
+    past Wo; one that fits, and any with CUs to spare, up to the limits."""
+    out = _run(tmp_path, r"""
+#include "few_rules.h"
+#include <cstdio>
+using namespace mg;
+int main() {
+    const int q4 = %d, dim = %d, kvDim = %d, ffn = %d, hd = %d;
+    const void* w = reinterpret_cast<const void*>(16ull << 30);         // (an address for the plan, not for reading)
+    const FewNext next[4] = {{FEW_RESID, w, nullptr, nullptr, dim, 0, dim, q4}, {FEW_SWIGLU, w, w, nullptr, ffn, 0, dim, q4},
+                             {FEW_RESID, w, nullptr, nullptr, dim, 0, ffn, q4}, {FEW_QKV, w, w, w, dim, kvDim, dim, q4}};
+    const double wb = q4 ? 9.0 / 16 : 1.0, wo = wb * dim * dim, layer = wb * (wo / wb + 3.0 * dim * ffn + (q4 ? 0 : (double)dim * (dim + 2 * kvDim)));
+    for (int n = 1; n <= 4; n++)
+        for (int grid = 8; grid <= 512; grid += 8) {
+            const FewAhead a = few_plan(grid, next, n, hd, [&](const FewNext& m) { return m.mode == FEW_SWIGLU ? 64 : 16; });
+            double read = 0, all = 0;
+            for (int i = 0; i < a.n; i++) read += (double)a.r[i].run * a.r[i].tiles;
+            for (int i = 0; i < n; i++) all += i == 1 ? wb * 2.0 * ffn * dim : i == 2 ? wb * dim * ffn : i == 0 ? wo : layer - wo - wb * 3.0 * dim * ffn;
+            const double most = (double)(grid <= 160 ? 256 - grid : 96) * FEW_AHEAD_EACH, cap = most < FEW_AHEAD_MOST ? most : FEW_AHEAD_MOST;
+            const double want = all <= cap ? all : grid > 160 && wo + (4 << 20) < cap ? wo + (4 << 20) : cap;
+            // (a matrix in part goes by eight tiles an XCD: of up to 64 rows of two matrices)
+            const double least = want - wb * 8 * 128 * dim;
+            if (read > want * (1 + 1e-9) || (all <= cap ? read < want * (1 - 1e-9) : read < least)) return std::printf("%%d launches behind %%d: %%.0f of %%.0f bytes\n", n, grid, read, want), 0;
+        }
+    std::puts("ok");
+}
+""" % (q4, dim, kvDim, ffn, head_dim))
+    assert out == "ok\n", out
