@@ -169,8 +169,8 @@ __device__ __forceinline__ float dot_q4_half(int2 w, float d, const float4 (&av)
 }
 // The same without the activations' sum, which takes as many additions as half of the products: a nibble in the upper half of a
 // byte, its highest bit flipped, is (nib - 8) * 16 as a signed byte, which converts in one instruction.  For the persistent
-// launch (flow.hip), whose phases are bound by their instructions (8B shape in Q4_0, six layers 340.5 -> 330.5 us a token, at 900 positions
-// 391 -> 383; 1.1B, eight layers 151.2 -> 150.2, at 600 169.9 -> 168.0); the separate launches wait for their loads instead and
+// launch (flow.hip), whose phases are bound by their instructions (8B shape in Q4_0, six layers 338.2 -> 328.4 us a token, at 900 positions
+// 389.8 -> 379.3; 1.1B, eight layers 146.9 -> 145.9, at 600 169.1 -> 167.4); the separate launches wait for their loads instead and
 // are no faster by it (5632 x 2048 5.3 -> 5.7 us, 32000 x 2048 14.5 -> 14.9, 4096 x 14336 15.5 -> 14.9).  Its error against
 // a shadow of the same roundings is half that of dot_q4_half (two layers of three shapes: 7e-7 -> 3.5e-7), whose sum has to cancel.
 __device__ __forceinline__ int nib_bytes(unsigned q) {

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(FR_WG) void few_rows_kernel(FewParams p) {
             }
         }
         // (every load is unconditional: one under a branch, even a branch that is always taken, makes the compiler's waits
-        // drain the ring; rows past T are whatever the buffer holds, and their results are dropped)
+        // drain the ring; rows past T are the last one's again, and their results are dropped)
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -463,8 +463,9 @@ static hipError_t launch_few_t(const FewParams& p, hipStream_t s) {
 // two workgroups (Q4_0 0.5B shape, down at 400 rows: 252 workgroups of 3 x 2, 288 launched, 11 us longer than 196 of 4 x 2).  Short rows
 // go through two workgroups a CU at once; tiles of more than four blocks take too many registers for that (1.5), which matters where
 // there are two, and 128 weight rows at any number.  The constants are a fit to every tile of gate | up, Wo and down at 16 to 512
-// rows of the benchmark shapes, both formats: what it picks is within 2 % of a prefill of the best one at all of them (without matrix
-// instructions, made-up tiles and the line at one workgroup a CU 10 %: 0.5B shape, 301 rows 1,808 -> 1,718 us, Q4_0 400 rows 2,642 -> 2,310).
+// rows of the benchmark shapes, both formats: what it picks is within 2 % of a prefill of the best one at all but one of 160 points (8B at
+// 77 rows 3 %; without matrix instructions, made-up tiles and the line at one workgroup a CU 10 %: 0.5B shape, 301 rows 1,808 -> 1,718 us, Q4_0
+// 400 rows 2,642 -> 2,330).
 struct FewTile { int mt, nb; };
 // With three terms an activation row is half as many bytes again, and a tile has at most FEW_MT3 row blocks.
 static double few_tile_cost(int rowsN, int T, int K, int nbFirst, int nbLast, int q4, int terms, FewTile& best) {
@@ -681,8 +682,8 @@ static hipError_t launch_few_swiglu(FewParams& p, hipStream_t s) {
 // 0: gate | up of T rows is few_rows_kernel's; else the activation rows of a workgroup's tile in few_swiglu_kernel.  The least of three
 // models in microseconds: few_tile's, and for tiles of 64 and 128 rows a start and end and so much a chunk of 64 k, times the
 // workgroups of the busiest CU (of 64 rows two run on it together and hide each other's waits).  Fitted to the launches of five
-// shapes at 16 to 1,000 rows; what it picks is within 6 % of the best at all but three of 123 points (15 %), and none of it is slower than few_rows_kernel.  Microseconds a launch, old / 64 /
-// 128 rows, Q8 and Q4_0: 0.5B shape 77 rows 12.6 / 14.8 / 20.3 and 15.0 / 17.0 / 24.0, 301 31.6 / 20.7 / 21.5 and 36.0 / 24.6 / 24.8, 512 47.0 /
+// shapes at 16 to 1,000 rows; what it picks is within 6 % of the best at all but three of 114 points (9, 12 and 15 %), and none of it is slower than
+// few_rows_kernel.  Microseconds a launch, old / 64 / 128 rows, Q8 and Q4_0: 0.5B shape 77 rows 12.6 / 14.8 / 20.3 and 15.0 / 17.0 / 24.0, 301 31.6 / 20.7 / 21.5 and 36.0 / 24.6 / 24.8, 512 47.0 /
 // 29.1 / 37.3 and 51.8 / 33.7 / 43.3; 1.1B 64 rows 19.1 / 23.0 / 34.2 and 27.7 / 27.6 / 42.8, 200 41.1 / 34.9 / 35.0 and 58.2 / 43.4 / 42.6; 8B
 // 16 rows 32.4 / 46.1 / 71.0, 37 62.8 / 42.6 / 63.0, 128 109.5 / 69.8 / 67.6, Q4_0 144.1 / 87.0 / 83.0.
 static int few_swiglu_rows(int N, int T, int K, int q4, int terms) {
