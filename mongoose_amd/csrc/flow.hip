@@ -1955,6 +1955,9 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 // Vectors past 2,048 elements, several pieces a thread: when the splits no longer fit a round of the merge (PB; us a token without / with
 // it, eight layers of 8B at three splits Q8 425 / 430, Q4_0 406 / 419, fp16 rows 435 / 424, at four 445 / 436, 420 / 421, 452 / 428, at
 // five 444 / 437, 424 / 421, 452 / 428, at eight 463 / 446, 451 / 423, 479 / 434; 24 heads on 8 at four 155.3 / 154.8, 150.5 / 151.2, 151.9 / 152.3).
+// A second round of up to 11K elements costs less than the hand-over: vectors up to 2,816 at four splits, four layers, Q8 and fp16 rows, 40 heads of 64
+// on 8 143.7 / 144.9 and 142.9 / 143.8, 36 on 6 129.5 / 130.7 and 129.1 / 131.1, 20 of 128 on 5 149.0 / 149.7 and 146.8 / 148.5, 18 on 6 135.3 /
+// 135.2 and 134.0 / 134.2; at five 149.4 / 145.0, 133.3 / 130.7, 151.9 / 149.9, 137.0 / 135.6; 48 of 64 on 8 (3,072) at four 158.8 / 157.5.
 // Query heads in pairs share least: there when the splits do not fit a second round of five, or it would merge more than 15K elements, or
 // the launch is five eighths full.  Four layers, 20 heads of 128 on 10, Q8, Q4_0 and fp16 rows at four splits 143.1 / 147.2, 152.4 / 152.4,
 // 141.2 / 144.8, five 144.9 / 147.7, 154.4 / 152.9, 142.7 / 144.9, six 146.1 / 148.4, 156.0 / 153.7, 143.3 / 145.0, seven 152.1 / 148.9, 162.2 /
@@ -1967,7 +1970,7 @@ __global__ __launch_bounds__(FWG) void flow_layers_kernel(FlowParams p) {
 int flow_plain_most(int nC, int cus, int nHeads, int nKVHeads, int dim) {
     if (nC != cus) return nC;
     if (dim <= 2048) return nC * 3 / 4;
-    const int splits = nHeads == 2 * nKVHeads ? std::min((15 << 10) / dim, 5) : 0;
+    const int splits = nHeads == 2 * nKVHeads ? std::min((15 << 10) / dim, 5) : std::min((11 << 10) / dim, 4);
     return std::min(nC, std::max(PB * nHeads, std::min(splits * nHeads, nC * 5 / 8)));
 }
 

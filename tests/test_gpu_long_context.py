@@ -125,7 +125,7 @@ def test_grouped_attention_before_the_launch_is_full(hip, shape, maxSeq, check):
 
 
 @pytest.mark.parametrize("heads,kv,hd,fmt,kv_f16,first", [
-    (32, 8, 128, "q8", False, 384), (18, 6, 128, "q4_0", True, 384), (20, 10, 128, "q8", False, 640), (24, 12, 128, "q4_0", False, 640),
+    (32, 8, 128, "q8", False, 384), (18, 6, 128, "q4_0", True, 512), (40, 8, 64, "q8", False, 512), (20, 5, 128, "q8", True, 512), (22, 11, 128, "q4_0", False, 640), (48, 8, 64, "q8", False, 384), (20, 10, 128, "q8", False, 640), (24, 12, 128, "q4_0", False, 640),
     (28, 14, 128, "q8", True, 512), (32, 16, 128, "q4_0", False, 384), (40, 20, 64, "q8", False, 512), (44, 22, 64, "q4_0", True, 384),
     (32, 4, 64, "q8", False, 768)])
 def test_where_grouped_attention_starts(hip, heads, kv, hd, fmt, kv_f16, first):
