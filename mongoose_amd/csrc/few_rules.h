@@ -63,7 +63,7 @@ struct FewNext { FewMode mode; const void* W0; const void* W1; const void* W2; i
 // have 64 KB each.  There a layer that does not fit whole is read up to 4 MB past its first matrix: the attention waits for its CUs, and what many
 // rows are multiplied by is wanted too slowly for a cold start to matter past the first tiles.  Nothing read / 8 / 12 / 19.2 MB, us a
 // call, Q8: eight 1.1B layers (44 MB), 100 rows 549 / 545 / 549 / 562, 128 573 / 566 / 571 / 583, 256 788 / 786 / 796 / 806; six of 2048 x 8192, heads of 64, 100 rows
-// 465 / 460 / 463 / 475; eight of 1536 x 6144 (38) 521 / 514 / 521 / 532; four of 3072 x 8192, heads of 128 (101; Wo alone 9.4) 441 / 443 / 437 / 438; 1.1B Q4_0 (22) 975 /
+// 465 / 460 / 463 / 475; eight of 1536 x 6144 (34) 521 / 514 / 521 / 532; four of 3072 x 8192, heads of 128 (101; Wo alone 9.4) 441 / 443 / 437 / 438; 1.1B Q4_0 (22) 975 /
 // 974 / 982 / 987.  Layers that fit: 0.5B, 100 behind 300, 1,137 / 1,128 / 1,129 / 1,092, 1536 x 6144 Q4_0 (17) 256 rows 1,513 / 1,486 / 1,485 / 1,463.
 constexpr long long FEW_AHEAD_EACH = 200 << 10, FEW_AHEAD_MOST = 20 << 20, FEW_AHEAD_LEAST = 64 << 10, FEW_AHEAD_SHARED = 4 << 20;
 constexpr long long few_ahead_bytes(const FewNext& m) {
